@@ -1,0 +1,42 @@
+"""Edges of the kernels' tiles and of the dispatch rules: remainders, smallest and largest sizes, each against
+the oracle or an exact integer / fp32 reference (integers and packed words: equality, no tolerance)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def G():
+    import gpu_util
+    return gpu_util
+
+
+# Packers: one wave owns 8 words of a small tensor and 64 of a large one (from 131072 words); rows with padding
+# (C < cpad) and without; one-word rows, where the two halves of a wave work on different rows.
+@pytest.mark.parametrize("rows,C,cpad", [(1, 32, 32), (7, 1, 32), (9, 31, 32), (33, 33, 64), (5, 96, 96), (131071, 32, 32),
+                                         (131075, 30, 32), (26216, 160, 160), (26219, 129, 160), (65537, 64, 64)])
+@pytest.mark.parametrize("bits,lo,hi", [(2, -10.0, 10.0), (5, -0.3, 0.7), (1, 0.0, 3.0), (3, -1e-20, 3e-20)])
+def test_float_packer_edges(G, rows, C, cpad, bits, lo, hi):
+    """Every operation of the quantizer is one fp32 rounding, so numpy's fp32 arithmetic is the exact reference; the
+    last range is below 2^-60 and takes the kernel's dividing form."""
+    rng = np.random.default_rng(8100 + rows + bits)
+    lo, hi = np.float32(lo), np.float32(hi)
+    span = np.float32(hi - lo)
+    x = rng.uniform(float(lo) - 0.2 * float(span), float(hi) + 0.2 * float(span), size=(rows, C)).astype(np.float32)
+    flat = x.reshape(-1)
+    ties = (lo + span * (np.arange(min(flat.size, 64)) + 0.5).astype(np.float32) / np.float32(2 ** bits)).astype(np.float32)
+    flat[:ties.size] = ties
+    if flat.size > 70:
+        flat[64:70] = [np.nan, np.inf, -np.inf, lo, hi, -0.0]
+    d = torch.from_numpy(x).cuda()
+    planes = G.dev_empty_i32(bits * rows * cpad // 32, fill=-7)
+    G.A.check(G.A.lib().apnn_quantize_pack(G.ptr(d), G.ptr(planes), rows, C, cpad, bits, float(lo), float(hi), None), "quantize_pack")
+    c = np.where(np.isnan(x), lo, np.clip(x, lo, hi)).astype(np.float32)
+    q = (((c - lo) * np.float32(2 ** bits)) / span).astype(np.float32)
+    codes = np.minimum(np.rint(q), 2 ** bits - 1).astype(np.uint32)
+    expect = O.pack_bits(codes, rows, C, cpad, bits)
+    assert np.array_equal(G.to_host(planes, np.uint32).reshape(expect.shape), expect)
