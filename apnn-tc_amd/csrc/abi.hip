@@ -375,7 +375,7 @@ int from_hip(hipError_t e) { return e == hipErrorNotSupported ? APNN_EUNSUPPORTE
 // compute unit still gets a work-group; when even 64x64 tiles leave most of the chip idle and the
 // reduction is long, the 32-row tiles whose four waves split K.
 int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, int planes = 3, int planesW = 1) {
-  const bool wide = planes > 5 || planes == 2;  // the reduced tile set (see mfma_tile_enabled)
+  const bool wide = planes > 5 || planes == 2;
   int cus = device_cus();
   if (cus <= 0) cus = 256;
   auto ntiles = [&](int t) {
@@ -386,11 +386,7 @@ int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, i
   auto fill = [&](int t) {
     return (double)rowsA * rowsB / ((double)ntiles(t) * apnn::kMfmaTileA[t] * apnn::kMfmaTileB[t]);
   };
-  if (wide) {  // more than five planes in all, or w1a1: 128x128, 64x64 and the 32x32 split-K tile are built
-    if (conv && vw != 4) return 2;
-    if (KW >= 32 && ntiles(4) <= 256) return 4;
-    return (ntiles(1) >= cus && fill(1) >= 0.8) ? 1 : 2;
-  }
+  if (wide && conv && vw != 4) return 2;  // the only tile built (see mfma_tile_enabled)
   if (i8 && conv) {  // int8 core, convolution: 128x256, 128x128, 128x64, 64x64, 32x32 split-K (128-bit loads)
     if (vw != 4) return 2;
     if (KW >= 32 && ntiles(4) <= 256) return 4;
@@ -487,6 +483,11 @@ bool auto_prefers_mfma_gemm(const KParams &p) {
   return outputs > 256LL * 256 || (outputs == 256LL * 256 && p.KW > 32);
 }
 
+// Precisions without a popcount kernel of their own (w1a1 and everything beyond five planes) reach the VALU only
+// through the any-precision kernel, which takes 30-100 us for products the matrix cores finish in 3 us (w1a1 at
+// 111x67x1792 105 us, w2a8 at 52x72x128 31 us): they take the matrix cores at every size.
+bool has_popcount_kernel(int wb, int xb) { return (wb == 1 && xb >= 2 && xb <= 4) || (wb == 2 && xb == 2); }
+
 valu_fn valu_gemm_fn(int wb, int xb) {
   if (wb == 1 && xb == 2) return apnn::valu_gemm_1_2_x;
   if (wb == 1 && xb == 3) return apnn::valu_gemm_1_3_x;
@@ -573,7 +574,7 @@ int run_gemm(const apnn_gemm_desc *d, hipStream_t stream, apnn_plan *plan = null
   // operand planes of 4 GiB or more: the matrix-core kernels address rows with 32-bit offsets and refuse
   if ((path == APNN_PATH_MFMA || path == APNN_PATH_MFMA_I8) && !p.addr32) return APNN_EUNSUPPORTED;
   if (path == APNN_PATH_MFMA || path == APNN_PATH_MFMA_I8 ||
-      (path == APNN_PATH_AUTO && p.addr32 && auto_prefers_mfma_gemm(p))) {
+      (path == APNN_PATH_AUTO && p.addr32 && (auto_prefers_mfma_gemm(p) || !has_popcount_kernel(d->wb, d->xb)))) {
     // AUTO: FP4 operands while their fp32 accumulation is exact, the int8 core (int32 accumulate) beyond
     const bool i8 = path == APNN_PATH_MFMA_I8 || (path == APNN_PATH_AUTO && !f4ok);
     valu_fn fn = mfma_gemm_fn(d->wb, d->xb, i8);
@@ -737,7 +738,7 @@ int run_conv(const apnn_conv_desc *d, hipStream_t stream, apnn_plan *plan = null
   }
   // operand planes of 4 GiB or more, or a filter beyond the kernels' 24-bit index arithmetic: refused
   if ((path == APNN_PATH_MFMA || path == APNN_PATH_MFMA_I8) && !p.addr32) return APNN_EUNSUPPORTED;
-  if (path == APNN_PATH_MFMA || path == APNN_PATH_MFMA_I8 || (path == APNN_PATH_AUTO && p.addr32 && auto_prefers_mfma(p))) {
+  if (path == APNN_PATH_MFMA || path == APNN_PATH_MFMA_I8 || (path == APNN_PATH_AUTO && p.addr32 && (auto_prefers_mfma(p) || !has_popcount_kernel(d->wb, d->xb)))) {
     const bool i8 = path == APNN_PATH_MFMA_I8 || (path == APNN_PATH_AUTO && !f4ok);
     valu_fn fn = mfma_conv_fn(d->xb, d->wb, i8);
     if (fn != nullptr) {

@@ -89,16 +89,13 @@ enum MfmaTile { MT_256x256 = 0, MT_128x128 = 1, MT_64x64 = 2, MT_128x64 = 3, MT_
 //   FP4 core  : GEMM: all but 256x256 / 128x256;  convolution: all but 256x256 / 256x128, and only
 //               the two small tiles when the stored channel count allows 32-bit loads only;
 //               plus, for convolution with 128-bit loads, the 32x128 split-K tile;
-//               more than five planes in all (w4a4, w1a8, w2a8): 128x128, 64x64, 32x32 split-K
-//               (convolution with narrower loads: 64x64 only); the int8 core is not built for those.
+//               precisions with more than five planes in all (w4a4, w1a8, w2a8, ...) and w1a1: FP4 / FP6 operands
+//               only, and for convolution with narrower loads the 64x64 tile only.
 constexpr bool mfma_tile_enabled(int core, bool conv, int vw, int tile, int pa, int pb) {
-  // two wave groups: FP4 core, 128-bit loads, the four benchmark precisions
-  if (tile == MT_128x128_G2) return core == CORE_F4 && pa + pb <= 5 && pa + pb > 2 && (!conv || vw == 4);
-  if (pa + pb > 5 || pa + pb == 2) {
-    if (core == CORE_I8) return false;
-    if (conv && vw != 4) return tile == MT_64x64;
-    return tile == MT_128x128 || tile == MT_64x64 || tile == MT_32x32_K4;
-  }
+  const bool wide = pa + pb > 5 || pa + pb == 2;
+  if (wide && core == CORE_I8) return false;
+  if (wide && conv && vw != 4) return tile == MT_64x64;
+  if (tile == MT_128x128_G2) return core == CORE_F4 && (!conv || vw == 4);  // two wave groups: 128-bit loads
   if (core == CORE_I8) {
     if (!conv) return tile == MT_128x128 || tile == MT_64x64 || tile == MT_256x128;
     if (vw != 4) return tile == MT_64x64;

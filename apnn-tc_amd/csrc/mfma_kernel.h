@@ -11,6 +11,11 @@
 //           weight 4^(da+db) applied by the instruction's E8M0 block scale.  Products are multiples
 //           of 1/4 and the host only launches this core while K * (2^w - 1) * (2^a - 1) < 2^24, so the
 //           fp32 accumulators are exact and the result is acc * 4.
+//           With more than two planes on either side both operands are FP6 (e2m3) digits of up to four planes
+//           (expand_fp6): same instruction and rate, half the matrix instructions (a quarter for w4a4), about
+//           the same expansion work.  w1a4 at 4096^3 58.1 -> 48.0 us, w4a4 at 4096 x 333 x 4096 71.9 -> 23.6 us
+//           (there the double set of staging registers had also spilled), w1a3 3x3 convolution of 512
+//           channels on 16x16 maps at batch 16 13.5 -> 12.8 us.
 //
 // Work-group = 4 waves arranged WA x WB, each wave owning an (FA*32) x (FB*32) output tile
 // (FA*FB accumulator blocks of 16 registers).  The *packed* planes are staged through LDS
@@ -77,6 +82,100 @@ __device__ __forceinline__ v8i expand_fp4(const uint32_t (&w)[P]) {
   return out;
 }
 
+// bits of a word whose index is congruent to c modulo 6
+constexpr uint32_t every_sixth(int c) {
+  uint32_t m = 0;
+  for (int b = 0; b < 32; ++b)
+    if ((b - c) % 6 == 0) m |= 1u << b;
+  return m;
+}
+
+__device__ __forceinline__ uint32_t rotl32(uint32_t x, int n) { return __builtin_amdgcn_alignbit(x, x, (32 - n) & 31); }
+
+// FP6 (e2m3) operand for digit D (planes 4D .. 4D+3, as far as there are any) of a P-plane row word.  The codes
+// 0..15 of e2m3 are the values code / 8, so a digit of up to four planes is simply the low four bits of a 6-bit
+// field; field f of a lane occupies bits 6f .. 6f+5 of the six operand words (32 mod 6 = 2, so the fields of
+// word j start at bits congruent to -2j modulo 6).  The elements are dealt to the fields so that a plane
+// reaches its words by rotations alone: the even elements of the word, in place, fill operand words 0..2 (bit b
+// of the word is the field that starts at bit b of one of them), the odd ones, one bit to the right, words
+// 3..5.  Which element sits in which field does not matter as long as both operands of the product agree.
+// One plane 7 operations per 32 elements, two 10 (merged into 2-bit digits first, as in expand_fp4), three 18,
+// four 22 -- against 17 and 20 for three and four planes as two FP4 digits, which need twice the matrix
+// instructions (both formats run at the same rate).
+template <int P, int D>
+__device__ __forceinline__ v8i expand_fp6(const uint32_t (&w)[P]) {
+  constexpr int N = P - 4 * D < 4 ? P - 4 * D : 4;  // planes of this digit
+  constexpr uint32_t EVEN = 0x55555555u;
+  v8i out = {0, 0, 0, 0, 0, 0, 0, 0};
+  uint32_t qe = w[4 * D], qo = w[4 * D] >> 1;
+  if constexpr (N >= 2) {
+    const uint32_t x0 = w[4 * D], x1 = w[4 * D + 1];
+    qe = (x0 & EVEN) | ((x1 << 1) & ~EVEN);
+    qo = ((x0 >> 1) & EVEN) | (x1 & ~EVEN);
+  }
+  asm("" : "+v"(qe));  // keep the merged words (see expand_fp4)
+  asm("" : "+v"(qo));
+  uint32_t re = 0, ro = 0;
+  if constexpr (N >= 3) {
+    re = rotl32(w[4 * D + 2], 2);
+    ro = rotl32(w[4 * D + 2], 1);
+    if constexpr (N == 4) {
+      re = (re & EVEN) | (rotl32(w[4 * D + 3], 3) & ~EVEN);
+      ro = (ro & EVEN) | (rotl32(w[4 * D + 3], 2) & ~EVEN);
+    }
+    asm("" : "+v"(re));
+    asm("" : "+v"(ro));
+  }
+  auto word = [&](auto jc) {
+    constexpr int j = decltype(jc)::value % 3;
+    constexpr uint32_t lo = every_sixth(-2 * j) | (N >= 2 ? every_sixth(1 - 2 * j) : 0u);
+    const uint32_t q = decltype(jc)::value < 3 ? qe : qo;
+    if constexpr (N >= 3) {
+      constexpr uint32_t hi = every_sixth(2 - 2 * j) | (N >= 4 ? every_sixth(3 - 2 * j) : 0u);
+      const uint32_t r = decltype(jc)::value < 3 ? re : ro;
+      return (int)((q & lo) | (r & hi));
+    } else {
+      return (int)(q & lo);
+    }
+  };
+  out[0] = word(std::integral_constant<int, 0>{});
+  out[1] = word(std::integral_constant<int, 1>{});
+  out[2] = word(std::integral_constant<int, 2>{});
+  out[3] = word(std::integral_constant<int, 3>{});
+  out[4] = word(std::integral_constant<int, 4>{});
+  out[5] = word(std::integral_constant<int, 5>{});
+  return out;
+}
+
+// Operand encoding of the CORE_F4 kernels, by the planes of the two operands: FP4 digits of two planes where
+// neither operand has more, else FP6 digits of four planes for both (one instruction takes two formats, but
+// the two expansions deal the elements differently).  A digit code v means v / 2 or v / 8.
+constexpr int digit_planes(int PA, int PB) { return PA > 2 || PB > 2 ? 4 : 2; }
+// accumulator units: result = acc * fp_scale
+constexpr int fp_scale(int PA, int PB) { return digit_planes(PA, PB) == 4 ? 64 : 4; }
+
+template <int DIG, int P, int D>
+__device__ __forceinline__ v8i expand_digit(const uint32_t (&w)[P]) {
+  if constexpr (DIG == 4) {
+    return expand_fp6<P, D>(w);
+  } else {
+    return expand_fp4<P, D>(w);
+  }
+}
+
+// acc += digit product of weight 2^(DIG * SUM) on one 32x32 block and 64 k
+template <int DIG, int SUM>
+__device__ __forceinline__ v16f mfma_digits(const v8i &a, const v8i &b, const v16f &acc) {
+  constexpr int fmt = DIG == 4 ? 2 : 4;  // cbsz / blgp: 2 = FP6 e2m3, 4 = FP4 e2m1
+  if constexpr (SUM == 0) {
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, acc, fmt, fmt, 0, 0, 0, 0);
+  } else {
+    // E8M0 block scales: 127 = 2^0 on A, 127 + DIG * SUM on B
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, acc, fmt, fmt, 0, 0x7F7F7F7F, 0,
+                                                           0x7F7F7F7F + 0x01010101 * (DIG * SUM));
+  }
+}
+
 template <int P>
 __device__ __forceinline__ v4i expand_planes(const uint32_t (&w)[P], const uint32_t (&rot)[P]) {
   uint32_t ys[P];
@@ -136,11 +235,12 @@ __device__ __forceinline__ int write_lane_pair(int lo, int hi, int old) {
 //   lds[FA*32 + FA*64*FB ...)                threshold table [k][FB*32] (TABLE only), filled here
 // Q0, Q1: the register quads (rows 8q .. 8q+7 of a block) this call finishes; the split-K tiles give
 // each of their four waves one quad of the summed block.
-template <bool F4, int FA, int FB, bool CONV, bool TABLE, int Q0 = 0, int Q1 = 4, class AccT>
+template <int FS, int FA, int FB, bool CONV, bool TABLE, int Q0 = 0, int Q1 = 4, class AccT>
 __device__ __forceinline__ void direct_epilogue(const KParams &p, AccT (&acc)[FA][FB],
                                                 const int (&ssum)[CONV ? FA : FB], uint32_t *lds, int rbase,
                                                 int cbase, int lane, const int (&T)[FB][3], const int (&fm)[FB],
                                                 bool shortcut, const int *shared_table = nullptr) {
+  constexpr bool F4 = FS != 0;
   constexpr int NCOLS = FB * 32;
   constexpr int NPARK = TABLE ? 2 : 1;
   const int li = lane & 31, g = lane >> 5;
@@ -190,7 +290,7 @@ __device__ __forceinline__ void direct_epilogue(const KParams &p, AccT (&acc)[FA
     }
     fast = bn && p.epi_float != 0 && p.pool != APNN_POOL_AVG2X2 && __ballot(anyflip != 0) == 0ull;
   }
-  const float vscale = p.sym ? 8.0f : 4.0f;
+  const float vscale = (float)(p.sym ? 2 * FS : FS);
 
   // The epilogue mode (thresholds or low bits, pooled or not) is the same for the whole launch: the
   // value loop is instantiated once per mode and entered through one branch, so the per-value code
@@ -383,10 +483,11 @@ __device__ __forceinline__ void direct_epilogue(const KParams &p, AccT (&acc)[FA
 // wave writes two full 128-byte rows of the block (one per lane half): no LDS round trip, two vector
 // operations per value (scale, convert) and one address update per output row.  lds[0 .. FA*32) holds
 // the activation row sums times the weight range (convolution with symmetric weights; unused otherwise).
-template <bool F4, int FA, int FB, bool CONV, class AccT>
+template <int FS, int FA, int FB, bool CONV, class AccT>
 __device__ __forceinline__ void store_int32_direct(const KParams &p, AccT (&acc)[FA][FB],
                                                    const int (&ssum)[CONV ? FA : FB], const uint32_t *lds,
                                                    int rbase, int cbase, int lane) {
+  constexpr bool F4 = FS != 0;
   const int li = lane & 31, g = lane >> 5;
   const int sh = p.sym ? 1 : 0;
   const int wmax = p.sym ? p.wmax : 0;
@@ -400,7 +501,7 @@ __device__ __forceinline__ void store_int32_direct(const KParams &p, AccT (&acc)
   }
   // FP4 core: value = acc * 4 * 2^sym - correction as one fused multiply-add in fp32 and one conversion
   // (the host launches this core only while every such value is an integer below 2^24, so both are exact)
-  const float vscale = p.sym ? 8.0f : 4.0f;
+  const float vscale = (float)(p.sym ? 2 * FS : FS);
   int *out = reinterpret_cast<int *>(p.out);
   const long long pitch = p.rowsB;
   const bool full = rbase + FA * 32 <= p.rowsA && cbase + FB * 32 <= p.rowsB;  // same for the whole wave
@@ -508,11 +609,12 @@ __device__ __forceinline__ void wave_epilogue(const KParams &p, const int *slab,
 // resid_scale = t0 + t1 with t = +-{1, 3} * 2^j (the host finds the terms: KParams::fold, 0 when there
 // are none or fp32 would round).  res: the wave's published shortcut words, index
 // ((x * 2 + plane) * FB + y) * 32 + row.
-template <int FA, int FB>
+template <int FS, int FA, int FB>
 __device__ __forceinline__ void fold_shortcut(const KParams &p, v16f (&acc)[FA][FB], const uint32_t *res, int lane) {
   const int li = lane & 31, g = lane >> 5;
   const uint32_t nib = (p.fold >> (4 * g)) & 0xfu;
-  const uint32_t e8 = (p.fold >> (8 + 8 * g)) & 0xffu;
+  // KParams::fold holds the block scale for accumulators in units of 1/4; units of 1/64 take 2^-4 of it
+  const uint32_t e8 = ((p.fold >> (8 + 8 * g)) & 0xffu) - (FS == 64 ? 4u : 0u);
   const int scale_b = (int)(e8 * 0x01010101u);
   // identity column li: the shortcut planes hold channel c at bit 31 - c%32, and element e of a packed word
   // is nibble e / 4 of operand word e % 4 (expand_fp4), so channel li pairs with element e = 31 - li
@@ -600,10 +702,11 @@ __device__ __forceinline__ void epi_prefetch(const KParams &p, int rbase, int cb
 // K).  acc: this wave's FA x FB accumulator blocks; ssum: activation sums of the lane's row li of each
 // row block (convolution) or column li of each column block (GEMM entry points), complete in every
 // lane.  smem: the work-group's LDS, free for reuse after the barrier at the top.
-template <bool F4, int KS, bool CONV, int DIRECT_BITS, bool LAZY, int FA, int FB, class AccT>
+template <int FS, int KS, bool CONV, int DIRECT_BITS, bool LAZY, int FA, int FB, class AccT>
 __device__ __forceinline__ void epi_finish(const KParams &p, AccT (&acc)[FA][FB], const int (&ssum)[CONV ? FA : FB],
                                            uint32_t *smem, int wave, int lane, int a0, int b0, int wa, int wb,
                                            EpiOperands<FA, FB> &eo) {
+  constexpr bool F4 = FS != 0;
   const int li = lane & 31, g = lane >> 5;
   if (LAZY) epi_load<KS>(p, a0 + wa * FA * 32, b0 + wb * FB * 32, lane, eo);
   constexpr int RES_REGS = FB;
@@ -655,7 +758,7 @@ __device__ __forceinline__ void epi_finish(const KParams &p, AccT (&acc)[FA][FB]
           // the shortcut term enters one of the partial sums (wave 0's) on the matrix cores
           if (wave == 0) {
             shortcut_publish<RES_REGS>(area + 32, lane, 64, res_regs[0]);
-            fold_shortcut<1, FB>(p, acc, area + 32, lane);
+            fold_shortcut<FS, 1, FB>(p, acc, area + 32, lane);
           }
           shortcut_vec = false;
         }
@@ -709,12 +812,12 @@ __device__ __forceinline__ void epi_finish(const KParams &p, AccT (&acc)[FA][FB]
         });
         if constexpr (DIRECT_BITS > 2) {
           if (use_table) {
-            direct_epilogue<F4, 1, FB, CONV, true, q, q + 1>(p, accr, stot, area, rb, cb, lane, thrT, flipm,
+            direct_epilogue<FS, 1, FB, CONV, true, q, q + 1>(p, accr, stot, area, rb, cb, lane, thrT, flipm,
                                                              shortcut_vec, table);
             return;
           }
         }
-        direct_epilogue<F4, 1, FB, CONV, false, q, q + 1>(p, accr, stot, area, rb, cb, lane, thrT, flipm, shortcut_vec);
+        direct_epilogue<FS, 1, FB, CONV, false, q, q + 1>(p, accr, stot, area, rb, cb, lane, thrT, flipm, shortcut_vec);
       };
       static_assert(KS == 4, "one register quad per wave");
       switch (wave) {
@@ -735,7 +838,7 @@ __device__ __forceinline__ void epi_finish(const KParams &p, AccT (&acc)[FA][FB]
           for (int x = 0; x < FA; ++x) area[x * 32 + li] = (uint32_t)(p.wmax * ssum[CONV ? x : 0]);
         }
       }
-      store_int32_direct<F4, FA, FB, CONV>(p, acc, ssum, area, a0 + wa * FA * 32, b0 + wb * FB * 32, lane);
+      store_int32_direct<FS, FA, FB, CONV>(p, acc, ssum, area, a0 + wa * FA * 32, b0 + wb * FB * 32, lane);
       return;
     }
     if (direct) {
@@ -753,15 +856,15 @@ __device__ __forceinline__ void epi_finish(const KParams &p, AccT (&acc)[FA][FB]
       if constexpr (F4 && FA * FB <= 4) {
         if (res_prefetched && p.fold != 0u) {
           // LDS operations of one wave complete in order: the words published above are visible here
-          fold_shortcut<FA, FB>(p, acc, area + FA * 32, lane);
+          fold_shortcut<FS, FA, FB>(p, acc, area + FA * 32, lane);
           shortcut_vec = false;
         }
       }
       const int rb = a0 + wa * FA * 32, cb = b0 + wb * FB * 32;
       if (DIRECT_BITS == 2 || p.out_bits <= 2) {
-        direct_epilogue<F4, FA, FB, CONV, false>(p, acc, ssum, area, rb, cb, lane, thrT, flipm, shortcut_vec);
+        direct_epilogue<FS, FA, FB, CONV, false>(p, acc, ssum, area, rb, cb, lane, thrT, flipm, shortcut_vec);
       } else if constexpr (DIRECT_BITS > 2) {
-        direct_epilogue<F4, FA, FB, CONV, true>(p, acc, ssum, area, rb, cb, lane, thrT, flipm, shortcut_vec);
+        direct_epilogue<FS, FA, FB, CONV, true>(p, acc, ssum, area, rb, cb, lane, thrT, flipm, shortcut_vec);
       }
       return;
     }
@@ -785,7 +888,7 @@ __device__ __forceinline__ void epi_finish(const KParams &p, AccT (&acc)[FA][FB]
         constexpr int r = decltype(rc)::value;
         int v;
         if constexpr (F4) {
-          v = __float2int_rn(acc[x][y][r] * 4.0f);
+          v = __float2int_rn(acc[x][y][r] * (float)FS);
         } else {
           v = acc[x][y][r];
         }
@@ -817,7 +920,8 @@ __device__ __forceinline__ void epi_finish(const KParams &p, AccT (&acc)[FA][FB]
 // work (im2col addressing, LDS staging, barrier) is a large share of a short K loop, and k-steps past the
 // end of K are skipped, so a longer chunk wastes nothing.
 constexpr int mfma_chunk_words(int PA, int PB, int FA, int FB, int WA, int WB, bool conv, int vw, int ksx = 1) {
-  if (ksx > 1) return 16;  // two wave groups share the k-steps of a chunk: four each
+  // two wave groups share the k-steps of a chunk: four each (two where 16 words would not fit the LDS twice)
+  if (ksx > 1) return PA + PB <= 8 ? 16 : 8;
   if (WA * WB == 1) return 32;
   if (conv && FA * FB <= 2 && vw == 4) return 16;
   if (!conv && FA * FB >= 8 && (PA * WA * FA + PB * WB * FB) * 32 <= 512) return 16;
@@ -857,8 +961,10 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
   constexpr bool F4 = CORE == CORE_F4;
   static_assert(KSX == 1 || (KSX == 2 && KS == 1 && F4 && FA % 2 == 0), "wave groups: FP4 core, even row blocks");
   constexpr int WPS = F4 ? 2 : 1;                 // packed words per row consumed by one k-step
-  constexpr int DA = F4 ? (PA + 1) / 2 : 1;       // operand digits (FP4: plane pairs)
-  constexpr int DB = F4 ? (PB + 1) / 2 : 1;
+  constexpr int DIG = digit_planes(PA, PB);       // bit-planes per operand digit (FP4: 2, FP6: 4)
+  constexpr int DA = F4 ? (PA + DIG - 1) / DIG : 1;
+  constexpr int DB = F4 ? (PB + DIG - 1) / DIG : 1;
+  constexpr int FSC = F4 ? fp_scale(PA, PB) : 0;
   using AccT = typename std::conditional<F4, v16f, v16i>::type;
   using FragT = typename std::conditional<F4, v8i, v4i>::type;
   constexpr int NT = 256 * KSX;
@@ -1075,7 +1181,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
   // register sets, so a chunk's loads are issued two chunk iterations before they are staged (one iteration
   // does not cover the memory latency when a wave runs only a few k-steps per chunk); the larger tiles have
   // no registers to spare for a second set.
-  constexpr int PF = (FA * FB <= 4 && VW == 4) ? 2 : 1;
+  constexpr int PF = (FA * FB <= 4 && VW == 4 && PA + PB <= 5) ? 2 : 1;
   uint32_t ra_[PF][NIA][PA][VW], rb_[PF][NIB][PB][VW];
 
   auto fetch = [&](int k0, auto set_c) {
@@ -1190,7 +1296,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
         for (int pl = 0; pl < PA; ++pl) psum[x][pl] += __popc(wA[x][pl]);
       }
       if constexpr (F4) {
-        static_for<0, DA>([&](auto dc) { a[x][decltype(dc)::value] = expand_fp4<PA, decltype(dc)::value>(wA[x]); });
+        static_for<0, DA>([&](auto dc) { a[x][decltype(dc)::value] = expand_digit<DIG, PA, decltype(dc)::value>(wA[x]); });
       } else {
         a[x][0] = expand_planes<PA>(wA[x], rotA);
       }
@@ -1202,7 +1308,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
         for (int pl = 0; pl < PB; ++pl) psum[y][pl] += __popc(wB[y][pl]);
       }
       if constexpr (F4) {
-        static_for<0, DB>([&](auto dc) { b[y][decltype(dc)::value] = expand_fp4<PB, decltype(dc)::value>(wB[y]); });
+        static_for<0, DB>([&](auto dc) { b[y][decltype(dc)::value] = expand_digit<DIG, PB, decltype(dc)::value>(wB[y]); });
       } else {
         b[y][0] = expand_planes<PB>(wB[y], rotB);
       }
@@ -1217,14 +1323,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
           static_for<0, DA>([&](auto dac) {
             static_for<0, DB>([&](auto dbc) {
               constexpr int da = decltype(dac)::value, db = decltype(dbc)::value;
-              if constexpr (da + db == 0) {
-                acc[x][y] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af[x][da], bf[y][db], acc[x][y], 4, 4,
-                                                                            0, 0, 0, 0);
-              } else {
-                // E8M0 block scales: 127 = 2^0 on A, 127 + 2*(da+db) = 4^(da+db) on B
-                acc[x][y] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                    af[x][da], bf[y][db], acc[x][y], 4, 4, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F + 0x02020202 * (da + db));
-              }
+              acc[x][y] = mfma_digits<DIG, da + db>(af[x][da], bf[y][db], acc[x][y]);
             });
           });
         } else {
@@ -1238,8 +1337,10 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
   // the last k-step of chunk ch).  Global loads run two chunks ahead, LDS holds two chunks.
   constexpr int NKS = KC / WPS;  // k-steps per chunk
   constexpr int N_MFMA = FA * FB * DA * DB;
-  // expansion cost per row word: FP4 10 operations per plane pair + 7 for an odd plane, int8 8 per plane
-  constexpr int XA = F4 ? 10 * (PA / 2) + 7 * (PA % 2) : 8 * PA, XB = F4 ? 10 * (PB / 2) + 7 * (PB % 2) : 8 * PB;
+  // expansion cost per row word: digits of one to four planes 7, 10, 18, 22 operations, int8 8 per plane
+  constexpr int XDIG[5] = {0, 7, 10, 18, 22};
+  constexpr int XA = F4 ? XDIG[DIG] * (PA / DIG) + XDIG[PA % DIG] : 8 * PA;
+  constexpr int XB = F4 ? XDIG[DIG] * (PB / DIG) + XDIG[PB % DIG] : 8 * PB;
   constexpr int N_VALU = FA * XA + FB * XB + FS * PS;
   constexpr int VALU_PER_MFMA = (N_VALU + N_MFMA - 1) / N_MFMA;
 
@@ -1384,7 +1485,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
   }
 
   if constexpr (KSX == 1) {
-    epi_finish<F4, KS, CONV, (CONV ? PA : PB) >= 3 ? 4 : 2, EPI_LAZY>(p, acc, ssum, smem, wave, lane, a0, b0, wa, wb, eo);
+    epi_finish<FSC, KS, CONV, (CONV ? PA : PB) >= 3 ? 4 : 2, EPI_LAZY>(p, acc, ssum, smem, wave, lane, a0, b0, wa, wb, eo);
   } else {
     // The two wave groups hold partial sums over their k-steps for the same outputs.  Group 0 finishes the
     // first HA row blocks of every wave tile, group 1 the last HA: each wave parks the blocks it gives away
@@ -1444,7 +1545,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
       own_sum[x] = xsum[(wave * FS + idx) * 64 + lane] + xsum[(partner * FS + idx) * 64 + lane];
     }
     // epi_finish opens with a barrier: nobody overwrites the exchange area before every wave has read it
-    epi_finish<F4, 1, CONV, (CONV ? PA : PB) >= 3 ? 4 : 2, EPI_LAZY>(p, own, own_sum, smem, wave, lane, own_rbase, b0, 0,
+    epi_finish<FSC, 1, CONV, (CONV ? PA : PB) >= 3 ? 4 : 2, EPI_LAZY>(p, own, own_sum, smem, wave, lane, own_rbase, b0, 0,
                                                                        wb, eo);
   }
 }

@@ -330,7 +330,7 @@ __global__ __launch_bounds__(256, OCC) void apnn_mfma_xs_kernel(const KParams pk
 #pragma unroll
   for (int x = 0; x < FS; ++x) ssum[x] = sumbuf[((CONV ? wa * FA : wb * FB) + x) * 32 + li];
 
-  epi_finish<true, 1, CONV, DIRECT_BITS, EPI_LAZY>(p, acc, ssum, smem, wave, lane, a0, b0, wa, wb, eo);
+  epi_finish<4, 1, CONV, DIRECT_BITS, EPI_LAZY>(p, acc, ssum, smem, wave, lane, a0, b0, wa, wb, eo);
 }
 
 constexpr size_t mfma_xs_smem_bytes(int PA, int PB, int FA, int FB, int WA, int WB) {

@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256, OCC) void apnn_patch_conv_kernel(const KParams
       }
     }
   }
-  epi_finish<true, 1, true, DIRECT_BITS, false>(p, acc, ssum, smem, wave, lane, a0, b0, wa, wb, eo);
+  epi_finish<4, 1, true, DIRECT_BITS, false>(p, acc, ssum, smem, wave, lane, a0, b0, wa, wb, eo);
 }
 
 // LDS bytes of a launch: patch + filter block + pixel sums, at least the slab area of the output stage

@@ -40,3 +40,34 @@ def test_float_packer_edges(G, rows, C, cpad, bits, lo, hi):
     codes = np.minimum(np.rint(q), 2 ** bits - 1).astype(np.uint32)
     expect = O.pack_bits(codes, rows, C, cpad, bits)
     assert np.array_equal(G.to_host(planes, np.uint32).reshape(expect.shape), expect)
+
+
+# Precisions beyond five planes (FP6 digits of four planes) and w1a1 on every tile that is built: one row past a
+# tile, one short of it, reductions that end inside a chunk.
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 9])
+@pytest.mark.parametrize("wb,xb", [(1, 1), (1, 8), (2, 8), (4, 4)])
+@pytest.mark.parametrize("M,N,K,sym", [(129, 255, 640, 1), (31, 33, 128, 0), (257, 129, 1152, 0)])
+def test_wide_precision_gemm_tiles(G, wb, xb, tile, M, N, K, sym):
+    rng = np.random.default_rng(8200 + M + 10 * wb + xb)
+    W, X = O.random_planes(rng, wb, M, K // 32), O.random_planes(rng, xb, N, K // 32)
+    got = G.run_gemm(W, X, M, N, K, wb, xb, sym=sym, path=2, tile=tile).reshape(M, N)
+    assert np.array_equal(got, O.gemm(W, X, M, N, K, wb, xb, sym_w=sym))
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 7, 8, 9])
+@pytest.mark.parametrize("wb,xb", [(1, 5), (2, 6), (1, 8), (2, 8)])
+@pytest.mark.parametrize("H,C,cout,R,sym", [(13, 128, 96, 3, 1), (5, 256, 33, 1, 0)])
+def test_wide_precision_conv_tiles(G, wb, xb, tile, H, C, cout, R, sym):
+    rng = np.random.default_rng(8300 + H + 10 * wb + xb)
+    W, X = O.random_planes(rng, wb, cout * R * R, C // 32), O.random_planes(rng, xb, 2 * H * H, C // 32)
+    kw = dict(batch=2, H=H, W=H, cout=cout, R=R, S=R, stride=1, pad=R // 2, halo=0, wb=wb, xb=xb)
+    got = G.run_conv(W, X, cin_pad=C, sym=sym, path=2, tile=tile, **kw)
+    assert np.array_equal(got.reshape(-1, cout), O.conv(W, X, cwords=C // 32, sym_w=sym, **kw).reshape(-1, cout))
+
+
+@pytest.mark.parametrize("wb,xb,M,N,K", [(1, 1, 111, 67, 1792), (1, 1, 1, 1, 128), (2, 8, 52, 72, 128), (4, 4, 3, 5, 256), (1, 8, 16, 1, 8192)])
+def test_small_products_of_precisions_without_popcount_kernel(G, wb, xb, M, N, K):
+    """AUTO takes the matrix cores for these at every size (the any-precision popcount kernel is 5-16 times slower)."""
+    rng = np.random.default_rng(8400 + M + wb + xb)
+    W, X = O.random_planes(rng, wb, M, K // 32), O.random_planes(rng, xb, N, K // 32)
+    assert np.array_equal(G.run_gemm(W, X, M, N, K, wb, xb).reshape(M, N), O.gemm(W, X, M, N, K, wb, xb))
