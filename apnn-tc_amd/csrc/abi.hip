@@ -224,46 +224,48 @@ bool int32_range_ok(long long kwords, int wb, int xb, bool sym, const apnn_epilo
   return top < (1LL << 31);
 }
 
-// resid_scale as terms the matrix cores can apply to FP4 shortcut digits (KParams::fold).  A digit v means
-// v / 2 and the accumulator holds result / vscale (vscale = 4, or 8 with symmetric weights), so a term
-// t = s * m * 2^j (m = 1 or 3) needs the FP4 value s * m / 2 (codes 1 and 3, sign in bit 3) and the block
-// scale 2^(j - sym).  Two terms at most; 0 when the scale needs more, when there is no packed shortcut of
-// one or two bits, or when fp32 could round (accumulator range plus both terms' largest magnitude must stay
-// below 2^24, as for epilogue_float_ok).
+// resid_scale as terms the matrix cores can apply to FP4 shortcut digits (KParams::fold): one or two terms +-m * 2^j
+// with m up to 15.  An odd scale of more than four bits is split at its low k bits, taken as they are or as a
+// negative remainder.  0 when that finds no second term, when there is no packed shortcut of one or two bits, or when
+// fp32 could round (accumulator range plus both terms' largest magnitude must stay below 2^24, as for
+// epilogue_float_ok).
 uint32_t shortcut_fold(const KParams &p, int wb, int xb) {
   if (p.resid_planes == nullptr || p.resid_bits < 1 || p.resid_bits > 2 || p.resid_scale == 0) return 0u;
   if (p.epi == APNN_EPI_INT32 || p.pool != APNN_POOL_NONE) return 0u;
-  const long long S = p.resid_scale;
-  const int sym = p.sym ? 1 : 0;
-  auto term = [&](long long t, uint32_t *nib, uint32_t *e8) {  // t == +-{1,3} * 2^j with j >= 0?
-    if (t == 0) return false;
-    const long long a = t < 0 ? -t : t;
-    int j = 0;
-    long long m = a;
-    while ((m & 1) == 0) {
-      m >>= 1;
-      ++j;
+  struct Term {
+    uint32_t m, e8;  // m: magnitude and sign (bit 4)
+  };
+  auto term = [](long long t, Term *out) {  // t == +-m * 2^j?
+    if (t == 0) {
+      *out = Term{0u, 127u};
+      return true;
     }
-    if (m != 1 && m != 3) return false;
-    *nib = (m == 1 ? 1u : 3u) | (t < 0 ? 8u : 0u);
-    *e8 = (uint32_t)(127 + j - sym);
+    const unsigned long long a = (unsigned long long)(t < 0 ? -t : t);
+    const int j = __builtin_ctzll(a);
+    if ((a >> j) > 15) return false;
+    *out = Term{(uint32_t)(a >> j) | (t < 0 ? 16u : 0u), (uint32_t)(127 + j)};
     return true;
   };
   const long long acc = (long long)p.KW * 32 * ((1LL << wb) - 1) * ((1LL << xb) - 1);
   const long long cmax = (1LL << p.resid_bits) - 1;
-  auto fits = [&](long long t0, long long t1) {
-    const long long a0 = t0 < 0 ? -t0 : t0, a1 = t1 < 0 ? -t1 : t1;
-    return acc + (a0 + a1) * cmax < (1LL << 24);
+  auto code = [&](long long t0, long long t1) -> uint32_t {
+    Term a, b;
+    if (!term(t0, &a) || !term(t1, &b)) return 0u;
+    const long long size = (t0 < 0 ? -t0 : t0) + (t1 < 0 ? -t1 : t1);
+    // (unsigned one-plane weights accumulate -1 / +1 products, in units of half a result)
+    if (acc + size * cmax * (p.sym || wb > 1 ? 1 : 2) >= (1LL << 24)) return 0u;
+    return a.m | (b.m << 5) | (a.e8 << 10) | (b.e8 << 18);
   };
-  uint32_t n0 = 0, e0 = 127, n1 = 0, e1 = 127;
-  if (term(S, &n0, &e0)) return fits(S, 0) ? (n0 | (e0 << 8) | (127u << 16)) : 0u;
-  for (int j = 0; j < 24; ++j)
-    for (int m = 1; m <= 3; m += 2)
-      for (int sg = -1; sg <= 1; sg += 2) {
-        const long long t0 = (long long)sg * m * (1LL << j);
-        if (term(t0, &n0, &e0) && term(S - t0, &n1, &e1) && fits(t0, S - t0))
-          return n0 | (n1 << 4) | (e0 << 8) | (e1 << 16);
-      }
+  const long long S = p.resid_scale;
+  const int z = __builtin_ctzll((unsigned long long)(S < 0 ? -S : S));
+  const long long odd = S >> z;
+  if (odd >= -15 && odd <= 15) return code(S, 0);
+  for (int k = 1; k <= 5; ++k) {
+    const long long low = odd & ((1LL << k) - 1);
+    for (const long long t : {low, low - (1LL << k)})
+      if (t >= -15 && t <= 15)
+        if (const uint32_t f = code((odd - t) * (1LL << z), t * (1LL << z))) return f;
+  }
   return 0u;
 }
 

@@ -78,10 +78,10 @@ struct KParams {
   // 1: every value the quantizing epilogue compares (accumulator, correction, scaled shortcut code) is an
   // integer below 2^24 in magnitude, so the FP4 kernels may do the threshold compare in fp32
   int epi_float;
-  // Shortcut add on the matrix cores (FP4 kernels, see fold_shortcut in mfma_kernel.h): resid_scale as the
-  // sum of two terms +-{1, 3} * 2^j, each an FP4 value (sign and code in a nibble: bits 0-3 first term,
-  // bits 4-7 second term, 0 = no term) times an E8M0 block scale (bits 8-15 and 16-23).  0: the shortcut is
-  // added per value in the vector ALUs (scale not representable, fp32 would round, other core).
+  // Shortcut add on the matrix cores (FP4 / FP6 kernels, see fold_shortcut in mfma_kernel.h): resid_scale as the
+  // sum of two terms +-m * 2^j, m up to 15: bits 0-4 first m with its sign in bit 4, bits 5-9 second (0 = no term),
+  // bits 10-17 and 18-25 the E8M0 codes 127 + j.  0: the shortcut is added per value in the vector ALUs (scale not
+  // representable, fp32 would round, other core).
   uint32_t fold;
   void *out;
   long long out_plane;       // packed output: plane stride in words

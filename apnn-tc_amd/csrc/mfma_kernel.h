@@ -28,9 +28,10 @@
 //   i.e. 8 VALU operations per plane for 16 int8 operands; CORE_F4: see expand_fp4.
 //
 // Symmetric (+-) weights use the closed form  2*raw - wmax * (activation row sum); the row sums
-// come from popcounts of the packed words the wave already holds.
+// come from popcounts of the packed words the wave already holds.  (FP4 / FP6 convolution kernels with one weight
+// plane: -1 / +1 operands, see expand_sign.)
 //
-// Output: int32 results and codes of up to two bits (four where the waves tile the output) leave
+// Output of the FP4 / FP6 convolution kernels: conv_epilogue.h.  GEMM entry points and int8 core: int32 results and codes of up to two bits (four where the waves tile the output) leave
 // straight from the accumulator registers (store_int32_direct, direct_epilogue); int32 residuals, saved
 // accumulators and wider codes pass each wave's tile through an LDS slab, 32 rows at a time, which turns
 // the matrix-core register layout into row-major order.
@@ -39,6 +40,7 @@
 
 #include <type_traits>
 
+#include "conv_epilogue.h"
 #include "dispatch.h"
 #include "epilogue.h"
 #include "kparams.h"
@@ -50,6 +52,14 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
+}
 
 // FP4 operand for digit D (planes 2D and, if present, 2D+1) of a P-plane row word: nibble c of
 // result word t is the digit of element 4c + t.
@@ -147,6 +157,29 @@ __device__ __forceinline__ v8i expand_fp6(const uint32_t (&w)[P]) {
   return out;
 }
 
+// One-plane weights as -1 / +1: sign bit = complement of the weight bit, magnitude 1.0 (FP4 code 2, FP6 code 8), the
+// same elements in the same fields as expand_fp4 / expand_fp6.  With symmetric weights the accumulator is then the
+// result itself (in units), no activation sums are needed; unsigned weights u = (1 + s) / 2 take half of it plus
+// half the activation sum.
+template <int DIG>
+__device__ __forceinline__ v8i expand_sign(uint32_t x) {
+  v8i out = {0, 0, 0, 0, 0, 0, 0, 0};
+  if constexpr (DIG == 2) {
+    static_for<0, 4>([&](auto tc) {
+      constexpr int t = decltype(tc)::value;
+      out[t] = (int)(((x << (3 - t)) & 0x88888888u) ^ 0xAAAAAAAAu);
+    });
+  } else {
+    const uint32_t e = rotl32(x, 5), o = rotl32(x, 4);
+    static_for<0, 6>([&](auto jc) {
+      constexpr int jj = decltype(jc)::value, j = jj % 3;
+      constexpr uint32_t sign = every_sixth(5 - 2 * j), one = every_sixth(3 - 2 * j);
+      out[jj] = (int)(((jj < 3 ? e : o) & sign) ^ (sign | one));
+    });
+  }
+  return out;
+}
+
 // Operand encoding of the CORE_F4 kernels, by the planes of the two operands: FP4 digits of two planes where
 // neither operand has more, else FP6 digits of four planes for both (one instruction takes two formats, but
 // the two expansions deal the elements differently).  A digit code v means v / 2 or v / 8.
@@ -172,7 +205,7 @@ __device__ __forceinline__ v16f mfma_digits(const v8i &a, const v8i &b, const v1
   } else {
     // E8M0 block scales: 127 = 2^0 on A, 127 + DIG * SUM on B
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, acc, fmt, fmt, 0, 0x7F7F7F7F, 0,
-                                                           0x7F7F7F7F + 0x01010101 * (DIG * SUM));
+                                                           (int)(0x7F7F7F7Fu + 0x01010101u * (uint32_t)(DIG * SUM)));
   }
 }
 
@@ -190,14 +223,6 @@ __device__ __forceinline__ v4i expand_planes(const uint32_t (&w)[P], const uint3
     out[t] = (int)word;
   }
   return out;
-}
-
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F &&f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
-  }
 }
 
 // old with lanes LANE_LO / LANE_HI replaced by the wave-uniform values lo / hi (v_writelane_b32: one VALU
@@ -600,28 +625,45 @@ __device__ __forceinline__ void wave_epilogue(const KParams &p, const int *slab,
   }
 }
 
-// Shortcut add on the matrix cores (FP4 core, shortcut codes of one or two bits).  The term
+// Shortcut add on the matrix cores (FP4 / FP6 core, shortcut codes of one or two bits).  The term
 // resid_scale * code[row][channel] of a 32x32 block is the product of the 32x32 matrix of codes (an FP4
 // operand like any activation row: digit v means v/2) with a scaled identity, so one more matrix
 // instruction per block adds it to the accumulator -- instead of two bit extracts, a merge, a multiply, a
-// conversion and an add per output value in the vector ALUs.  The scale travels as FP4 value x E8M0 block
-// scale; the two lane halves (k positions 0..31 and 32..63) both see the codes and carry one term each, so
-// resid_scale = t0 + t1 with t = +-{1, 3} * 2^j (the host finds the terms: KParams::fold, 0 when there
-// are none or fp32 would round).  res: the wave's published shortcut words, index
-// ((x * 2 + plane) * FB + y) * 32 + row.
+// conversion and an add per output value in the vector ALUs.  The identity is an FP6 operand (e2m3: code m means
+// m / 8 up to 15) and its block scale a power of two; the two lane halves (k positions 0..31 and 32..63) both see
+// the codes and carry one term each, so resid_scale = t0 + t1 with t = +-m * 2^j, m up to 15: every scale of up to
+// eight bits and most larger ones (the host finds the terms: KParams::fold, 0 when there are none or fp32 would
+// round).  With FP4 identities (m = 1 or 3) a third of the scales above 32 had kept the vector form.
+//
+// Position p (0..31) of an FP4 operand is nibble p % 8 of word p / 8 and holds element 4 * (p % 8) + p / 8 of the
+// packed word (expand_fp4); the shortcut planes hold channel c at bit 31 - c%32, so channel c sits at the position
+// below, which in FP6 is the field at bits 6p .. 6p+5.
+__device__ __forceinline__ v8i fold_identity(const KParams &p, int lane) {
+  const int li = lane & 31, g = lane >> 5;
+  const uint32_t m = (p.fold >> (5 * g)) & 0x1fu;                      // sign in bit 4
+  const uint64_t code = (m & 15u) | (m & 16u ? 32u : 0u);              // e2m3: sign in bit 5
+  const int e = 31 - li, bit = 6 * (8 * (e & 3) + (e >> 2));
+  const uint64_t at = code << (bit & 31);
+  v8i d = {0, 0, 0, 0, 0, 0, 0, 0};
+  static_for<0, 6>([&](auto wc) {
+    constexpr int w = decltype(wc)::value;
+    d[w] = (int)((bit >> 5) == w ? (uint32_t)at : (bit >> 5) == w - 1 ? (uint32_t)(at >> 32) : 0u);
+  });
+  return d;
+}
+// E8M0 scale of this half's term for accumulators whose unit is worth 2^log2vs
+__device__ __forceinline__ int fold_scale(const KParams &p, int lane, int log2vs) {
+  const uint32_t e8 = ((p.fold >> (10 + 8 * (lane >> 5))) & 0xffu) + 4 - log2vs;  // (code / 2) * (m / 8)
+  return (int)(e8 * 0x01010101u);
+}
+
+// Lanes are channels (GEMM entry points, patch-resident and expand-while-staging kernels).  res: the wave's
+// published shortcut words, index ((x * 2 + plane) * FB + y) * 32 + row.
 template <int FS, int FA, int FB>
 __device__ __forceinline__ void fold_shortcut(const KParams &p, v16f (&acc)[FA][FB], const uint32_t *res, int lane) {
-  const int li = lane & 31, g = lane >> 5;
-  const uint32_t nib = (p.fold >> (4 * g)) & 0xfu;
-  // KParams::fold holds the block scale for accumulators in units of 1/4; units of 1/64 take 2^-4 of it
-  const uint32_t e8 = ((p.fold >> (8 + 8 * g)) & 0xffu) - (FS == 64 ? 4u : 0u);
-  const int scale_b = (int)(e8 * 0x01010101u);
-  // identity column li: the shortcut planes hold channel c at bit 31 - c%32, and element e of a packed word
-  // is nibble e / 4 of operand word e % 4 (expand_fp4), so channel li pairs with element e = 31 - li
-  const int e = 31 - li;
-  const uint32_t one = nib << (4 * (e >> 2));
-  const v8i bop = {(e & 3) == 0 ? (int)one : 0, (e & 3) == 1 ? (int)one : 0, (e & 3) == 2 ? (int)one : 0,
-                   (e & 3) == 3 ? (int)one : 0, 0, 0, 0, 0};
+  const int li = lane & 31;
+  const v8i bop = fold_identity(p, lane);
+  const int scale_b = fold_scale(p, lane, __builtin_ctz(FS) + (p.sym ? 1 : 0));
   static_for<0, FA>([&](auto xc) {
     constexpr int x = decltype(xc)::value;
     static_for<0, FB>([&](auto yc) {
@@ -630,7 +672,24 @@ __device__ __forceinline__ void fold_shortcut(const KParams &p, v16f (&acc)[FA][
       w[0] = res[((x * 2 + 0) * FB + y) * 32 + li];
       w[1] = p.resid_bits > 1 ? res[((x * 2 + 1) * FB + y) * 32 + li] : 0u;
       const v8i aop = expand_fp4<2, 0>(w);
-      acc[x][y] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aop, bop, acc[x][y], 4, 4, 0, 0x7F7F7F7F, 0, scale_b);
+      acc[x][y] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aop, bop, acc[x][y], 4, 2, 0, 0x7F7F7F7F, 0, scale_b);
+    });
+  });
+}
+
+// Lanes are pixels: the scaled identity is the first operand (its row li is channel li of the block), the codes of
+// the lane's pixel the second.
+template <int FA, int FB>
+__device__ __forceinline__ void fold_shortcut_lanes(const KParams &p, v16f (&acc)[FA][FB], const uint32_t (&sc)[FA][FB][2],
+                                                    int lane, int log2vs) {
+  const v8i aop = fold_identity(p, lane);
+  const int scale_a = fold_scale(p, lane, log2vs);
+  static_for<0, FA>([&](auto xc) {
+    constexpr int x = decltype(xc)::value;
+    static_for<0, FB>([&](auto yc) {
+      constexpr int y = decltype(yc)::value;
+      const v8i bop = expand_fp4<2, 0>(sc[x][y]);
+      acc[x][y] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aop, bop, acc[x][y], 2, 4, 0, scale_a, 0, 0x7F7F7F7F);
     });
   });
 }
@@ -921,11 +980,23 @@ __device__ __forceinline__ void epi_finish(const KParams &p, AccT (&acc)[FA][FB]
 // end of K are skipped, so a longer chunk wastes nothing.
 constexpr int mfma_chunk_words(int PA, int PB, int FA, int FB, int WA, int WB, bool conv, int vw, int ksx = 1) {
   // two wave groups share the k-steps of a chunk: four each (two where 16 words would not fit the LDS twice)
-  if (ksx > 1) return PA + PB <= 8 ? 16 : 8;
+  if (ksx > 1) return PA + PB <= (conv ? 6 : 8) ? 16 : 8;
   if (WA * WB == 1) return 32;
-  if (conv && FA * FB <= 2 && vw == 4) return 16;
+  if (conv && FA * FB <= 2 && vw == 4 && PA + PB <= 5) return 16;
   if (!conv && FA * FB >= 8 && (PA * WA * FA + PB * WB * FB) * 32 <= 512) return 16;
   return 8;
+}
+
+// Operand buffers of the FP4 / FP6 convolution kernels in LDS (words), or the exchange area of their partial sums
+// where that is larger; the threshold table lies behind it.
+constexpr int mfma_lp_stage_words(int PA, int PB, int FA, int FB, int WA, int WB, int vw, int ksx) {
+  const int ks = 4 / (WA * WB);
+  const int ld = mfma_chunk_words(PA, PB, FA, FB, WA, WB, true, vw, ksx) + 1;
+  const int stage = ks > 1 && vw == 4 ? 0 : 2 * (PA * WA * FA * 32 + PB * WB * FB * 32) * ld;
+  const int part = ks > 1 ? ks * FB * 4 * 64 * 4 + ks * 32 : 0;
+  const int xch = ksx > 1 ? 4 * ksx * ((FA / ksx) * FB * 16 + FA) * 64 : 0;
+  const int m = stage > part ? stage : part;
+  return ((m > xch ? m : xch) + 3) & ~3;
 }
 
 // longest reduction (32-bit words) the one- and two-block convolution tiles load without staging
@@ -965,6 +1036,12 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
   constexpr int DA = F4 ? (PA + DIG - 1) / DIG : 1;
   constexpr int DB = F4 ? (PB + DIG - 1) / DIG : 1;
   constexpr int FSC = F4 ? fp_scale(PA, PB) : 0;
+  // convolution on the FP4 / FP6 core: weights are the first operand of the matrix instructions, a lane of the
+  // accumulator is an output pixel (conv_epilogue.h), one-plane weights are -1 / +1
+  constexpr bool LP = CONV && F4;
+  constexpr bool SIGNED1 = LP && PB == 1;
+  constexpr int VSC = SIGNED1 ? (DIG == 4 ? 8 : 2) : FSC;
+  const bool need_sum = !LP || (SIGNED1 ? p.sym == 0 : p.sym != 0);  // activation sums enter the result
   using AccT = typename std::conditional<F4, v16f, v16i>::type;
   using FragT = typename std::conditional<F4, v8i, v4i>::type;
   constexpr int NT = 256 * KSX;
@@ -1038,6 +1115,14 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
     y0 = oy * p.stride - p.pad;
     x0 = ox * p.stride - p.pad;
   };
+
+  // value per accumulator unit; the thresholds of the tile's channels, behind the operand buffers
+  const int log2vs = __builtin_ctz(VSC > 0 ? VSC : 1) + (SIGNED1 ? (p.sym ? 0 : -1) : (p.sym ? 1 : 0));
+  const float inv_vs = __uint_as_float((uint32_t)(127 - log2vs) << 23), vs = __uint_as_float((uint32_t)(127 + log2vs) << 23);
+  uint32_t *tab = smem + (LP ? mfma_lp_stage_words(PA, PB, FA, FB, WA, WB, VW, KSX) : 0);
+  constexpr int MAXB = PA >= 3 ? 4 : 2;  // code widths the output stage has a path of its own for
+  ConvTable<TB, PA >= 3 ? 15 : 3, MAXB> table;
+  if constexpr (LP) table.load(p, b0);
 
   // how the operands reach the matrix core (see direct_loop below)
   constexpr bool DIRECT_K = F4 && KS > 1 && VW == 4;
@@ -1138,6 +1223,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
       baseB[y] = (uint32_t)grow * (uint32_t)p.KW;
     }
     direct_issue(gfirst);
+    if constexpr (LP) table.store(p, b0, tab, inv_vs);
   }
 
   // ---- staging bookkeeping (same scheme as the VALU kernel) ----------------------------------
@@ -1269,7 +1355,13 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
   const int own_rbase = a0 + (wa * FA + kq * HA) * 32;
   EpiOperands<HA, FB> eo;
   constexpr bool EPI_LAZY = HA * FB >= 8;
-  epi_prefetch<KS, (CONV ? PA : PB) >= 3 ? 4 : 2, EPI_LAZY>(p, own_rbase, b0 + wb * FB * 32, lane, eo);
+  uint32_t sc[HA][FB][2];  // shortcut words of the wave's pixels (split-K: wave 0 adds the shortcut)
+  const bool fold = LP && p.fold != 0u && (KS == 1 || wave == 0);
+  if constexpr (LP) {
+    if (fold && !EPI_LAZY) conv_shortcut_load<HA, FB>(p, own_rbase, b0 + wb * FB * 32, li, sc);
+  } else {
+    epi_prefetch<KS, (CONV ? PA : PB) >= 3 ? 4 : 2, EPI_LAZY>(p, own_rbase, b0 + wb * FB * 32, lane, eo);
+  }
 
   // packed words of this lane's rows for one k-step
   uint32_t wA[FA][PA], wB[FB][PB];
@@ -1288,10 +1380,11 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
       for (int pl = 0; pl < PB; ++pl) wB[y][pl] = Bs[(pl * TB + y * 32) * LD];
   };
   FragT af[FA][DA], bf[FB][DB];
-  auto expand_all = [&](FragT (&a)[FA][DA], FragT (&b)[FB][DB]) {
+  auto expand_all = [&](auto sum_c, FragT (&a)[FA][DA], FragT (&b)[FB][DB]) {
+    constexpr bool SUM = decltype(sum_c)::value;
 #pragma unroll
     for (int x = 0; x < FA; ++x) {
-      if (CONV) {
+      if (CONV && SUM) {
 #pragma unroll
         for (int pl = 0; pl < PA; ++pl) psum[x][pl] += __popc(wA[x][pl]);
       }
@@ -1303,11 +1396,13 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
     }
 #pragma unroll
     for (int y = 0; y < FB; ++y) {
-      if (!CONV) {
+      if (!CONV && SUM) {
 #pragma unroll
         for (int pl = 0; pl < PB; ++pl) psum[y][pl] += __popc(wB[y][pl]);
       }
-      if constexpr (F4) {
+      if constexpr (SIGNED1) {
+        b[y][0] = expand_sign<DIG>(wB[y][0]);
+      } else if constexpr (F4) {
         static_for<0, DB>([&](auto dc) { b[y][decltype(dc)::value] = expand_digit<DIG, PB, decltype(dc)::value>(wB[y]); });
       } else {
         b[y][0] = expand_planes<PB>(wB[y], rotB);
@@ -1323,7 +1418,11 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
           static_for<0, DA>([&](auto dac) {
             static_for<0, DB>([&](auto dbc) {
               constexpr int da = decltype(dac)::value, db = decltype(dbc)::value;
-              acc[x][y] = mfma_digits<DIG, da + db>(af[x][da], bf[y][db], acc[x][y]);
+              if constexpr (LP) {
+                acc[x][y] = mfma_digits<DIG, da + db>(bf[y][db], af[x][da], acc[x][y]);
+              } else {
+                acc[x][y] = mfma_digits<DIG, da + db>(af[x][da], bf[y][db], acc[x][y]);
+              }
             });
           });
         } else {
@@ -1350,6 +1449,15 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
 #pragma unroll
       for (int d = 0; d < GD; ++d) {
         if (gb + d * GSTEP < ngroups) {  // same for the whole wave
+          if constexpr (LP) {
+            // (unsigned one-plane or symmetric wider weights; one test per group of VW k-steps)
+            if (need_sum) {
+#pragma unroll
+              for (int pl = 0; pl < PA; ++pl)
+#pragma unroll
+                for (int i = 0; i < VW; ++i) psum[0][pl] += __popc(ga[d][pl][i]);
+            }
+          }
 #pragma unroll
           for (int i = 0; i < VW; ++i) {
 #pragma unroll
@@ -1358,18 +1466,14 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
             for (int y = 0; y < FB; ++y)
 #pragma unroll
               for (int pl = 0; pl < PB; ++pl) wB[y][pl] = gbw[d][y][pl][i];
-            expand_all(af, bf);
+            expand_all(std::integral_constant<bool, !LP>{}, af, bf);
             mfma_all();
           }
         }
       }
     }
   };
-  if constexpr (DIRECT_K) {
-    direct_loop();
-  } else if (direct_k) {
-    if constexpr (DIRECT_OPT) direct_loop();
-  } else {
+  auto k_loop = [&](auto sum_c) {
   const int nchunks = (p.KW + KC - 1) / KC;
   using Set0 = std::integral_constant<int, 0>;
   using Set1 = std::integral_constant<int, PF - 1>;
@@ -1377,13 +1481,14 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
   // (a fetch past the end of K is issued all the same, with every load disabled: the number of loads in
   // flight is then the same on every path, and the compiler's wait counts stay exact)
   fetch(0, Set0{});
+  if constexpr (LP) table.store(p, b0, tab, inv_vs);
   stage(smem, Set0{});
   if (PF == 2 || nchunks > 1) fetch(KC, Set0{});
   if (PF == 2) fetch(2 * KC, Set1{});
   __syncthreads();
   if constexpr (KS == 1) {
     read_words(smem, kq);
-    expand_all(af, bf);
+    expand_all(sum_c, af, bf);
   }
   // one chunk; par = ch % 2 is a compile-time constant (LDS buffer and register set of the iteration)
   auto chunk_body = [&](int ch, auto par_c) {
@@ -1406,7 +1511,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
 #pragma unroll
       for (int ks = 0; ks < NKS / KS; ++ks) {
         read_words(cur, wave + ks * KS);
-        expand_all(af, bf);
+        expand_all(sum_c, af, bf);
         mfma_all();
       }
       __syncthreads();
@@ -1414,7 +1519,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
     }
     auto advance = [&]() {
       FragT an[FA][DA], bn[FB][DB];
-      expand_all(an, bn);
+      expand_all(sum_c, an, bn);
 #pragma unroll
       for (int x = 0; x < FA; ++x)
 #pragma unroll
@@ -1473,6 +1578,16 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
   } else {
     for (int ch = 0; ch < nchunks; ++ch) chunk_body(ch, ch & 1);
   }
+  };
+  if constexpr (DIRECT_K) {
+    direct_loop();
+  } else if (direct_k) {
+    if constexpr (DIRECT_OPT) direct_loop();
+  } else if constexpr (LP) {
+    // with and without activation sums: the loop carries no test
+    if (need_sum) k_loop(std::true_type{}); else k_loop(std::false_type{});
+  } else {
+    k_loop(std::true_type{});
   }
   int ssum[FS];
 #pragma unroll
@@ -1484,7 +1599,139 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
     ssum[x] = t;
   }
 
-  if constexpr (KSX == 1) {
+  if constexpr (LP) {
+    // fp32 form of the activation-sum term, in accumulator units
+    const float sum_scale = SIGNED1 ? 1.0f / (float)VSC : -(float)p.wmax * inv_vs;
+    const int cb = b0 + wb * FB * 32;
+    auto block_access = [](const auto &a) {
+      return [&a](auto xc, auto yc, auto ic) { return (float)a[decltype(xc)::value][decltype(yc)::value][decltype(ic)::value]; };
+    };
+    auto add_sum = [&](v16f &a, int sum) {
+      const float c = (float)sum * sum_scale;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) a[r] += c;
+    };
+    if constexpr (KS > 1) {
+      // Split-K: the partial blocks meet in LDS in the accumulator's own register layout (16 bytes per lane and
+      // register quad); each wave then finishes FB of the tile's 4 * FB quads (8 channels of all 32 pixels each):
+      // a whole packed word of every pixel with FB = 4, half of one with 2, a byte with 1.
+      if (fold) fold_shortcut_lanes<1, FB>(p, acc, sc, lane, log2vs);
+      __syncthreads();  // the staging buffers are free, the table is complete
+      float4 *part = reinterpret_cast<float4 *>(smem);                 // [KS][FB][4 quads][64 lanes]
+      int *sums = reinterpret_cast<int *>(smem) + KS * FB * 4 * 64 * 4;  // [KS][32]
+      static_for<0, FB>([&](auto yc) {
+        constexpr int y = decltype(yc)::value;
+        static_for<0, 4>([&](auto qc) {
+          constexpr int q = decltype(qc)::value;
+          float4 v;
+          v.x = acc[0][y][4 * q];
+          v.y = acc[0][y][4 * q + 1];
+          v.z = acc[0][y][4 * q + 2];
+          v.w = acc[0][y][4 * q + 3];
+          part[((wave * FB + y) * 4 + q) * 64 + lane] = v;
+        });
+      });
+      if (need_sum && g == 0) sums[wave * 32 + li] = ssum[0];
+      __syncthreads();
+      const int first = wave * FB;  // first quad of this wave, over (channel block, quad)
+      const int yb = first >> 2, q0 = first & 3;
+      float own[4 * FB];
+      static_for<0, FB>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        float4 t = part[(first + q) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < KS; ++w) {
+          const float4 u = part[(w * FB * 4 + first + q) * 64 + lane];
+          t.x += u.x;
+          t.y += u.y;
+          t.z += u.z;
+          t.w += u.w;
+        }
+        own[4 * q] = t.x;
+        own[4 * q + 1] = t.y;
+        own[4 * q + 2] = t.z;
+        own[4 * q + 3] = t.w;
+      });
+      if (need_sum) {
+        int t = 0;
+#pragma unroll
+        for (int w = 0; w < KS; ++w) t += sums[w * 32 + li];
+        const float c = (float)t * sum_scale;
+#pragma unroll
+        for (int i = 0; i < 4 * FB; ++i) own[i] += c;
+      }
+      conv_output<1, 1, FB, TB, MAXB>(
+          p, [&](auto, auto, auto ic) { return own[decltype(ic)::value]; }, vs, tab, a0, b0 + yb * 32, b0, q0, lane);
+    } else if constexpr (KSX == 1) {
+      if (fold) {
+        if (EPI_LAZY) conv_shortcut_load<FA, FB>(p, own_rbase, cb, li, sc);
+        fold_shortcut_lanes<FA, FB>(p, acc, sc, lane, log2vs);
+      }
+      if (need_sum) {
+#pragma unroll
+        for (int x = 0; x < FA; ++x)
+#pragma unroll
+          for (int y = 0; y < FB; ++y) add_sum(acc[x][y], ssum[x]);
+      }
+      // (short reductions without staging have not met a barrier since the table was written)
+      if (direct_k) __syncthreads();
+      conv_output<FA, FB, 4, TB, MAXB>(p, block_access(acc), vs, tab, own_rbase, cb, b0, 0, lane);
+    } else {
+      // Two wave groups: see below; group 0 finishes the first HA pixel blocks of every wave tile, group 1 the last
+      static_assert(KSX == 2, "two wave groups");
+      __syncthreads();
+      float4 *xch = reinterpret_cast<float4 *>(smem);                        // [8 waves][HA][FB][4 quads][64 lanes]
+      int *xsum = reinterpret_cast<int *>(smem) + 8 * HA * FB * 4 * 64 * 4;  // [8 waves][FA][64 lanes]
+      auto quads = [&](auto f) {
+        static_for<0, HA>([&](auto xc) {
+          static_for<0, FB>([&](auto yc) { static_for<0, 4>([&](auto qc) { f(xc, yc, qc); }); });
+        });
+      };
+      auto give = [&](auto first_c) {
+        constexpr int first = decltype(first_c)::value;
+        quads([&](auto xc, auto yc, auto qc) {
+          constexpr int x = decltype(xc)::value, y = decltype(yc)::value, q = decltype(qc)::value;
+          float4 v;
+          v.x = acc[first + x][y][4 * q];
+          v.y = acc[first + x][y][4 * q + 1];
+          v.z = acc[first + x][y][4 * q + 2];
+          v.w = acc[first + x][y][4 * q + 3];
+          xch[(((wave * HA + x) * FB + y) * 4 + q) * 64 + lane] = v;
+        });
+      };
+      if (kq == 0) give(std::integral_constant<int, HA>{}); else give(std::integral_constant<int, 0>{});
+      if (need_sum) {
+#pragma unroll
+        for (int x = 0; x < FA; ++x) xsum[(wave * FA + x) * 64 + lane] = ssum[x];
+      }
+      __syncthreads();
+      const int partner = wave ^ 4;
+      v16f own[HA][FB];
+      auto take = [&](auto first_c) {
+        constexpr int first = decltype(first_c)::value;
+        quads([&](auto xc, auto yc, auto qc) {
+          constexpr int x = decltype(xc)::value, y = decltype(yc)::value, q = decltype(qc)::value;
+          const float4 v = xch[(((partner * HA + x) * FB + y) * 4 + q) * 64 + lane];
+          own[x][y][4 * q] = acc[first + x][y][4 * q] + v.x;
+          own[x][y][4 * q + 1] = acc[first + x][y][4 * q + 1] + v.y;
+          own[x][y][4 * q + 2] = acc[first + x][y][4 * q + 2] + v.z;
+          own[x][y][4 * q + 3] = acc[first + x][y][4 * q + 3] + v.w;
+        });
+      };
+      if (kq == 0) take(std::integral_constant<int, 0>{}); else take(std::integral_constant<int, HA>{});
+      if (need_sum) {
+#pragma unroll
+        for (int x = 0; x < HA; ++x) {
+          const int idx = kq * HA + x;
+          const int t = xsum[(wave * FA + idx) * 64 + lane] + xsum[(partner * FA + idx) * 64 + lane];
+#pragma unroll
+          for (int y = 0; y < FB; ++y) add_sum(own[x][y], t);
+        }
+      }
+      if (fold) fold_shortcut_lanes<HA, FB>(p, own, sc, lane, log2vs);
+      conv_output<HA, FB, 4, TB, MAXB>(p, block_access(own), vs, tab, own_rbase, cb, b0, 0, lane);
+    }
+  } else if constexpr (KSX == 1) {
     epi_finish<FSC, KS, CONV, (CONV ? PA : PB) >= 3 ? 4 : 2, EPI_LAZY>(p, acc, ssum, smem, wave, lane, a0, b0, wa, wb, eo);
   } else {
     // The two wave groups hold partial sums over their k-steps for the same outputs.  Group 0 finishes the
@@ -1552,6 +1799,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
 
 constexpr size_t mfma_smem_bytes(int core, int PA, int PB, int FA, int FB, int WA, int WB, bool conv, int vw,
                                  int ksx = 1) {
+  if (conv && core == CORE_F4) return mfma_lp_stage_words(PA, PB, FA, FB, WA, WB, vw, ksx) * sizeof(uint32_t);
   const size_t ld = mfma_chunk_words(PA, PB, FA, FB, WA, WB, conv, vw, ksx) + 1;
   // FP4 split-K tiles with 128-bit loads stage nothing (operands go from global memory to registers)
   const size_t stage = core == CORE_F4 && WA * WB == 1 && vw == 4
@@ -1575,15 +1823,19 @@ template <int CORE, int PA, int PB, int FA, int FB, int WA, int WB, int VW, bool
 inline hipError_t launch_mfma(const KParams &p, hipStream_t stream) {
   constexpr int TA = WA * FA * 32, TB = WB * FB * 32;
   constexpr size_t smem_bytes = mfma_smem_bytes(CORE, PA, PB, FA, FB, WA, WB, CONV, VW, KSX);
-  constexpr int OCC_FIT = (int)((160 * 1024) / smem_bytes);
+  constexpr bool LP = CONV && CORE == CORE_F4;
+  constexpr size_t most_bytes = smem_bytes + (LP ? conv_table_words(PA >= 3 ? 4 : 2, TB) * sizeof(uint32_t) : 0);
+  constexpr int OCC_FIT = (int)((160 * 1024) / most_bytes);
   constexpr int OCC = OCC_FIT < 1 ? 1 : (OCC_FIT < OCC_WANTED ? OCC_FIT : OCC_WANTED);
-  static_assert(smem_bytes * OCC <= 160 * 1024, "LDS budget of a gfx950 compute unit");
+  static_assert(smem_bytes + (LP ? (conv_table_words(4, TB) + 4) * 4 + 64 * 256 * KSX : 0) <= 160 * 1024, "LDS budget of a gfx950 compute unit");
   auto kern = apnn_mfma_kernel<CORE, PA, PB, FA, FB, WA, WB, VW, CONV, OCC, KSX>;
-  if (smem_bytes > 64 * 1024) {
+  const size_t launch_bytes = smem_bytes + (LP ? conv_epilogue_bytes(p, TB, 256 * KSX, PA >= 3 ? 4 : 2) : 0);
+  constexpr size_t attr_bytes = smem_bytes + (LP ? (conv_table_words(4, TB) + 4) * 4 + 64 * 256 * KSX : 0);
+  if (attr_bytes > 64 * 1024) {
     static bool raised = false;  // per instantiation; a repeated call is harmless
     if (!raised) {
       const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_bytes);
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)attr_bytes);
       if (e != hipSuccess) return e;
       raised = true;
     }
@@ -1595,8 +1847,8 @@ inline hipError_t launch_mfma(const KParams &p, hipStream_t stream) {
   // before the L2s matter, and the regrouping costs every work-group two scalar divisions)
   const long long tilesB = (p.rowsB + TB - 1) / TB;
   q.xcd_rows = (p.pair_tiles == 0 && tiles % 8 == 0 && tiles >= kXcdOrderMinTiles && tilesB >= 2) ? 8 : 0;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(q.pair_tiles != 0 ? 2 * tiles : tiles)), dim3(256 * KSX), smem_bytes, stream,
-                     q);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(q.pair_tiles != 0 ? 2 * tiles : tiles)), dim3(256 * KSX), launch_bytes,
+                     stream, q);
   return hipGetLastError();
 }
 

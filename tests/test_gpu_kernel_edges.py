@@ -71,3 +71,32 @@ def test_small_products_of_precisions_without_popcount_kernel(G, wb, xb, M, N, K
     rng = np.random.default_rng(8400 + M + wb + xb)
     W, X = O.random_planes(rng, wb, M, K // 32), O.random_planes(rng, xb, N, K // 32)
     assert np.array_equal(G.run_gemm(W, X, M, N, K, wb, xb).reshape(M, N), O.gemm(W, X, M, N, K, wb, xb))
+
+
+# The convolution output stage with pixels in the lanes: codes of one to four bits, flip flags, shortcut scales that
+# are one or two terms m * 2^j (m up to 15) and one that is not, pixel rows and channels that end inside a tile.
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 7, 8, 9])
+@pytest.mark.parametrize("xb,ob,scale", [(2, 2, 43), (2, 1, -171), (2, 3, 0), (3, 3, 203), (4, 4, 1365), (3, 2, 0), (4, 1, 15)])
+@pytest.mark.parametrize("sym", [0, 1])
+def test_conv_codes_flips_and_shortcuts(G, tile, xb, ob, scale, sym):
+    rng = np.random.default_rng(8500 + tile + 10 * xb + ob)
+    batch, H, C, cout = 3, 7, 128, 96
+    W, X = O.random_planes(rng, 1, cout * 9, C // 32), O.random_planes(rng, xb, batch * H * H, C // 32)
+    kw = dict(batch=batch, H=H, W=H, cout=cout, R=3, S=3, stride=1, pad=1, halo=0, wb=1, xb=xb)
+    v = O.conv(W, X, cwords=C // 32, sym_w=sym, **kw).reshape(-1, cout).astype(np.int64)
+    extra = {}
+    if scale:
+        short = rng.integers(0, 4, size=v.shape).astype(np.uint32)
+        v = v + scale * short.astype(np.int64)
+        d_short = G.to_dev(O.pack_bits(short, v.shape[0], cout, cout, 2))
+        extra = dict(resid_planes=d_short, resid_bits=2, resid_scale=scale)
+    thr = np.sort(rng.integers(v.min() - 5, v.max() + 6, size=(cout, 2 ** ob - 1)), axis=1).astype(np.int32)
+    thr[0, :] = np.iinfo(np.int32).min
+    thr[1, :] = np.iinfo(np.int32).max
+    flip = rng.integers(0, 2, size=cout).astype(np.uint8)
+    thr[flip != 0] = np.sort(-thr[flip != 0].astype(np.int64), axis=1).clip(-2 ** 31, 2 ** 31 - 1).astype(np.int32)
+    d_thr, d_flip = G.to_dev(thr), G.to_dev(flip)
+    epi = G.epilogue(mode=G.A.EPI_BN, out_bits=ob, thr=d_thr, flip=d_flip, **extra)
+    got = G.run_conv(W, X, cin_pad=C, sym=sym, epi=epi, path=2, tile=tile, **kw).view(np.uint32).reshape(ob, -1, cout // 32)
+    q = O.bn_quantize(v.astype(np.int32), None, thr, flip, ob)
+    assert np.array_equal(got, O.lowbits_pack(q, v.shape[0], cout, ob))
