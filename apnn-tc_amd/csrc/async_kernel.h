@@ -1,0 +1,297 @@
+// Large matrix products on FP4 / FP6 operands (GEMM entry points, tile 256x128): arithmetic and output stage of
+// mfma_kernel.h, another operand supply.
+//
+// What bounds it.  One 32x32x64 matrix instruction takes 32 clocks of a SIMD; measured with register-only loops, two
+// waves per SIMD hide up to six vector operations behind each (33 clocks per instruction), seven cost 36, eight 39,
+// and a wave alone pays eight clocks for every vector operation beyond four.  The vector operations per matrix
+// instruction are therefore what counts, and everything that is not expansion leaves the loop:
+//   - packed words go from global memory to LDS without passing registers (buffer_load ... lds, 16 bytes per lane),
+//     one chunk ahead of the products; a row's offset is computed once, the chunk is the scalar offset;
+//   - a lane reads four k-steps of a row with one 128-bit LDS read.  K is cut into groups of eight words, the lower
+//     lane half takes the first four, the upper the last four, for both operands alike (a permutation of the terms
+//     of each dot product);
+//   - symmetric one-plane weights are -1 / +1 operands and unsigned ones need no correction, so nothing is counted
+//     (wider symmetric weights: activation sums, as in mfma_kernel.h);
+//   - the last k-step of a chunk carries the barrier, and expands the first operands of the next chunk.
+// w1a2: 6.1 vector operations per matrix instruction instead of 6.75 plus staging, 212 registers.  8192^3 w1a2 229 ->
+// 221 us: the matrix pipes are busy 65 % of the time at the 1.85 GHz that the card holds under this load (2.2 GHz
+// where they are less busy).  4096^3 w1a4 58.2 -> 45.2 us (48.0 with FP6 digits alone): one round of tiles, whose
+// 67 MB of results leave the chip after the last product.
+//
+// LDS rows are KC words (64 or 32 bytes) without padding, as the loads fill them in lane order; the 16-byte units of a
+// row are permuted by its index so that any eight consecutive rows read from eight different bank groups.
+#pragma once
+#include "mfma_kernel.h"
+
+namespace apnn {
+
+typedef int rsrc4 __attribute__((ext_vector_type(4)));
+
+// words per row and chunk: the addresses a load may write (both buffers) stay below 64 KiB
+constexpr int async_chunk_words(int PA, int PB, int TA, int TB) {
+  return 2 * (PA * TA + PB * TB) * 16 * 4 <= 64 * 1024 ? 16 : 8;
+}
+
+template <int PA, int PB, int FA, int FB, int WA, int WB, bool SYM, int OCC>
+__global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) {
+  KParams p = pk;
+  static_assert(WA * WB == 4, "four waves tile the output");
+  constexpr int DIG = digit_planes(PA, PB);
+  constexpr int DA = (PA + DIG - 1) / DIG, DB = (PB + DIG - 1) / DIG;
+  constexpr bool SIGN = SYM && PA == 1;  // -1 / +1 operands: the accumulator is the result
+  constexpr bool SUM = SYM && PA > 1;    // activation sums enter the result
+  constexpr int FSC = SIGN ? (DIG == 4 ? 8 : 2) : fp_scale(PA, PB);
+  if (!SUM) p.sym = 0;
+  constexpr int TA = WA * FA * 32, TB = WB * FB * 32;
+  constexpr int KC = async_chunk_words(PA, PB, TA, TB);
+  constexpr int UPR = KC / 4, RPI = 64 / UPR;  // 16-byte units per row of a chunk, rows per load instruction
+  constexpr int NG = KC / 8;                   // groups of four k-steps
+  constexpr int RA = TA / RPI, RB = TB / RPI;  // row groups
+  static_assert(RA % 4 == 0 && RB % 4 == 0, "row groups go round the four waves");
+  constexpr int NA = RA / 4, NB = RB / 4;
+  constexpr int BUF = (PA * TA + PB * TB) * KC;  // words
+  extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 31, g = lane >> 5;
+  const int wa = wave / WB, wb = wave % WB;
+
+  const int bid = blockIdx.x;
+  const int tilesB = (p.rowsB + TB - 1) / TB;
+  int trow = bid / tilesB, tcol = bid % tilesB;
+  if (p.xcd_rows > 0) {
+    const int tilesA = (p.rowsA + TA - 1) / TA;
+    const int per_xcd = (tilesA * tilesB) >> 3;
+    const int lin = (bid & 7) * per_xcd + (bid >> 3);
+    const int per_band = p.xcd_rows * tilesB;
+    const int band = lin / per_band, w = lin - band * per_band;
+    const int rows_in_band = min(p.xcd_rows, tilesA - band * p.xcd_rows);
+    tcol = w / rows_in_band;
+    trow = band * p.xcd_rows + (w - tcol * rows_in_band);
+  }
+  const int a0 = trow * TA, b0 = tcol * TB;
+
+  auto resource = [](const uint32_t *base, long long words) {
+    const unsigned long long a = reinterpret_cast<unsigned long long>(base);
+    return rsrc4{(int)(uint32_t)a, (int)(uint32_t)((a >> 32) & 0xffffu), (int)(uint32_t)(words * 4), 0x00020000};
+  };
+  rsrc4 rsA[PA], rsB[PB];
+#pragma unroll
+  for (int pl = 0; pl < PA; ++pl) rsA[pl] = resource(p.A + pl * p.planeA, p.planeA);
+#pragma unroll
+  for (int pl = 0; pl < PB; ++pl) rsB[pl] = resource(p.B + pl * p.planeB, p.planeB);
+
+  // lane l of a load instruction fills the 16 bytes at 16 * l of a row group: row l / UPR, unit place l % UPR
+  const int lrow = lane / UPR;
+  const int unit = (lane % UPR) ^ (UPR == 4 ? (lrow >> 1) & 3 : (lrow >> 2) & 1);
+  uint32_t voA[NA], voB[NB];
+#pragma unroll
+  for (int n = 0; n < NA; ++n) {
+    const int row = a0 + (wave + 4 * n) * RPI + lrow;
+    voA[n] = row < p.rowsA ? ((uint32_t)row * (uint32_t)p.KW + 4u * unit) * 4u : 0xffffffffu;
+  }
+#pragma unroll
+  for (int n = 0; n < NB; ++n) {
+    const int row = b0 + (wave + 4 * n) * RPI + lrow;
+    voB[n] = row < p.rowsB ? ((uint32_t)row * (uint32_t)p.KW + 4u * unit) * 4u : 0xffffffffu;
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t *)smem;
+  // (m0 holds the LDS address; the compiler keeps nothing in it across statements)
+  auto load_lds = [](uint32_t lds, uint32_t voff, rsrc4 rs, uint32_t soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds), "v"(voff), "s"(rs), "s"(soff)
+                 : "memory");
+  };
+  auto fetch = [&](int ch, int buf) {
+    const bool ok = ch * KC + 4 * unit < p.KW;
+    const uint32_t soff = (uint32_t)(ch * KC * 4);
+    const uint32_t base = lds0 + (uint32_t)(buf * BUF * 4);
+#pragma unroll
+    for (int n = 0; n < NA; ++n) {
+      const uint32_t vo = ok ? voA[n] : 0xffffffffu;
+#pragma unroll
+      for (int pl = 0; pl < PA; ++pl) load_lds(base + (uint32_t)((pl * TA + (wave + 4 * n) * RPI) * KC * 4), vo, rsA[pl], soff);
+    }
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      const uint32_t vo = ok ? voB[n] : 0xffffffffu;
+#pragma unroll
+      for (int pl = 0; pl < PB; ++pl)
+        load_lds(base + (uint32_t)((PA * TA + pl * TB + (wave + 4 * n) * RPI) * KC * 4), vo, rsB[pl], soff);
+    }
+  };
+  // the loads above are invisible to the compiler's wait counts; a disabled one writes zeros
+  auto arrive = [&]() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  };
+
+  const int nchunks = (p.KW + KC - 1) / KC;
+  fetch(0, 0);
+
+  v16f acc[FA][FB];
+#pragma unroll
+  for (int x = 0; x < FA; ++x)
+#pragma unroll
+    for (int y = 0; y < FB; ++y)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[x][y][r] = 0;
+  int psum[FB][PB];
+#pragma unroll
+  for (int y = 0; y < FB; ++y)
+#pragma unroll
+    for (int pl = 0; pl < PB; ++pl) psum[y][pl] = 0;
+
+  // four k-steps of words of this lane's rows (lower lane half: the first four words of a group, upper: the last four)
+  uint4 qA[FA][PA], qB[FB][PB];
+  const int rowA = wa * FA * 32 + li, rowB = wb * FB * 32 + li;
+  const int swz = UPR == 4 ? (li >> 1) & 3 : (li >> 2) & 1;
+  auto read_group = [&](const uint32_t *buf, auto jc) {
+    constexpr int j = decltype(jc)::value;
+    const int place = ((2 * j + g) ^ swz) * 4;
+#pragma unroll
+    for (int x = 0; x < FA; ++x)
+#pragma unroll
+      for (int pl = 0; pl < PA; ++pl)
+        qA[x][pl] = *reinterpret_cast<const uint4 *>(buf + (pl * TA + rowA + x * 32) * KC + place);
+#pragma unroll
+    for (int y = 0; y < FB; ++y)
+#pragma unroll
+      for (int pl = 0; pl < PB; ++pl)
+        qB[y][pl] = *reinterpret_cast<const uint4 *>(buf + (PA * TA + pl * TB + rowB + y * 32) * KC + place);
+  };
+  v8i af[FA][DA], bf[FB][DB];
+  auto word = [](const uint4 &q, auto ic) -> uint32_t {
+    constexpr int i = decltype(ic)::value;
+    return i == 0 ? q.x : i == 1 ? q.y : i == 2 ? q.z : q.w;
+  };
+  auto expand_into = [&](auto ic, v8i (&a)[FA][DA], v8i (&b)[FB][DB]) {
+#pragma unroll
+    for (int x = 0; x < FA; ++x) {
+      uint32_t w[PA];
+#pragma unroll
+      for (int pl = 0; pl < PA; ++pl) w[pl] = word(qA[x][pl], ic);
+      if constexpr (SIGN) {
+        a[x][0] = expand_sign<DIG>(w[0]);
+      } else {
+        static_for<0, DA>([&](auto dc) { a[x][decltype(dc)::value] = expand_digit<DIG, PA, decltype(dc)::value>(w); });
+      }
+    }
+#pragma unroll
+    for (int y = 0; y < FB; ++y) {
+      uint32_t w[PB];
+#pragma unroll
+      for (int pl = 0; pl < PB; ++pl) {
+        w[pl] = word(qB[y][pl], ic);
+        if constexpr (SUM) psum[y][pl] += __popc(w[pl]);
+      }
+      static_for<0, DB>([&](auto dc) { b[y][decltype(dc)::value] = expand_digit<DIG, PB, decltype(dc)::value>(w); });
+    }
+  };
+  auto mfma_all = [&]() {
+#pragma unroll
+    for (int x = 0; x < FA; ++x)
+#pragma unroll
+      for (int y = 0; y < FB; ++y)
+        static_for<0, DA>([&](auto dac) {
+          static_for<0, DB>([&](auto dbc) {
+            constexpr int da = decltype(dac)::value, db = decltype(dbc)::value;
+            acc[x][y] = mfma_digits<DIG, da + db>(af[x][da], bf[y][db], acc[x][y]);
+          });
+        });
+  };
+  constexpr int N_MFMA = FA * FB * DA * DB;
+  constexpr int XDIG[5] = {0, 7, 10, 18, 22};
+  constexpr int XA = XDIG[DIG] * (PA / DIG) + XDIG[PA % DIG], XB = XDIG[DIG] * (PB / DIG) + XDIG[PB % DIG];
+  constexpr int N_VALU = FA * XA + FB * (XB + (SUM ? PB : 0));
+  constexpr int VALU_PER_MFMA = (N_VALU + N_MFMA - 1) / N_MFMA;
+  // matrix products of one k-step and, between them, the expansion of the next
+  auto step = [&](auto ic) {
+    v8i an[FA][DA], bn[FB][DB];
+    mfma_all();
+    expand_into(ic, an, bn);
+#pragma unroll
+    for (int x = 0; x < FA; ++x)
+#pragma unroll
+      for (int d = 0; d < DA; ++d) af[x][d] = an[x][d];
+#pragma unroll
+    for (int y = 0; y < FB; ++y)
+#pragma unroll
+      for (int d = 0; d < DB; ++d) bf[y][d] = bn[y][d];
+#pragma unroll
+    for (int i = 0; i < N_MFMA; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, VALU_PER_MFMA, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I3 = std::integral_constant<int, 3>;
+
+  arrive();
+  if (nchunks > 1) fetch(1, 1);
+  read_group(smem, I0{});
+  expand_into(I0{}, af, bf);
+#pragma unroll 1
+  for (int ch = 0; ch < nchunks; ++ch) {
+    const uint32_t *cur = smem + (ch & 1) * BUF;
+    step(I1{});
+    step(I2{});
+    step(I3{});
+    if constexpr (NG == 2) {
+      if (ch * KC + 8 < p.KW) {
+        read_group(cur, I1{});
+        step(I0{});
+        step(I1{});
+        step(I2{});
+        step(I3{});
+      }
+    }
+    // every wave holds its last words of this chunk in registers, the next chunk has arrived (after the last chunk the
+    // words read here are stale: their operands meet no product, their sums are taken back below)
+    if (ch + 1 < nchunks) {
+      arrive();
+      if (ch + 2 < nchunks) fetch(ch + 2, ch & 1);
+    }
+    read_group(smem + ((ch + 1) & 1) * BUF, I0{});
+    step(I0{});
+  }
+  int ssum[FB];
+#pragma unroll
+  for (int y = 0; y < FB; ++y) {
+    int t = 0;
+    if constexpr (SUM) {
+#pragma unroll
+      for (int pl = 0; pl < PB; ++pl) t += (psum[y][pl] - __popc(qB[y][pl].x)) << pl;
+      t += __shfl_xor(t, 32, 64);
+    }
+    ssum[y] = t;
+  }
+  EpiOperands<FA, FB> eo;
+  epi_prefetch<1, PB >= 3 ? 4 : 2, true>(p, a0 + wa * FA * 32, b0 + wb * FB * 32, lane, eo);
+  epi_finish<FSC, 1, false, PB >= 3 ? 4 : 2, true>(p, acc, ssum, smem, wave, lane, a0, b0, wa, wb, eo);
+}
+
+template <int PA, int PB, int FA, int FB, int WA, int WB, int OCC>
+inline hipError_t launch_async(const KParams &p, hipStream_t stream) {
+  constexpr int TA = WA * FA * 32, TB = WB * FB * 32;
+  constexpr int KC = async_chunk_words(PA, PB, TA, TB);
+  constexpr size_t slab = 4ull * (32 * (FB * 32 + 1) + 32 + FB * 32 + 2 * 32 * FB) * sizeof(int);
+  constexpr size_t stage = 2ull * (PA * TA + PB * TB) * KC * sizeof(uint32_t);
+  constexpr size_t bytes = stage > slab ? stage : slab;
+  static_assert(bytes <= 64 * 1024, "LDS addresses of the loads fit 16 bits");
+  const long long tilesB = (p.rowsB + TB - 1) / TB, tiles = (long long)((p.rowsA + TA - 1) / TA) * tilesB;
+  KParams q = p;
+  q.xcd_rows = (tiles % 8 == 0 && tiles >= kXcdOrderMinTiles && tilesB >= 2) ? 8 : 0;
+  if (p.sym)
+    hipLaunchKernelGGL((apnn_async_kernel<PA, PB, FA, FB, WA, WB, true, OCC>), dim3((unsigned)tiles), dim3(256), bytes, stream, q);
+  else
+    hipLaunchKernelGGL((apnn_async_kernel<PA, PB, FA, FB, WA, WB, false, OCC>), dim3((unsigned)tiles), dim3(256), bytes, stream, q);
+  return hipGetLastError();
+}
+
+}  // namespace apnn

@@ -1,5 +1,6 @@
 // One translation unit per (INST_CORE, INST_PA, INST_PB, INST_CONV): tile-shape instantiations of
 // the MFMA kernel.  INST_CORE 0 = int8 operands, 1 = FP4 operands.
+#include "async_kernel.h"
 #include "mfma_kernel.h"
 
 #ifndef INST_PA
@@ -27,6 +28,11 @@ hipError_t APNN_CAT(APNN_PFX(conv_), INST_PA, INST_PB, x)(int vw, int tile, cons
 #else
 hipError_t APNN_CAT(APNN_PFX(gemm_), INST_PA, INST_PB, x)(int vw, int tile, const KParams &p, hipStream_t s) {
   (void)vw;
+#if INST_CORE == 1
+  if constexpr (gemm_async_built(INST_PA, INST_PB)) {
+    if (tile == MT_256x128) return launch_async<INST_PA, INST_PB, 4, 2, 2, 2, 2>(p, s);
+  }
+#endif
   return launch_mfma_tile<INST_CORE, INST_PA, INST_PB, 4, false>(tile, p, s);
 }
 #endif

@@ -1854,7 +1854,8 @@ inline hipError_t launch_mfma(const KParams &p, hipStream_t stream) {
 
 template <int CORE, int PA, int PB, int FA, int FB, int WA, int WB, int VW, bool CONV, int OCC, int TILE, int KSX = 1>
 inline hipError_t launch_mfma_if_enabled(const KParams &p, hipStream_t stream) {
-  if constexpr (mfma_tile_enabled(CORE, CONV, VW, TILE, PA, PB)) {
+  if constexpr (mfma_tile_enabled(CORE, CONV, VW, TILE, PA, PB) &&
+                !(CORE == CORE_F4 && !CONV && TILE == MT_256x128 && gemm_async_built(PA, PB))) {
     return launch_mfma<CORE, PA, PB, FA, FB, WA, WB, VW, CONV, OCC, KSX>(p, stream);
   } else {
     return hipErrorNotSupported;

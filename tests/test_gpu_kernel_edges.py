@@ -100,3 +100,16 @@ def test_conv_codes_flips_and_shortcuts(G, tile, xb, ob, scale, sym):
     got = G.run_conv(W, X, cin_pad=C, sym=sym, epi=epi, path=2, tile=tile, **kw).view(np.uint32).reshape(ob, -1, cout // 32)
     q = O.bn_quantize(v.astype(np.int32), None, thr, flip, ob)
     assert np.array_equal(got, O.lowbits_pack(q, v.shape[0], cout, ob))
+
+
+# GEMM tile 256x128 (operands loaded straight to LDS): rows and columns around the tile, reductions of half a group,
+# one group, one chunk and a few words more; -1 / +1, unsigned and two-plane weights.
+@pytest.mark.parametrize("wb,xb", [(1, 1), (1, 2), (1, 3), (1, 4), (2, 2)])
+@pytest.mark.parametrize("sym", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 128), (255, 127, 256), (257, 129, 384), (256, 128, 512), (300, 130, 640),
+                                   (511, 257, 1024), (513, 96, 1152), (40, 300, 2176)])
+def test_async_gemm_tile(G, wb, xb, sym, M, N, K):
+    rng = np.random.default_rng(8400 + M + 10 * wb + xb)
+    W, X = O.random_planes(rng, wb, M, K // 32), O.random_planes(rng, xb, N, K // 32)
+    got = G.run_gemm(W, X, M, N, K, wb, xb, sym=sym, path=2, tile=6).reshape(M, N)
+    assert np.array_equal(got, O.gemm(W, X, M, N, K, wb, xb, sym_w=sym))
