@@ -403,18 +403,27 @@ int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, i
   }
   if (conv && vw == 1) return (ntiles(2) >= cus / 2 || KW < 16) ? 2 : 4;  // 32-bit loads: two tiles built
   // About one 128x128 tile per compute unit over a long reduction (16x16 maps at batch 16 with 1024 channels,
-  // 14x14x256 at batch 64, 2048^2 outputs): plain 128x128 work-groups would leave one wave per SIMD, so two
-  // wave groups share each tile's k-steps.  Measured 11-18 % ahead of the best other tile there; with fewer
-  // tiles than that the idle compute units cost more than the split-K tiles' extra operand traffic.  How
-  // many units may idle depends on what the 32x64 split-K tile costs instead: in convolutions with one
-  // weight plane it stays ahead until 9/10 of the units have a tile (16x16 maps with 640..896 channels;
-  // 14x14x256 at batch 64: 5 % ahead for w1a2 with quantized output, 17 % for w1a3 / w1a4); with two weight
-  // planes, whose expansion the small tiles repeat per 64 channels, and for the GEMM entry points 3/4 suffice
-  // (w2a2 on 16x16 maps: 17 % ahead at 768 channels, 34 % at 896).
+  // 14x14x256 at batch 64, 2048^2 outputs).  GEMM entry points and the wide precisions: a plain work-group leaves one
+  // wave per SIMD, so two wave groups share each tile's k-steps, 11-18 % ahead of the best other tile.
+  // Convolutions of up to five planes: the plain tile loads straight to LDS (async_kernel.h).  The two groups stay
+  // level or ahead over long reductions while one round holds all tiles (16x16x1024 at batch 16: w1a2 24.6 us both,
+  // w1a4 37.8 against 41.6), and lose once there is a second round (14x14x384 at batch 64, 294 tiles: w1a2 23.9
+  // against 17.6 us, w1a4 38.6 against 29.9).  Fewer tiles than compute units: the 32x64 split-K tile holds out below
+  // 9/10 of the units with one weight plane (16x16x768 at batch 16: 18.9 against 19.9 us); with two, whose expansion
+  // the small tiles repeat, 3/4 suffice.  Over at most 128 words the plain tile is ahead of both from 3/4 on
+  // (14x14x256 at batch 64: w1a2 9.6 us against 10.4 for the groups and 11.2 for split-K, w1a4 16.7 against 17.1 and
+  // 17.2, w2a2 10.9 against 11.6 and 12.5).
   if ((!conv || vw == 4) && planes > 2 && KW >= 64 && fill(1) >= 0.8) {
     const long long nt1 = ntiles(1);
-    const bool strict = conv && planesW == 1;
-    if (2 * nt1 < 3 * cus && (strict ? 10 * nt1 >= 9 * cus : 4 * nt1 >= 3 * cus)) return apnn::MT_128x128_G2;
+    if (!conv || wide) {
+      const bool strict = conv && planesW == 1;
+      if (2 * nt1 < 3 * cus && (strict ? 10 * nt1 >= 9 * cus : 4 * nt1 >= 3 * cus)) return apnn::MT_128x128_G2;
+    } else if (2 * nt1 < 3 * cus && 4 * nt1 >= 3 * cus) {
+      const bool most = 10 * nt1 >= 9 * cus;
+      if (KW <= 128) return 1;
+      if ((planesW > 1 || most) && nt1 <= cus) return apnn::MT_128x128_G2;
+      if (planesW > 1 || most) return 1;
+    }
   }
   // Few outputs over a long reduction (batch-1 / batch-8 layers, 7x7 maps): the split-K tiles give
   // every 32x32 (32x64) block a work-group of its own and the four waves share K.  Measured

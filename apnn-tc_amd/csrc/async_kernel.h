@@ -1,5 +1,5 @@
-// Large matrix products on FP4 / FP6 operands (GEMM entry points, tile 256x128): arithmetic and output stage of
-// mfma_kernel.h, another operand supply.
+// Large tiles on FP4 / FP6 operands (GEMM entry points 256x128; convolution 128x256 and 128x128): arithmetic and output
+// stages of mfma_kernel.h and conv_epilogue.h, another operand supply.
 //
 // What bounds it.  One 32x32x64 matrix instruction takes 32 clocks of a SIMD; measured with register-only loops, two
 // waves per SIMD hide up to six vector operations behind each (33 clocks per instruction), seven cost 36, eight 39,
@@ -17,6 +17,11 @@
 // 221 us: the matrix pipes are busy 65 % of the time at the 1.85 GHz that the card holds under this load (2.2 GHz
 // where they are less busy).  4096^3 w1a4 58.2 -> 45.2 us (48.0 with FP6 digits alone): one round of tiles, whose
 // 67 MB of results leave the chip after the last product.
+// Convolution: a load's lane decodes the tap of its 16 bytes once per chunk; padding pixels are disabled loads, which
+// write zeros.  Two tiles of 128x256 per compute unit, three of 128x128.  3x3 convolutions at batch
+// 64: 56x56x256 76 -> 66 us, 28x28x512 78 -> 64, 14x14x512 28 -> 23 (bounded by vector work, 9.8 operations per matrix
+// instruction with the output stage, and by the last round: 784 tiles of 128x256 on 512 places); the VGG variant at
+// batch 64 541 -> 489 us.
 //
 // LDS rows are KC words (64 or 32 bytes) without padding, as the loads fill them in lane order; the 16-byte units of a
 // row are permuted by its index so that any eight consecutive rows read from eight different bank groups.
@@ -32,14 +37,30 @@ constexpr int async_chunk_words(int PA, int PB, int TA, int TB) {
   return 2 * (PA * TA + PB * TB) * 16 * 4 <= 64 * 1024 ? 16 : 8;
 }
 
-template <int PA, int PB, int FA, int FB, int WA, int WB, bool SYM, int OCC>
+template <int PA, int PB, int FA, int FB, int WA, int WB, bool CONV, bool SYM, int OCC>
 __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) {
   KParams p = pk;
+  int bid = blockIdx.x;
+  if (CONV && pk.pair_tiles > 0 && bid >= pk.pair_tiles) {  // paired launch, see apnn_mfma_kernel
+    bid -= pk.pair_tiles;
+    p.B = pk.B2;
+    p.KW = pk.KW2;
+    p.S = pk.S2;
+    p.pad = pk.pad2;
+    p.magicS = pk.magicS2;
+    p.magicS16 = pk.magicS16_2;
+    p.planeB = pk.planeB2;
+    p.thr = pk.thr2;
+    p.flip = pk.flip2;
+    p.out = pk.out2;
+  }
   static_assert(WA * WB == 4, "four waves tile the output");
   constexpr int DIG = digit_planes(PA, PB);
   constexpr int DA = (PA + DIG - 1) / DIG, DB = (PB + DIG - 1) / DIG;
-  constexpr bool SIGN = SYM && PA == 1;  // -1 / +1 operands: the accumulator is the result
-  constexpr bool SUM = SYM && PA > 1;    // activation sums enter the result
+  constexpr int PW = CONV ? PB : PA;     // planes of the weights, of the activations
+  constexpr int PX = CONV ? PA : PB;
+  constexpr bool SIGN = SYM && PW == 1;  // -1 / +1 operands: the accumulator is the result
+  constexpr bool SUM = SYM && PW > 1;    // activation sums enter the result
   constexpr int FSC = SIGN ? (DIG == 4 ? 8 : 2) : fp_scale(PA, PB);
   if (!SUM) p.sym = 0;
   constexpr int TA = WA * FA * 32, TB = WB * FB * 32;
@@ -57,7 +78,6 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
   const int li = lane & 31, g = lane >> 5;
   const int wa = wave / WB, wb = wave % WB;
 
-  const int bid = blockIdx.x;
   const int tilesB = (p.rowsB + TB - 1) / TB;
   int trow = bid / tilesB, tcol = bid % tilesB;
   if (p.xcd_rows > 0) {
@@ -85,10 +105,18 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
   // lane l of a load instruction fills the 16 bytes at 16 * l of a row group: row l / UPR, unit place l % UPR
   const int lrow = lane / UPR;
   const int unit = (lane % UPR) ^ (UPR == 4 ? (lrow >> 1) & 3 : (lrow >> 2) & 1);
-  uint32_t voA[NA], voB[NB];
+  uint32_t voA[NA], voB[NB];  // byte offset of the row's unit (convolution: word offset of the pixel's tap (0, 0), mod 2^32)
+  int y0[NA], x0[NA];
 #pragma unroll
   for (int n = 0; n < NA; ++n) {
     const int row = a0 + (wave + 4 * n) * RPI + lrow;
+    y0[n] = x0[n] = 0;
+    if constexpr (CONV) {
+      int b = 0;
+      pixel_origin(p, row, b, y0[n], x0[n]);
+      voA[n] = (((uint32_t)b * (uint32_t)p.Hs + (uint32_t)y0[n]) * (uint32_t)p.Ws + (uint32_t)x0[n]) * (uint32_t)p.C32;
+      if (row >= p.rowsA) y0[n] = 1 << 30;  // no tap of it lies in the image
+    } else
     voA[n] = row < p.rowsA ? ((uint32_t)row * (uint32_t)p.KW + 4u * unit) * 4u : 0xffffffffu;
   }
 #pragma unroll
@@ -108,11 +136,26 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
     const bool ok = ch * KC + 4 * unit < p.KW;
     const uint32_t soff = (uint32_t)(ch * KC * 4);
     const uint32_t base = lds0 + (uint32_t)(buf * BUF * 4);
+    uint32_t r = 0, sx = 0, toff = 0;
+    if constexpr (CONV) {  // a unit of four words lies within one tap
+      const uint32_t kw0 = (uint32_t)(ch * KC + 4 * unit);
+      const uint32_t tap = p.c32_shift >= 0 ? kw0 >> p.c32_shift : fast_div(kw0, (uint32_t)p.C32, p.magicC32);
+      r = __umul24(tap, p.magicS16) >> 16;
+      sx = tap - __umul24(r, (uint32_t)p.S);
+      toff = __umul24(__umul24(r, (uint32_t)p.Ws) + sx, (uint32_t)p.C32) + kw0 - __umul24(tap, (uint32_t)p.C32);
+    }
 #pragma unroll
     for (int n = 0; n < NA; ++n) {
-      const uint32_t vo = ok ? voA[n] : 0xffffffffu;
+      uint32_t vo;
+      if constexpr (CONV) {
+        const bool in = ok && (uint32_t)(y0[n] + (int)r) < (uint32_t)p.Hs && (uint32_t)(x0[n] + (int)sx) < (uint32_t)p.Ws;
+        vo = in ? (voA[n] + toff) << 2 : 0xffffffffu;
+      } else {
+        vo = ok ? voA[n] : 0xffffffffu;
+      }
 #pragma unroll
-      for (int pl = 0; pl < PA; ++pl) load_lds(base + (uint32_t)((pl * TA + (wave + 4 * n) * RPI) * KC * 4), vo, rsA[pl], soff);
+      for (int pl = 0; pl < PA; ++pl)
+        load_lds(base + (uint32_t)((pl * TA + (wave + 4 * n) * RPI) * KC * 4), vo, rsA[pl], CONV ? 0u : soff);
     }
 #pragma unroll
     for (int n = 0; n < NB; ++n) {
@@ -129,7 +172,21 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
   };
 
   const int nchunks = (p.KW + KC - 1) / KC;
+  // convolution: value per accumulator unit, thresholds of the tile's channels behind the operand buffers
+  constexpr int log2vs = __builtin_ctz(FSC) + (SUM ? 1 : 0);
+  const float inv_vs = 1.0f / (float)(1 << log2vs);
+  uint32_t *tab = smem + 2 * BUF;
+  constexpr int MAXB = PA >= 3 ? 4 : 2;
+  ConvTable<TB, PA >= 3 ? 15 : 3, MAXB> table;
+  if constexpr (CONV) table.load(p, b0);
   fetch(0, 0);
+  const int rbase = a0 + wa * FA * 32, cbase = b0 + wb * FB * 32;
+  constexpr bool LAZY = FA * FB >= 8;
+  uint32_t sc[FA][FB][2];
+  if constexpr (CONV) {
+    if (p.fold != 0u && !LAZY) conv_shortcut_load<FA, FB>(p, rbase, cbase, li, sc);
+    table.store(p, b0, tab, inv_vs);
+  }
 
   v16f acc[FA][FB];
 #pragma unroll
@@ -138,11 +195,12 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
     for (int y = 0; y < FB; ++y)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[x][y][r] = 0;
-  int psum[FB][PB];
+  constexpr int FX = CONV ? FA : FB;
+  int psum[FX][PX];  // activation sums (SUM)
 #pragma unroll
-  for (int y = 0; y < FB; ++y)
+  for (int y = 0; y < FX; ++y)
 #pragma unroll
-    for (int pl = 0; pl < PB; ++pl) psum[y][pl] = 0;
+    for (int pl = 0; pl < PX; ++pl) psum[y][pl] = 0;
 
   // four k-steps of words of this lane's rows (lower lane half: the first four words of a group, upper: the last four)
   uint4 qA[FA][PA], qB[FB][PB];
@@ -172,8 +230,11 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
     for (int x = 0; x < FA; ++x) {
       uint32_t w[PA];
 #pragma unroll
-      for (int pl = 0; pl < PA; ++pl) w[pl] = word(qA[x][pl], ic);
-      if constexpr (SIGN) {
+      for (int pl = 0; pl < PA; ++pl) {
+        w[pl] = word(qA[x][pl], ic);
+        if constexpr (CONV && SUM) psum[x][pl] += __popc(w[pl]);
+      }
+      if constexpr (!CONV && SIGN) {
         a[x][0] = expand_sign<DIG>(w[0]);
       } else {
         static_for<0, DA>([&](auto dc) { a[x][decltype(dc)::value] = expand_digit<DIG, PA, decltype(dc)::value>(w); });
@@ -185,9 +246,13 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
 #pragma unroll
       for (int pl = 0; pl < PB; ++pl) {
         w[pl] = word(qB[y][pl], ic);
-        if constexpr (SUM) psum[y][pl] += __popc(w[pl]);
+        if constexpr (!CONV && SUM) psum[y][pl] += __popc(w[pl]);
       }
-      static_for<0, DB>([&](auto dc) { b[y][decltype(dc)::value] = expand_digit<DIG, PB, decltype(dc)::value>(w); });
+      if constexpr (CONV && SIGN) {
+        b[y][0] = expand_sign<DIG>(w[0]);
+      } else {
+        static_for<0, DB>([&](auto dc) { b[y][decltype(dc)::value] = expand_digit<DIG, PB, decltype(dc)::value>(w); });
+      }
     }
   };
   auto mfma_all = [&]() {
@@ -198,14 +263,18 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
         static_for<0, DA>([&](auto dac) {
           static_for<0, DB>([&](auto dbc) {
             constexpr int da = decltype(dac)::value, db = decltype(dbc)::value;
-            acc[x][y] = mfma_digits<DIG, da + db>(af[x][da], bf[y][db], acc[x][y]);
+            if constexpr (CONV) {
+              acc[x][y] = mfma_digits<DIG, da + db>(bf[y][db], af[x][da], acc[x][y]);
+            } else {
+              acc[x][y] = mfma_digits<DIG, da + db>(af[x][da], bf[y][db], acc[x][y]);
+            }
           });
         });
   };
   constexpr int N_MFMA = FA * FB * DA * DB;
   constexpr int XDIG[5] = {0, 7, 10, 18, 22};
   constexpr int XA = XDIG[DIG] * (PA / DIG) + XDIG[PA % DIG], XB = XDIG[DIG] * (PB / DIG) + XDIG[PB % DIG];
-  constexpr int N_VALU = FA * XA + FB * (XB + (SUM ? PB : 0));
+  constexpr int N_VALU = FA * XA + FB * XB + (SUM ? FX * PX : 0);
   constexpr int VALU_PER_MFMA = (N_VALU + N_MFMA - 1) / N_MFMA;
   // matrix products of one k-step and, between them, the expansion of the next
   auto step = [&](auto ic) {
@@ -260,37 +329,68 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
     read_group(smem + ((ch + 1) & 1) * BUF, I0{});
     step(I0{});
   }
-  int ssum[FB];
+  int ssum[FX];
 #pragma unroll
-  for (int y = 0; y < FB; ++y) {
+  for (int y = 0; y < FX; ++y) {
     int t = 0;
     if constexpr (SUM) {
 #pragma unroll
-      for (int pl = 0; pl < PB; ++pl) t += (psum[y][pl] - __popc(qB[y][pl].x)) << pl;
+      for (int pl = 0; pl < PX; ++pl) t += (psum[y][pl] - __popc((CONV ? qA[CONV ? y : 0][CONV ? pl : 0] : qB[CONV ? 0 : y][CONV ? 0 : pl]).x)) << pl;
       t += __shfl_xor(t, 32, 64);
     }
     ssum[y] = t;
   }
-  EpiOperands<FA, FB> eo;
-  epi_prefetch<1, PB >= 3 ? 4 : 2, true>(p, a0 + wa * FA * 32, b0 + wb * FB * 32, lane, eo);
-  epi_finish<FSC, 1, false, PB >= 3 ? 4 : 2, true>(p, acc, ssum, smem, wave, lane, a0, b0, wa, wb, eo);
+  if constexpr (CONV) {
+    if (p.fold != 0u) {
+      if (LAZY) conv_shortcut_load<FA, FB>(p, rbase, cbase, li, sc);
+      fold_shortcut_lanes<FA, FB>(p, acc, sc, lane, log2vs);
+    }
+    if constexpr (SUM) {
+#pragma unroll
+      for (int x = 0; x < FA; ++x) {
+        const float c = (float)ssum[x] * (-(float)p.wmax * inv_vs);
+#pragma unroll
+        for (int y = 0; y < FB; ++y)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[x][y][r] += c;
+      }
+    }
+    conv_output<FA, FB, 4, TB, MAXB>(
+        p, [&](auto xc, auto yc, auto ic) { return (float)acc[decltype(xc)::value][decltype(yc)::value][decltype(ic)::value]; },
+        (float)(1 << log2vs), tab, rbase, cbase, b0, 0, lane);
+  } else {
+    EpiOperands<FA, FB> eo;
+    epi_prefetch<1, PB >= 3 ? 4 : 2, true>(p, rbase, cbase, lane, eo);
+    epi_finish<FSC, 1, false, PB >= 3 ? 4 : 2, true>(p, acc, ssum, smem, wave, lane, a0, b0, wa, wb, eo);
+  }
 }
 
-template <int PA, int PB, int FA, int FB, int WA, int WB, int OCC>
+template <int PA, int PB, int FA, int FB, int WA, int WB, bool CONV, int OCC>
 inline hipError_t launch_async(const KParams &p, hipStream_t stream) {
   constexpr int TA = WA * FA * 32, TB = WB * FB * 32;
   constexpr int KC = async_chunk_words(PA, PB, TA, TB);
-  constexpr size_t slab = 4ull * (32 * (FB * 32 + 1) + 32 + FB * 32 + 2 * 32 * FB) * sizeof(int);
+  constexpr size_t slab = CONV ? 0 : 4ull * (32 * (FB * 32 + 1) + 32 + FB * 32 + 2 * 32 * FB) * sizeof(int);
   constexpr size_t stage = 2ull * (PA * TA + PB * TB) * KC * sizeof(uint32_t);
   constexpr size_t bytes = stage > slab ? stage : slab;
-  static_assert(bytes <= 64 * 1024, "LDS addresses of the loads fit 16 bits");
+  static_assert(stage <= 64 * 1024, "LDS addresses of the loads fit 16 bits");
+  constexpr int MAXB = PA >= 3 ? 4 : 2;
+  constexpr size_t most = bytes + (CONV ? (conv_table_words(4, TB) + 4) * 4 + 64 * 256 : 0);
+  static_assert(most <= 160 * 1024, "LDS of a compute unit");
+  auto kern = p.sym ? apnn_async_kernel<PA, PB, FA, FB, WA, WB, CONV, true, OCC> : apnn_async_kernel<PA, PB, FA, FB, WA, WB, CONV, false, OCC>;
+  if (most > 64 * 1024) {
+    static bool raised[2] = {false, false};  // a repeated call is harmless
+    if (!raised[p.sym != 0]) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
+      if (e != hipSuccess) return e;
+      raised[p.sym != 0] = true;
+    }
+  }
   const long long tilesB = (p.rowsB + TB - 1) / TB, tiles = (long long)((p.rowsA + TA - 1) / TA) * tilesB;
   KParams q = p;
-  q.xcd_rows = (tiles % 8 == 0 && tiles >= kXcdOrderMinTiles && tilesB >= 2) ? 8 : 0;
-  if (p.sym)
-    hipLaunchKernelGGL((apnn_async_kernel<PA, PB, FA, FB, WA, WB, true, OCC>), dim3((unsigned)tiles), dim3(256), bytes, stream, q);
-  else
-    hipLaunchKernelGGL((apnn_async_kernel<PA, PB, FA, FB, WA, WB, false, OCC>), dim3((unsigned)tiles), dim3(256), bytes, stream, q);
+  if (p.pair_tiles != 0) q.pair_tiles = (int)tiles;
+  q.xcd_rows = (p.pair_tiles == 0 && tiles % 8 == 0 && tiles >= kXcdOrderMinTiles && tilesB >= 2) ? 8 : 0;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(q.pair_tiles != 0 ? 2 * tiles : tiles)), dim3(256),
+                     bytes + (CONV ? conv_epilogue_bytes(p, TB, 256, MAXB) : 0), stream, q);
   return hipGetLastError();
 }
 

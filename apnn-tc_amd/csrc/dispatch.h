@@ -108,8 +108,12 @@ constexpr bool mfma_tile_enabled(int core, bool conv, int vw, int tile, int pa, 
   return tile != MT_256x256 && tile != MT_256x128;
 }
 
-// the FP4 / FP6 GEMM tile 256x128 of these precisions is the kernel of async_kernel.h
-constexpr bool gemm_async_built(int pa, int pb) { return pa + pb <= 5; }
+// FP4 / FP6 tiles that run on the kernel of async_kernel.h (loads straight to LDS)
+constexpr bool async_built(int pa, int pb) { return pa + pb <= 5; }
+constexpr bool async_tile(bool conv, int vw, int tile, int pa, int pb) {
+  if (!async_built(pa, pb)) return false;
+  return conv ? vw == 4 && (tile == MT_128x256 || tile == MT_128x128) : tile == MT_256x128;
+}
 
 // tiles of the kernel that expands operands while staging (mfma_xs_kernel.h), by their MfmaTile index:
 // the shapes whose four waves tile the output; convolution with 128-bit loads only

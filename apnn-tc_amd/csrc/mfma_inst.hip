@@ -19,6 +19,12 @@ namespace apnn {
 
 #if INST_CONV
 hipError_t APNN_CAT(APNN_PFX(conv_), INST_PA, INST_PB, x)(int vw, int tile, const KParams &p, hipStream_t s) {
+#if INST_CORE == 1
+  if constexpr (async_built(INST_PA, INST_PB)) {
+    if (vw == 4 && tile == MT_128x256) return launch_async<INST_PA, INST_PB, 2, 4, 2, 2, true, 2>(p, s);
+    if (vw == 4 && tile == MT_128x128) return launch_async<INST_PA, INST_PB, 2, 2, 2, 2, true, 2>(p, s);
+  }
+#endif
   switch (vw) {
     case 4: return launch_mfma_tile<INST_CORE, INST_PA, INST_PB, 4, true>(tile, p, s);
     case 2: return launch_mfma_tile<INST_CORE, INST_PA, INST_PB, 2, true>(tile, p, s);
@@ -29,8 +35,8 @@ hipError_t APNN_CAT(APNN_PFX(conv_), INST_PA, INST_PB, x)(int vw, int tile, cons
 hipError_t APNN_CAT(APNN_PFX(gemm_), INST_PA, INST_PB, x)(int vw, int tile, const KParams &p, hipStream_t s) {
   (void)vw;
 #if INST_CORE == 1
-  if constexpr (gemm_async_built(INST_PA, INST_PB)) {
-    if (tile == MT_256x128) return launch_async<INST_PA, INST_PB, 4, 2, 2, 2, 2>(p, s);
+  if constexpr (async_built(INST_PA, INST_PB)) {
+    if (tile == MT_256x128) return launch_async<INST_PA, INST_PB, 4, 2, 2, 2, false, 2>(p, s);
   }
 #endif
   return launch_mfma_tile<INST_CORE, INST_PA, INST_PB, 4, false>(tile, p, s);

@@ -1002,6 +1002,37 @@ constexpr int mfma_lp_stage_words(int PA, int PB, int FA, int FB, int WA, int WB
 // longest reduction (32-bit words) the one- and two-block convolution tiles load without staging
 constexpr int kDirectMaxKW = 40;
 
+// output pixel (row of A) -> image index and the input coordinates of its filter tap (0, 0)
+__device__ __forceinline__ void pixel_origin(const KParams &p, int pix, int &b, int &y0, int &x0) {
+  int oy, ox;
+  if (p.geo_fast) {
+    // multiply-high by ceil(2^32 / d) is the exact quotient here (the host checked the range)
+    const int gw = p.pool_order ? p.Wo >> 1 : p.Wo, gh = p.pool_order ? p.Ho >> 1 : p.Ho;
+    const int cell = p.pool_order ? pix >> 2 : pix, sub = pix & 3;
+    const int t = (int)fast_div((uint32_t)cell, (uint32_t)gw, p.magicGW);
+    const int px = cell - t * gw;
+    b = (int)fast_div((uint32_t)t, (uint32_t)gh, p.magicGH);
+    const int py = t - b * gh;
+    oy = p.pool_order ? 2 * py + (sub >> 1) : py;
+    ox = p.pool_order ? 2 * px + (sub & 1) : px;
+  } else if (p.pool_order) {
+    const int win = pix >> 2, sub = pix & 3;
+    const int hw = p.Wo >> 1, hh = p.Ho >> 1;
+    const int px = win % hw, t = win / hw;
+    const int py = t % hh;
+    b = t / hh;
+    oy = 2 * py + (sub >> 1);
+    ox = 2 * px + (sub & 1);
+  } else {
+    ox = pix % p.Wo;
+    const int t = pix / p.Wo;
+    oy = t % p.Ho;
+    b = t / p.Ho;
+  }
+  y0 = oy * p.stride - p.pad;
+  x0 = ox * p.stride - p.pad;
+}
+
 // KSX > 1: KSX groups of four waves each (work-groups of 256 * KSX threads).  Every group tiles the whole
 // output tile WA x WB like the four waves of the other kernels and takes every KSX-th k-step of each
 // staged chunk; after the K loop the groups exchange partial accumulators through LDS so that each group
@@ -1084,37 +1115,6 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
   }
   const int a0 = trow * TA;
   const int b0 = tcol * TB;
-
-  // output pixel (row of A) -> image index and the input coordinates of its filter tap (0, 0)
-  auto pixel_origin = [&](int pix, int &b, int &y0, int &x0) {
-    int oy, ox;
-    if (p.geo_fast) {
-      // multiply-high by ceil(2^32 / d) is the exact quotient here (the host checked the range)
-      const int gw = p.pool_order ? p.Wo >> 1 : p.Wo, gh = p.pool_order ? p.Ho >> 1 : p.Ho;
-      const int cell = p.pool_order ? pix >> 2 : pix, sub = pix & 3;
-      const int t = (int)fast_div((uint32_t)cell, (uint32_t)gw, p.magicGW);
-      const int px = cell - t * gw;
-      b = (int)fast_div((uint32_t)t, (uint32_t)gh, p.magicGH);
-      const int py = t - b * gh;
-      oy = p.pool_order ? 2 * py + (sub >> 1) : py;
-      ox = p.pool_order ? 2 * px + (sub & 1) : px;
-    } else if (p.pool_order) {
-      const int win = pix >> 2, sub = pix & 3;
-      const int hw = p.Wo >> 1, hh = p.Ho >> 1;
-      const int px = win % hw, t = win / hw;
-      const int py = t % hh;
-      b = t / hh;
-      oy = 2 * py + (sub >> 1);
-      ox = 2 * px + (sub & 1);
-    } else {
-      ox = pix % p.Wo;
-      const int t = pix / p.Wo;
-      oy = t % p.Ho;
-      b = t / p.Ho;
-    }
-    y0 = oy * p.stride - p.pad;
-    x0 = ox * p.stride - p.pad;
-  };
 
   // value per accumulator unit; the thresholds of the tile's channels, behind the operand buffers
   const int log2vs = __builtin_ctz(VSC > 0 ? VSC : 1) + (SIGNED1 ? (p.sym ? 0 : -1) : (p.sym ? 1 : 0));
@@ -1213,7 +1213,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
     const int growA = a0 + wa * FA * 32 + li;
     okA = growA < p.rowsA;
     int ab = 0;
-    if (CONV) pixel_origin(growA, ab, ay0, ax0);
+    if (CONV) pixel_origin(p, growA, ab, ay0, ax0);
     baseA = CONV ? (((uint32_t)ab * (uint32_t)p.Hs + (uint32_t)ay0) * (uint32_t)p.Ws + (uint32_t)ax0) * (uint32_t)p.C32
                  : (uint32_t)growA * (uint32_t)p.KW;
 #pragma unroll
@@ -1248,7 +1248,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
     a_ok[it] = (u < UA) && (grow < p.rowsA);
     int ab = 0;
     a_y0[it] = a_x0[it] = 0;
-    if (CONV) pixel_origin(grow, ab, a_y0[it], a_x0[it]);
+    if (CONV) pixel_origin(p, grow, ab, a_y0[it], a_x0[it]);
     a_base[it] = CONV ? (((uint32_t)ab * (uint32_t)p.Hs + (uint32_t)a_y0[it]) * (uint32_t)p.Ws + (uint32_t)a_x0[it]) *
                             (uint32_t)p.C32
                       : (uint32_t)grow * (uint32_t)p.KW;
@@ -1855,7 +1855,7 @@ inline hipError_t launch_mfma(const KParams &p, hipStream_t stream) {
 template <int CORE, int PA, int PB, int FA, int FB, int WA, int WB, int VW, bool CONV, int OCC, int TILE, int KSX = 1>
 inline hipError_t launch_mfma_if_enabled(const KParams &p, hipStream_t stream) {
   if constexpr (mfma_tile_enabled(CORE, CONV, VW, TILE, PA, PB) &&
-                !(CORE == CORE_F4 && !CONV && TILE == MT_256x128 && gemm_async_built(PA, PB))) {
+                !(CORE == CORE_F4 && async_tile(CONV, VW, TILE, PA, PB))) {
     return launch_mfma<CORE, PA, PB, FA, FB, WA, WB, VW, CONV, OCC, KSX>(p, stream);
   } else {
     return hipErrorNotSupported;

@@ -113,3 +113,38 @@ def test_async_gemm_tile(G, wb, xb, sym, M, N, K):
     W, X = O.random_planes(rng, wb, M, K // 32), O.random_planes(rng, xb, N, K // 32)
     got = G.run_gemm(W, X, M, N, K, wb, xb, sym=sym, path=2, tile=6).reshape(M, N)
     assert np.array_equal(got, O.gemm(W, X, M, N, K, wb, xb, sym_w=sym))
+
+
+# Convolution tiles 128x256 and 128x128 (operands loaded straight to LDS): images smaller and larger than a tile,
+# channel words that are and are not a power of two, taps that straddle a chunk, stride, padding, every output form.
+@pytest.mark.parametrize("tile", [1, 7])
+@pytest.mark.parametrize("wb,xb", [(1, 2), (1, 3), (1, 4), (2, 2)])
+@pytest.mark.parametrize("batch,H,C,cout,R,stride,pad", [(1, 5, 128, 32, 3, 1, 1), (2, 9, 384, 288, 3, 1, 1),
+                                                         (3, 13, 256, 160, 3, 2, 1), (1, 16, 640, 256, 1, 1, 0),
+                                                         (2, 8, 128, 96, 5, 1, 2)])
+@pytest.mark.parametrize("sym,mode", [(0, "int32"), (1, "int32"), (1, "bn"), (0, "shortcut")])
+def test_async_conv_tiles(G, wb, xb, tile, batch, H, C, cout, R, stride, pad, sym, mode):
+    rng = np.random.default_rng(8500 + C + cout + 10 * wb + xb)
+    Ho = (H + 2 * pad - R) // stride + 1
+    rows = batch * Ho * Ho
+    X = O.random_planes(rng, xb, batch * H * H, C // 32)
+    Wt = O.random_planes(rng, wb, cout * R * R, C // 32)
+    kw = dict(batch=batch, H=H, W=H, cout=cout, R=R, S=R, stride=stride, pad=pad, halo=0, wb=wb, xb=xb)
+    acc = O.conv(Wt, X, cwords=C // 32, sym_w=sym, **kw).reshape(-1, cout)
+    if mode == "int32":
+        got = G.run_conv(Wt, X, cin_pad=C, sym=sym, path=2, tile=tile, **kw).reshape(rows, cout)
+        assert np.array_equal(got, acc)
+        return
+    lo, hi = int(acc.min()), int(acc.max())
+    thr = np.sort(rng.integers(lo, hi + 1, size=(cout, (1 << xb) - 1)), axis=1).astype(np.int32)
+    keep = [G.to_dev(thr)]
+    extra, value = {}, acc
+    if mode == "shortcut":
+        codes = rng.integers(0, 4, size=(rows, cout)).astype(np.uint32)
+        keep.append(G.to_dev(O.pack_bits(codes, rows, cout, cout, 2)))
+        extra = dict(resid_planes=keep[1], resid_bits=2, resid_scale=5)
+        value = acc + 5 * codes.astype(np.int32)
+    epi = G.epilogue(mode=G.A.EPI_BN, out_bits=xb, thr=keep[0], **extra)
+    got = G.run_conv(Wt, X, cin_pad=C, sym=sym, epi=epi, path=2, tile=tile, **kw).view(np.uint32).reshape(xb, rows, cout // 32)
+    q = O.bn_quantize(value, None, thr, None, xb)
+    assert np.array_equal(got, O.lowbits_pack(q, rows, cout, xb))
