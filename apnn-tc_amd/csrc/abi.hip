@@ -495,9 +495,12 @@ bool auto_prefers_mfma_gemm(const KParams &p) {
 }
 
 // Precisions without a popcount kernel of their own (w1a1 and everything beyond five planes) reach the VALU only
-// through the any-precision kernel, which takes 30-100 us for products the matrix cores finish in 3 us (w1a1 at
-// 111x67x1792 105 us, w2a8 at 52x72x128 31 us): they take the matrix cores at every size.
-bool has_popcount_kernel(int wb, int xb) { return (wb == 1 && xb >= 2 && xb <= 4) || (wb == 2 && xb == 2); }
+// through the any-precision kernel, which takes 30-100 us for products the matrix cores finish in 6 us (w1a1 at
+// 111x67x1792 105.7 against 6.4 us, w2a8 at 52x72x128 31.0 against 6.6 us): they take the matrix cores at every size.
+// A pinned tile names one of the popcount kernel's below the cross-over, as it does for the other precisions.
+bool any_precision_only(int wb, int xb, int tile_pin) {
+  return tile_pin == 0 && !((wb == 1 && xb >= 2 && xb <= 4) || (wb == 2 && xb == 2));
+}
 
 valu_fn valu_gemm_fn(int wb, int xb) {
   if (wb == 1 && xb == 2) return apnn::valu_gemm_1_2_x;
@@ -585,7 +588,7 @@ int run_gemm(const apnn_gemm_desc *d, hipStream_t stream, apnn_plan *plan = null
   // operand planes of 4 GiB or more: the matrix-core kernels address rows with 32-bit offsets and refuse
   if ((path == APNN_PATH_MFMA || path == APNN_PATH_MFMA_I8) && !p.addr32) return APNN_EUNSUPPORTED;
   if (path == APNN_PATH_MFMA || path == APNN_PATH_MFMA_I8 ||
-      (path == APNN_PATH_AUTO && p.addr32 && (auto_prefers_mfma_gemm(p) || !has_popcount_kernel(d->wb, d->xb)))) {
+      (path == APNN_PATH_AUTO && p.addr32 && (auto_prefers_mfma_gemm(p) || any_precision_only(d->wb, d->xb, tile_pin)))) {
     // AUTO: FP4 operands while their fp32 accumulation is exact, the int8 core (int32 accumulate) beyond
     const bool i8 = path == APNN_PATH_MFMA_I8 || (path == APNN_PATH_AUTO && !f4ok);
     valu_fn fn = mfma_gemm_fn(d->wb, d->xb, i8);
@@ -749,7 +752,7 @@ int run_conv(const apnn_conv_desc *d, hipStream_t stream, apnn_plan *plan = null
   }
   // operand planes of 4 GiB or more, or a filter beyond the kernels' 24-bit index arithmetic: refused
   if ((path == APNN_PATH_MFMA || path == APNN_PATH_MFMA_I8) && !p.addr32) return APNN_EUNSUPPORTED;
-  if (path == APNN_PATH_MFMA || path == APNN_PATH_MFMA_I8 || (path == APNN_PATH_AUTO && p.addr32 && (auto_prefers_mfma(p) || !has_popcount_kernel(d->wb, d->xb)))) {
+  if (path == APNN_PATH_MFMA || path == APNN_PATH_MFMA_I8 || (path == APNN_PATH_AUTO && p.addr32 && (auto_prefers_mfma(p) || any_precision_only(d->wb, d->xb, tile_pin)))) {
     const bool i8 = path == APNN_PATH_MFMA_I8 || (path == APNN_PATH_AUTO && !f4ok);
     valu_fn fn = mfma_conv_fn(d->xb, d->wb, i8);
     if (fn != nullptr) {

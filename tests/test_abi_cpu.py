@@ -308,6 +308,21 @@ def test_plan_reports_the_dispatchers_choices():
     assert A.lib().apnn_gemm_plan(ctypes.byref(g), None) == A.ENULL
 
 
+@pytest.mark.parametrize("wb,xb", [(1, 1), (1, 8), (2, 8), (4, 4), (1, 2), (2, 2)])
+@pytest.mark.parametrize("tile", [1, 2, 3, 4])
+def test_pinned_tile_below_the_crossover_names_a_popcount_tile(wb, xb, tile):
+    """AUTO with a pinned tile: below the matrix-core cross-over the pin is one of the popcount kernels' tiles at every
+    precision, also where AUTO without a pin takes the matrix cores for any size."""
+    rc, plan = _plan_gemm(M=52, N=72, K=128, wb=wb, xb=xb, path=A.PATH_AUTO | (tile << 8))
+    assert rc == 0 and plan.path == A.PATH_VALU
+    rc, plan = _plan_conv(batch=1, H=5, Wd=5, cin_pad=64, COUT=32, R=1, S=1, stride=1, pad=0, wb=wb, xb=xb,
+                          path=A.PATH_AUTO | (tile << 8))
+    assert rc == 0 and plan.path == A.PATH_VALU
+    if (wb, xb) in ((1, 1), (1, 8), (2, 8), (4, 4)):
+        rc, plan = _plan_gemm(M=52, N=72, K=128, wb=wb, xb=xb, path=A.PATH_AUTO)
+        assert rc == 0 and plan.kernel == A.KERNEL_MFMA_FP4
+
+
 def test_patch_capacity_bounds_every_tile():
     """The patch-resident convolution kernel stages, per work-group, the contiguous range of padded-frame
     pixels that its tile of consecutive output rows reads; the host sizes that range from a closed-form
