@@ -318,22 +318,40 @@ __device__ __forceinline__ void static_for_n(F &&f) {
   }
 }
 
-// old with lanes L0, L0 + 4 replaced by the halves of m0 and lanes L0 + 32, L0 + 36 by the halves of m1
-// (wave-uniform compare masks).  A vector instruction that takes a scalar register written by the vector
-// instruction just before it needs two wait states, which the compiler inserts only for instructions it
-// can see -- not for this opaque assembly, hence the leading s_nop.
-template <int L0>
-__device__ __forceinline__ int write_mask_lanes(unsigned long long m0, unsigned long long m1, int old) {
-  static_assert(L0 >= 0 && L0 + 36 < 64, "lane index");
-  asm("s_nop 1\n\t"
-      "v_writelane_b32 %0, %1, %5\n\t"
-      "v_writelane_b32 %0, %2, %6\n\t"
-      "v_writelane_b32 %0, %3, %7\n\t"
-      "v_writelane_b32 %0, %4, %8"
-      : "+v"(old)
-      : "s"((int)(uint32_t)m0), "s"((int)(uint32_t)(m0 >> 32)), "s"((int)(uint32_t)m1), "s"((int)(uint32_t)(m1 >> 32)),
-        "n"(L0), "n"(L0 + 4), "n"(L0 + 32), "n"(L0 + 36));
-  return old;
+// w = 16 w + four code bits, first value on top, for bit 1 and bit 0 of a 2-bit code: bit1 = v >= t1,
+// bit0 = v >= (bit1 ? t2 : t0).  One block, because a vector instruction must not read a scalar register within
+// two instructions of the vector instruction that wrote it, and the compiler does not see into assembly: each
+// mask here is used at least three instructions after its compare.
+__device__ __forceinline__ void append_int_codes(int v0, int v1, int v2, int v3, const v4i_t &a, const v4i_t &b,
+                                                 const v4i_t &c, uint32_t &w1, uint32_t &w0) {
+  unsigned long long s0, s1, s2, s3;
+  int x0, x1, x2, x3;
+  asm("v_cmp_ge_i32_e64 %[s0], %[v0], %[b0]\n\t"
+      "v_cmp_ge_i32_e64 %[s1], %[v1], %[b1]\n\t"
+      "v_cmp_ge_i32_e64 %[s2], %[v2], %[b2]\n\t"
+      "v_cmp_ge_i32_e64 %[s3], %[v3], %[b3]\n\t"
+      "v_cndmask_b32_e64 %[x0], %[a0], %[c0], %[s0]\n\t"
+      "v_cndmask_b32_e64 %[x1], %[a1], %[c1], %[s1]\n\t"
+      "v_cndmask_b32_e64 %[x2], %[a2], %[c2], %[s2]\n\t"
+      "v_cndmask_b32_e64 %[x3], %[a3], %[c3], %[s3]\n\t"
+      "v_addc_co_u32_e64 %[w1], vcc, %[w1], %[w1], %[s0]\n\t"
+      "v_addc_co_u32_e64 %[w1], vcc, %[w1], %[w1], %[s1]\n\t"
+      "v_addc_co_u32_e64 %[w1], vcc, %[w1], %[w1], %[s2]\n\t"
+      "v_addc_co_u32_e64 %[w1], vcc, %[w1], %[w1], %[s3]\n\t"
+      "v_cmp_ge_i32_e64 %[s0], %[v0], %[x0]\n\t"
+      "v_cmp_ge_i32_e64 %[s1], %[v1], %[x1]\n\t"
+      "v_cmp_ge_i32_e64 %[s2], %[v2], %[x2]\n\t"
+      "v_cmp_ge_i32_e64 %[s3], %[v3], %[x3]\n\t"
+      "v_addc_co_u32_e64 %[w0], vcc, %[w0], %[w0], %[s0]\n\t"
+      "v_addc_co_u32_e64 %[w0], vcc, %[w0], %[w0], %[s1]\n\t"
+      "v_addc_co_u32_e64 %[w0], vcc, %[w0], %[w0], %[s2]\n\t"
+      "v_addc_co_u32_e64 %[w0], vcc, %[w0], %[w0], %[s3]"
+      : [s0] "=&s"(s0), [s1] "=&s"(s1), [s2] "=&s"(s2), [s3] "=&s"(s3), [x0] "=&v"(x0), [x1] "=&v"(x1), [x2] "=&v"(x2),
+        [x3] "=&v"(x3), [w1] "+v"(w1), [w0] "+v"(w0)
+      : [v0] "v"(v0), [v1] "v"(v1), [v2] "v"(v2), [v3] "v"(v3), [a0] "v"(a[0]), [a1] "v"(a[1]), [a2] "v"(a[2]),
+        [a3] "v"(a[3]), [b0] "v"(b[0]), [b1] "v"(b[1]), [b2] "v"(b[2]), [b3] "v"(b[3]), [c0] "v"(c[0]), [c1] "v"(c[1]),
+        [c2] "v"(c[2]), [c3] "v"(c[3])
+      : "vcc");
 }
 
 // ---- int8 first convolution for images, filter rows taken straight from the image bytes ------------
@@ -344,19 +362,26 @@ __device__ __forceinline__ int write_mask_lanes(unsigned long long m0, unsigned 
 // output row) is R image-row segments copied to LDS as aligned dwords -- no per-pixel repacking -- with
 // the zero point removed by an XOR (x - 128 == x ^ 0x80 as int8) and out-of-image dwords set to zero.
 // A lane's 16 operand bytes start at byte lead + pixel*stride*C + 16*half of its row segment: five
-// aligned dword reads and four v_alignbyte.  With NKS > 0 the wave keeps its 64 x (NKS*32) weight
-// block in registers for the whole (persistent) kernel; with NKS == 0 weights are read from LDS.
-// The epilogue is the compare-is-ballot scheme of the matrix-core kernels: per accumulator register
-// two compares and a select give both bit-plane masks of two output pixels.  Lane li of a column block
-// works on output channel 31 - li (its filter row and thresholds are read in that order), so a compare
-// mask already is the packed word (channel c at bit 31 - c%32) and needs no bit reversal.
+// aligned dword reads and four v_alignbyte.  NKS > 0: the number of k-steps is known, the loop is unrolled and a
+// lane keeps the patch offset of each step; with WREG the wave also keeps its 64 x (NKS*32) weight block in
+// registers for the whole (persistent) kernel, otherwise weights are read from LDS.
+// Weights are the first operand, so a lane of the accumulator owns one output pixel and its registers hold
+// channels: code bits are appended to the lane's own words, thresholds come from a table in LDS.  Filter row
+// 8q + 4h + j of a block of 32 holds channel 16h + 4q + j, which gives lane half h the channels 16h .. 16h + 15 in
+// order; one half-wave swap joins the two halves of both planes' words.
+// What bounds it: vector issue and LDS reads share the time of a group of 32 pixels about evenly.  Five vector
+// operations per value (compare, select, compare, two appends) instead of eight with lane writes alone gain little,
+// because the table adds 24 LDS reads (11x11 filter at batch 8 15.1 -> 14.8 us); with the unrolled loop, which drops
+// the decode of every k-step, 7x7 stride 2 on 224x224x3 at batch 64 39.7 -> 36.0 us, 3x3 to 96 channels 53.0 -> 48.1.
 // Requires C <= 4, (W*C) % 4 == 0, X 4-byte aligned, bits <= 2, COUT % 32 == 0.
 // NWAV waves per work-group share one filter block in LDS (each wave has its own patch and walks its
 // own pixel groups): eight waves where the filter block is large, so that its LDS cost per wave halves
 // and four waves per SIMD stay resident (two work-groups per compute unit: the register budget of that
 // variant is held to 128 by its launch bounds).
-template <int NKS, int NSLOT, int NWAV>
-__global__ __launch_bounds__(64 * NWAV, NWAV == 8 ? 4 : 1) void conv_i8_rows_kernel(const uint8_t *__restrict__ X, const int8_t *__restrict__ Wt,
+constexpr int kRowsTable = 3 * 64 * 4;  // bytes of thresholds in LDS, [3][64]
+
+template <int NKS, bool WREG, int NSLOT, int NWAV>
+__global__ __launch_bounds__(64 * NWAV, WREG ? 3 : 4) void conv_i8_rows_kernel(const uint8_t *__restrict__ X, const int8_t *__restrict__ Wt,
                                                            const int32_t *__restrict__ thr,
                                                            uint32_t *__restrict__ planes, int B, int H, int W, int C,
                                                            int COUT, int R, int S, int stride, int pad, int Ho, int Wo,
@@ -369,12 +394,13 @@ __global__ __launch_bounds__(64 * NWAV, NWAV == 8 ? 4 : 1) void conv_i8_rows_ker
   const int NH = R * HPR;
   const int nks = (NH + 1) / 2;
   const int KB = nks * 32, KPL = KB + 16;
-  int8_t *wl = reinterpret_cast<int8_t *>(lds);  // [64][KPL]
+  int *table = reinterpret_cast<int *>(lds);                  // [3][64]
+  int8_t *wl = reinterpret_cast<int8_t *>(lds + kRowsTable);  // [64][KPL]
   // the wave index is the same in all 64 lanes: as a scalar it keeps the pixel-group arithmetic below
   // (group -> image, output row, image row addresses) on the scalar unit
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 31, g = lane >> 5;
-  uint32_t *patch = reinterpret_cast<uint32_t *>(lds + 64 * KPL) + wave * (R * PWD);
+  uint32_t *patch = reinterpret_cast<uint32_t *>(lds + kRowsTable + 64 * KPL) + wave * (R * PWD);
   const int co0 = blockIdx.y * 64;
   const int SC = S * C;
 
@@ -390,7 +416,8 @@ __global__ __launch_bounds__(64 * NWAV, NWAV == 8 ? 4 : 1) void conv_i8_rows_ker
       const int task = t0 + u * 64 * NWAV + tid;
       const int col = (int)quot((uint32_t)task, (uint32_t)(nks * 2), magic_nh2), hh = task - col * (nks * 2);
       const int r = (int)quot((uint32_t)hh, (uint32_t)HPR, magic_hpr), hq = hh - r * HPR;
-      dst_off[u] = col * KPL + hh * 16;
+      const int row = (col & 0x23) | ((col & 0xc) << 1) | ((col & 0x10) >> 2);
+      dst_off[u] = row * KPL + hh * 16;
       const int co = co0 + col;
       const int nvalid = (task < ntasks && co < COUT && r < R) ? min(max(SC - hq * 16, 0), 16) : 0;
       const int8_t *src = Wt + ((long long)co * R + r) * SC + hq * 16;
@@ -423,33 +450,25 @@ __global__ __launch_bounds__(64 * NWAV, NWAV == 8 ? 4 : 1) void conv_i8_rows_ker
       if (task < ntasks) *reinterpret_cast<uint4 *>(wl + dst_off[u]) = make_uint4(w[u][0], w[u][1], w[u][2], w[u][3]);
     }
   }
+  const int nt = (1 << bits) - 1;
+  if (tid < 3 * 64) {
+    const int co = co0 + (tid & 63), k = tid >> 6;
+    table[tid] = co < COUT ? thr[co * nt + (k < nt ? k : 0)] : 0x7fffffff;
+  }
   __syncthreads();
 
   constexpr int NW = NKS > 0 ? NKS : 1;
-  v4i_t wreg[2][NW];
+  v4i_t wreg[2][WREG ? NW : 1];
   int koff[NW];  // byte offset of this lane's half of k-step ks inside the patch
   if (NKS > 0) {
 #pragma unroll
     for (int ks = 0; ks < NW; ++ks) {
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
-        wreg[nb][ks] = *reinterpret_cast<const v4i_t *>(wl + (nb * 32 + 31 - li) * KPL + ks * 32 + g * 16);
+      for (int nb = 0; nb < (WREG ? 2 : 0); ++nb)
+        wreg[nb][WREG ? ks : 0] = *reinterpret_cast<const v4i_t *>(wl + (nb * 32 + li) * KPL + ks * 32 + g * 16);
       const int hh = 2 * ks + g;
       const int r = min(hh / HPR, R - 1);
       koff[ks] = r * PWD * 4 + (hh % HPR) * 16;
-    }
-  }
-
-  const int nt = (1 << bits) - 1;
-  int t0[2], t1[2], t2[2];
-#pragma unroll
-  for (int nb = 0; nb < 2; ++nb) {
-    const int co = co0 + nb * 32 + 31 - li;
-    t0[nb] = t1[nb] = t2[nb] = 0x7fffffff;
-    if (co < COUT) {
-      t0[nb] = thr[co * nt];
-      t1[nb] = nt > 1 ? thr[co * nt + 1] : t0[nb];
-      t2[nb] = nt > 2 ? thr[co * nt + 2] : t0[nb];
     }
   }
 
@@ -573,7 +592,12 @@ __global__ __launch_bounds__(64 * NWAV, NWAV == 8 ? 4 : 1) void conv_i8_rows_ker
       for (int ks = 0; ks < NW; ++ks) {
         const v4i_t af = operand(koff[ks]);
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) acc[nb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, wreg[nb][ks], acc[nb], 0, 0, 0);
+        for (int nb = 0; nb < 2; ++nb) {
+          v4i_t w;
+          if constexpr (WREG) w = wreg[nb][ks];
+          else w = *reinterpret_cast<const v4i_t *>(wl + (nb * 32 + li) * KPL + ks * 32 + g * 16);
+          acc[nb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w, af, acc[nb], 0, 0, 0);
+        }
       }
     } else {
       int r = 0, h = g;  // half index 2ks + g = r * HPR + h
@@ -585,10 +609,10 @@ __global__ __launch_bounds__(64 * NWAV, NWAV == 8 ? 4 : 1) void conv_i8_rows_ker
       // clearing 32 accumulator registers per pixel group (this loop's trip count is a run-time value)
       auto k_step = [&](int ks, const v16i_t &c0, const v16i_t &c1) {
         const v4i_t af = operand(min(r, R - 1) * PWD * 4 + h * 16);
-        const v4i_t b0 = *reinterpret_cast<const v4i_t *>(wl + (31 - li) * KPL + ks * 32 + g * 16);
-        const v4i_t b1 = *reinterpret_cast<const v4i_t *>(wl + (63 - li) * KPL + ks * 32 + g * 16);
-        acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, b0, c0, 0, 0, 0);
-        acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, b1, c1, 0, 0, 0);
+        const v4i_t b0 = *reinterpret_cast<const v4i_t *>(wl + li * KPL + ks * 32 + g * 16);
+        const v4i_t b1 = *reinterpret_cast<const v4i_t *>(wl + (32 + li) * KPL + ks * 32 + g * 16);
+        acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b0, af, c0, 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b1, af, c1, 0, 0, 0);
         h += 2;
         while (h >= HPR) {
           h -= HPR;
@@ -600,29 +624,35 @@ __global__ __launch_bounds__(64 * NWAV, NWAV == 8 ? 4 : 1) void conv_i8_rows_ker
       for (int ks = 1; ks < nks; ++ks) k_step(ks, acc[0], acc[1]);
     }
 
-    // ---- thresholds -> bit-plane words, parked at lane = pixel (+32 for plane 1) -------------------
-    int park[2] = {0, 0};
+    // ---- thresholds -> bit-plane words: lane half 0 ends with the pixel's word of plane 0, half 1 of plane 1 ----
+    // wait states between the last matrix instruction and a vector instruction that reads its result (19 for sixteen
+    // passes): the compiler adds them for instructions it can see, not for the assembly of append_int_codes
+    asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]), "+v"(acc[1]));
+    __builtin_amdgcn_sched_barrier(0);  // (keeps the threshold reads from piling up in registers)
+    const int *tab = table + 16 * g;
+    uint32_t word[2];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
-      static_for_n<0, 16>([&](auto rc) {
-        constexpr int r = decltype(rc)::value;
-        constexpr int rlo = 8 * (r >> 2) + (r & 3);  // lane half 0's pixel; lane half 1's is rlo + 4
-        const int v = acc[nb][r];
-        const bool hi1 = v >= t1[nb];
-        const unsigned long long m1 = __ballot(hi1);
-        const int tsel = hi1 ? t2[nb] : t0[nb];
-        const unsigned long long m0 = __ballot(v >= tsel);
-        park[nb] = write_mask_lanes<rlo>(m0, m1, park[nb]);
+      uint32_t w0 = 0, w1 = 0;
+      static_for_n<0, 4>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        const v4i_t a = *reinterpret_cast<const v4i_t *>(tab + nb * 32 + 4 * q);
+        const v4i_t b1 = *reinterpret_cast<const v4i_t *>(tab + 64 + nb * 32 + 4 * q);
+        const v4i_t c2 = *reinterpret_cast<const v4i_t *>(tab + 128 + nb * 32 + 4 * q);
+        append_int_codes(acc[nb][4 * q], acc[nb][4 * q + 1], acc[nb][4 * q + 2], acc[nb][4 * q + 3], a, b1, c2, w1, w0);
+        __builtin_amdgcn_sched_barrier(0);
       });
+      const auto s = __builtin_amdgcn_permlane32_swap(w0, w1, false, false);
+      word[nb] = (s[0] << 16) | s[1];
     }
     const int ox = ox0 + li, plane = g;
     if (ox < Wo && plane < bits) {
       uint32_t *dst = planes + plane * rows_total * cw32 + (((long long)b * Ho + oy) * Wo + ox) * cw32 + (co0 >> 5);
       if ((cw32 & 1) == 0) {
-        *reinterpret_cast<uint2 *>(dst) = make_uint2((uint32_t)park[0], (uint32_t)park[1]);
+        *reinterpret_cast<uint2 *>(dst) = make_uint2(word[0], word[1]);
       } else {
-        dst[0] = (uint32_t)park[0];
-        if (co0 + 32 < COUT) dst[1] = (uint32_t)park[1];
+        dst[0] = word[0];
+        if (co0 + 32 < COUT) dst[1] = word[1];
       }
     }
   }
@@ -950,30 +980,30 @@ hipError_t launch_conv_i8_bn(const int8_t *X, const int8_t *Wt, const int32_t *t
     const int nwav = wide_patch ? 8 : 4;
     const size_t lds = (size_t)64 * (nks * 32 + 16) + (size_t)nwav * R * PWD * 4;
     if (lds <= (wide_patch ? 80 * 1024 : 64 * 1024)) {
+      const size_t all = lds + kRowsTable;
       // persistent grid: exactly as many work-groups as the device holds at once
       // Filter block in registers (two work-groups per compute unit fit) while one or two rounds of
       // work-groups cover all pixel groups; beyond that the variant that re-reads the filter from LDS
       // wins through its higher occupancy (four per compute unit).
+      // Unrolled loops for the k-steps of 7x7x3 and 3x3x3 filters (see the kernel); any other number runs the loop with a
+      // decode per step, the 11x11 one because its 17 offsets do not fit the 128 registers of four waves per SIMD.
       const bool wreg = nks == 7 && grid.x <= 1024 && !wide_patch;
-      auto kern = wreg ? conv_i8_rows_kernel<7, 8, 4>
-                       : (wide_patch ? conv_i8_rows_kernel<0, 18, 8> : conv_i8_rows_kernel<0, 8, 4>);
-      if (wide_patch) {
-        grid.x = (unsigned)((groups + 7) / 8);
-        if (lds > 64 * 1024) {
-          static bool raised = false;
-          if (!raised) {
-            const hipError_t e0 = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
-            if (e0 != hipSuccess) return e0;
-            raised = true;
-          }
-        }
+      auto kern = wreg ? conv_i8_rows_kernel<7, true, 8, 4>
+                  : wide_patch ? conv_i8_rows_kernel<0, false, 18, 8>
+                  : nks == 7   ? conv_i8_rows_kernel<7, false, 8, 4>
+                  : nks == 2   ? conv_i8_rows_kernel<2, false, 8, 4>
+                               : conv_i8_rows_kernel<0, false, 8, 4>;
+      if (wide_patch) grid.x = (unsigned)((groups + 7) / 8);
+      if (all > 64 * 1024) {
+        const hipError_t e0 = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024 + kRowsTable);
+        if (e0 != hipSuccess) return e0;
       }
       int per_cu = 0, cus = 0, dev = 0;
       hipError_t e = hipGetDevice(&dev);
       if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
       if (e == hipSuccess)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kern), 64 * nwav, lds);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kern), 64 * nwav, all);
       if (e != hipSuccess) return e;
       unsigned resident = (unsigned)(per_cu > 0 ? per_cu : 1) * (unsigned)(cus > 0 ? cus : 256);
       const unsigned slices = grid.y > 0 ? grid.y : 1;
@@ -992,7 +1022,7 @@ hipError_t launch_conv_i8_bn(const int8_t *X, const int8_t *Wt, const int32_t *t
       const uint32_t mn = small_magic(NDW), mt = small_magic(nks * 2), mp = small_magic(HPR);
       // the filter array as aligned dwords: base 4-byte aligned and a whole number of dwords long
       const int wt_dwords = (reinterpret_cast<uintptr_t>(Wt) & 3u) == 0 && ((long long)COUT * R * S * C) % 4 == 0;
-      hipLaunchKernelGGL(kern, g2, dim3(64 * nwav), lds, s, Xu, Wt, thr, planes, B, H, W, C, COUT, R, S, stride, pad, Ho,
+      hipLaunchKernelGGL(kern, g2, dim3(64 * nwav), all, s, Xu, Wt, thr, planes, B, H, W, C, COUT, R, S, stride, pad, Ho,
                          Wo, bits, xm, HPR, NDW, PWD, mg, mh, mn, mt, mp, wt_dwords);
       return hipGetLastError();
     }

@@ -148,3 +148,25 @@ def test_async_conv_tiles(G, wb, xb, tile, batch, H, C, cout, R, stride, pad, sy
     got = G.run_conv(Wt, X, cin_pad=C, sym=sym, epi=epi, path=2, tile=tile, **kw).view(np.uint32).reshape(xb, rows, cout // 32)
     q = O.bn_quantize(value, None, thr, None, xb)
     assert np.array_equal(got, O.lowbits_pack(q, rows, cout, xb))
+
+
+# First layer on image rows: seven k-steps with the filter in registers and (beyond 4096 pixel groups) in LDS, two, three
+# and seventeen k-steps; an odd number of channel words, one and two bits, thresholds at the ends of int32.
+@pytest.mark.parametrize("B,H,W,C,cout,R,stride,pad", [(2, 30, 36, 3, 96, 7, 2, 3), (42, 200, 8, 3, 96, 7, 2, 3), (3, 9, 36, 3, 64, 3, 1, 1),
+                                                       (1, 12, 72, 4, 160, 3, 2, 0), (2, 13, 40, 3, 32, 5, 1, 2),
+                                                       (2, 33, 64, 3, 96, 11, 4, 5)])
+@pytest.mark.parametrize("bits", [1, 2])
+def test_first_layer_filter_supply(G, B, H, W, C, cout, R, stride, pad, bits):
+    rng = np.random.default_rng(8600 + H + R + bits)
+    X = rng.integers(0, 256, size=(B, H, W, C)).astype(np.uint8)
+    Wt = rng.integers(-128, 128, size=(cout, R, R, C)).astype(np.int8)
+    acc = O.conv_i8(Wt, (X.astype(np.int16) - 128).astype(np.int8), stride, pad).reshape(-1, cout)
+    rows = acc.shape[0]
+    thr = np.sort(rng.integers(acc.min(), acc.max() + 1, size=(cout, 2 ** bits - 1)), axis=1).astype(np.int32)
+    thr[0, :], thr[17, :] = np.iinfo(np.int32).min, np.iinfo(np.int32).max
+    dX, dW, dT = torch.from_numpy(X).cuda(), G.to_dev(Wt), G.to_dev(thr)
+    planes = G.dev_empty_i32(bits * rows * cout // 32, fill=-7)
+    G.A.check(G.A.lib().apnn_conv_i8_bn_pack(G.ptr(dX), G.ptr(dW), G.ptr(dT), G.ptr(planes), B, H, W, C, cout, R, R, stride, pad,
+                                             bits, 128, None), "conv_i8_bn_pack")
+    expect = O.pack_bits(O.bn_quantize(acc, None, thr, None, bits).astype(np.uint32), rows, cout, cout, bits)
+    assert np.array_equal(G.to_host(planes, np.uint32).reshape(expect.shape), expect)
