@@ -227,8 +227,10 @@ bool int32_range_ok(long long kwords, int wb, int xb, bool sym, const apnn_epilo
 // resid_scale as terms the matrix cores can apply to FP4 shortcut digits (KParams::fold): one or two terms +-m * 2^j
 // with m up to 15.  An odd scale of more than four bits is split at its low k bits, taken as they are or as a
 // negative remainder.  0 when that finds no second term, when there is no packed shortcut of one or two bits, or when
-// fp32 could round (accumulator range plus both terms' largest magnitude must stay below 2^24, as for
-// epilogue_float_ok).
+// fp32 could round.  With symmetric weights the accumulator may hold the raw sum of unsigned products, worth two
+// results each, when the terms are added: half units have to be exact, so 2 * raw + terms must stay below 2^24.
+// (One-plane weights multiplied as -1 / +1 would do with half of that; they reach it only beyond K = 32896 even with
+// eight activation planes.)
 uint32_t shortcut_fold(const KParams &p, int wb, int xb) {
   if (p.resid_planes == nullptr || p.resid_bits < 1 || p.resid_bits > 2 || p.resid_scale == 0) return 0u;
   if (p.epi == APNN_EPI_INT32 || p.pool != APNN_POOL_NONE) return 0u;
@@ -252,8 +254,8 @@ uint32_t shortcut_fold(const KParams &p, int wb, int xb) {
     Term a, b;
     if (!term(t0, &a) || !term(t1, &b)) return 0u;
     const long long size = (t0 < 0 ? -t0 : t0) + (t1 < 0 ? -t1 : t1);
-    // (unsigned one-plane weights accumulate -1 / +1 products, in units of half a result)
-    if (acc + size * cmax * (p.sym || wb > 1 ? 1 : 2) >= (1LL << 24)) return 0u;
+    // (unsigned one-plane weights of the convolutions accumulate -1 / +1 products, in units of half a result)
+    if ((p.sym ? 2 : 1) * acc + size * cmax * (p.sym || wb > 1 ? 1 : 2) >= (1LL << 24)) return 0u;
     return a.m | (b.m << 5) | (a.e8 << 10) | (b.e8 << 18);
   };
   const long long S = p.resid_scale;

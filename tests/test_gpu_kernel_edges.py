@@ -170,3 +170,36 @@ def test_first_layer_filter_supply(G, B, H, W, C, cout, R, stride, pad, bits):
                                              bits, 128, None), "conv_i8_bn_pack")
     expect = O.pack_bits(O.bn_quantize(acc, None, thr, None, bits).astype(np.uint32), rows, cout, cout, bits)
     assert np.array_equal(G.to_host(planes, np.uint32).reshape(expect.shape), expect)
+
+
+# A packed shortcut beside sums near the 2^24 limit of fp32: with symmetric weights the matrix cores may hold the raw sum of
+# unsigned products, worth two results, and an odd shortcut term is half a unit of it.  All-ones operands make every
+# result K * wmax * amax (raw sums between 2^23 and 2^24 units), so the codes equal the shortcut's codes exactly when
+# no half unit was rounded away.
+_LARGE_SUMS = [(2, 8, 12800), (2, 6, 51200), (2, 2, 1024000), (4, 4, 41600), (1, 8, 64000), (1, 4, 640000), (1, 2, 3200000)]
+
+
+@pytest.mark.parametrize("gemm,path,tile,wb,xb,K", [
+    (gemm, path, tile, wb, xb, K) for gemm in (0, 1) for path, tile in ((0, None), (2, 1), (2, 2), (2, 4), (2, 5), (2, 9), (5, 2))
+    for wb, xb, K in _LARGE_SUMS
+    # precisions that the expand-while-staging kernel (path 5) and the GEMM matrix-core kernels are built for
+    if (path != 5 or (wb, xb) in ((1, 2), (1, 4), (2, 2))) and not (gemm and (wb, xb) == (2, 6))])
+def test_shortcut_beside_large_sums(G, gemm, path, tile, wb, xb, K):
+    wmax, amax, rows, cols = 2 ** wb - 1, 2 ** xb - 1, 32, 32
+    assert 2 ** 23 < K * wmax * amax < 2 ** 24 - 64
+    v = K * wmax * amax
+    rng = np.random.default_rng(8700 + wb + 10 * xb)
+    codes = rng.integers(0, 4, size=(rows, cols)).astype(np.uint32)
+    d_short = G.to_dev(O.pack_bits(codes, rows, cols, cols, 2))
+    W, X = np.full((wb, cols, K // 32), 0xFFFFFFFF, np.uint32), np.full((xb, rows, K // 32), 0xFFFFFFFF, np.uint32)
+    for scale in (1, -3):
+        thr = np.sort(v + scale * np.repeat(np.arange(1, 4, dtype=np.int64)[None, :], cols, axis=0), axis=1)
+        d_thr = G.to_dev((thr + (scale < 0)).astype(np.int32))
+        expect = codes if scale > 0 else 3 - codes
+        epi = G.epilogue(mode=G.A.EPI_BN, out_bits=2, thr=d_thr, resid_planes=d_short, resid_bits=2, resid_scale=scale)
+        if gemm:
+            got = G.run_gemm(W, X, rows, cols, K, wb, xb, sym=1, epi=epi, path=path, tile=tile)
+        else:
+            got = G.run_conv(W, X, batch=1, H=4, W=8, cin_pad=K, cout=cols, R=1, S=1, stride=1, pad=0, halo=0, wb=wb, xb=xb,
+                             sym=1, epi=epi, path=path, tile=tile)
+        assert np.array_equal(got.view(np.uint32).reshape(2, rows, cols // 32), O.lowbits_pack(expect, rows, cols, 2)), scale
