@@ -355,6 +355,7 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
           for (int r = 0; r < 16; ++r) acc[x][y][r] += c;
       }
     }
+    settle_results(acc);
     conv_output<FA, FB, 4, TB, MAXB>(
         p, [&](auto xc, auto yc, auto ic) { return (float)acc[decltype(xc)::value][decltype(yc)::value][decltype(ic)::value]; },
         (float)(1 << log2vs), tab, rbase, cbase, b0, 0, lane);

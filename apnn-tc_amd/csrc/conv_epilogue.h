@@ -111,7 +111,8 @@ struct ConvTable {
 // w = 16 w + four code bits, first value on top, for bit 1 and bit 0 of a 2-bit code: bit1 = v >= t1,
 // bit0 = v >= (bit1 ? t2 : t0).  One block, because a vector instruction must not read a scalar register within
 // two instructions of the vector instruction that wrote it, and the compiler does not see into assembly: each
-// mask here is used at least three instructions after its compare.
+// mask here is used at least three instructions after its compare.  For the same reason values that come straight from
+// matrix instructions have to be settled by the caller (settle_results).
 __device__ __forceinline__ void append_codes2(const float (&v)[4], const float (&t0)[4], const float (&t1)[4],
                                               const float (&t2)[4], uint32_t &w1, uint32_t &w0) {
   unsigned long long s0, s1, s2, s3;

@@ -677,6 +677,22 @@ __device__ __forceinline__ void fold_shortcut(const KParams &p, v16f (&acc)[FA][
   });
 }
 
+// Wait states between the last matrix instruction and a vector instruction that reads its result (19 for sixteen
+// passes).  The compiler adds them for instructions it can see, not for the assembly of append_codes2: every block is
+// complete before the wait and is not read until after it.  24 clocks per work-group.
+template <int FA, int FB>
+__device__ __forceinline__ void settle_results(v16f (&acc)[FA][FB]) {
+#pragma unroll
+  for (int x = 0; x < FA; ++x)
+#pragma unroll
+    for (int y = 0; y < FB; ++y) asm volatile("" : "+v"(acc[x][y]));
+  asm volatile("s_nop 15\n\ts_nop 7");
+#pragma unroll
+  for (int x = 0; x < FA; ++x)
+#pragma unroll
+    for (int y = 0; y < FB; ++y) asm volatile("" : "+v"(acc[x][y]));
+}
+
 // Lanes are pixels: the scaled identity is the first operand (its row li is channel li of the block), the codes of
 // the lane's pixel the second.
 template <int FA, int FB>
@@ -1675,6 +1691,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
       }
       // (short reductions without staging have not met a barrier since the table was written)
       if (direct_k) __syncthreads();
+      settle_results(acc);
       conv_output<FA, FB, 4, TB, MAXB>(p, block_access(acc), vs, tab, own_rbase, cb, b0, 0, lane);
     } else {
       // Two wave groups: see below; group 0 finishes the first HA pixel blocks of every wave tile, group 1 the last
@@ -1729,6 +1746,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
         }
       }
       if (fold) fold_shortcut_lanes<HA, FB>(p, own, sc, lane, log2vs);
+      settle_results(own);
       conv_output<HA, FB, 4, TB, MAXB>(p, block_access(own), vs, tab, own_rbase, cb, b0, 0, lane);
     }
   } else if constexpr (KSX == 1) {
