@@ -254,8 +254,7 @@ uint32_t shortcut_fold(const KParams &p, int wb, int xb) {
     Term a, b;
     if (!term(t0, &a) || !term(t1, &b)) return 0u;
     const long long size = (t0 < 0 ? -t0 : t0) + (t1 < 0 ? -t1 : t1);
-    // (unsigned one-plane weights of the convolutions accumulate -1 / +1 products, in units of half a result)
-    if ((p.sym ? 2 : 1) * acc + size * cmax * (p.sym || wb > 1 ? 1 : 2) >= (1LL << 24)) return 0u;
+    if ((p.sym ? 2 : 1) * acc + size * cmax >= (1LL << 24)) return 0u;
     return a.m | (b.m << 5) | (a.e8 << 10) | (b.e8 << 18);
   };
   const long long S = p.resid_scale;

@@ -28,8 +28,8 @@
 //   i.e. 8 VALU operations per plane for 16 int8 operands; CORE_F4: see expand_fp4.
 //
 // Symmetric (+-) weights use the closed form  2*raw - wmax * (activation row sum); the row sums
-// come from popcounts of the packed words the wave already holds.  (FP4 / FP6 convolution kernels with one weight
-// plane: -1 / +1 operands, see expand_sign.)
+// come from popcounts of the packed words the wave already holds.  (FP4 / FP6 convolution kernels, symmetric weights
+// of one plane: -1 / +1 operands, see expand_sign.)
 //
 // Output of the FP4 / FP6 convolution kernels: conv_epilogue.h.  GEMM entry points and int8 core: int32 results and codes of up to two bits (four where the waves tile the output) leave
 // straight from the accumulator registers (store_int32_direct, direct_epilogue); int32 residuals, saved
@@ -157,10 +157,9 @@ __device__ __forceinline__ v8i expand_fp6(const uint32_t (&w)[P]) {
   return out;
 }
 
-// One-plane weights as -1 / +1: sign bit = complement of the weight bit, magnitude 1.0 (FP4 code 2, FP6 code 8), the
-// same elements in the same fields as expand_fp4 / expand_fp6.  With symmetric weights the accumulator is then the
-// result itself (in units), no activation sums are needed; unsigned weights u = (1 + s) / 2 take half of it plus
-// half the activation sum.
+// Symmetric one-plane weights as -1 / +1: sign bit = complement of the weight bit, magnitude 1.0 (FP4 code 2, FP6
+// code 8), the same elements in the same fields as expand_fp4 / expand_fp6.  The accumulator is then the result itself
+// (in units), no activation sums are needed.
 template <int DIG>
 __device__ __forceinline__ v8i expand_sign(uint32_t x) {
   v8i out = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -175,6 +174,49 @@ __device__ __forceinline__ v8i expand_sign(uint32_t x) {
       constexpr int jj = decltype(jc)::value, j = jj % 3;
       constexpr uint32_t sign = every_sixth(5 - 2 * j), one = every_sixth(3 - 2 * j);
       out[jj] = (int)(((jj < 3 ? e : o) & sign) ^ (sign | one));
+    });
+  }
+  return out;
+}
+
+// Unsigned one-plane weights as 0 / 1.0, in the same fields and units as expand_sign.
+template <int DIG>
+__device__ __forceinline__ v8i expand_unit(uint32_t x) {
+  v8i out = {0, 0, 0, 0, 0, 0, 0, 0};
+  if constexpr (DIG == 2) {
+    out[0] = (int)((x << 1) & 0x22222222u);
+    out[1] = (int)(x & 0x22222222u);
+    out[2] = (int)((x >> 1) & 0x22222222u);
+    out[3] = (int)((x >> 2) & 0x22222222u);
+  } else {
+    const uint32_t e = rotl32(x, 3), o = rotl32(x, 2);
+    static_for<0, 6>([&](auto jc) {
+      constexpr int jj = decltype(jc)::value, j = jj % 3;
+      out[jj] = (int)((jj < 3 ? e : o) & every_sixth(3 - 2 * j));
+    });
+  }
+  return out;
+}
+
+// expand_sign or expand_unit by a run-time choice, for loops that hold their loads in registers: two copies of such a
+// loop make the compiler wait in each for the loads of the other (16x16x256 maps at batch 16, w1a2: 6.2 -> 9.3 us).
+template <int DIG>
+__device__ __forceinline__ v8i expand_w1(uint32_t x, bool sign) {
+  v8i out = {0, 0, 0, 0, 0, 0, 0, 0};
+  if constexpr (DIG == 2) {
+    const uint32_t y = __builtin_amdgcn_alignbit(x, x, sign ? 0 : 2);
+    const uint32_t mask = sign ? 0x88888888u : 0x22222222u, flip = sign ? 0xAAAAAAAAu : 0u;
+    out[0] = (int)((rotl32(y, 3) & mask) ^ flip);
+    out[1] = (int)((rotl32(y, 2) & mask) ^ flip);
+    out[2] = (int)((rotl32(y, 1) & mask) ^ flip);
+    out[3] = (int)((y & mask) ^ flip);
+  } else {
+    const uint32_t e = __builtin_amdgcn_alignbit(x, x, sign ? 27 : 29), o = __builtin_amdgcn_alignbit(x, x, sign ? 28 : 30);
+    static_for<0, 6>([&](auto jc) {
+      constexpr int jj = decltype(jc)::value, j = jj % 3;
+      constexpr uint32_t top = every_sixth(5 - 2 * j), one = every_sixth(3 - 2 * j);
+      const uint32_t mask = sign ? top : one, flip = sign ? top | one : 0u;
+      out[jj] = (int)(((jj < 3 ? e : o) & mask) ^ flip);
     });
   }
   return out;
@@ -1084,11 +1126,11 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
   constexpr int DB = F4 ? (PB + DIG - 1) / DIG : 1;
   constexpr int FSC = F4 ? fp_scale(PA, PB) : 0;
   // convolution on the FP4 / FP6 core: weights are the first operand of the matrix instructions, a lane of the
-  // accumulator is an output pixel (conv_epilogue.h), one-plane weights are -1 / +1
+  // accumulator is an output pixel (conv_epilogue.h), symmetric one-plane weights are -1 / +1
   constexpr bool LP = CONV && F4;
-  constexpr bool SIGNED1 = LP && PB == 1;
-  constexpr int VSC = SIGNED1 ? (DIG == 4 ? 8 : 2) : FSC;
-  const bool need_sum = !LP || (SIGNED1 ? p.sym == 0 : p.sym != 0);  // activation sums enter the result
+  constexpr bool W1 = LP && PB == 1;
+  const bool sign = W1 && p.sym != 0;
+  const bool need_sum = !LP || (!W1 && p.sym != 0);  // activation sums enter the result
   using AccT = typename std::conditional<F4, v16f, v16i>::type;
   using FragT = typename std::conditional<F4, v8i, v4i>::type;
   constexpr int NT = 256 * KSX;
@@ -1133,7 +1175,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
   const int b0 = tcol * TB;
 
   // value per accumulator unit; the thresholds of the tile's channels, behind the operand buffers
-  const int log2vs = __builtin_ctz(VSC > 0 ? VSC : 1) + (SIGNED1 ? (p.sym ? 0 : -1) : (p.sym ? 1 : 0));
+  const int log2vs = W1 ? (DIG == 4 ? 3 : 1) : __builtin_ctz(FSC > 0 ? FSC : 1) + (p.sym ? 1 : 0);
   const float inv_vs = __uint_as_float((uint32_t)(127 - log2vs) << 23), vs = __uint_as_float((uint32_t)(127 + log2vs) << 23);
   uint32_t *tab = smem + (LP ? mfma_lp_stage_words(PA, PB, FA, FB, WA, WB, VW, KSX) : 0);
   constexpr int MAXB = PA >= 3 ? 4 : 2;  // code widths the output stage has a path of its own for
@@ -1396,8 +1438,11 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
       for (int pl = 0; pl < PB; ++pl) wB[y][pl] = Bs[(pl * TB + y * 32) * LD];
   };
   FragT af[FA][DA], bf[FB][DB];
-  auto expand_all = [&](auto sum_c, FragT (&a)[FA][DA], FragT (&b)[FB][DB]) {
-    constexpr bool SUM = decltype(sum_c)::value;
+  // form_c 1: activation sums are counted (one-plane weights of the convolutions: they are -1 / +1);  0: they are not
+  // (0 / 1);  2, one-plane weights only: by the weight mode
+  auto expand_all = [&](auto form_c, FragT (&a)[FA][DA], FragT (&b)[FB][DB]) {
+    constexpr int FORM = decltype(form_c)::value;
+    constexpr bool SUM = !W1 && FORM == 1;
 #pragma unroll
     for (int x = 0; x < FA; ++x) {
       if (CONV && SUM) {
@@ -1416,8 +1461,10 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
 #pragma unroll
         for (int pl = 0; pl < PB; ++pl) psum[y][pl] += __popc(wB[y][pl]);
       }
-      if constexpr (SIGNED1) {
-        b[y][0] = expand_sign<DIG>(wB[y][0]);
+      if constexpr (W1) {
+        if constexpr (FORM == 1) b[y][0] = expand_sign<DIG>(wB[y][0]);
+        else if constexpr (FORM == 0) b[y][0] = expand_unit<DIG>(wB[y][0]);
+        else b[y][0] = expand_w1<DIG>(wB[y][0], sign);
       } else if constexpr (F4) {
         static_for<0, DB>([&](auto dc) { b[y][decltype(dc)::value] = expand_digit<DIG, PB, decltype(dc)::value>(wB[y]); });
       } else {
@@ -1465,8 +1512,8 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
 #pragma unroll
       for (int d = 0; d < GD; ++d) {
         if (gb + d * GSTEP < ngroups) {  // same for the whole wave
-          if constexpr (LP) {
-            // (unsigned one-plane or symmetric wider weights; one test per group of VW k-steps)
+          if constexpr (LP && !W1) {
+            // (symmetric weights; one test per group of VW k-steps)
             if (need_sum) {
 #pragma unroll
               for (int pl = 0; pl < PA; ++pl)
@@ -1482,14 +1529,14 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
             for (int y = 0; y < FB; ++y)
 #pragma unroll
               for (int pl = 0; pl < PB; ++pl) wB[y][pl] = gbw[d][y][pl][i];
-            expand_all(std::integral_constant<bool, !LP>{}, af, bf);
+            expand_all(std::integral_constant<int, W1 ? 2 : LP ? 0 : 1>{}, af, bf);
             mfma_all();
           }
         }
       }
     }
   };
-  auto k_loop = [&](auto sum_c) {
+  auto k_loop = [&](auto form_c) {
   const int nchunks = (p.KW + KC - 1) / KC;
   using Set0 = std::integral_constant<int, 0>;
   using Set1 = std::integral_constant<int, PF - 1>;
@@ -1504,7 +1551,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
   __syncthreads();
   if constexpr (KS == 1) {
     read_words(smem, kq);
-    expand_all(sum_c, af, bf);
+    expand_all(form_c, af, bf);
   }
   // one chunk; par = ch % 2 is a compile-time constant (LDS buffer and register set of the iteration)
   auto chunk_body = [&](int ch, auto par_c) {
@@ -1527,7 +1574,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
 #pragma unroll
       for (int ks = 0; ks < NKS / KS; ++ks) {
         read_words(cur, wave + ks * KS);
-        expand_all(sum_c, af, bf);
+        expand_all(form_c, af, bf);
         mfma_all();
       }
       __syncthreads();
@@ -1535,7 +1582,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
     }
     auto advance = [&]() {
       FragT an[FA][DA], bn[FB][DB];
-      expand_all(sum_c, an, bn);
+      expand_all(form_c, an, bn);
 #pragma unroll
       for (int x = 0; x < FA; ++x)
 #pragma unroll
@@ -1595,15 +1642,17 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
     for (int ch = 0; ch < nchunks; ++ch) chunk_body(ch, ch & 1);
   }
   };
+  using Form0 = std::integral_constant<int, 0>;
+  using Form1 = std::integral_constant<int, 1>;
   if constexpr (DIRECT_K) {
     direct_loop();
   } else if (direct_k) {
     if constexpr (DIRECT_OPT) direct_loop();
   } else if constexpr (LP) {
-    // with and without activation sums: the loop carries no test
-    if (need_sum) k_loop(std::true_type{}); else k_loop(std::false_type{});
+    // one loop per form: it carries no test
+    if (W1 ? sign : need_sum) k_loop(Form1{}); else k_loop(Form0{});
   } else {
-    k_loop(std::true_type{});
+    k_loop(Form1{});
   }
   int ssum[FS];
 #pragma unroll
@@ -1617,7 +1666,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
 
   if constexpr (LP) {
     // fp32 form of the activation-sum term, in accumulator units
-    const float sum_scale = SIGNED1 ? 1.0f / (float)VSC : -(float)p.wmax * inv_vs;
+    const float sum_scale = -(float)p.wmax * inv_vs;
     const int cb = b0 + wb * FB * 32;
     auto block_access = [](const auto &a) {
       return [&a](auto xc, auto yc, auto ic) { return (float)a[decltype(xc)::value][decltype(yc)::value][decltype(ic)::value]; };

@@ -203,3 +203,22 @@ def test_shortcut_beside_large_sums(G, gemm, path, tile, wb, xb, K):
             got = G.run_conv(W, X, batch=1, H=4, W=8, cin_pad=K, cout=cols, R=1, S=1, stride=1, pad=0, halo=0, wb=wb, xb=xb,
                              sym=1, epi=epi, path=path, tile=tile)
         assert np.array_equal(got.view(np.uint32).reshape(2, rows, cols // 32), O.lowbits_pack(expect, rows, cols, 2)), scale
+
+
+# Unsigned one-plane weights are plain digits: the shortcut folds while the raw sum and the terms stay below 2^24.
+@pytest.mark.parametrize("tile", [None, 1, 2, 4, 5, 9])
+@pytest.mark.parametrize("xb", [2, 4, 8])
+def test_unsigned_shortcut_beside_large_sums(G, tile, xb):
+    amax, rows, cols = 2 ** xb - 1, 32, 32
+    K = 1 << (((2 ** 24 - 64) // amax).bit_length() - 1)
+    v = K * amax
+    rng = np.random.default_rng(8800 + xb)
+    codes = rng.integers(0, 4, size=(rows, cols)).astype(np.uint32)
+    d_short = G.to_dev(O.pack_bits(codes, rows, cols, cols, 2))
+    W, X = np.full((1, cols, K // 32), 0xFFFFFFFF, np.uint32), np.full((xb, rows, K // 32), 0xFFFFFFFF, np.uint32)
+    thr = v + np.repeat(np.arange(1, 4, dtype=np.int32)[None, :], cols, axis=0)
+    d_thr = G.to_dev(thr.astype(np.int32))
+    epi = G.epilogue(mode=G.A.EPI_BN, out_bits=2, thr=d_thr, resid_planes=d_short, resid_bits=2, resid_scale=1)
+    got = G.run_conv(W, X, batch=1, H=4, W=8, cin_pad=K, cout=cols, R=1, S=1, stride=1, pad=0, halo=0, wb=1, xb=xb, sym=0,
+                     epi=epi, path=0 if tile is None else 2, tile=tile)
+    assert np.array_equal(got.view(np.uint32).reshape(2, rows, cols // 32), O.lowbits_pack(codes, rows, cols, 2))
