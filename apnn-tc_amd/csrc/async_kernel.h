@@ -358,7 +358,7 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
     settle_results(acc);
     conv_output<FA, FB, 4, TB, MAXB>(
         p, [&](auto xc, auto yc, auto ic) { return (float)acc[decltype(xc)::value][decltype(yc)::value][decltype(ic)::value]; },
-        (float)(1 << log2vs), tab, rbase, cbase, b0, 0, lane);
+        (float)(1 << log2vs), tab, smem, rbase, cbase, b0, 0, lane);
   } else {
     EpiOperands<FA, FB> eo;
     epi_prefetch<1, PB >= 3 ? 4 : 2, true>(p, rbase, cbase, lane, eo);

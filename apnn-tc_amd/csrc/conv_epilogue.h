@@ -15,7 +15,10 @@
 //   * the words of a packed shortcut are the lane's own, read straight into the operand of fold_shortcut_lanes;
 //   * the four pixels of a 2x2 pooling window are four neighbouring lanes: the maximum of their codes is taken on
 //     the finished bit-planes, two bitwise steps per word pair;
-//   * an int32 result leaves as 16-byte stores of four consecutive channels.
+//   * int32 results of whole blocks pass 4 KB of LDS per wave, which turns them into rows: a store instruction writes
+//     eight rows of 128 bytes.  Stored as a lane holds them, 16 bytes of 64 places, a short reduction with a large
+//     result is bound by the partial lines (56x56x64 to 256 channels, 1x1 at batch 64, w1a2: 42.7 us, 35.4 in rows; 3x3
+//     on 28x28x512 at batch 64: 69.8 and 62.5).  The shares of the split-K tiles are stored that way.
 // With pixels in the registers and channels in the lanes, as these kernels were first built, a compare mask had
 // to be reversed and moved to its row by four lane writes per 64 values: 128 vector and about 100 other
 // operations per 32x32 block against 88 and 12 LDS reads here.  With the -1 / +1 weights this layout makes free of
@@ -32,6 +35,7 @@
 namespace apnn {
 
 // 4-byte-aligned vectors: output and residual rows need not start on 16 bytes
+typedef int i4 __attribute__((ext_vector_type(4)));
 typedef int i4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u2u __attribute__((ext_vector_type(2), aligned(4)));
@@ -266,11 +270,48 @@ __device__ __forceinline__ void conv_shortcut_codes(const KParams &p, long long 
 //   vs               value per accumulator unit (fp32 kernels)
 //   rbase            first pixel row;  cbase: first channel of block 0;  q0: first quad of the share
 //   MAXB             code widths with a path of their own; wider ones take the general integer path
+//   slab             NQ = 4: the work-group's operand buffers (4 KB per wave are used, after a barrier)
 template <int NX, int NY, int NQ, int TB, int MAXB, class Value>
-__device__ __forceinline__ void conv_output(const KParams &p, Value value, float vs, const uint32_t *tab, int rbase,
-                                            int cbase, int b0, int q0, int lane) {
+__device__ __forceinline__ void conv_output(const KParams &p, Value value, float vs, const uint32_t *tab, uint32_t *slab,
+                                            int rbase, int cbase, int b0, int q0, int lane) {
   const int li = lane & 31, g = lane >> 5;
   if (p.epi == APNN_EPI_INT32) {
+    if constexpr (NQ == 4) {
+      __syncthreads();  // every wave is done with the operand buffers
+      // 16-byte unit u (channels 4u ..) of row r lies at place u ^ (r % 8): no bank is met twice by eight lanes
+      i4 *mine = reinterpret_cast<i4 *>(slab) + (threadIdx.x >> 6) * 256;
+      const int r8 = lane >> 3, u = lane & 7;
+      static_for_e<0, NX * NY>([&](auto xyc) {
+        constexpr int x = decltype(xyc)::value / NY, y = decltype(xyc)::value % NY;
+        using X = std::integral_constant<int, x>;
+        using Y = std::integral_constant<int, y>;
+        static_for_e<0, 4>([&](auto qc) {
+          constexpr int q = decltype(qc)::value;
+          const i4 v = {(int)(value(X{}, Y{}, std::integral_constant<int, 4 * q>{}) * vs),
+                        (int)(value(X{}, Y{}, std::integral_constant<int, 4 * q + 1>{}) * vs),
+                        (int)(value(X{}, Y{}, std::integral_constant<int, 4 * q + 2>{}) * vs),
+                        (int)(value(X{}, Y{}, std::integral_constant<int, 4 * q + 3>{}) * vs)};
+          mine[li * 8 + ((2 * q + g) ^ (li & 7))] = v;
+        });
+        // (LDS operations of one wave complete in order)
+        const int col = cbase + y * 32 + 4 * u;
+        int *dst = reinterpret_cast<int *>(p.out) + (long long)(rbase + x * 32 + r8) * p.rowsB + col;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const i4 v = mine[(8 * k + r8) * 8 + (u ^ r8)];
+          if (rbase + x * 32 + 8 * k + r8 < p.rowsA) {
+            if (col + 4 <= p.rowsB) {
+              *reinterpret_cast<i4u *>(dst + (long long)(8 * k) * p.rowsB) = v;
+            } else {
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+                if (col + j < p.rowsB) dst[(long long)(8 * k) * p.rowsB + j] = v[j];
+            }
+          }
+        }
+      });
+      return;
+    }
     const bool full = cbase + NY * 32 <= p.rowsB;  // same for the whole wave
     static_for_e<0, NX>([&](auto xc) {
       constexpr int x = decltype(xc)::value;

@@ -1053,8 +1053,9 @@ constexpr int mfma_lp_stage_words(int PA, int PB, int FA, int FB, int WA, int WB
   const int stage = ks > 1 && vw == 4 ? 0 : 2 * (PA * WA * FA * 32 + PB * WB * FB * 32) * ld;
   const int part = ks > 1 ? ks * FB * 4 * 64 * 4 + ks * 32 : 0;
   const int xch = ksx > 1 ? 4 * ksx * ((FA / ksx) * FB * 16 + FA) * 64 : 0;
-  const int m = stage > part ? stage : part;
-  return ((m > xch ? m : xch) + 3) & ~3;
+  const int rows = ks > 1 ? 0 : 4 * ksx * 1024;  // 4 KB per wave for int32 results (conv_output)
+  const int m = stage > part ? stage : part, n = xch > rows ? xch : rows;
+  return ((m > n ? m : n) + 3) & ~3;
 }
 
 // longest reduction (32-bit words) the one- and two-block convolution tiles load without staging
@@ -1726,7 +1727,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
         for (int i = 0; i < 4 * FB; ++i) own[i] += c;
       }
       conv_output<1, 1, FB, TB, MAXB>(
-          p, [&](auto, auto, auto ic) { return own[decltype(ic)::value]; }, vs, tab, a0, b0 + yb * 32, b0, q0, lane);
+          p, [&](auto, auto, auto ic) { return own[decltype(ic)::value]; }, vs, tab, smem, a0, b0 + yb * 32, b0, q0, lane);
     } else if constexpr (KSX == 1) {
       if (fold) {
         if (EPI_LAZY) conv_shortcut_load<FA, FB>(p, own_rbase, cb, li, sc);
@@ -1741,7 +1742,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
       // (short reductions without staging have not met a barrier since the table was written)
       if (direct_k) __syncthreads();
       settle_results(acc);
-      conv_output<FA, FB, 4, TB, MAXB>(p, block_access(acc), vs, tab, own_rbase, cb, b0, 0, lane);
+      conv_output<FA, FB, 4, TB, MAXB>(p, block_access(acc), vs, tab, smem, own_rbase, cb, b0, 0, lane);
     } else {
       // Two wave groups: see below; group 0 finishes the first HA pixel blocks of every wave tile, group 1 the last
       static_assert(KSX == 2, "two wave groups");
@@ -1796,7 +1797,7 @@ __global__ __launch_bounds__(256 * KSX, OCC) void apnn_mfma_kernel(const KParams
       }
       if (fold) fold_shortcut_lanes<HA, FB>(p, own, sc, lane, log2vs);
       settle_results(own);
-      conv_output<HA, FB, 4, TB, MAXB>(p, block_access(own), vs, tab, own_rbase, cb, b0, 0, lane);
+      conv_output<HA, FB, 4, TB, MAXB>(p, block_access(own), vs, tab, smem, own_rbase, cb, b0, 0, lane);
     }
   } else if constexpr (KSX == 1) {
     epi_finish<FSC, KS, CONV, (CONV ? PA : PB) >= 3 ? 4 : 2, EPI_LAZY>(p, acc, ssum, smem, wave, lane, a0, b0, wa, wb, eo);

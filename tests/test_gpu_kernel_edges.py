@@ -222,3 +222,18 @@ def test_unsigned_shortcut_beside_large_sums(G, tile, xb):
     got = G.run_conv(W, X, batch=1, H=4, W=8, cin_pad=K, cout=cols, R=1, S=1, stride=1, pad=0, halo=0, wb=1, xb=xb, sym=0,
                      epi=epi, path=0 if tile is None else 2, tile=tile)
     assert np.array_equal(got.view(np.uint32).reshape(2, rows, cols // 32), O.lowbits_pack(codes, rows, cols, 2))
+
+
+# int32 results pass LDS into rows of 128 bytes: channels that end inside a block and inside a 16-byte unit, pixel rows that
+# end inside a tile, output rows that do not start on 16 bytes.
+@pytest.mark.parametrize("tile", [1, 2, 3, 7, 9])
+@pytest.mark.parametrize("wb,xb,C", [(1, 2, 128), (2, 2, 256), (1, 4, 64), (2, 8, 128)])
+@pytest.mark.parametrize("H,cout", [(3, 1), (7, 31), (9, 34), (13, 130), (8, 256)])
+def test_conv_int32_rows(G, tile, wb, xb, C, H, cout):
+    if C == 64 and tile == 9:
+        pytest.skip("two wave groups need 128-bit loads")
+    rng = np.random.default_rng(8900 + cout + wb)
+    W, X = O.random_planes(rng, wb, cout, C // 32), O.random_planes(rng, xb, 3 * H * H, C // 32)
+    kw = dict(batch=3, H=H, W=H, cout=cout, R=1, S=1, stride=1, pad=0, halo=0, wb=wb, xb=xb)
+    got = G.run_conv(W, X, cin_pad=C, sym=1, path=2, tile=tile, **kw)
+    assert np.array_equal(got.reshape(-1, cout), O.conv(W, X, cwords=C // 32, sym_w=1, **kw).reshape(-1, cout))
