@@ -374,8 +374,7 @@ inline hipError_t launch_async(const KParams &p, hipStream_t stream) {
   constexpr size_t stage = 2ull * (PA * TA + PB * TB) * KC * sizeof(uint32_t);
   constexpr size_t bytes = stage > slab ? stage : slab;
   static_assert(stage <= 64 * 1024, "LDS addresses of the loads fit 16 bits");
-  constexpr int MAXB = PA >= 3 ? 4 : 2;
-  constexpr size_t most = bytes + (CONV ? (conv_table_words(4, TB) + 4) * 4 + 64 * 256 : 0);
+  constexpr size_t most = bytes + (CONV ? (conv_table_words(4, TB) + 4) * 4 : 0);
   static_assert(most <= 160 * 1024, "LDS of a compute unit");
   auto kern = p.sym ? apnn_async_kernel<PA, PB, FA, FB, WA, WB, CONV, true, OCC> : apnn_async_kernel<PA, PB, FA, FB, WA, WB, CONV, false, OCC>;
   if (most > 64 * 1024) {
@@ -391,7 +390,7 @@ inline hipError_t launch_async(const KParams &p, hipStream_t stream) {
   if (p.pair_tiles != 0) q.pair_tiles = (int)tiles;
   q.xcd_rows = (p.pair_tiles == 0 && tiles % 8 == 0 && tiles >= kXcdOrderMinTiles && tilesB >= 2) ? 8 : 0;
   hipLaunchKernelGGL(kern, dim3((unsigned)(q.pair_tiles != 0 ? 2 * tiles : tiles)), dim3(256),
-                     bytes + (CONV ? conv_epilogue_bytes(p, TB, 256, MAXB) : 0), stream, q);
+                     bytes + (CONV ? conv_epilogue_bytes(p, TB) : 0), stream, q);
   return hipGetLastError();
 }
 

@@ -40,30 +40,24 @@ typedef int i4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u2u __attribute__((ext_vector_type(2), aligned(4)));
 
-// Threshold table of a work-group's channels, in LDS behind the operand buffers: float or int32 [nt][TB], then
-// one word per 32 channels with the flip flags (channel c at bit 31 - c%32).  Present for BN codes of up to four
+// Threshold table of a work-group's channels, in LDS behind the operand buffers: float or int32 [nt][TB + 4] (a channel's
+// thresholds lie in different banks: a search reads them with another index in every lane), then one word per 32 channels with the flip flags (channel c at bit 31 - c%32).  Present for BN codes of up to four
 // bits; wider codes search the thresholds in memory.
-__host__ __device__ constexpr int conv_table_words(int out_bits, int TB) { return ((1 << out_bits) - 1) * TB + TB / 32; }
+__host__ __device__ constexpr int conv_table_words(int out_bits, int TB) { return ((1 << out_bits) - 1) * (TB + 4) + TB / 32; }
 
-// words the table takes in a launch (0 where there is none), and the area of the general path behind it: 16 values per
-// lane of every wave
+// words the table takes in a launch (0 where there is none)
 __host__ __device__ inline int conv_table_words_of(const KParams &p, int TB) {
   return p.epi == APNN_EPI_BN && p.out_bits <= 4 ? (conv_table_words(p.out_bits, TB) + 3) & ~3 : 0;
 }
-// (keep in step with conv_float_codes)
-inline bool conv_general_path(const KParams &p, int max_bits) {
-  return p.epi != APNN_EPI_INT32 && !(p.epi == APNN_EPI_BN && p.out_bits <= max_bits && p.epi_float != 0 &&
-                                      p.pool != APNN_POOL_AVG2X2 && p.resid == nullptr && p.save_acc == nullptr &&
-                                      (p.resid_planes == nullptr || p.fold != 0u));
-}
-inline size_t conv_epilogue_bytes(const KParams &p, int TB, int threads, int max_bits) {
-  return 4ull * conv_table_words_of(p, TB) + (conv_general_path(p, max_bits) ? 64ull * threads : 0ull);
-}
-
-// Whether values are compared in fp32 accumulator units (float table) or as int32.
-__device__ __forceinline__ bool conv_float_codes(const KParams &p, int max_bits) {
-  return p.epi == APNN_EPI_BN && p.out_bits <= max_bits && p.epi_float != 0 && p.pool != APNN_POOL_AVG2X2 && p.resid == nullptr && p.save_acc == nullptr &&
+// Whether codes are found by comparing fp32 values in accumulator units (float table); everything but these and int32
+// results takes the general path over int32 values.
+__host__ __device__ inline bool conv_float_codes(const KParams &p, int max_bits) {
+  return p.epi == APNN_EPI_BN && p.out_bits <= max_bits && p.epi_float != 0 && p.pool != APNN_POOL_AVG2X2 &&
+         !(p.pool == APNN_POOL_MAX2X2 && p.out_bits > 2) && p.resid == nullptr && p.save_acc == nullptr &&
          (p.resid_planes == nullptr || p.fold != 0u);
+}
+inline size_t conv_epilogue_bytes(const KParams &p, int TB) {
+  return 4ull * conv_table_words_of(p, TB);
 }
 
 // The table is filled by one thread per channel.  load() requests the thresholds (first thing in the kernel, so that
@@ -97,9 +91,9 @@ struct ConvTable {
       if (as_float) {
         const int lim = 1 << 24;  // no value reaches it
         const int cl = min(max(v, -lim), lim);
-        tab[(fl ? nt - 1 - k : k) * TB + c] = __float_as_uint((float)(fl ? 1 - cl : cl) * inv);
+        tab[(fl ? nt - 1 - k : k) * (TB + 4) + c] = __float_as_uint((float)(fl ? 1 - cl : cl) * inv);
       } else {
-        tab[k * TB + c] = (uint32_t)v;
+        tab[k * (TB + 4) + c] = (uint32_t)v;
       }
     };
 #pragma unroll
@@ -108,7 +102,7 @@ struct ConvTable {
     const int32_t *src = p.thr + (long long)min(b0 + c, p.rowsB - 1) * nt;
     for (int k = MAXT; k < nt; ++k) put(k, src[k]);
     const unsigned long long m = __ballot(fl);
-    if ((c & 31) == 0) tab[nt * TB + (c >> 5)] = __brev((uint32_t)(m >> (c & 32)));
+    if ((c & 31) == 0) tab[nt * (TB + 4) + (c >> 5)] = __brev((uint32_t)(m >> (c & 32)));
   }
 };
 
@@ -194,7 +188,7 @@ __device__ __forceinline__ void conv_append_quad(const float (&v)[NX][4], const 
     float v[4];
   };
   auto thr = [&](int k) {
-    const float4 t = *reinterpret_cast<const float4 *>(at + k * TB);
+    const float4 t = *reinterpret_cast<const float4 *>(at + k * (TB + 4));
     return F4{{t.x, t.y, t.z, t.w}};
   };
   if constexpr (NB == 2) {
@@ -250,27 +244,13 @@ __device__ __forceinline__ void conv_shortcut_load(const KParams &p, int rbase, 
   }
 }
 
-// Codes of the packed shortcut for the four channels of register quad q of a share, as integers (any width).
-__device__ __forceinline__ void conv_shortcut_codes(const KParams &p, long long row, int word, int quad, int g, int (&code)[4]) {
-  const int w32 = p.rowsB >> 5;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) code[j] = 0;
-  if (word >= w32) return;
-  const uint32_t *src = p.resid_planes + row * w32 + word;
-  for (int b = 0; b < p.resid_bits; ++b) {
-    const uint32_t nib = src[(long long)b * p.rowsA * w32] >> (28 - 8 * quad - 4 * g);  // channel 0 of four at bit 3
-#pragma unroll
-    for (int j = 0; j < 4; ++j) code[j] |= (int)((nib >> (3 - j)) & 1u) << b;
-  }
-}
-
 // Output stage of one wave for NX pixel blocks of NY channel blocks (NQ = 4: whole blocks of 32 channels) or for a
 // share of NQ quads of one channel block (NY = 1, NQ < 4; the split-K tiles).
 //   value(x, y, i)   accumulator of channel 8 (i/4) + 4g + i%4 of the share, final except for `vs` (x, y, i: constants)
 //   vs               value per accumulator unit (fp32 kernels)
 //   rbase            first pixel row;  cbase: first channel of block 0;  q0: first quad of the share
 //   MAXB             code widths with a path of their own; wider ones take the general integer path
-//   slab             NQ = 4: the work-group's operand buffers (4 KB per wave are used, after a barrier)
+//   slab             the work-group's operand buffers (1 KB per quad of the share and wave are used, after a barrier)
 template <int NX, int NY, int NQ, int TB, int MAXB, class Value>
 __device__ __forceinline__ void conv_output(const KParams &p, Value value, float vs, const uint32_t *tab, uint32_t *slab,
                                             int rbase, int cbase, int b0, int q0, int lane) {
@@ -352,7 +332,7 @@ __device__ __forceinline__ void conv_output(const KParams &p, Value value, float
     for (int y = 0; y < NW; ++y) {
       if (flips && p.flip != nullptr) {
         // flip flags of the share's channels, this half's nibbles in the layout of w
-        const uint32_t f = tab[nt * TB + ((cbase - b0) >> 5) + y0 + y] >> (8 * (4 - q0 - NQ));
+        const uint32_t f = tab[nt * (TB + 4) + ((cbase - b0) >> 5) + y0 + y] >> (8 * (4 - q0 - NQ));
         const uint32_t fs = (g == 0 ? f >> 4 : f) & (0x0f0f0f0fu >> (8 * (4 - NQ)));
 #pragma unroll
         for (int b = 0; b < NB; ++b) w[y][b] ^= fs;
@@ -436,74 +416,192 @@ __device__ __forceinline__ void conv_output(const KParams &p, Value value, float
     return;
   }
 
-  // int32 values: low bits, int32 residual maps, saved sums, average pooling, values fp32 could round, wider codes.
-  // A block's values pass through the wave's part of an LDS area so that the loop over them can stay rolled: this
-  // path covers every mode and width, and unrolled over the registers it would dwarf the kernel around it.
-  int *mine = reinterpret_cast<int *>(const_cast<uint32_t *>(tab) + conv_table_words_of(p, TB)) + (threadIdx.x >> 6) * (64 * 4 * NQ) + lane * 4;
-  static_for_e<0, NX * NY>([&](auto xyc) {
-    constexpr int x = decltype(xyc)::value / NY, y = decltype(xyc)::value % NY;
-    const int row = rbase + x * 32 + li;
-    static_for_e<0, NQ>([&](auto qc) {
-      constexpr int q = decltype(qc)::value;
-      using X = std::integral_constant<int, x>;
-      using Y = std::integral_constant<int, y>;
-      int4 v;
-      v.x = (int)(value(X{}, Y{}, std::integral_constant<int, 4 * q>{}) * vs);
-      v.y = (int)(value(X{}, Y{}, std::integral_constant<int, 4 * q + 1>{}) * vs);
-      v.z = (int)(value(X{}, Y{}, std::integral_constant<int, 4 * q + 2>{}) * vs);
-      v.w = (int)(value(X{}, Y{}, std::integral_constant<int, 4 * q + 3>{}) * vs);
-      *reinterpret_cast<int4 *>(mine + q * 256) = v;  // LDS operations of one wave complete in order
-    });
-    uint32_t w[1][8];
-#pragma unroll
-    for (int b = 0; b < 8; ++b) w[0][b] = 0;
-    const bool bn = p.epi == APNN_EPI_BN, table = bn && nb <= 4;
+  // int32 values: low bits, int32 residual maps, saved sums, average pooling, maxima of three- and four-bit codes,
+  // values fp32 could round, wider codes.  A block's values pass through 4 KB of LDS per wave, so that one body
+  // (per range of code widths) serves all blocks: unrolled over the registers it would dwarf the kernel around it.  Waves
+  // of eight blocks, whose registers are full, take half a block at a time.
+  // Pooled thresholds: the four lanes of a window hold the same four pooled values, so each searches one of them and
+  // the bits meet in an OR over the quad.
+  __syncthreads();  // every wave is done with the operand buffers (split K: with the partial sums)
+  int *mine = reinterpret_cast<int *>(slab) + (threadIdx.x >> 6) * (64 * 4 * NQ) + lane * 4;
+  const bool bn = p.epi == APNN_EPI_BN;
+  auto blocks = [&](auto nb_c) {
+    constexpr int NB = decltype(nb_c)::value;
+    constexpr int QG = NX * NY >= 8 ? 2 : NQ;  // quads at a time
+    // first two planes of the shortcut words, one block ahead
+    uint32_t ahead[2] = {0, 0};
+    auto request = [&](int blk) {
+      const int row = min(rbase + (blk / NY) * 32 + li, p.rowsA - 1), word = min((cbase >> 5) + blk % NY, w32 - 1);
+      const uint32_t *src = p.resid_planes + (long long)row * w32 + word;
+      ahead[0] = src[0];
+      if (p.resid_bits > 1) ahead[1] = src[(long long)p.rowsA * w32];
+    };
+    if (pending) request(0);
 #pragma unroll 1
-    for (int q = 0; q < NQ; ++q) {
-      const int4 r = *reinterpret_cast<const int4 *>(mine + q * 256);
-      i4u v = {r.x, r.y, r.z, r.w};
-      const int c = cbase - b0 + y * 32 + 8 * (q0 + q) + 4 * g;  // four channels, all inside or all outside
-      const int gcol = b0 + c;
-      const bool ok = row < p.rowsA && gcol < p.rowsB;
-      const long long o = (long long)row * p.rowsB + gcol;
-      if (pending) {
-        int code[4];
-        conv_shortcut_codes(p, min(row, p.rowsA - 1), (cbase >> 5) + y, q0 + q, g, code);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] += code[j] * p.resid_scale;
-      }
-      if (p.resid != nullptr && ok) v += *reinterpret_cast<const i4u *>(p.resid + o);
-      if (p.save_acc != nullptr && ok) *reinterpret_cast<i4u *>(p.save_acc + o) = v;
-      const uint32_t flips = table ? tab[nt * TB + (c >> 5)] << (c & 31) : 0u;
-      uint32_t nib[8];
-#pragma unroll
-      for (int b = 0; b < 8; ++b) nib[b] = 0;
-      static_for_e<0, 4>([&](auto jc) {
-        constexpr int j = decltype(jc)::value;
-        int t = v[j];
-        if (p.pool == APNN_POOL_AVG2X2) {
-          t += (int)quad_xor1((uint32_t)t);
-          t += (int)quad_xor2((uint32_t)t);
-          t /= 4;
+    for (int blk = 0; blk < NX * NY; ++blk) {
+      const int x = blk / NY, y = blk - x * NY;
+      const int word = (cbase >> 5) + y;
+      const uint32_t first[2] = {ahead[0], ahead[1]};
+      if (pending && blk + 1 < NX * NY) request(blk + 1);
+      if (word >= w32) continue;  // same for the whole wave
+      static_for_e<0, NX * NY>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        if (blk == k) {
+          using X = std::integral_constant<int, k / NY>;
+          using Y = std::integral_constant<int, k % NY>;
+          static_for_e<0, NQ>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            const i4 v = {(int)(value(X{}, Y{}, std::integral_constant<int, 4 * q>{}) * vs),
+                          (int)(value(X{}, Y{}, std::integral_constant<int, 4 * q + 1>{}) * vs),
+                          (int)(value(X{}, Y{}, std::integral_constant<int, 4 * q + 2>{}) * vs),
+                          (int)(value(X{}, Y{}, std::integral_constant<int, 4 * q + 3>{}) * vs)};
+            *reinterpret_cast<i4 *>(mine + q * 256) = v;  // LDS operations of one wave complete in order
+          });
         }
-        uint32_t code = 0;
-        if (!bn) {
-          code = (uint32_t)t;
-        } else if (table) {
-          const int s = (int)(flips << j) < 0 ? -t : t;
-          for (int h = (nt + 1) >> 1; h > 0; h >>= 1)
-            if (s >= (int)tab[(code + h - 1) * TB + c + j]) code += h;
-        } else if (gcol < p.rowsB) {
-          code = (uint32_t)quantize_code(p, t, gcol + j);
-        }
-#pragma unroll
-        for (int b = 0; b < 8; ++b) nib[b] = (nib[b] << 1) | ((code >> b) & 1u);
       });
+      uint32_t w[1][NB];
 #pragma unroll
-      for (int b = 0; b < 8; ++b) w[0][b] = (w[0][b] << (q > 0 ? 8 : 0)) | nib[b];
+      for (int b = 0; b < NB; ++b) w[0][b] = 0;
+#pragma unroll 1
+      for (int qb = 0; qb < NQ; qb += QG) {
+        i4 v[QG];
+#pragma unroll
+        for (int q = 0; q < QG; ++q) v[q] = *reinterpret_cast<const i4 *>(mine + (qb + q) * 256);
+        const int row = rbase + x * 32 + li;
+        const int gcol = cbase + y * 32 + 8 * (q0 + qb) + 4 * g;  // of quad 0
+        const long long o = (long long)row * p.rowsB + gcol;
+        if (pending) {
+          const uint32_t *src = p.resid_planes + (long long)min(row, p.rowsA - 1) * w32 + word;
+          for (int b = 0; b < p.resid_bits; ++b) {
+            const uint32_t bits = (b == 0 ? first[0] : b == 1 ? first[1] : src[(long long)b * p.rowsA * w32]) << (8 * (q0 + qb) + 4 * g);
+            const int part = (int)((uint32_t)p.resid_scale << b);
+#pragma unroll
+            for (int q = 0; q < QG; ++q)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) v[q][j] += ((int)(bits << (8 * q + j)) >> 31) & part;
+          }
+        }
+        if (p.resid != nullptr && row < p.rowsA) {
+#pragma unroll
+          for (int q = 0; q < QG; ++q) v[q] += *reinterpret_cast<const i4u *>(p.resid + o + 8 * q);
+        }
+        if (p.save_acc != nullptr && row < p.rowsA) {
+#pragma unroll
+          for (int q = 0; q < QG; ++q) *reinterpret_cast<i4u *>(p.save_acc + o + 8 * q) = v[q];
+        }
+        if (p.pool == APNN_POOL_AVG2X2) {
+#pragma unroll
+          for (int q = 0; q < QG; ++q)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              int t = v[q][j];
+              t += (int)quad_xor1((uint32_t)t);
+              t += (int)quad_xor2((uint32_t)t);
+              v[q][j] = t / 4;
+            }
+        }
+        auto append = [&](const int (&code)[QG][4]) {
+#pragma unroll
+          for (int q = 0; q < QG; ++q)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+              w[0][b] <<= 4;  // the other lane half's nibble
+#pragma unroll
+              for (int j = 0; j < 4; ++j) w[0][b] = __builtin_amdgcn_alignbit(w[0][b], (uint32_t)code[q][j] << (31 - b), 31);
+            }
+        };
+        if (!bn) {
+          int code[QG][4];
+#pragma unroll
+          for (int q = 0; q < QG; ++q)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) code[q][j] = v[q][j];
+          append(code);
+        } else {
+          const int c0 = gcol - b0;
+          if (p.flip != nullptr) {
+            uint32_t flips = 0;  // flag of channel j of quad q at bit 31 - 8q - j
+            if constexpr (NB <= 4) {
+              flips = tab[nt * (TB + 4) + (c0 >> 5)] << (c0 & 31);
+            } else {
+#pragma unroll
+              for (int q = 0; q < QG; ++q)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) flips |= (p.flip[gcol + 8 * q + j] ? 0x80000000u : 0u) >> (8 * q + j);
+            }
+#pragma unroll
+            for (int q = 0; q < QG; ++q)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const int m = (int)(flips << (8 * q + j)) >> 31;
+                v[q][j] = (int)(((uint32_t)v[q][j] ^ (uint32_t)m) - (uint32_t)m);
+              }
+          }
+          // codes of N values each, of channels c0 + 8q + at(j)
+          auto search = [&](auto &code, const auto &s, int shift) {
+            constexpr int N = sizeof(s[0]) / sizeof(int);
+            const int *thr = NB <= 4 ? reinterpret_cast<const int *>(tab) + c0 + shift : p.thr + (long long)(gcol + shift) * nt;
+            const int pitch = NB <= 4 ? 1 : nt;  // of a channel
+#pragma unroll
+            for (int q = 0; q < QG; ++q)
+#pragma unroll
+              for (int j = 0; j < N; ++j) code[q][j] = 0;
+            for (int h = (nt + 1) >> 1; h > 0; h >>= 1) {
+              int t[QG][N];  // all reads of a level before its first compare
+#pragma unroll
+              for (int q = 0; q < QG; ++q)
+#pragma unroll
+                for (int j = 0; j < N; ++j) t[q][j] = thr[(8 * q + j) * pitch + (code[q][j] + h - 1) * (NB <= 4 ? TB + 4 : 1)];
+#pragma unroll
+              for (int q = 0; q < QG; ++q)
+#pragma unroll
+                for (int j = 0; j < N; ++j) code[q][j] += s[q][j] >= t[q][j] ? h : 0;
+            }
+          };
+          if (pooled) {
+            const int l = li & 3;
+            int s[QG][1], code[QG][1];
+#pragma unroll
+            for (int q = 0; q < QG; ++q) {
+              if (p.pool == APNN_POOL_MAX2X2) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                  int t = v[q][j];
+                  t = max(t, (int)quad_xor1((uint32_t)t));
+                  v[q][j] = max(t, (int)quad_xor2((uint32_t)t));
+                }
+              }
+              s[q][0] = l < 2 ? (l == 0 ? v[q][0] : v[q][1]) : (l == 2 ? v[q][2] : v[q][3]);
+            }
+            search(code, s, l);
+#pragma unroll
+            for (int q = 0; q < QG; ++q) {
+              uint32_t m = 0;  // plane b: nibble b, channel 0 on top
+#pragma unroll
+              for (int b = 0; b < NB; ++b) m |= (((uint32_t)code[q][0] >> b) & 1u) << (4 * b);
+              m <<= 3 - l;
+              m |= quad_xor1(m);
+              m |= quad_xor2(m);
+#pragma unroll
+              for (int b = 0; b < NB; ++b) w[0][b] = (w[0][b] << 8) | ((m >> (4 * b)) & 15u);
+            }
+          } else {
+            int s[QG][4], code[QG][4];
+#pragma unroll
+            for (int q = 0; q < QG; ++q)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) s[q][j] = v[q][j];
+            search(code, s, 0);
+            append(code);
+          }
+        }
+      }
+      finish(x, y, w, false);
     }
-    finish(x, y, w, false);
-  });
+  };
+  if (nb <= 2) blocks(std::integral_constant<int, 2>{});
+  else if (nb <= 4) blocks(std::integral_constant<int, 4>{});
+  else blocks(std::integral_constant<int, 8>{});
 }
 
 }  // namespace apnn

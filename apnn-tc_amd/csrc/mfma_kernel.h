@@ -1053,7 +1053,7 @@ constexpr int mfma_lp_stage_words(int PA, int PB, int FA, int FB, int WA, int WB
   const int stage = ks > 1 && vw == 4 ? 0 : 2 * (PA * WA * FA * 32 + PB * WB * FB * 32) * ld;
   const int part = ks > 1 ? ks * FB * 4 * 64 * 4 + ks * 32 : 0;
   const int xch = ksx > 1 ? 4 * ksx * ((FA / ksx) * FB * 16 + FA) * 64 : 0;
-  const int rows = ks > 1 ? 0 : 4 * ksx * 1024;  // 4 KB per wave for int32 results (conv_output)
+  const int rows = ks > 1 ? 0 : 4 * ksx * 1024;  // 4 KB per wave for conv_output
   const int m = stage > part ? stage : part, n = xch > rows ? xch : rows;
   return ((m > n ? m : n) + 3) & ~3;
 }
@@ -1895,10 +1895,10 @@ inline hipError_t launch_mfma(const KParams &p, hipStream_t stream) {
   constexpr size_t most_bytes = smem_bytes + (LP ? conv_table_words(PA >= 3 ? 4 : 2, TB) * sizeof(uint32_t) : 0);
   constexpr int OCC_FIT = (int)((160 * 1024) / most_bytes);
   constexpr int OCC = OCC_FIT < 1 ? 1 : (OCC_FIT < OCC_WANTED ? OCC_FIT : OCC_WANTED);
-  static_assert(smem_bytes + (LP ? (conv_table_words(4, TB) + 4) * 4 + 64 * 256 * KSX : 0) <= 160 * 1024, "LDS budget of a gfx950 compute unit");
+  static_assert(smem_bytes + (LP ? (conv_table_words(4, TB) + 4) * 4 : 0) <= 160 * 1024, "LDS budget of a gfx950 compute unit");
   auto kern = apnn_mfma_kernel<CORE, PA, PB, FA, FB, WA, WB, VW, CONV, OCC, KSX>;
-  const size_t launch_bytes = smem_bytes + (LP ? conv_epilogue_bytes(p, TB, 256 * KSX, PA >= 3 ? 4 : 2) : 0);
-  constexpr size_t attr_bytes = smem_bytes + (LP ? (conv_table_words(4, TB) + 4) * 4 + 64 * 256 * KSX : 0);
+  const size_t launch_bytes = smem_bytes + (LP ? conv_epilogue_bytes(p, TB) : 0);
+  constexpr size_t attr_bytes = smem_bytes + (LP ? (conv_table_words(4, TB) + 4) * 4 : 0);
   if (attr_bytes > 64 * 1024) {
     static bool raised = false;  // per instantiation; a repeated call is harmless
     if (!raised) {

@@ -237,3 +237,52 @@ def test_conv_int32_rows(G, tile, wb, xb, C, H, cout):
     kw = dict(batch=3, H=H, W=H, cout=cout, R=1, S=1, stride=1, pad=0, halo=0, wb=wb, xb=xb)
     got = G.run_conv(W, X, cin_pad=C, sym=1, path=2, tile=tile, **kw)
     assert np.array_equal(got.reshape(-1, cout), O.conv(W, X, cwords=C // 32, sym_w=1, **kw).reshape(-1, cout))
+
+
+# Every output form of the convolutions that is not a plain threshold code, on every tile: low bits, pooled averages and
+# maxima, flip flags, codes of one to eight bits, a shortcut scale the matrix cores do not take, an int32 map with the sums
+# saved.
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 7, 8, 9])
+@pytest.mark.parametrize("wb,xb,ob", [(1, 2, 2), (1, 2, 3), (1, 4, 4), (2, 2, 1), (1, 5, 5), (2, 8, 8)])
+@pytest.mark.parametrize("bn,pool", [(0, 0), (0, 1), (0, 2), (1, 0), (1, 1), (1, 2)])
+def test_conv_output_forms(G, tile, wb, xb, ob, bn, pool):
+    rng = np.random.default_rng(9000 + 100 * tile + 10 * xb + ob + 3 * bn + pool)
+    batch, H, C, cout = 3, 6, 128, 96
+    W, X = O.random_planes(rng, wb, cout * 9, C // 32), O.random_planes(rng, xb, batch * H * H, C // 32)
+    kw = dict(batch=batch, H=H, W=H, cout=cout, R=3, S=3, stride=1, pad=1, halo=0, wb=wb, xb=xb)
+    v = O.conv(W, X, cwords=C // 32, sym_w=1, **kw).reshape(-1, cout).astype(np.int64)
+    extra, keep = {}, []
+    if pool == 0 and ob != 3:
+        short = rng.integers(0, 4, size=v.shape).astype(np.uint32)
+        v = v + 1365 * short.astype(np.int64)
+        keep.append(G.to_dev(O.pack_bits(short, v.shape[0], cout, cout, 2)))
+        extra = dict(resid_planes=keep[-1], resid_bits=2, resid_scale=1365)
+    elif pool == 0:
+        res = rng.integers(-500, 500, size=v.shape).astype(np.int32)
+        v = v + res
+        keep += [G.to_dev(res), G.dev_empty_i32(v.size, fill=-7)]
+        extra = dict(resid=keep[0], save=keep[1])
+    if pool:  # windows in raster order, four values each
+        v = v.reshape(batch, H // 2, 2, H // 2, 2, cout).transpose(0, 1, 3, 2, 4, 5).reshape(-1, 4, cout)
+    if pool == 1:
+        s = v.sum(axis=1)
+        v = np.where(s < 0, -(-s // 4), s // 4)[:, None, :]
+    v = v.reshape(-1, cout)
+    if bn:
+        thr = np.sort(rng.integers(v.min() - 5, v.max() + 6, size=(cout, 2 ** ob - 1)), axis=1).astype(np.int32)
+        thr[0, :], thr[1, :] = np.iinfo(np.int32).min, np.iinfo(np.int32).max
+        flip = rng.integers(0, 2, size=cout).astype(np.uint8)
+        thr[flip != 0] = np.sort(-thr[flip != 0].astype(np.int64), axis=1).clip(-2 ** 31, 2 ** 31 - 1).astype(np.int32)
+        keep += [G.to_dev(thr), G.to_dev(flip)]
+        epi = G.epilogue(mode=G.A.EPI_BN, out_bits=ob, pool=pool, thr=keep[-2], flip=keep[-1], **extra)
+        q = O.bn_quantize(v.astype(np.int32), None, thr, flip, ob)
+    else:
+        epi = G.epilogue(mode=G.A.EPI_LOWBITS, out_bits=ob, pool=pool, **extra)
+        q = v & (2 ** ob - 1)
+    q = np.asarray(q).astype(np.uint32).reshape(-1, cout)
+    if pool == 2:
+        q = np.ascontiguousarray(q.reshape(-1, 4, cout).max(axis=1))
+    got = G.run_conv(W, X, cin_pad=C, sym=1, epi=epi, path=2, tile=tile, **kw).view(np.uint32).reshape(ob, -1, cout // 32)
+    assert np.array_equal(got, O.lowbits_pack(q, q.shape[0], cout, ob))
+    if "save" in extra:
+        assert np.array_equal(G.to_host(keep[1]).reshape(v.shape), v)
