@@ -125,12 +125,12 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
     voB[n] = row < p.rowsB ? ((uint32_t)row * (uint32_t)p.KW + 4u * unit) * 4u : 0xffffffffu;
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t *)smem;
-  // (m0 holds the LDS address; the compiler keeps nothing in it across statements)
+  // (m0 holds the LDS address)
   auto load_lds = [](uint32_t lds, uint32_t voff, rsrc4 rs, uint32_t soff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :
                  : "s"(lds), "v"(voff), "s"(rs), "s"(soff)
-                 : "memory");
+                 : "memory", "m0");
   };
   auto fetch = [&](int ch, int buf) {
     const bool ok = ch * KC + 4 * unit < p.KW;
