@@ -40,10 +40,10 @@ __device__ __forceinline__ int park_words(int i, unsigned long long mask, int ol
 
 template <int UNITS, bool FLAT, class Src>
 __global__ __launch_bounds__(256) void pack_planes_kernel(Src src, uint32_t *__restrict__ planes, long long words, int C,
-                                                          int cw, int first, int bits) {
+                                                          int cw, int first, int bits, long long block0) {
   const int lane = threadIdx.x & 63, half = lane >> 5;
   const int ch = 31 - (lane & 31);
-  const long long wave = (long long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long long wave = (block0 + blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long long w0 = wave * (2 * UNITS);
   if (w0 >= words) return;
   typename Src::Raw raw[UNITS];
@@ -151,8 +151,11 @@ static hipError_t launch_pack_planes(const Src &src, uint32_t *planes, int rows,
     constexpr int UNITS = decltype(units_c)::value;
     constexpr bool FLAT = decltype(flat_c)::value;
     const long long blocks = (words + 8 * UNITS - 1) / (8 * UNITS);
-    hipLaunchKernelGGL((pack_planes_kernel<UNITS, FLAT, Src>), dim3((unsigned)blocks), dim3(256), 0, s, src, planes, words, C,
-                       cw, first, bits);
+    // a grid holds fewer than 2^32 threads; tensors of more words go out in parts
+    constexpr long long most = (1ll << 24) - 1;
+    for (long long b0 = 0; b0 < blocks; b0 += most)
+      hipLaunchKernelGGL((pack_planes_kernel<UNITS, FLAT, Src>), dim3((unsigned)(blocks - b0 < most ? blocks - b0 : most)), dim3(256),
+                         0, s, src, planes, words, C, cw, first, bits, b0);
   };
   using std::integral_constant;
   if (words >= 64 * 2048) {

@@ -286,3 +286,18 @@ def test_conv_output_forms(G, tile, wb, xb, ob, bn, pool):
     assert np.array_equal(got, O.lowbits_pack(q, q.shape[0], cout, ob))
     if "save" in extra:
         assert np.array_equal(G.to_host(keep[1]).reshape(v.shape), v)
+
+
+def test_packer_beyond_one_grid(G):
+    """More than 2^32 words: the packers' grid of one wave per 64 words would exceed the threads one launch may have."""
+    rows, words = (2 ** 32 + 3 * 4096) // 3, 3
+    if torch.cuda.mem_get_info()[0] < 40 * 2 ** 30:
+        pytest.skip("needs 40 GB of device memory")
+    x = torch.randint(0, 256, (rows,), dtype=torch.uint8, device="cuda")
+    planes = torch.full((rows, words), -7, dtype=torch.int32, device="cuda")
+    G.A.check(G.A.lib().apnn_quantize_pack_u8(G.ptr(x), G.ptr(planes), rows, 1, 32 * words, 1, None), "quantize_pack_u8")
+    step = 1 << 28
+    for r in range(0, rows, step):
+        got = planes[r:r + step]
+        assert torch.equal(got[:, 0] != 0, x[r:r + step] >= 128) and bool(((got[:, 0] == 0) | (got[:, 0] == -2 ** 31)).all())
+        assert not bool(got[:, 1:].any())
