@@ -3,6 +3,7 @@
 // of packed codes, code unpacking and the int8 classifier.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <type_traits>
 
 #include "../../include/apnn_tc.h"
@@ -993,14 +994,20 @@ hipError_t launch_conv_i8_bn(const int8_t *X, const int8_t *Wt, const int32_t *t
                   : nks == 7   ? conv_i8_rows_kernel<7, false, 8, 4>
                   : nks == 2   ? conv_i8_rows_kernel<2, false, 8, 4>
                                : conv_i8_rows_kernel<0, false, 8, 4>;
+      const int variant = wreg ? 0 : wide_patch ? 1 : nks == 7 ? 2 : nks == 2 ? 3 : 4;
       if (wide_patch) grid.x = (unsigned)((groups + 7) / 8);
-      if (all > 64 * 1024) {
-        const hipError_t e0 = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024 + kRowsTable);
-        if (e0 != hipSuccess) return e0;
-      }
       int per_cu = 0, cus = 0, dev = 0;
       hipError_t e = hipGetDevice(&dev);
+      if (all > 64 * 1024 && e == hipSuccess) {
+        // once per kernel and device (a bit each; a repeated call is harmless)
+        static std::atomic<unsigned long long> raised[5];
+        const unsigned long long bit = 1ull << (dev & 63);
+        if ((raised[variant].load(std::memory_order_relaxed) & bit) == 0) {
+          e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  80 * 1024 + kRowsTable);
+          if (e == hipSuccess) raised[variant].fetch_or(bit, std::memory_order_relaxed);
+        }
+      }
       if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
       if (e == hipSuccess)
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kern), 64 * nwav, all);
