@@ -448,6 +448,10 @@ int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, i
     if (KW >= 32 && nb32 <= 640) return 5;
     if (KW >= 64 && nb32 <= 14 * cus) return 5;  // up to 3584 blocks: 16x16 maps at batch 16, 896 channels
   }
+  // w1a1 products of up to two 64x64 tiles per compute unit: one plane on either side leaves nothing that a larger or a
+  // split tile would save (int32, 512^3 3.4 against 3.8-4.0 us on 32x64 split K, 1000x2016x2048 7.7 against 8.2 us on 128x64;
+  // 2048^3, 1024 tiles: 11.1 against 10.5 us)
+  if (!conv && planes == 2 && ntiles(2) <= 2 * cus && !(KW >= 32 && ntiles(4) <= cus)) return 2;
   if (rowsB <= 64 && ntiles(3) >= cus) return 3;
   if (rowsB > 64) {
     const int big = conv ? 7 : 6;

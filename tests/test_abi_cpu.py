@@ -323,6 +323,15 @@ def test_pinned_tile_below_the_crossover_names_a_popcount_tile(wb, xb, tile):
         assert rc == 0 and plan.kernel == A.KERNEL_MFMA_FP4
 
 
+@pytest.mark.parametrize("M,N,K,small", [(512, 512, 512, True), (1024, 1024, 1024, True), (1000, 2016, 2048, True),
+                                         (100, 8192, 1024, True), (128, 512, 4096, False), (2048, 2048, 2048, False)])
+def test_w1a1_products_take_64x64_tiles_up_to_two_per_unit(M, N, K, small):
+    """One plane on either side: the 64x64 tile (2) is ahead of the split and the larger ones while there are at most two
+    per compute unit and the 32x32 split-K tile does not give every unit one block."""
+    rc, plan = _plan_gemm(M=M, N=N, K=K, wb=1, xb=1, path=A.PATH_AUTO)
+    assert rc == 0 and plan.kernel == A.KERNEL_MFMA_FP4 and (plan.tile == 2) == small
+
+
 def test_patch_capacity_bounds_every_tile():
     """The patch-resident convolution kernel stages, per work-group, the contiguous range of padded-frame
     pixels that its tile of consecutive output rows reads; the host sizes that range from a closed-form
