@@ -116,7 +116,8 @@ def test_async_gemm_tile(G, wb, xb, sym, M, N, K):
 
 
 # Convolution tiles 128x256 and 128x128 (operands loaded straight to LDS): images smaller and larger than a tile,
-# channel words that are and are not a power of two, taps that straddle a chunk, stride, padding, every output form.
+# channel words that are and are not a power of two, taps that straddle a chunk, stride, padding, int32 results,
+# thresholds and a shortcut (the other output forms: test_conv_output_forms).
 @pytest.mark.parametrize("tile", [1, 7])
 @pytest.mark.parametrize("wb,xb", [(1, 2), (1, 3), (1, 4), (2, 2)])
 @pytest.mark.parametrize("batch,H,C,cout,R,stride,pad", [(1, 5, 128, 32, 3, 1, 1), (2, 9, 384, 288, 3, 1, 1),
@@ -301,3 +302,23 @@ def test_packer_beyond_one_grid(G):
         got = planes[r:r + step]
         assert torch.equal(got[:, 0] != 0, x[r:r + step] >= 128) and bool(((got[:, 0] == 0) | (got[:, 0] == -2 ** 31)).all())
         assert not bool(got[:, 1:].any())
+
+
+# Sums just below 2^24 on the kernels that load straight to LDS, on convolutions and with FP6 digits: all-ones operands
+# give the largest value the host admits, random ones are checked with the oracle.
+@pytest.mark.parametrize("wb,xb", [(1, 2), (1, 4), (2, 2), (2, 8), (4, 4)])
+@pytest.mark.parametrize("gemm,tile", [(1, 6), (1, 2), (0, 1), (0, 7), (0, 2), (0, 9)])
+@pytest.mark.parametrize("sym", [0, 1])
+def test_exact_just_below_the_limit(G, gemm, tile, wb, xb, sym):
+    span = (2 ** wb - 1) * (2 ** xb - 1)
+    K = 128 * (1 << ((2 ** 24 - 1) // span // 128).bit_length() - 1)  # words per pixel a power of two
+    rows = cols = 32
+    rng = np.random.default_rng(9100 + 10 * wb + xb)
+    for W, X in ((np.full((wb, cols, K // 32), 0xFFFFFFFF, np.uint32), np.full((xb, rows, K // 32), 0xFFFFFFFF, np.uint32)),
+                 (O.random_planes(rng, wb, cols, K // 32), O.random_planes(rng, xb, rows, K // 32))):
+        if gemm:
+            got = G.run_gemm(W, X, cols, rows, K, wb, xb, sym=sym, path=2, tile=tile).reshape(cols, rows)
+        else:
+            got = G.run_conv(W, X, batch=1, H=4, W=8, cin_pad=K, cout=cols, R=1, S=1, stride=1, pad=0, halo=0, wb=wb, xb=xb,
+                             sym=sym, path=2, tile=tile).reshape(rows, cols).T
+        assert np.array_equal(got, O.gemm(W, X, cols, rows, K, wb, xb, sym_w=sym, nthreads=8))

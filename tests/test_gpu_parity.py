@@ -505,13 +505,13 @@ def test_conv_packed_residual(G, path, tile):
     assert np.array_equal(got, O.lowbits_pack(q, acc.shape[0], C, ob))
 
 
-@pytest.mark.parametrize("scale", [1, 3, 8, 7, 11, 21, -5, -12, 37, 1 << 14])
+@pytest.mark.parametrize("scale", [1, 3, 8, 7, 11, 21, -5, -12, 37, 1 << 14, 1365, -1365])
 @pytest.mark.parametrize("path,tile", [(0, None), (2, 1), (2, 2), (2, 3), (2, 4), (2, 5), (2, 8), (2, 9), (3, 2), (4, 0), (4, 3),
                                        (5, 1)])
 def test_conv_packed_shortcut_scales(G, path, tile, scale):
     """Shortcut codes of two bits and of one bit times an integer scale, added before the thresholds.  The FP4
-    kernels add the term on the matrix cores when the scale is a sum of two terms +-{1, 3} * 2^j (every
-    scale here but 37, which takes the per-value path like the other cores), symmetric and unsigned
+    kernels add the term on the matrix cores when the scale is a sum of two terms +-m * 2^j, m up to 15 (every
+    scale here but +-1365, which take the per-value path like the other cores), symmetric and unsigned
     weights, every kind of tile (waves tile the output, split K, two wave groups, patch-resident,
     expanded while staging)."""
     rng = np.random.default_rng(1980 + path + 7 * (tile or 0) + (scale & 1023))
