@@ -190,7 +190,7 @@ int choose_xs_tile(int rowsA, int rowsB, bool conv) {
   return 2;
 }
 
-// The FP4 matrix-core kernels accumulate in fp32: every partial sum is a multiple of 1/4 and stays
+// The FP4 / FP6 matrix-core kernels accumulate in fp32: every partial sum is a multiple of 1/4 (FP6: 1/64) and stays
 // exact while the largest possible result, K * (2^w - 1) * (2^a - 1), is below 2^24.
 bool fp4_exact(long long kwords, int wb, int xb) {
   return kwords * 32 * ((1LL << wb) - 1) * ((1LL << xb) - 1) < (1LL << 24);

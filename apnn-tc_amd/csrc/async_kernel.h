@@ -13,10 +13,11 @@
 //   - symmetric one-plane weights are -1 / +1 operands and unsigned ones need no correction, so nothing is counted
 //     (wider symmetric weights: activation sums, as in mfma_kernel.h);
 //   - the last k-step of a chunk carries the barrier, and expands the first operands of the next chunk.
-// w1a2: 6.1 vector operations per matrix instruction instead of 6.75 plus staging, 212 registers.  8192^3 w1a2 229 ->
-// 221 us: the matrix pipes are busy 65 % of the time at the 1.85 GHz that the card holds under this load (2.2 GHz
-// where they are less busy).  4096^3 w1a4 58.2 -> 45.2 us (48.0 with FP6 digits alone): one round of tiles, whose
-// 67 MB of results leave the chip after the last product.
+// w1a2: 6.1 vector operations per matrix instruction in the loop instead of 6.75 plus staging, 212 registers.  8192^3 w1a2
+// 226 -> 220 us.  Counters there: matrix pipes 64 % busy, vector pipes 63 %, waves waiting 14 % of their lifetime, 1.89
+// GHz.  The loop alone would leave the matrix pipes above 90 % busy; what takes the rest (a chunk's wait and barrier, the
+// output stage, 268 MB of results) has not been separated.  4096^3 w1a4 58.2 -> 45.2 us (48.0 with FP6 digits alone):
+// one round of tiles, whose 67 MB of results leave the chip after the last product.
 // Convolution: a load's lane decodes the tap of its 16 bytes once per chunk; padding pixels are disabled loads, which
 // write zeros.  Two tiles of 128x256 per compute unit, three of 128x128.  3x3 convolutions at batch
 // 64: 56x56x256 76 -> 66 us, 28x28x512 78 -> 64, 14x14x512 28 -> 23 (bounded by vector work, 9.8 operations per matrix

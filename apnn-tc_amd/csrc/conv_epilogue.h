@@ -14,7 +14,8 @@
 //   * corrections that depend on the pixel (activation sums) are one register per pixel block;
 //   * the words of a packed shortcut are the lane's own, read straight into the operand of fold_shortcut_lanes;
 //   * the four pixels of a 2x2 pooling window are four neighbouring lanes: the maximum of their codes is taken on
-//     the finished bit-planes, two bitwise steps per word pair;
+//     the finished bit-planes, two bitwise steps per word pair (codes of three and four bits: on the values, before
+//     the search);
 //   * int32 results of whole blocks pass 4 KB of LDS per wave, which turns them into rows: a store instruction writes
 //     eight rows of 128 bytes.  Stored as a lane holds them, 16 bytes of 64 places, a short reduction with a large
 //     result is bound by the partial lines (56x56x64 to 256 channels, 1x1 at batch 64, w1a2: 42.7 us, 35.4 in rows; 3x3

@@ -9,8 +9,8 @@
 //           2-bit digits (plane pairs); digit pair (da, db) is one instruction per 32x32 block and
 //           64 k -- at the same issue cost as the int8 instruction, so twice its rate -- with the
 //           weight 4^(da+db) applied by the instruction's E8M0 block scale.  Products are multiples
-//           of 1/4 and the host only launches this core while K * (2^w - 1) * (2^a - 1) < 2^24, so the
-//           fp32 accumulators are exact and the result is acc * 4.
+//           of 1/4 (FP6: of 1/64) and the host only launches this core while K * (2^w - 1) * (2^a - 1) < 2^24, so the
+//           fp32 accumulators are exact and the result is acc * fp_scale.
 //           With more than two planes on either side both operands are FP6 (e2m3) digits of up to four planes
 //           (expand_fp6): same instruction and rate, half the matrix instructions (a quarter for w4a4), about
 //           the same expansion work.  w1a4 at 4096^3 58.1 -> 48.0 us, w4a4 at 4096 x 333 x 4096 71.9 -> 23.6 us
