@@ -669,7 +669,7 @@ int build_conv_params(const apnn_conv_desc *d, KParams &p, int *vw_out) {
   p.S = d->S;
   p.stride = d->stride;
   p.pad = d->halo ? 0 : d->pad;
-  p.magicC32 = magic_of(C32);
+  p.magicC32 = d->R * d->S == 1 ? 0u : magic_of(C32);  // one tap: every word belongs to tap 0, however many there are
   p.magicS = magic_of(d->S);
   p.pool_order = d->epi.pool != APNN_POOL_NONE;
   p.sym = d->weight_mode == APNN_WEIGHT_SYMMETRIC;

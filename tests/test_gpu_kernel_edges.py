@@ -322,3 +322,13 @@ def test_exact_just_below_the_limit(G, gemm, tile, wb, xb, sym):
             got = G.run_conv(W, X, batch=1, H=4, W=8, cin_pad=K, cout=cols, R=1, S=1, stride=1, pad=0, halo=0, wb=wb, xb=xb,
                              sym=sym, path=2, tile=tile).reshape(rows, cols).T
         assert np.array_equal(got, O.gemm(W, X, cols, rows, K, wb, xb, sym_w=sym, nthreads=8))
+
+
+@pytest.mark.parametrize("path,tile", [(0, None), (1, 0), (1, 2), (2, 1), (2, 2), (2, 4), (2, 7), (2, 9), (3, 2), (5, 2)])
+def test_very_long_single_tap(G, path, tile):
+    """A 1x1 filter over 174760 words per pixel: the multiply-high that finds a word's tap is exact up to 65536 words."""
+    K, rows, cols = 32 * 174760, 32, 32
+    W, X = np.full((1, cols, K // 32), 0xFFFFFFFF, np.uint32), np.full((2, rows, K // 32), 0xFFFFFFFF, np.uint32)
+    got = G.run_conv(W, X, batch=1, H=4, W=8, cin_pad=K, cout=cols, R=1, S=1, stride=1, pad=0, halo=0, wb=1, xb=2, sym=0,
+                     path=path, tile=tile)
+    assert np.all(got == 3 * K)
