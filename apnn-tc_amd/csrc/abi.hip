@@ -327,9 +327,7 @@ int patch_pixels(const KParams &p, int R, int rows) {
 // Tile of the patch-resident convolution kernel, or -1 when it does not apply: the patch (at most
 // 1024 pixels) and the filter block of all taps must fit in LDS twice per compute unit.  When the
 // library chooses (`automatic`) the kernel is taken only where it measures faster than the
-// implicit-GEMM kernel: at most 64 output channels over at most 64 input channels (one channel
-// chunk, e.g. the first stage of ResNet18) with enough 128x64 tiles to occupy the chip, and layers whose
-// channel words are odd in number.
+// implicit-GEMM kernels; the figures below are microseconds in graph replay, theirs first, w1a2 with threshold codes.
 int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
   int cus = device_cus();
   if (cus <= 0) cus = 256;
@@ -347,14 +345,31 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
   };
   if (automatic) {
     if (tile_pin != 0) return -1;  // a pinned tile names a tile of the implicit-GEMM families
-    const int t = 3;               // 128 x 64
-    if (p.rowsB <= 64 && p.C32 <= 2 && taps > 1 && fits(t) && ntiles(t) >= 2 * cus) return t;
-    // An odd number of channel words (96 channels: the second layer of the VGG variant) leaves the
-    // implicit-GEMM kernel with 32-bit loads and its two smallest tiles; this kernel reads pixels, not
-    // k-chunks, and is 22-34 % ahead there (56x56x96 -> 256 at batch 8 / 64).
-    // (256x64 tiles while 128x64 would give fewer than four work-groups per compute unit: 9 % ahead at batch 8)
-    if ((p.C32 & 1) && p.C32 >= 3 && taps > 1 && fits(t) && ntiles(t) >= 2 * cus)
-      return (ntiles(t) < 4 * cus && fits(1)) ? 1 : t;
+    if (taps == 1 || !fits(3)) return -1;
+    // 256x64 tiles (three work-groups per unit at a time, against four of 128x64) where they save a round: 56x56x96 to
+    // 256 channels at batch 64 39.8 against 42.9, 27x27x96 to 256 12.6 against 14.9.  Not with four activation planes,
+    // whose patch is twice as large (107 against 92); with two weight planes over many chunks of channels also at equal
+    // rounds, as each tile expands its filter block again (28x28x320 to 256 at batch 64 31.9 against 39.1).
+    const long long n128 = ntiles(3), r128 = (n128 + 4 * cus - 1) / (4 * cus), r256 = (ntiles(1) + 3 * cus - 1) / (3 * cus);
+    const bool tall = p.planesA <= 3 && fits(1) && (r256 < r128 || (p.planesB > 1 && p.C32 > 8 && r256 == r128));
+    const int t = tall ? 1 : 3;
+    const bool plain = taps == 9 && p.S == 3 && p.stride == 1;  // the filters with an unrolled loop, the densest patches
+    // One chunk of channels (56x56x64 to 64 at batch 8 5.3 -> 4.6, 196 tiles; 28x28x64 to 192 at batch 64 11.8 -> 9.1;
+    // below half a tile per unit 128x64 leaves too much idle: 4.3 -> 4.6 with 98), or channel words without 128-bit
+    // loads, which leave the others their 32- and 64-bit forms (56x56x96 to 256 at batch 4 / 64 11.4 -> 7.4 / 68.9 -> 40.6,
+    // 14x14x960 to 1024 at batch 16 33.4 -> 27.0, 7x7x480 to 512 at batch 64 18.2 -> 13.4).  A single channel word fills
+    // half a chunk: to many channels it loses (32x32x32 to 1024 at batch 3 6.3 -> 6.7).
+    if ((p.C32 <= 2 || p.C32 % 4 != 0) && (p.C32 > 1 || p.rowsB <= 64)) {
+      if (plain && 2 * n128 >= cus) return t;
+      // other filter sizes and strides
+      if (((p.rowsB <= 64 && p.C32 <= 2) || (p.C32 & 1)) && n128 >= 2 * cus) return t;
+    }
+    // 128 channels to at most 128 from 1.5 tiles per unit (28x28 at batch 64 9.9 -> 8.9, 56x56 at batch 64 28.0 -> 22.0; to
+    // 256 channels the 128x256 tile of async_kernel.h is ahead, 13.6 -> 14.8)
+    if (plain && p.C32 == 4 && p.rowsB <= 128 && 2 * n128 >= 3 * cus) return t;
+    // 256 channels at 1.5 to 2 tiles per unit, all resident at once (14x14 to 256 at batch 64 9.9 -> 9.3, w1a4 17.4 -> 15.5;
+    // w1a3, whose two FP4 digits cost as much as w1a4's, is level: 13.1 -> 13.4 on 28x28 at batch 16)
+    if (plain && p.C32 == 8 && p.planesA != 3 && 2 * n128 >= 3 * cus && n128 <= 2 * cus) return t;
     return -1;
   }
   if (tile_pin != 0) {

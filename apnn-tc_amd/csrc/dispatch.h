@@ -127,6 +127,14 @@ constexpr int kPatchTileCount = 5;
 constexpr int kPatchTileRows[kPatchTileCount] = {128, 256, 64, 128, 64};
 constexpr int kPatchTileCols[kPatchTileCount] = {128, 64, 128, 64, 64};
 
+// LDS words a work-group of that kernel stages: patch, filter block of all taps, pixel sums (two weight planes); at
+// least the 16 KB that the output stage uses
+constexpr size_t patch_stage_words(int PA, int PB, int TB, int taps, int cap) {
+  const size_t da = (PA + 1) / 2, db = (PB + 1) / 2;
+  const size_t words = (da * cap * 8 + db * (size_t)taps * TB * 8 + (PB > 1 ? ((size_t)cap + 3) / 4 * 4 : 0));
+  return words > 4096 ? words : 4096;
+}
+
 // aux_kernels.hip
 hipError_t launch_pack_bits(const uint32_t *values, uint32_t *planes, int rows, int C, int cpad, int bits,
                             hipStream_t s);

@@ -699,7 +699,7 @@ __device__ __forceinline__ int fold_scale(const KParams &p, int lane, int log2vs
   return (int)(e8 * 0x01010101u);
 }
 
-// Lanes are channels (GEMM entry points, patch-resident and expand-while-staging kernels).  res: the wave's
+// Lanes are channels (GEMM entry points and the expand-while-staging kernel).  res: the wave's
 // published shortcut words, index ((x * 2 + plane) * FB + y) * 32 + row.
 template <int FS, int FA, int FB>
 __device__ __forceinline__ void fold_shortcut(const KParams &p, v16f (&acc)[FA][FB], const uint32_t *res, int lane) {

@@ -1,9 +1,8 @@
 // Patch-resident convolution on the matrix cores (FP4 operands, see mfma_kernel.h for the encoding).
 //
-// The implicit-GEMM kernel in mfma_kernel.h gathers, for every filter tap, the packed activation
-// words of every output pixel of its tile and expands them to matrix-core operands in registers --
-// R*S times per input pixel and once more per column tile.  Here the input pixels a tile needs are
-// expanded ONCE into LDS and every tap reads them in place:
+// The implicit-GEMM kernels gather, for every filter tap, the packed activation words of every output pixel of
+// their tile and expand them to matrix-core operands in registers -- R*S times per input pixel and once more per
+// column tile.  Here the input pixels a tile needs are expanded ONCE into LDS and every tap reads them in place:
 //
 //   * In the zero-padded frame (stored frame plus `pad` pixels on every side, PHs x PWs per image) the
 //     input pixel of output pixel (b, oy, ox) and tap (r, s) has the linear index
@@ -13,47 +12,78 @@
 //   * Per chunk of 64 channels the work-group stages the patch (bit-plane words -> FP4 digit
 //     operands, 16 bytes per pixel, 32-channel word and digit; padding pixels are zeros) and the
 //     filter block of its output channels for all taps (same encoding), then runs
-//     taps k-steps of pure LDS reads + MFMA:  A operand = patch[base(row) + tap offset], B operand =
-//     filter[tap][column].
-//   * Per-pixel activation sums (for the symmetric-weight correction) are taken once per patch pixel
-//     while staging; a row's window sum is the sum over taps of those.
+//     taps k-steps of pure LDS reads + MFMA: first operand = filter[tap][channel], second = patch[base(pixel) + tap
+//     offset].  The packed words of the next chunk are requested before the k-steps of this one.
+//   * One-plane weights are -1 / +1 or 0 / 1 operands (expand_w1) and need no correction.  With two planes, symmetric:
+//     per-pixel activation sums are taken once per patch pixel while staging; a pixel's window sum is the sum over taps.
 //
-// Output stage, tile-to-row mapping, epilogue operands and all quantizing modes are the ones of the
-// implicit-GEMM kernel (epi_prefetch / epi_finish).
+// The accumulator holds pixels in the lanes and channels in the registers; the output stage is conv_output.
+//
+// What bounds it.  With pixels in the registers and channels in the lanes, activation sums for one-plane weights and
+// a filter address per word, vector issue did: 62 vector operations per matrix instruction on 56x56x64.  What they became:
+// the lane-local output stage, -1 / +1 weights (no sums), filter words at a constant stride from one offset per thread, tap
+// loops unrolled for 3x3 (addresses are immediates), operands of a tap read behind the products of the one before.  Then
+// residency: the staging of one work-group hides behind the products of others, so registers are cut for four
+// work-groups per compute unit (three where a wave has four blocks; what spills is the general output path alone).
+// us before -> without and with the cut, w1a2 with threshold codes in graph replay: 56x56x64 to 64 at batch 64 14.6 -> 11.6 ->
+// 10.6; 56x56x96 to 256 at batch 64 68.9 -> 53.6 -> 40.0 (256x64 tiles); w1a4 there 169 -> 90.  Left: the two LDS reads per
+// matrix instruction pair of a 2x2-block wave are the LDS rate (128 bytes a clock), so long reductions stay level with
+// async_kernel.h (56x56x256 at batch 64 59 against 61 us).  A 256x128 tile of 4x2 blocks reads less, but two of them per
+// unit leave their last round emptier: 62 us there, 68 against 60 on 28x28x512.
 #pragma once
 #include "mfma_kernel.h"
 
 namespace apnn {
 
+// What is known of the filter when the kernel is built.  One kernel for all, with the forms on branches, joins the
+// accumulators of both tap loops by copies and the loads of both widths by waits (56x56x64 at batch 64 13.6 -> 12.4 us,
+// 56x56x256 81 -> 75, on 256x64 tiles before the cut).
+//   PF_ANY        any filter, any number of channel words: a loop over the taps
+//   PF_3x3_ODD    3x3, an odd number of channel words: 32-bit loads
+//   PF_3x3_PAIRS  3x3, an even number of channel words: 64-bit loads
+enum PatchForm { PF_ANY = 0, PF_3x3_ODD = 1, PF_3x3_PAIRS = 2 };
+
+// Work-groups per compute unit that the registers are cut for, by the 32x32 blocks of a wave (measured above).
+constexpr int patch_occupancy(int blocks) { return blocks == 4 ? 3 : 4; }
+
 constexpr int PATCH_NPT = 4;  // patch pixels per thread (patch capacity = 4 * 256 pixels)
 
-template <int PA, int PB, int FA, int FB, int WA, int WB, int OCC>
-__global__ __launch_bounds__(256, OCC) void apnn_patch_conv_kernel(const KParams p) {
+template <int PA, int PB, int FA, int FB, int WA, int WB, int FORM>
+__global__ __launch_bounds__(256, patch_occupancy(FA * FB)) void apnn_patch_conv_kernel(const KParams p) {
   static_assert(WA * WB == 4, "four waves tile the output");
   constexpr int DA = (PA + 1) / 2, DB = (PB + 1) / 2;
   constexpr int NT = 256;
   constexpr int TA = WA * FA * 32, TB = WB * FB * 32;
-  constexpr int DIRECT_BITS = PA >= 3 ? 4 : 2;
+  static_assert(NT % TB == 0, "a thread stages the filter words of one channel");
+  constexpr int MAXB = PA >= 3 ? 4 : 2;
+  constexpr bool ONE = PB == 1;  // -1 / +1 or 0 / 1 operands: the accumulator is the result
 
   extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 31, g = lane >> 5;
   const int wa = wave / WB, wb = wave % WB;
   const int tilesB = (p.rowsB + TB - 1) / TB;
   const int a0 = (blockIdx.x / tilesB) * TA;
   const int b0 = (blockIdx.x % tilesB) * TB;
-  const int taps = p.KW / p.C32;
+  const int taps = FORM != PF_ANY ? 9 : p.KW / p.C32;
   const int cap = p.patch_cap;
 
-  uint32_t *patchA = smem;                                 // [DA][cap][2 words][4 dwords]
-  uint32_t *filtB = patchA + DA * cap * 8;                 // [DB][taps][TB][2 words][4 dwords]
-  int *pixsum = reinterpret_cast<int *>(filtB + DB * taps * TB * 8);  // [cap]
+  uint32_t *patchA = smem;                                 // [DA][2 words][cap][4 dwords]
+  uint32_t *filtB = patchA + DA * cap * 8;                 // [DB][2 words][taps][TB][4 dwords]
+  int *pixsum = reinterpret_cast<int *>(filtB + DB * taps * TB * 8);  // [cap], two weight planes only
+  uint32_t *tab = smem + patch_stage_words(PA, PB, TB, taps, cap);    // thresholds of the tile's channels
+  const bool need_sum = !ONE && p.sym != 0;
+  const int log2vs = ONE ? 1 : need_sum ? 3 : 2;  // value per accumulator unit
+  const float inv_vs = ONE ? 0.5f : need_sum ? 0.125f : 0.25f;
+
+  ConvTable<TB, PA >= 3 ? 15 : 3, MAXB> table;
+  table.load(p, b0);
 
   // ---- tile geometry.  Only the tile's first row is decoded with full divisions (uniform); every
   // other row and patch pixel is a small offset from it, for which the multiply-high quotients are
   // exact. -----------------------------------------------------------------------------------------
   const int last_row = min(a0 + TA, p.rowsA) - 1;
-  const int R = taps / p.S;
+  const int R = FORM != PF_ANY ? 3 : taps / p.S;
   const bool pooled = p.pool_order != 0;
   const int gw = pooled ? p.Wo >> 1 : p.Wo, gh = pooled ? p.Ho >> 1 : p.Ho;  // row grid (windows when pooling)
   const int gst = pooled ? 2 * p.stride : p.stride;                          // its step in the padded frame
@@ -83,7 +113,7 @@ __global__ __launch_bounds__(256, OCC) void apnn_patch_conv_kernel(const KParams
     return;
   }
 
-  // this lane's rows: patch-relative pixel index of row li of each of its FA row blocks
+  // this lane's pixels: LDS word of pixel li of each of its FA blocks
   int prow[FA];
 #pragma unroll
   for (int x = 0; x < FA; ++x) prow[x] = row_base(min((wa * FA + x) * 32 + li, last_row - a0)) - q_lo;
@@ -102,16 +132,16 @@ __global__ __launch_bounds__(256, OCC) void apnn_patch_conv_kernel(const KParams
   for (int pl = 0; pl < PB; ++pl)
     rsrcB[pl] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t *>(p.B + pl * p.planeB), 0,
                                                   (int)(uint32_t)(p.planeB * 4), 0x00020000);
-  // word pair at byte offset boff (kOff: zeros); without 64-bit loads (odd number of channel words) the
+  // word pair at byte offset boff + soff (boff kOff: zeros); without 64-bit loads (odd number of channel words) the
   // second word of the last pair does not exist
-  auto load_pair = [&](__amdgpu_buffer_rsrc_t rsrc, uint32_t boff, auto pair_c, bool second, uint32_t &w0,
+  auto load_pair = [&](__amdgpu_buffer_rsrc_t rsrc, uint32_t boff, uint32_t soff, auto pair_c, bool second, uint32_t &w0,
                        uint32_t &w1) {
     if constexpr (decltype(pair_c)::value) {
-      const auto v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)boff, 0, 0);
+      const auto v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)boff, (int)soff, 0);
       w0 = v[0], w1 = v[1];
     } else {
-      w0 = __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)boff, 0, 0);
-      w1 = __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(second && boff != kOff ? boff + 4 : kOff), 0, 0);
+      w0 = __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)boff, (int)soff, 0);
+      w1 = __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(second && boff != kOff ? boff + 4 : kOff), (int)soff, 0);
     }
   };
 
@@ -124,7 +154,7 @@ __global__ __launch_bounds__(256, OCC) void apnn_patch_conv_kernel(const KParams
   for (int j = 0; j < PATCH_NPT; ++j) {
     const int q = tid + j * NT;
     poff[j] = kOff;
-    if (q < npp) {
+    if (j * NT < npp && q < npp) {
       int xp = xp0 + q;
       const int cy = (int)fast_div((uint32_t)xp, (uint32_t)p.PWs, p.magicPW);
       xp -= cy * p.PWs;
@@ -137,6 +167,67 @@ __global__ __launch_bounds__(256, OCC) void apnn_patch_conv_kernel(const KParams
         poff[j] = ((((uint32_t)img * (uint32_t)p.Hs + (uint32_t)iy) * (uint32_t)p.Ws + (uint32_t)ix) * (uint32_t)p.C32) << 2;
     }
   }
+  // filter words this thread stages: one channel, taps tap0, tap0 + TSTEP, ...; FT of them held in registers
+  constexpr int TSTEP = NT / TB, FT = TSTEP >= 4 ? 3 : 5;
+  const int fcol = tid % TB, tap0 = tid / TB;
+  const uint32_t foff = b0 + fcol < p.rowsB
+                            ? ((uint32_t)(b0 + fcol) * (uint32_t)taps + (uint32_t)tap0) * (uint32_t)p.C32 << 2
+                            : kOff;
+
+  const bool pair_ok = FORM == PF_3x3_PAIRS || (FORM == PF_ANY && (p.C32 & 1) == 0);  // 64-bit loads of a channel-word pair
+  const int nchunks = (p.C32 + 1) >> 1;
+  uint32_t pw0[PATCH_NPT][PA], pw1[PATCH_NPT][PA], fw0[FT][PB], fw1[FT][PB];
+  auto filter_load_w = [&](int cw, int first, auto pair_c) {
+#pragma unroll
+    for (int j = 0; j < FT; ++j) {
+      const uint32_t boff = tap0 + first + j * TSTEP < taps ? foff : kOff;
+      const uint32_t soff = (uint32_t)((first + j * TSTEP) * p.C32 + cw) << 2;
+#pragma unroll
+      for (int pl = 0; pl < PB; ++pl) load_pair(rsrcB[pl], boff, soff, pair_c, cw + 1 < p.C32, fw0[j][pl], fw1[j][pl]);
+    }
+  };
+  // packed words of a chunk: patch pixels and the first batch of filter words (one branch on the load width around
+  // all of them)
+  auto request_w = [&](int cw, auto pair_c) {
+#pragma unroll
+    for (int j = 0; j < PATCH_NPT; ++j) {
+      if (j * NT < npp) {
+#pragma unroll
+        for (int pl = 0; pl < PA; ++pl)
+          load_pair(rsrcA[pl], poff[j], (uint32_t)cw << 2, pair_c, cw + 1 < p.C32, pw0[j][pl], pw1[j][pl]);
+      }
+    }
+    filter_load_w(cw, 0, pair_c);
+  };
+  auto request = [&](int cw) {
+    if (pair_ok) request_w(cw, std::true_type{}); else request_w(cw, std::false_type{});
+  };
+  // Operands of a pixel's (channel's) two words; the words lie in blocks of their own, so that consecutive lanes read and
+  // write consecutive 16-byte units (level with the words side by side: reads 32 bytes apart meet no bank twice either).
+  auto put = [](uint32_t *at, int block, const v8i &e0, const v8i &e1) {
+    *reinterpret_cast<uint4 *>(at) = make_uint4((uint32_t)e0[0], (uint32_t)e0[1], (uint32_t)e0[2], (uint32_t)e0[3]);
+    *reinterpret_cast<uint4 *>(at + block) = make_uint4((uint32_t)e1[0], (uint32_t)e1[1], (uint32_t)e1[2], (uint32_t)e1[3]);
+  };
+  auto filter_store = [&](int first) {
+#pragma unroll
+    for (int j = 0; j < FT; ++j) {
+      const int tap = tap0 + first + j * TSTEP;
+      if (tap < taps) {
+        if constexpr (ONE) {
+          put(filtB + (tap * TB + fcol) * 4, taps * TB * 4, expand_w1<2>(fw0[j][0], p.sym != 0), expand_w1<2>(fw1[j][0], p.sym != 0));
+        } else {
+          static_for<0, DB>([&](auto dc) {
+            constexpr int d = decltype(dc)::value;
+            put(filtB + ((2 * d * taps + tap) * TB + fcol) * 4, taps * TB * 4, expand_fp4<PB, d>(fw0[j]), expand_fp4<PB, d>(fw1[j]));
+          });
+        }
+      }
+    }
+  };
+
+  request(0);
+  const int rbase = a0 + wa * FA * 32, cbase = b0 + wb * FB * 32;
+  table.store(p, b0, tab, inv_vs);
 
   v16f acc[FA][FB];
 #pragma unroll
@@ -149,160 +240,135 @@ __global__ __launch_bounds__(256, OCC) void apnn_patch_conv_kernel(const KParams
 #pragma unroll
   for (int x = 0; x < FA; ++x) ssum[x] = 0;
 
-  EpiOperands<FA, FB> eo;
-  epi_prefetch<1, DIRECT_BITS, false>(p, a0 + wa * FA * 32, b0 + wb * FB * 32, lane, eo);
+  // operands of one tap: patch at pa (and sums at ps), filter block at fb
+  auto tap_read = [&](const uint32_t *pa, const uint32_t *fb, const int *ps, int dstride, v8i (&af)[FA][DA],
+                      v8i (&bf)[FB][DB]) {
+#pragma unroll
+    for (int x = 0; x < FA; ++x) {
+      if constexpr (!ONE) ssum[x] += ps[prow[x]];
+#pragma unroll
+      for (int d = 0; d < DA; ++d) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(pa + (2 * d * cap + prow[x]) * 4);
+        af[x][d] = v8i{(int)v.x, (int)v.y, (int)v.z, (int)v.w, 0, 0, 0, 0};
+      }
+    }
+#pragma unroll
+    for (int y = 0; y < FB; ++y)
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(fb + d * dstride + y * 32 * 4);
+        bf[y][d] = v8i{(int)v.x, (int)v.y, (int)v.z, (int)v.w, 0, 0, 0, 0};
+      }
+  };
+  auto tap_products = [&](const v8i (&af)[FA][DA], const v8i (&bf)[FB][DB]) {
+#pragma unroll
+    for (int x = 0; x < FA; ++x)
+#pragma unroll
+      for (int y = 0; y < FB; ++y)
+        static_for<0, DA>([&](auto dac) {
+          static_for<0, DB>([&](auto dbc) {
+            constexpr int da = decltype(dac)::value, db = decltype(dbc)::value;
+            acc[x][y] = mfma_digits<2, da + db>(bf[y][db], af[x][da], acc[x][y]);
+          });
+        });
+  };
 
-  const bool pair_ok = (p.C32 & 1) == 0;  // 64-bit loads of a channel-word pair
-  const int nchunks = (p.C32 + 1) >> 1;
   for (int cc = 0; cc < nchunks; ++cc) {
     const int cw = cc * 2;
     if (cc > 0) __syncthreads();  // every wave has finished reading the previous chunk
-    // ---- global loads of the chunk: patch pixels, then the first batch of filter tasks; all are in
-    // flight before the first one is consumed ----------------------------------------------------
-    uint32_t pw0[PATCH_NPT][PA], pw1[PATCH_NPT][PA];
-    const bool second = cw + 1 < p.C32;
-    // (one branch on the load width around each batch of loads, not one per load)
-    auto patch_load = [&](auto pair_c) {
-#pragma unroll
-      for (int j = 0; j < PATCH_NPT; ++j) {
-        const uint32_t boff = poff[j] != kOff ? poff[j] + ((uint32_t)cw << 2) : kOff;
-#pragma unroll
-        for (int pl = 0; pl < PA; ++pl) load_pair(rsrcA[pl], boff, pair_c, second, pw0[j][pl], pw1[j][pl]);
-      }
-    };
-    if (pair_ok) patch_load(std::true_type{}); else patch_load(std::false_type{});
-    constexpr int FT = 4;  // filter tasks (tap, column) per thread and batch
-    const int ntask = taps * TB;
-    uint32_t fw0[FT][PB], fw1[FT][PB];
-    auto filter_load_w = [&](int first, auto pair_c) {
-#pragma unroll
-      for (int j = 0; j < FT; ++j) {
-        const int t = first + tid + j * NT;
-        const int tap = t / TB, col = t % TB;
-        const int gcol = b0 + col;
-        const uint32_t boff = t < ntask && gcol < p.rowsB
-                                  ? (((uint32_t)gcol * (uint32_t)taps + (uint32_t)tap) * (uint32_t)p.C32 + (uint32_t)cw) << 2
-                                  : kOff;
-#pragma unroll
-        for (int pl = 0; pl < PB; ++pl) load_pair(rsrcB[pl], boff, pair_c, second, fw0[j][pl], fw1[j][pl]);
-      }
-    };
-    auto filter_load = [&](int first) {
-      if (pair_ok) filter_load_w(first, std::true_type{}); else filter_load_w(first, std::false_type{});
-    };
-    auto filter_store = [&](int first) {
-#pragma unroll
-      for (int j = 0; j < FT; ++j) {
-        const int t = first + tid + j * NT;
-        if (t < ntask) {
-          const int tap = t / TB, col = t % TB;
-          static_for<0, DB>([&](auto dc) {
-            constexpr int d = decltype(dc)::value;
-            const v8i e0 = expand_fp4<PB, d>(fw0[j]), e1 = expand_fp4<PB, d>(fw1[j]);
-            uint4 *dst = reinterpret_cast<uint4 *>(filtB + (((d * taps + tap) * TB + col) * 2) * 4);
-            dst[0] = make_uint4((uint32_t)e0[0], (uint32_t)e0[1], (uint32_t)e0[2], (uint32_t)e0[3]);
-            dst[1] = make_uint4((uint32_t)e1[0], (uint32_t)e1[1], (uint32_t)e1[2], (uint32_t)e1[3]);
-          });
-        }
-      }
-    };
-    filter_load(0);
-    // ---- patch chunk: packed words -> FP4 digit operands --------------------------------------
 #pragma unroll
     for (int j = 0; j < PATCH_NPT; ++j) {
       const int q = tid + j * NT;
-      if (q < npp) {
-        int ps = 0;
+      if (j * NT < npp && q < npp) {
+        if constexpr (!ONE) {
+          int ps = 0;
 #pragma unroll
-        for (int pl = 0; pl < PA; ++pl) ps += (__popc(pw0[j][pl]) + __popc(pw1[j][pl])) << pl;
-        pixsum[q] = ps;
+          for (int pl = 0; pl < PA; ++pl) ps += (__popc(pw0[j][pl]) + __popc(pw1[j][pl])) << pl;
+          pixsum[q] = ps;
+        }
         static_for<0, DA>([&](auto dc) {
           constexpr int d = decltype(dc)::value;
-          const v8i e0 = expand_fp4<PA, d>(pw0[j]), e1 = expand_fp4<PA, d>(pw1[j]);
-          uint4 *dst = reinterpret_cast<uint4 *>(patchA + ((d * cap + q) * 2) * 4);
-          dst[0] = make_uint4((uint32_t)e0[0], (uint32_t)e0[1], (uint32_t)e0[2], (uint32_t)e0[3]);
-          dst[1] = make_uint4((uint32_t)e1[0], (uint32_t)e1[1], (uint32_t)e1[2], (uint32_t)e1[3]);
+          put(patchA + (2 * d * cap + q) * 4, cap * 4, expand_fp4<PA, d>(pw0[j]), expand_fp4<PA, d>(pw1[j]));
         });
       }
     }
-    // ---- filter chunk ----------------------------------------------------------------------
-    for (int first = 0; first < ntask; first += FT * NT) {
+    filter_store(0);
+    for (int first = FT * TSTEP; first < taps; first += FT * TSTEP) {
+      if (pair_ok) filter_load_w(cw, first, std::true_type{}); else filter_load_w(cw, first, std::false_type{});
       filter_store(first);
-      if (first + FT * NT < ntask) filter_load(first + FT * NT);
     }
     __syncthreads();
+    if (cc + 1 < nchunks) request(cw + 2);
 
-    // ---- taps k-steps: operands straight from LDS --------------------------------------------
-    int r = 0, sx = 0;
-    for (int tap = 0; tap < taps; ++tap) {
-      const int toff = r * p.PWs + sx;
-      v8i af[FA][DA], bf[FB][DB];
-#pragma unroll
-      for (int x = 0; x < FA; ++x) {
-        const int pix = prow[x] + toff;
-        ssum[x] += pixsum[pix];
-#pragma unroll
-        for (int d = 0; d < DA; ++d) {
-          const uint4 v = *reinterpret_cast<const uint4 *>(patchA + ((d * cap + pix) * 2 + g) * 4);
-          af[x][d] = v8i{(int)v.x, (int)v.y, (int)v.z, (int)v.w, 0, 0, 0, 0};
+    const uint32_t *pa = patchA + g * cap * 4;
+    const uint32_t *fb = filtB + (g * taps * TB + wb * FB * 32 + li) * 4;
+    if constexpr (FORM != PF_ANY) {
+      // a tap's operands are read while the one before is multiplied; the scheduler does not see past a tap, or it
+      // would hoist the reads of all nine and spill
+      v8i af[2][FA][DA], bf[2][FB][DB];
+      int pitch = p.PWs;
+      asm("" : "+s"(pitch));  // keeps the addresses of the nine taps from being held in registers over all chunks
+      auto read = [&](auto tc) {
+        constexpr int tap = decltype(tc)::value;
+        const int toff = tap / 3 * pitch + tap % 3;
+        tap_read(pa + toff * 4, fb + tap * TB * 4, pixsum + toff, 9 * TB * 8, af[tap & 1], bf[tap & 1]);
+      };
+      read(std::integral_constant<int, 0>{});
+      static_for<0, 9>([&](auto tc) {
+        constexpr int tap = decltype(tc)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (tap < 8) read(std::integral_constant<int, tap + 1>{});
+        tap_products(af[tap & 1], bf[tap & 1]);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      int toff = 0, sx = 0;
+#pragma unroll 1
+      for (int tap = 0; tap < taps; ++tap) {
+        v8i af[FA][DA], bf[FB][DB];
+        tap_read(pa + toff * 4, fb + tap * TB * 4, pixsum + toff, taps * TB * 8, af, bf);
+        tap_products(af, bf);
+        ++toff;
+        if (++sx == p.S) {
+          sx = 0;
+          toff += p.PWs - p.S;
         }
-      }
-#pragma unroll
-      for (int y = 0; y < FB; ++y) {
-#pragma unroll
-        for (int d = 0; d < DB; ++d) {
-          const uint4 v = *reinterpret_cast<const uint4 *>(
-              filtB + (((d * taps + tap) * TB + (wb * FB + y) * 32 + li) * 2 + g) * 4);
-          bf[y][d] = v8i{(int)v.x, (int)v.y, (int)v.z, (int)v.w, 0, 0, 0, 0};
-        }
-      }
-#pragma unroll
-      for (int x = 0; x < FA; ++x)
-#pragma unroll
-        for (int y = 0; y < FB; ++y) {
-          static_for<0, DA>([&](auto dac) {
-            static_for<0, DB>([&](auto dbc) {
-              constexpr int da = decltype(dac)::value, db = decltype(dbc)::value;
-              if constexpr (da + db == 0) {
-                acc[x][y] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af[x][da], bf[y][db], acc[x][y], 4, 4, 0,
-                                                                            0, 0, 0);
-              } else {
-                acc[x][y] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                    af[x][da], bf[y][db], acc[x][y], 4, 4, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F + 0x02020202 * (da + db));
-              }
-            });
-          });
-        }
-      if (++sx == p.S) {
-        sx = 0;
-        ++r;
       }
     }
   }
-  epi_finish<4, 1, true, DIRECT_BITS, false>(p, acc, ssum, smem, wave, lane, a0, b0, wa, wb, eo);
-}
 
-// LDS bytes of a launch: patch + filter block + pixel sums, at least the slab area of the output stage
-constexpr size_t patch_smem_bytes(int PA, int PB, int FB, int TB, int taps, int cap) {
-  const size_t da = (PA + 1) / 2, db = (PB + 1) / 2;
-  const size_t stage = (da * cap * 8 + db * (size_t)taps * TB * 8 + cap) * sizeof(uint32_t);
-  const size_t slab = 4ull * (32 * (FB * 32 + 1) + 32 + FB * 32 + 2 * 32 * FB) * sizeof(int);
-  return stage > slab ? stage : slab;
+  if (p.fold != 0u) {
+    uint32_t sc[FA][FB][2];
+    conv_shortcut_load<FA, FB>(p, rbase, cbase, li, sc);
+    fold_shortcut_lanes<FA, FB>(p, acc, sc, lane, log2vs);
+  }
+  if (need_sum) {
+#pragma unroll
+    for (int x = 0; x < FA; ++x) {
+      const float c = (float)ssum[x] * (-(float)p.wmax * inv_vs);
+#pragma unroll
+      for (int y = 0; y < FB; ++y)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[x][y][r] += c;
+    }
+  }
+  settle_results(acc);
+  conv_output<FA, FB, 4, TB, MAXB>(
+      p, [&](auto xc, auto yc, auto ic) { return (float)acc[decltype(xc)::value][decltype(yc)::value][decltype(ic)::value]; },
+      (float)(1 << log2vs), tab, smem, rbase, cbase, b0, 0, lane);
 }
 
 enum PatchTile { PT_128x128 = 0, PT_256x64 = 1, PT_64x128 = 2, PT_128x64 = 3, PT_64x64 = 4, PT_COUNT = 5 };
-constexpr int kPatchTileA[PT_COUNT] = {128, 256, 64, 128, 64};
-constexpr int kPatchTileB[PT_COUNT] = {128, 64, 128, 64, 64};
+static_assert(PT_COUNT == kPatchTileCount, "tile tables of dispatch.h");
 
-template <int PA, int PB, int FA, int FB, int WA, int WB>
-inline hipError_t launch_patch(const KParams &p, hipStream_t stream) {
+template <int PA, int PB, int FA, int FB, int WA, int WB, int FORM>
+inline hipError_t launch_patch_form(const KParams &p, hipStream_t stream) {
   constexpr int TA = WA * FA * 32, TB = WB * FB * 32;
-  const int taps = p.KW / p.C32;
-  const size_t smem_bytes = patch_smem_bytes(PA, PB, FB, TB, taps, p.patch_cap);
+  const size_t smem_bytes = patch_stage_words(PA, PB, TB, p.KW / p.C32, p.patch_cap) * 4 + conv_epilogue_bytes(p, TB);
   if (smem_bytes > 160 * 1024 || p.patch_cap > PATCH_NPT * 256) return hipErrorNotSupported;
-  auto kern = apnn_patch_conv_kernel<PA, PB, FA, FB, WA, WB, 2>;
+  auto kern = apnn_patch_conv_kernel<PA, PB, FA, FB, WA, WB, FORM>;
   if (smem_bytes > 64 * 1024) {
-    static bool raised = false;
+    static bool raised = false;  // a repeated call is harmless
     if (!raised) {
       const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -315,13 +381,22 @@ inline hipError_t launch_patch(const KParams &p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <int PA, int PB, int FA, int FB, int WA, int WB, bool ODD = false>
+inline hipError_t launch_patch(const KParams &p, hipStream_t stream) {
+  if (p.KW == 9 * p.C32 && p.S == 3) {
+    if ((p.C32 & 1) == 0) return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_3x3_PAIRS>(p, stream);
+    if constexpr (ODD) return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_3x3_ODD>(p, stream);
+  }
+  return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_ANY>(p, stream);
+}
+
 template <int PA, int PB>
 inline hipError_t launch_patch_tile(int tile, const KParams &p, hipStream_t stream) {
   switch (tile) {
     case PT_128x128: return launch_patch<PA, PB, 2, 2, 2, 2>(p, stream);
-    case PT_256x64: return launch_patch<PA, PB, 2, 2, 4, 1>(p, stream);
+    case PT_256x64: return launch_patch<PA, PB, 2, 2, 4, 1, true>(p, stream);
     case PT_64x128: return launch_patch<PA, PB, 1, 2, 2, 2>(p, stream);
-    case PT_128x64: return launch_patch<PA, PB, 1, 2, 4, 1>(p, stream);
+    case PT_128x64: return launch_patch<PA, PB, 1, 2, 4, 1, true>(p, stream);
     case PT_64x64: return launch_patch<PA, PB, 1, 1, 2, 2>(p, stream);
     default: return hipErrorNotSupported;
   }

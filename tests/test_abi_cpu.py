@@ -308,6 +308,24 @@ def test_plan_reports_the_dispatchers_choices():
     assert A.lib().apnn_gemm_plan(ctypes.byref(g), None) == A.ENULL
 
 
+@pytest.mark.parametrize("batch,H,C,cout,R,stride,wb,xb,tile", [
+    (8, 56, 64, 64, 3, 1, 1, 2, (128, 64)), (4, 56, 64, 64, 3, 1, 1, 2, None),          # half a 128x64 tile per unit
+    (64, 28, 64, 192, 3, 1, 1, 2, (256, 64)), (64, 28, 64, 192, 3, 1, 1, 4, (128, 64)),  # 256x64 saves a round
+    (64, 28, 64, 192, 5, 1, 1, 2, None), (64, 56, 64, 128, 3, 2, 1, 2, None),            # other filters, strides
+    (64, 28, 128, 128, 3, 1, 1, 2, (128, 64)), (16, 28, 128, 128, 3, 1, 1, 2, None), (64, 28, 128, 256, 3, 1, 1, 2, None),
+    (64, 14, 256, 256, 3, 1, 1, 2, (128, 64)), (64, 14, 256, 256, 3, 1, 1, 3, None), (64, 28, 256, 256, 3, 1, 1, 2, None),
+    (16, 14, 960, 1024, 3, 1, 2, 2, (256, 64)), (16, 14, 960, 1024, 3, 1, 1, 2, (128, 64)),
+    (3, 32, 32, 1024, 3, 1, 1, 2, None), (64, 56, 32, 64, 3, 1, 1, 2, (128, 64)), (64, 14, 512, 512, 3, 1, 1, 2, None),
+    (64, 56, 64, 64, 1, 1, 1, 2, None),
+])
+def test_patch_resident_tile_rule(batch, H, C, cout, R, stride, wb, xb, tile):
+    """Where AUTO takes the patch-resident convolution, on which tile, and where it leaves a layer to the others."""
+    rc, plan = _plan_conv(batch=batch, H=H, Wd=H, cin_pad=C, COUT=cout, R=R, S=R, stride=stride, pad=R // 2, halo=0, wb=wb,
+                          xb=xb, path=A.PATH_AUTO)
+    assert rc == 0
+    assert ((plan.tile_rows, plan.tile_cols) if plan.kernel == A.KERNEL_PATCH_FP4 else None) == tile
+
+
 @pytest.mark.parametrize("wb,xb", [(1, 1), (1, 8), (2, 8), (4, 4), (1, 2), (2, 2)])
 @pytest.mark.parametrize("tile", [1, 2, 3, 4])
 def test_pinned_tile_below_the_crossover_names_a_popcount_tile(wb, xb, tile):

@@ -332,3 +332,34 @@ def test_very_long_single_tap(G, path, tile):
     got = G.run_conv(W, X, batch=1, H=4, W=8, cin_pad=K, cout=cols, R=1, S=1, stride=1, pad=0, halo=0, wb=1, xb=2, sym=0,
                      path=path, tile=tile)
     assert np.all(got == 3 * K)
+
+
+# Patch-resident convolution: the three forms of its kernel (any filter; 3x3 over an odd and over an even number of channel
+# words), one chunk of 64 channels and several, rows one past a tile and one short of it, a last column tile that is
+# mostly empty, raw sums and codes with flips.
+@pytest.mark.parametrize("tile", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("wb,xb", [(1, 2), (1, 3), (1, 4), (2, 2)])
+@pytest.mark.parametrize("H,Wd,C,cout,R,S,stride,sym", [
+    (3, 43, 64, 96, 3, 3, 1, 1),     # 129 rows
+    (15, 17, 192, 64, 3, 3, 1, 0),   # 255 rows, three chunks
+    (11, 12, 96, 160, 3, 3, 1, 1),   # an odd last word
+    (4, 16, 32, 32, 3, 3, 1, 0),     # one word
+    (9, 14, 160, 64, 4, 2, 1, 1),    # general form, odd words
+    (10, 10, 128, 32, 1, 1, 1, 1),   # one tap
+])
+def test_patch_conv_forms(G, wb, xb, tile, H, Wd, C, cout, R, S, stride, sym):
+    rng = np.random.default_rng(8700 + H + 10 * C + tile)
+    pad = 1 if R > 1 else 0
+    X, W = O.random_planes(rng, xb, H * Wd, C // 32), O.random_planes(rng, wb, cout * R * S, C // 32)
+    kw = dict(batch=1, H=H, W=Wd, cout=cout, R=R, S=S, stride=stride, pad=pad, halo=0, wb=wb, xb=xb)
+    acc = O.conv(W, X, cwords=C // 32, sym_w=sym, **kw).reshape(-1, cout)
+    got = G.run_conv(W, X, cin_pad=C, sym=sym, path=G.A.PATH_MFMA_PATCH, tile=tile, **kw).reshape(acc.shape)
+    assert np.array_equal(got, acc)
+    sigma = max(int(acc.std()), 2)
+    thr = np.sort(rng.integers(-sigma, sigma, size=(cout, (1 << xb) - 1)) + int(acc.mean()), axis=1).astype(np.int32)
+    flip = rng.integers(0, 2, size=cout).astype(np.uint8)
+    d_thr, d_flip = G.to_dev(thr), G.to_dev(flip)
+    epi = G.epilogue(mode=G.A.EPI_BN, out_bits=xb, thr=d_thr, flip=d_flip)
+    got = G.run_conv(W, X, cin_pad=C, sym=sym, epi=epi, path=G.A.PATH_MFMA_PATCH, tile=tile, **kw).view(np.uint32)
+    expect = O.lowbits_pack(O.bn_quantize(acc, None, thr, flip, xb), acc.shape[0], cout, xb)
+    assert np.array_equal(got.reshape(expect.shape), expect)
