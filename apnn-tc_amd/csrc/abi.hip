@@ -354,6 +354,13 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     const bool tall = p.planesA <= 3 && fits(1) && (r256 < r128 || (p.planesB > 1 && p.C32 > 8 && r256 == r128));
     const int t = tall ? 1 : 3;
     const bool plain = taps == 9 && p.S == 3 && p.stride == 1;  // the filters with an unrolled loop, the densest patches
+    // 5x5 over an even number of channel words, on the tile its unrolled form is built for: one chunk to at most 256 channels
+    // from half a tile per unit (28x28x64 to 192 at batch 8 / 16 / 64 7.9 -> 5.9 / 10.9 -> 7.0 / 20.0 -> 16.4, w1a4 at batch 8
+    // 12.1 -> 10.0; level at batch 4 and to 512 channels), several without 128-bit loads from one tile per unit (14x14x192 to
+    // 256 at batch 64 21.5 -> 13.3; with 100 tiles 9.4 -> 10.2)
+    if (taps == 25 && p.S == 5 && p.stride == 1 &&
+        (p.C32 == 2 ? p.rowsB <= 256 && 2 * n128 >= cus : p.C32 % 4 == 2 && n128 >= cus))
+      return 3;
     // One chunk of channels (56x56x64 to 64 at batch 8 5.3 -> 4.6, 196 tiles; 28x28x64 to 192 at batch 64 11.8 -> 9.1;
     // below half a tile per unit 128x64 leaves too much idle: 4.3 -> 4.6 with 98), or channel words without 128-bit
     // loads, which leave the others their 32- and 64-bit forms (56x56x96 to 256 at batch 4 / 64 11.4 -> 7.4 / 68.9 -> 40.6,

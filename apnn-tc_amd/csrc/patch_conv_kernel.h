@@ -30,6 +30,8 @@
 // matrix instruction pair of a 2x2-block wave are the LDS rate (128 bytes a clock), so long reductions stay level with
 // async_kernel.h (56x56x256 at batch 64 59 against 61 us).  A 256x128 tile of 4x2 blocks reads less, but two of them per
 // unit leave their last round emptier: 62 us there, 68 against 60 on 28x28x512.
+// 5x5 filters in a form of their own, all filter words of a chunk in flight at once: 28x28x64 to 192 at batch 64 21.2 us in
+// the general form, 16.4 in this one (two work-groups per unit, by the LDS).
 #pragma once
 #include "mfma_kernel.h"
 
@@ -41,7 +43,9 @@ namespace apnn {
 //   PF_ANY        any filter, any number of channel words: a loop over the taps
 //   PF_3x3_ODD    3x3, an odd number of channel words: 32-bit loads
 //   PF_3x3_PAIRS  3x3, an even number of channel words: 64-bit loads
-enum PatchForm { PF_ANY = 0, PF_3x3_ODD = 1, PF_3x3_PAIRS = 2 };
+//   PF_5x5_PAIRS  5x5, an even number of channel words
+enum PatchForm { PF_ANY = 0, PF_3x3_ODD = 1, PF_3x3_PAIRS = 2, PF_5x5_PAIRS = 3 };
+constexpr int patch_form_side(int form) { return form == PF_ANY ? 0 : form == PF_5x5_PAIRS ? 5 : 3; }
 
 // Work-groups per compute unit that the registers are cut for, by the 32x32 blocks of a wave (measured above).
 constexpr int patch_occupancy(int blocks) { return blocks == 4 ? 3 : 4; }
@@ -65,7 +69,8 @@ __global__ __launch_bounds__(256, patch_occupancy(FA * FB)) void apnn_patch_conv
   const int tilesB = (p.rowsB + TB - 1) / TB;
   const int a0 = (blockIdx.x / tilesB) * TA;
   const int b0 = (blockIdx.x % tilesB) * TB;
-  const int taps = FORM != PF_ANY ? 9 : p.KW / p.C32;
+  constexpr int SIDE = patch_form_side(FORM), TAPS = SIDE * SIDE;  // 0: not known
+  const int taps = FORM != PF_ANY ? TAPS : p.KW / p.C32;
   const int cap = p.patch_cap;
 
   uint32_t *patchA = smem;                                 // [DA][2 words][cap][4 dwords]
@@ -83,7 +88,7 @@ __global__ __launch_bounds__(256, patch_occupancy(FA * FB)) void apnn_patch_conv
   // other row and patch pixel is a small offset from it, for which the multiply-high quotients are
   // exact. -----------------------------------------------------------------------------------------
   const int last_row = min(a0 + TA, p.rowsA) - 1;
-  const int R = FORM != PF_ANY ? 3 : taps / p.S;
+  const int R = FORM != PF_ANY ? SIDE : taps / p.S;
   const bool pooled = p.pool_order != 0;
   const int gw = pooled ? p.Wo >> 1 : p.Wo, gh = pooled ? p.Ho >> 1 : p.Ho;  // row grid (windows when pooling)
   const int gst = pooled ? 2 * p.stride : p.stride;                          // its step in the padded frame
@@ -168,13 +173,13 @@ __global__ __launch_bounds__(256, patch_occupancy(FA * FB)) void apnn_patch_conv
     }
   }
   // filter words this thread stages: one channel, taps tap0, tap0 + TSTEP, ...; FT of them held in registers
-  constexpr int TSTEP = NT / TB, FT = TSTEP >= 4 ? 3 : 5;
+  constexpr int TSTEP = NT / TB, FT = FORM == PF_5x5_PAIRS ? (TAPS + TSTEP - 1) / TSTEP : TSTEP >= 4 ? 3 : 5;
   const int fcol = tid % TB, tap0 = tid / TB;
   const uint32_t foff = b0 + fcol < p.rowsB
                             ? ((uint32_t)(b0 + fcol) * (uint32_t)taps + (uint32_t)tap0) * (uint32_t)p.C32 << 2
                             : kOff;
 
-  const bool pair_ok = FORM == PF_3x3_PAIRS || (FORM == PF_ANY && (p.C32 & 1) == 0);  // 64-bit loads of a channel-word pair
+  const bool pair_ok = FORM == PF_3x3_PAIRS || FORM == PF_5x5_PAIRS || (FORM == PF_ANY && (p.C32 & 1) == 0);  // 64-bit loads of a channel-word pair
   const int nchunks = (p.C32 + 1) >> 1;
   uint32_t pw0[PATCH_NPT][PA], pw1[PATCH_NPT][PA], fw0[FT][PB], fw1[FT][PB];
   auto filter_load_w = [&](int cw, int first, auto pair_c) {
@@ -304,20 +309,20 @@ __global__ __launch_bounds__(256, patch_occupancy(FA * FB)) void apnn_patch_conv
     const uint32_t *fb = filtB + (g * taps * TB + wb * FB * 32 + li) * 4;
     if constexpr (FORM != PF_ANY) {
       // a tap's operands are read while the one before is multiplied; the scheduler does not see past a tap, or it
-      // would hoist the reads of all nine and spill
+      // would hoist the reads of all of them and spill
       v8i af[2][FA][DA], bf[2][FB][DB];
       int pitch = p.PWs;
-      asm("" : "+s"(pitch));  // keeps the addresses of the nine taps from being held in registers over all chunks
+      asm("" : "+s"(pitch));  // keeps the addresses of the taps from being held in registers over all chunks
       auto read = [&](auto tc) {
         constexpr int tap = decltype(tc)::value;
-        const int toff = tap / 3 * pitch + tap % 3;
-        tap_read(pa + toff * 4, fb + tap * TB * 4, pixsum + toff, 9 * TB * 8, af[tap & 1], bf[tap & 1]);
+        const int toff = tap / SIDE * pitch + tap % SIDE;
+        tap_read(pa + toff * 4, fb + tap * TB * 4, pixsum + toff, TAPS * TB * 8, af[tap & 1], bf[tap & 1]);
       };
       read(std::integral_constant<int, 0>{});
-      static_for<0, 9>([&](auto tc) {
+      static_for<0, TAPS>([&](auto tc) {
         constexpr int tap = decltype(tc)::value;
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (tap < 8) read(std::integral_constant<int, tap + 1>{});
+        if constexpr (tap + 1 < TAPS) read(std::integral_constant<int, tap + 1>{});
         tap_products(af[tap & 1], bf[tap & 1]);
       });
       __builtin_amdgcn_sched_barrier(0);
@@ -381,11 +386,15 @@ inline hipError_t launch_patch_form(const KParams &p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <int PA, int PB, int FA, int FB, int WA, int WB, bool ODD = false>
+// ODD, BIG: whether the forms for odd channel words and for 5x5 filters are built
+template <int PA, int PB, int FA, int FB, int WA, int WB, bool ODD = false, bool BIG = false>
 inline hipError_t launch_patch(const KParams &p, hipStream_t stream) {
   if (p.KW == 9 * p.C32 && p.S == 3) {
     if ((p.C32 & 1) == 0) return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_3x3_PAIRS>(p, stream);
     if constexpr (ODD) return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_3x3_ODD>(p, stream);
+  }
+  if constexpr (BIG) {
+    if (p.KW == 25 * p.C32 && p.S == 5 && (p.C32 & 1) == 0) return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_5x5_PAIRS>(p, stream);
   }
   return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_ANY>(p, stream);
 }
@@ -396,7 +405,7 @@ inline hipError_t launch_patch_tile(int tile, const KParams &p, hipStream_t stre
     case PT_128x128: return launch_patch<PA, PB, 2, 2, 2, 2>(p, stream);
     case PT_256x64: return launch_patch<PA, PB, 2, 2, 4, 1, true>(p, stream);
     case PT_64x128: return launch_patch<PA, PB, 1, 2, 2, 2>(p, stream);
-    case PT_128x64: return launch_patch<PA, PB, 1, 2, 4, 1, true>(p, stream);
+    case PT_128x64: return launch_patch<PA, PB, 1, 2, 4, 1, true, true>(p, stream);
     case PT_64x64: return launch_patch<PA, PB, 1, 1, 2, 2>(p, stream);
     default: return hipErrorNotSupported;
   }

@@ -334,8 +334,8 @@ def test_very_long_single_tap(G, path, tile):
     assert np.all(got == 3 * K)
 
 
-# Patch-resident convolution: the three forms of its kernel (any filter; 3x3 over an odd and over an even number of channel
-# words), one chunk of 64 channels and several, rows one past a tile and one short of it, a last column tile that is
+# Patch-resident convolution: the forms of its kernel (any filter; 3x3 over an odd and over an even number of channel words; 5x5
+# over an even one, run on the narrow tiles), one chunk of 64 channels and several, rows one past a tile and one short of it, a last column tile that is
 # mostly empty, raw sums and codes with flips.
 @pytest.mark.parametrize("tile", [0, 1, 2, 3, 4])
 @pytest.mark.parametrize("wb,xb", [(1, 2), (1, 3), (1, 4), (2, 2)])
@@ -346,8 +346,12 @@ def test_very_long_single_tap(G, path, tile):
     (4, 16, 32, 32, 3, 3, 1, 0),     # one word
     (9, 14, 160, 64, 4, 2, 1, 1),    # general form, odd words
     (10, 10, 128, 32, 1, 1, 1, 1),   # one tap
+    (12, 15, 64, 96, 5, 5, 1, 1),    # 130 rows
+    (7, 9, 192, 64, 5, 5, 1, 0),     # three chunks
 ])
 def test_patch_conv_forms(G, wb, xb, tile, H, Wd, C, cout, R, S, stride, sym):
+    if R == 5 and tile not in (3, 4):
+        pytest.skip("patch and filter block of 25 taps are built for the narrow tiles only")
     rng = np.random.default_rng(8700 + H + 10 * C + tile)
     pad = 1 if R > 1 else 0
     X, W = O.random_planes(rng, xb, H * Wd, C // 32), O.random_planes(rng, wb, cout * R * S, C // 32)
