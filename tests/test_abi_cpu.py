@@ -312,7 +312,7 @@ def test_plan_reports_the_dispatchers_choices():
     (8, 56, 64, 64, 3, 1, 1, 2, (128, 64)), (4, 56, 64, 64, 3, 1, 1, 2, None),          # half a 128x64 tile per unit
     (64, 28, 64, 192, 3, 1, 1, 2, (256, 64)), (64, 28, 64, 192, 3, 1, 1, 4, (128, 64)),  # 256x64 saves a round
     (8, 28, 64, 192, 5, 1, 1, 2, (128, 64)), (4, 28, 64, 192, 5, 1, 1, 2, None), (16, 28, 64, 512, 5, 1, 1, 2, None),
-    (64, 14, 192, 256, 5, 1, 1, 2, (128, 64)), (64, 14, 128, 128, 5, 1, 1, 2, None), (8, 56, 64, 64, 5, 1, 1, 2, None),
+    (64, 14, 192, 256, 5, 1, 1, 2, (128, 64)), (64, 14, 128, 128, 5, 1, 1, 2, None), (8, 56, 64, 64, 5, 1, 1, 2, (128, 64)),
     (64, 28, 64, 192, 7, 1, 1, 2, None), (64, 56, 64, 128, 3, 2, 1, 2, None),            # other filters, strides
     (64, 28, 128, 128, 3, 1, 1, 2, (128, 64)), (16, 28, 128, 128, 3, 1, 1, 2, None), (64, 28, 128, 256, 3, 1, 1, 2, None),
     (64, 14, 256, 256, 3, 1, 1, 2, (128, 64)), (64, 14, 256, 256, 3, 1, 1, 3, None), (64, 28, 256, 256, 3, 1, 1, 2, None),
