@@ -335,10 +335,10 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
   auto fits = [&](int t) {
     const int cap = patch_pixels(p, R, apnn::kPatchTileRows[t]);
     if (cap > 1024) return false;
-    // digits: one per plane pair, for a pinned tile as in the widest case; the byte counts of patch_stage_words().  (A
-    // pooled 5x5 layer of 28x28x64 has a patch of 464 pixels: it fits with the one digit of two planes.  5x5 on 56x56x64 to 64
-    // at batch 8 / 64 8.0 -> 5.9 / 25.7 -> 20.9 us, w2a2 at batch 8 8.7 -> 6.7.)
-    const size_t digits = automatic ? (p.planesA + 1) / 2 : 2;
+    // One digit per pair of activation planes, for a pinned tile as for AUTO: a plan's tile can be pinned.  (A pooled 5x5
+    // layer of 28x28x64 has a patch of 464 pixels: it fits with the one digit of two planes.  5x5 on 56x56x64 to 64 at batch
+    // 8 / 64 8.0 -> 5.9 / 25.7 -> 20.9 us, w2a2 at batch 8 8.7 -> 6.7.)
+    const size_t digits = (p.planesA + 1) / 2;
     const size_t bytes = (digits * cap * 8 + (size_t)taps * apnn::kPatchTileCols[t] * 8 + cap) * 4;
     return bytes <= 80 * 1024;
   };

@@ -328,6 +328,21 @@ def test_patch_resident_tile_rule(batch, H, C, cout, R, stride, wb, xb, tile):
     assert ((plan.tile_rows, plan.tile_cols) if plan.kernel == A.KERNEL_PATCH_FP4 else None) == tile
 
 
+@pytest.mark.parametrize("batch,H,C,cout,R,wb,xb", [(8, 56, 64, 64, 5, 1, 2), (64, 27, 96, 256, 5, 1, 2), (64, 56, 96, 256, 5, 1, 2),
+                                                    (8, 28, 64, 192, 5, 1, 4), (16, 32, 64, 192, 5, 1, 4), (64, 28, 64, 192, 3, 1, 2)])
+def test_patch_tile_of_auto_can_be_pinned(batch, H, C, cout, R, wb, xb):
+    """A plan's tile is the value that pins it: what AUTO takes, a caller can name, whatever the digits of the precision."""
+    kw = dict(batch=batch, H=H, Wd=H, cin_pad=C, COUT=cout, R=R, S=R, stride=1, pad=R // 2, halo=0, wb=wb, xb=xb,
+              epi=A.Epilogue(mode=A.EPI_BN, out_bits=xb, thresholds=0x1000))
+    rc, auto = _plan_conv(path=A.PATH_AUTO, **kw)
+    assert rc == 0
+    rc, free = _plan_conv(path=A.PATH_MFMA_PATCH, **kw)
+    assert rc == 0 and free.kernel == A.KERNEL_PATCH_FP4
+    if auto.kernel == A.KERNEL_PATCH_FP4:
+        rc, pinned = _plan_conv(path=A.PATH_MFMA_PATCH | ((auto.tile + 1) << 8), **kw)
+        assert rc == 0 and (pinned.tile, pinned.patch_pixels) == (auto.tile, auto.patch_pixels)
+
+
 @pytest.mark.parametrize("wb,xb", [(1, 1), (1, 8), (2, 8), (4, 4), (1, 2), (2, 2)])
 @pytest.mark.parametrize("tile", [1, 2, 3, 4])
 def test_pinned_tile_below_the_crossover_names_a_popcount_tile(wb, xb, tile):
@@ -363,6 +378,7 @@ def test_patch_capacity_bounds_every_tile():
         (3, 28, 28, 1, 1, 2, 0, 0), (2, 13, 11, 5, 5, 1, 2, 0), (2, 12, 20, 3, 3, 1, 1, 1), (3, 8, 8, 5, 3, 1, 1, 2),
         (9, 5, 6, 3, 3, 1, 1, 0), (2, 30, 9, 3, 1, 1, 0, 0), (7, 6, 6, 3, 3, 1, 1, 1), (2, 24, 24, 5, 5, 2, 2, 1),
         (70, 3, 3, 3, 3, 1, 1, 0), (1, 40, 6, 1, 5, 1, 2, 0), (6, 10, 10, 3, 3, 1, 0, 1),
+        (1, 9, 60, 5, 5, 1, 1, 0), (2, 10, 58, 5, 5, 1, 2, 1), (2, 12, 58, 5, 5, 1, 1, 0),  # patches beyond 512 pixels with 25 taps
     ]
     checked = 0
     for (batch, H, W, R, S, stride, pad, pool) in geoms:

@@ -348,10 +348,12 @@ def test_very_long_single_tap(G, path, tile):
     (10, 10, 128, 32, 1, 1, 1, 1),   # one tap
     (12, 15, 64, 96, 5, 5, 1, 1),    # 130 rows
     (7, 9, 192, 64, 5, 5, 1, 0),     # three chunks
+    (9, 60, 64, 96, 5, 5, 1, 1),     # patches of 640 (128x64) and 776 (256x64) pixels: they fit with the one digit of two planes
+    (10, 58, 96, 64, 5, 5, 1, 0),    # the same over an odd number of words
 ])
 def test_patch_conv_forms(G, wb, xb, tile, H, Wd, C, cout, R, S, stride, sym):
-    if R == 5 and tile not in (3, 4):
-        pytest.skip("patch and filter block of 25 taps are built for the narrow tiles only")
+    if R == 5 and tile not in ((1, 3, 4) if xb == 2 else (3, 4)) or Wd > 50 and xb > 2:
+        pytest.skip("the patch and the filter block of 25 taps do not fit")
     rng = np.random.default_rng(8700 + H + 10 * C + tile)
     pad = 1 if R > 1 else 0
     X, W = O.random_planes(rng, xb, H * Wd, C // 32), O.random_planes(rng, wb, cout * R * S, C // 32)
