@@ -7,6 +7,7 @@
 #include <atomic>
 
 #include "../../include/apnn_tc.h"
+#include "conv_epilogue.h"
 #include "dispatch.h"
 
 // One error word per device (each device holds its own copy of a __device__ variable).
@@ -332,15 +333,18 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
   int cus = device_cus();
   if (cus <= 0) cus = 256;
   const int taps = p.KW / p.C32;
-  auto fits = [&](int t) {
+  // Staged bytes of a tile, with the digits of the precision for a pinned tile as for AUTO: a plan's tile can be pinned.  (A
+  // pooled 5x5 layer of 28x28x64 has a patch of 464 pixels: it fits with the one digit of two planes.  5x5 on 56x56x64 to 64
+  // at batch 8 / 64 8.0 -> 5.9 / 25.7 -> 20.9 us, w2a2 at batch 8 8.7 -> 6.7.)
+  auto staged = [&](int t) {
     const int cap = patch_pixels(p, R, apnn::kPatchTileRows[t]);
-    if (cap > 1024) return false;
-    // One digit per pair of activation planes, for a pinned tile as for AUTO: a plan's tile can be pinned.  (A pooled 5x5
-    // layer of 28x28x64 has a patch of 464 pixels: it fits with the one digit of two planes.  5x5 on 56x56x64 to 64 at batch
-    // 8 / 64 8.0 -> 5.9 / 25.7 -> 20.9 us, w2a2 at batch 8 8.7 -> 6.7.)
-    const size_t digits = (p.planesA + 1) / 2;
-    const size_t bytes = (digits * cap * 8 + (size_t)taps * apnn::kPatchTileCols[t] * 8 + cap) * 4;
-    return bytes <= 80 * 1024;
+    return cap > 1024 ? ~(size_t)0 : apnn::patch_stage_words(p.planesA, p.planesB, apnn::kPatchTileCols[t], taps, cap) * 4;
+  };
+  // AUTO counts the threshold table too: with it, a 5x5 tile of four planes over a patch of 417 pixels or more stays alone on
+  // its unit (32x32x64 to 160 at batch 25, w1a4 threshold codes: 25.1 us, 20.2 on the 128x64 implicit-GEMM tile).
+  auto fits = [&](int t) {
+    const size_t bytes = staged(t);
+    return bytes <= 80 * 1024 && (!automatic || bytes + apnn::conv_epilogue_bytes(p, apnn::kPatchTileCols[t]) <= 80 * 1024);
   };
   auto ntiles = [&](int t) {
     return (long long)((p.rowsA + apnn::kPatchTileRows[t] - 1) / apnn::kPatchTileRows[t]) *

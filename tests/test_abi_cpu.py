@@ -343,6 +343,20 @@ def test_patch_tile_of_auto_can_be_pinned(batch, H, C, cout, R, wb, xb):
         assert rc == 0 and (pinned.tile, pinned.patch_pixels) == (auto.tile, auto.patch_pixels)
 
 
+@pytest.mark.parametrize("H", [28, 32, 60, 64, 66, 68, 70, 72, 74])
+@pytest.mark.parametrize("xb,out_bits", [(2, 2), (2, 4), (3, 3), (4, 4), (4, 2)])
+def test_auto_takes_5x5_patches_that_fit_twice(H, xb, out_bits):
+    """Two work-groups of 80 KB a compute unit: patch, filter block of 25 taps and the threshold table of 64 channels."""
+    rc, plan = _plan_conv(batch=16, H=H, Wd=H, cin_pad=64, COUT=192, R=5, S=5, stride=1, pad=2, halo=0, wb=1, xb=xb,
+                          epi=A.Epilogue(mode=A.EPI_BN, out_bits=out_bits, thresholds=0x1000), path=A.PATH_AUTO)
+    assert rc == 0
+    if plan.kernel == A.KERNEL_PATCH_FP4:
+        table = 4 * ((2 ** out_bits - 1) * (64 + 4) + 2)
+        assert plan.patch_pixels * 32 * ((xb + 1) // 2) + 25 * 64 * 32 + table <= 80 * 1024, plan.patch_pixels
+    else:
+        assert xb > 2  # one digit a pixel fits at all of these
+
+
 @pytest.mark.parametrize("wb,xb", [(1, 1), (1, 8), (2, 8), (4, 4), (1, 2), (2, 2)])
 @pytest.mark.parametrize("tile", [1, 2, 3, 4])
 def test_pinned_tile_below_the_crossover_names_a_popcount_tile(wb, xb, tile):
