@@ -47,13 +47,22 @@ namespace apnn {
 enum PatchForm { PF_ANY = 0, PF_3x3_ODD = 1, PF_3x3_PAIRS = 2, PF_5x5_PAIRS = 3 };
 constexpr int patch_form_side(int form) { return form == PF_ANY ? 0 : form == PF_5x5_PAIRS ? 5 : 3; }
 
-// Work-groups per compute unit that the registers are cut for, by the 32x32 blocks of a wave (measured above).
-constexpr int patch_occupancy(int blocks) { return blocks == 4 ? 3 : 4; }
+// Work-groups per compute unit that the registers are cut for, by the 32x32 blocks of a wave, the form and the activation planes.
+// The 5x5 form stages 50 KB of filter: LDS holds two work-groups, and a cut to 128 registers made it reload up to 12 in every
+// chunk.  28x28x64 to 192 at batch 8 / 64, us with four work-groups and with two: w1a4 9.9 -> 9.3 / 30.2 -> 28.4, w1a3 8.1 ->
+// 7.7 / 24.1 -> 23.0.  2x2 blocks of the 3x3 forms with four planes reloaded 8 to 16: 256x64 tiles on 56x56x96 to 256 at batch
+// 64 108 -> 95 with two work-groups instead of three, 14x14x960 to 1024 185 -> 124.  The general form with four planes still
+// reloads 8 to 18 a chunk: three work-groups without them are ahead where the filter fills the LDS (16 taps, 27x27x96 to 256 at
+// batch 16 18.6 -> 16.8; 25 taps 72.9 -> 67.1) and behind where it does not (2x2 at batch 32 17.9 -> 20.4).
+constexpr int patch_occupancy(int blocks, int form, int planes) {
+  if (form == PF_5x5_PAIRS || (blocks == 4 && planes == 4 && form != PF_ANY)) return 2;
+  return blocks == 4 ? 3 : 4;
+}
 
 constexpr int PATCH_NPT = 4;  // patch pixels per thread (patch capacity = 4 * 256 pixels)
 
 template <int PA, int PB, int FA, int FB, int WA, int WB, int FORM>
-__global__ __launch_bounds__(256, patch_occupancy(FA * FB)) void apnn_patch_conv_kernel(const KParams p) {
+__global__ __launch_bounds__(256, patch_occupancy(FA * FB, FORM, PA)) void apnn_patch_conv_kernel(const KParams p) {
   static_assert(WA * WB == 4, "four waves tile the output");
   constexpr int DA = (PA + 1) / 2, DB = (PB + 1) / 2;
   constexpr int NT = 256;
