@@ -340,15 +340,17 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     const int cap = patch_pixels(p, R, apnn::kPatchTileRows[t]);
     return cap > 1024 ? ~(size_t)0 : apnn::patch_stage_words(p.planesA, p.planesB, apnn::kPatchTileCols[t], taps, cap) * 4;
   };
-  // AUTO counts the threshold table too: with it, a 5x5 tile of four planes over a patch of 417 pixels or more stays alone on
-  // its unit (32x32x64 to 160 at batch 25, w1a4 threshold codes: 25.1 us, 20.2 on the 128x64 implicit-GEMM tile).
-  auto fits = [&](int t) {
-    const size_t bytes = staged(t);
-    return bytes <= 80 * 1024 && (!automatic || bytes + apnn::conv_epilogue_bytes(p, apnn::kPatchTileCols[t]) <= 80 * 1024);
-  };
   auto ntiles = [&](int t) {
     return (long long)((p.rowsA + apnn::kPatchTileRows[t] - 1) / apnn::kPatchTileRows[t]) *
            ((p.rowsB + apnn::kPatchTileCols[t] - 1) / apnn::kPatchTileCols[t]);
+  };
+  // AUTO counts the threshold table too where a unit gets a second tile: with it, a 5x5 tile of four planes over a patch of 417
+  // pixels or more stays alone (w1a4 threshold codes, 32x32x64 to 160 at batch 25, 600 tiles: 25.1 us, 20.2 on the 128x64
+  // implicit-GEMM tile; at batch 7, 168 tiles, 9.6 against 12.4).
+  auto fits = [&](int t) {
+    const size_t bytes = staged(t);
+    const bool table = automatic && ntiles(t) > cus;
+    return bytes <= 80 * 1024 && (!table || bytes + apnn::conv_epilogue_bytes(p, apnn::kPatchTileCols[t]) <= 80 * 1024);
   };
   if (automatic) {
     if (tile_pin != 0) return -1;  // a pinned tile names a tile of the implicit-GEMM families

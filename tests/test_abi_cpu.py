@@ -328,6 +328,27 @@ def test_patch_resident_tile_rule(batch, H, C, cout, R, stride, wb, xb, tile):
     assert ((plan.tile_rows, plan.tile_cols) if plan.kernel == A.KERNEL_PATCH_FP4 else None) == tile
 
 
+@pytest.mark.parametrize("batch,H,C,cout,R,stride,wb,xb,out,tile", [
+    # 5x5 of four planes: the threshold table counts where a unit gets a second tile
+    (7, 32, 64, 160, 5, 1, 1, 4, "bn", (128, 64)), (25, 32, 64, 160, 5, 1, 1, 4, "bn", None),
+])
+def test_patch_resident_tile_rule_by_output(batch, H, C, cout, R, stride, wb, xb, out, tile):
+    """The rule where results other than two-bit codes, long reductions or rounds of the other tiles decide.  out: int32, bn,
+    low bits, pooled averages, a shortcut that folds (near) or not (far), an int32 map."""
+    epi = A.Epilogue()
+    if out != "int32":
+        epi = A.Epilogue(mode=A.EPI_LOWBITS if out == "low" else A.EPI_BN, out_bits=xb, thresholds=0x1000)
+        epi.pool = A.POOL_AVG2X2 if out == "avg" else A.POOL_NONE
+        if out in ("near", "far"):
+            epi.residual_planes, epi.residual_bits, epi.residual_scale = 0x1000, 2, 12 if out == "near" else 1365
+        if out == "map":
+            epi.residual, epi.save_acc = 0x1000, 0x1000
+    rc, plan = _plan_conv(batch=batch, H=H, Wd=H, cin_pad=C, COUT=cout, R=R, S=R, stride=stride, pad=(R - 1) // 2, halo=0, wb=wb,
+                          xb=xb, weight_mode=A.WEIGHT_SYMMETRIC, epi=epi, path=A.PATH_AUTO)
+    assert rc == 0
+    assert ((plan.tile_rows, plan.tile_cols) if plan.kernel == A.KERNEL_PATCH_FP4 else None) == tile
+
+
 @pytest.mark.parametrize("batch,H,C,cout,R,wb,xb", [(8, 56, 64, 64, 5, 1, 2), (64, 27, 96, 256, 5, 1, 2), (64, 56, 96, 256, 5, 1, 2),
                                                     (8, 28, 64, 192, 5, 1, 4), (16, 32, 64, 192, 5, 1, 4), (64, 28, 64, 192, 3, 1, 2)])
 def test_patch_tile_of_auto_can_be_pinned(batch, H, C, cout, R, wb, xb):
