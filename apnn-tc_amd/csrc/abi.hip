@@ -355,20 +355,31 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
   if (automatic) {
     if (tile_pin != 0) return -1;  // a pinned tile names a tile of the implicit-GEMM families
     if (taps == 1 || !fits(3)) return -1;
-    // 256x64 tiles (three work-groups per unit at a time, against four of 128x64) where they save a round: 56x56x96 to
-    // 256 channels at batch 64 39.8 against 42.9, 27x27x96 to 256 12.6 against 14.9.  Not with four activation planes,
-    // whose patch is twice as large (107 against 92); with two weight planes over many chunks of channels also at equal
-    // rounds, as each tile expands its filter block again (28x28x320 to 256 at batch 64 31.9 against 39.1).
-    const long long n128 = ntiles(3), r128 = (n128 + 4 * cus - 1) / (4 * cus), r256 = (ntiles(1) + 3 * cus - 1) / (3 * cus);
-    const bool tall = p.planesA <= 3 && fits(1) && (r256 < r128 || (p.planesB > 1 && p.C32 > 8 && r256 == r128));
-    const int t = tall ? 1 : 3;
+    const long long n = ntiles(3), n256 = ntiles(1);  // 128x64 and 256x64 tiles
     const bool plain = taps == 9 && p.S == 3 && p.stride == 1;  // the filters with an unrolled loop, the densest patches
+    // Results that leave over the output stage's general path (its values pass LDS, and 2x2 blocks keep part of them in
+    // scratch).
+    const bool general = p.epi != APNN_EPI_INT32 && !apnn::conv_float_codes(p, p.planesA >= 3 ? 4 : 2);
+    // 3x3: 256x64 tiles (three work-groups per unit at a time, against four of 128x64; LDS holds as many, but three of either
+    // with two digits a pixel) where they save a round: 56x56x96 to 256 channels at batch 64 39.8 against 42.9, 27x27x96 to 256
+    // 12.6 against 14.9, w1a3 level.  Not with four activation planes, whose patch is twice as large (97 against 92), nor for
+    // general results (1.1 to 1.6 times the 128x64 tile's time: 56x56x64 to 64 at batch 62, w1a3 averages 27.6 against 19.2),
+    // unless the reduction is long (27x27x960 to 896 at batch 48 187 against 221; w1a3, the other way round, 832 to 192 at batch
+    // 64 on 32x32 117 against 102).  With two weight planes over many chunks of
+    // channels also at equal rounds, as each tile expands its filter block again (28x28x320 to 256 at batch 64 31.9 against
+    // 39.1), from 9/16 of a tile per unit (14x14x960 to 192 at batch 64, 147 tiles, 31.3 against 39.1; 28x28x320 to 32 at batch
+    // 25, 77 tiles, 14.6 against 9.4), general results from one.
+    const long long r128 = (n + 4 * cus - 1) / (4 * cus), r256 = (n256 + 3 * cus - 1) / (3 * cus);
+    const bool long_w2 = p.planesB > 1 && p.C32 > 8 && r256 <= r128 && 16 * n256 >= (general ? 16 : 9) * cus;
+    const bool tall = p.planesA <= 3 && fits(1) &&
+                      (long_w2 || (r256 < r128 && (p.planesA == 2 ? !general || p.C32 >= 20 : !general && p.C32 < 20)));
+    const int t = tall ? 1 : 3;
     // 5x5 over an even number of channel words, on the tile its unrolled form is built for: one chunk to at most 256 channels
     // from half a tile per unit (28x28x64 to 192 at batch 8 / 16 / 64 7.9 -> 5.9 / 10.9 -> 7.0 / 20.0 -> 16.4, w1a4 at batch 8
     // 12.1 -> 10.0; level at batch 4 and to 512 channels), several without 128-bit loads from one tile per unit (14x14x192 to
     // 256 at batch 64 21.5 -> 13.3; with 100 tiles 9.4 -> 10.2)
     if (taps == 25 && p.S == 5 && p.stride == 1 &&
-        (p.C32 == 2 ? p.rowsB <= 256 && 2 * n128 >= cus : p.C32 % 4 == 2 && n128 >= cus))
+        (p.C32 == 2 ? p.rowsB <= 256 && 2 * n >= cus : p.C32 % 4 == 2 && n >= cus))
       return 3;
     // One chunk of channels (56x56x64 to 64 at batch 8 5.3 -> 4.6, 196 tiles; 28x28x64 to 192 at batch 64 11.8 -> 9.1;
     // below half a tile per unit 128x64 leaves too much idle: 4.3 -> 4.6 with 98), or channel words without 128-bit
@@ -376,16 +387,16 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     // 14x14x960 to 1024 at batch 16 33.4 -> 27.0, 7x7x480 to 512 at batch 64 18.2 -> 13.4).  A single channel word fills
     // half a chunk: to many channels it loses (32x32x32 to 1024 at batch 3 6.3 -> 6.7).
     if ((p.C32 <= 2 || p.C32 % 4 != 0) && (p.C32 > 1 || p.rowsB <= 64)) {
-      if (plain && 2 * n128 >= cus) return t;
+      if (plain && 2 * n >= cus) return t;
       // other filter sizes and strides
-      if (((p.rowsB <= 64 && p.C32 <= 2) || (p.C32 & 1)) && n128 >= 2 * cus) return t;
+      if (((p.rowsB <= 64 && p.C32 <= 2) || (p.C32 & 1)) && n >= 2 * cus) return t;
     }
     // 128 channels to at most 128 from 1.5 tiles per unit (28x28 at batch 64 9.9 -> 8.9, 56x56 at batch 64 28.0 -> 22.0; to
     // 256 channels the 128x256 tile of async_kernel.h is ahead, 13.6 -> 14.8)
-    if (plain && p.C32 == 4 && p.rowsB <= 128 && 2 * n128 >= 3 * cus) return t;
+    if (plain && p.C32 == 4 && p.rowsB <= 128 && 2 * n >= 3 * cus) return t;
     // 256 channels at 1.5 to 2 tiles per unit, all resident at once (14x14 to 256 at batch 64 9.9 -> 9.3, w1a4 17.4 -> 15.5;
     // w1a3, whose two FP4 digits cost as much as w1a4's, is level: 13.1 -> 13.4 on 28x28 at batch 16)
-    if (plain && p.C32 == 8 && p.planesA != 3 && 2 * n128 >= 3 * cus && n128 <= 2 * cus) return t;
+    if (plain && p.C32 == 8 && p.planesA != 3 && 2 * n >= 3 * cus && n <= 2 * cus) return t;
     return -1;
   }
   if (tile_pin != 0) {

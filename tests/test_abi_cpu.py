@@ -329,6 +329,11 @@ def test_patch_resident_tile_rule(batch, H, C, cout, R, stride, wb, xb, tile):
 
 
 @pytest.mark.parametrize("batch,H,C,cout,R,stride,wb,xb,out,tile", [
+    # 256x64 tiles save a round, or cut the filter expansion of two weight planes; not for general results
+    (62, 56, 64, 64, 3, 1, 1, 3, "avg", (128, 64)), (64, 56, 128, 128, 3, 1, 2, 2, "far", (128, 64)),
+    (64, 56, 128, 128, 3, 1, 2, 2, "bn", (256, 64)), (64, 14, 960, 192, 3, 1, 2, 2, "bn", (256, 64)),
+    (8, 16, 480, 896, 3, 1, 2, 2, "bn", (128, 64)), (48, 27, 960, 896, 3, 1, 1, 2, "far", (256, 64)),
+    (64, 32, 832, 192, 3, 1, 1, 3, "bn", (128, 64)),
     # 5x5 of four planes: the threshold table counts where a unit gets a second tile
     (7, 32, 64, 160, 5, 1, 1, 4, "bn", (128, 64)), (25, 32, 64, 160, 5, 1, 1, 4, "bn", None),
 ])
