@@ -325,6 +325,8 @@ int patch_pixels(const KParams &p, int R, int rows) {
   return span > 0x7fffffff ? 0x7fffffff : (int)span;
 }
 
+int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, int planes, int planesW);
+
 // Tile of the patch-resident convolution kernel, or -1 when it does not apply: the patch (at most
 // 1024 pixels) and the filter block of all taps must fit in LDS twice per compute unit.  When the
 // library chooses (`automatic`) the kernel is taken only where it measures faster than the
@@ -358,8 +360,16 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     const long long n = ntiles(3), n256 = ntiles(1);  // 128x64 and 256x64 tiles
     const bool plain = taps == 9 && p.S == 3 && p.stride == 1;  // the filters with an unrolled loop, the densest patches
     // Results that leave over the output stage's general path (its values pass LDS, and 2x2 blocks keep part of them in
-    // scratch).
+    // scratch), and those of them that are searched codes: pooled averages, unfolded shortcuts, int32 maps, pooled maxima
+    // of three and four bits.
     const bool general = p.epi != APNN_EPI_INT32 && !apnn::conv_float_codes(p, p.planesA >= 3 ? 4 : 2);
+    const bool searched = general && p.epi == APNN_EPI_BN;
+    // the tile that takes the layer otherwise, and whether its 128x256 tiles would fill one round of the units
+    const int vw = p.C32 % 4 == 0 ? 4 : p.C32 % 2 == 0 ? 2 : 1;
+    const int other = choose_mfma_tile(p.rowsA, p.rowsB, p.KW, true, vw, false, p.planesA + p.planesB, p.planesB);
+    auto others = [&](int ta, int tb) { return (long long)((p.rowsA + ta - 1) / ta) * ((p.rowsB + tb - 1) / tb); };
+    const long long big = others(128, 256);
+    const bool full_round = other == apnn::MT_128x256 && big <= 2 * cus && 10 * big >= 19 * cus;
     // 3x3: 256x64 tiles (three work-groups per unit at a time, against four of 128x64; LDS holds as many, but three of either
     // with two digits a pixel) where they save a round: 56x56x96 to 256 channels at batch 64 39.8 against 42.9, 27x27x96 to 256
     // 12.6 against 14.9, w1a3 level.  Not with four activation planes, whose patch is twice as large (97 against 92), nor for
@@ -374,6 +384,9 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     const bool tall = p.planesA <= 3 && fits(1) &&
                       (long_w2 || (r256 < r128 && (p.planesA == 2 ? !general || p.C32 >= 20 : !general && p.C32 < 20)));
     const int t = tall ? 1 : 3;
+    // Nowhere against the 32x32 split-K tile, which wins where half of a 64-channel tile is empty: 3x3 on 56x56x192 to 32 at
+    // batch 6, w1a4 8.0 -> 10.1, 5x5 on 28x28x64 to 32 at batch 24 8.5 -> 9.2.
+    if (other == apnn::MT_32x32_K4) return -1;
     // 5x5 over an even number of channel words, on the tile its unrolled form is built for: one chunk to at most 256 channels
     // from half a tile per unit (28x28x64 to 192 at batch 8 / 16 / 64 7.9 -> 5.9 / 10.9 -> 7.0 / 20.0 -> 16.4, w1a4 at batch 8
     // 12.1 -> 10.0; level at batch 4 and to 512 channels), several without 128-bit loads from one tile per unit (14x14x192 to
@@ -381,22 +394,45 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     if (taps == 25 && p.S == 5 && p.stride == 1 &&
         (p.C32 == 2 ? p.rowsB <= 256 && 2 * n >= cus : p.C32 % 4 == 2 && n >= cus))
       return 3;
-    // One chunk of channels (56x56x64 to 64 at batch 8 5.3 -> 4.6, 196 tiles; 28x28x64 to 192 at batch 64 11.8 -> 9.1;
-    // below half a tile per unit 128x64 leaves too much idle: 4.3 -> 4.6 with 98), or channel words without 128-bit
-    // loads, which leave the others their 32- and 64-bit forms (56x56x96 to 256 at batch 4 / 64 11.4 -> 7.4 / 68.9 -> 40.6,
-    // 14x14x960 to 1024 at batch 16 33.4 -> 27.0, 7x7x480 to 512 at batch 64 18.2 -> 13.4).  A single channel word fills
-    // half a chunk: to many channels it loses (32x32x32 to 1024 at batch 3 6.3 -> 6.7).
-    if ((p.C32 <= 2 || p.C32 % 4 != 0) && (p.C32 > 1 || p.rowsB <= 64)) {
-      if (plain && 2 * n >= cus) return t;
-      // other filter sizes and strides
-      if (((p.rowsB <= 64 && p.C32 <= 2) || (p.C32 & 1)) && n >= 2 * cus) return t;
+    // 3x3 over one chunk of channels (56x56x64 to 64 at batch 8 5.3 -> 4.6, 196 tiles; 28x28x64 to 192 at batch 64 11.8 -> 9.1;
+    // below half a tile per unit 128x64 leaves too much idle: 4.3 -> 4.6 with 98; searched codes from one tile per unit: 56x56x64
+    // to 64 at batch 6 with an int32 map 7.0 -> 8.0, averages of 28x28x64 to 640 at batch 4 7.1 -> 7.9, of 16x16x64 to 416 at batch
+    // 20, 280 tiles, 8.7 -> 7.4).  A single channel word fills half a chunk: to many channels it loses (32x32x32 to 1024 at batch
+    // 3 6.3 -> 6.7), and so does a layer whose 128x256 tiles fill one round (56x56x64 to 224 at batch 20, 490 tiles, w1a3
+    // 16.3 -> 20.1, w2a2 to 256 12.2 -> 12.7).
+    if (plain && p.C32 <= 2 && (p.C32 > 1 || p.rowsB <= 64) && !full_round && (searched ? n > cus : 2 * n >= cus)) return t;
+    // 3x3 over channel words without 128-bit loads, which leave the others their 32- and 64-bit forms (56x56x96 to 256 at batch
+    // 4 / 64 11.4 -> 7.4 / 68.9 -> 40.6, 14x14x960 to 1024 at batch 16 33.4 -> 27.0, 7x7x480 to 512 at batch 64 18.2 -> 13.4).
+    // An odd number: from half a tile per unit (searched codes: just above it).  Pairs: from half a tile over 192 channels,
+    // whose other kernel is the plain 64x64 tile; from 3/4 where that is the 32x64 split-K tile (27x27x320 to 704 at batch 2, 132
+    // tiles, w1a3 8.9 -> 10.8, 16x16x320 to 576 at batch 14, 252 tiles, w1a4 16.8 -> 13.6), w1a4 from half (7x7x320 to 704 at
+    // batch 32, 143 tiles, 16.5 -> 14.1).  Not long reductions of two digits a pixel against 128x256 tiles (14x14x960 to 1024 at
+    // batch 64 w1a3 / w1a4 86 -> 118 / 98 -> 133) or of w1a3 against 128x128 (28x28x960 to 384 at batch 48 128 -> 141); nor general
+    // results of two weight planes but on 256x64 tiles (28x28x928 to 320 at batch 7 33.2 -> 38.9) and not against 128x256 ones
+    // (low bits of 28x28x832 to 256 at batch 64 82 -> 98).
+    const bool w2_general = p.planesB > 1 && general && p.C32 > 16 && !tall;
+    if (plain && (p.C32 & 1) && p.C32 >= 3 && !w2_general && (searched ? 2 * n > cus : 2 * n >= cus)) return t;
+    if (plain && p.C32 % 4 == 2 && p.C32 > 2 && !full_round && !w2_general) {
+      const bool enough = p.C32 == 6 ? 2 * n >= cus : p.planesA == 4 && !general ? 2 * n > cus : 4 * n > 3 * cus;
+      const bool heavy = p.planesA >= 3 || (p.planesB > 1 && general);
+      const bool beaten = p.C32 >= 20 && heavy && (other == apnn::MT_128x256 ||
+                          (other == apnn::MT_128x128 && (p.planesA == 3 || (p.planesA == 4 && general))));
+      if (enough && !beaten) return t;
     }
+    // Other filter sizes and strides, over a single chunk to few channels or an odd number of words
+    if (((p.rowsB <= 64 && p.C32 <= 2) || (p.C32 & 1)) && !plain && n >= 2 * cus) return t;
     // 128 channels to at most 128 from 1.5 tiles per unit (28x28 at batch 64 9.9 -> 8.9, 56x56 at batch 64 28.0 -> 22.0; to
     // 256 channels the 128x256 tile of async_kernel.h is ahead, 13.6 -> 14.8)
     if (plain && p.C32 == 4 && p.rowsB <= 128 && 2 * n >= 3 * cus) return t;
     // 256 channels at 1.5 to 2 tiles per unit, all resident at once (14x14 to 256 at batch 64 9.9 -> 9.3, w1a4 17.4 -> 15.5;
-    // w1a3, whose two FP4 digits cost as much as w1a4's, is level: 13.1 -> 13.4 on 28x28 at batch 16)
-    if (plain && p.C32 == 8 && p.planesA != 3 && 2 * n >= 3 * cus && n <= 2 * cus) return t;
+    // w1a3, whose two FP4 digits cost as much as w1a4's, is level: 13.1 -> 13.4 on 28x28 at batch 16; w2a2 loses where 128x128
+    // tiles fill one round of the units, 28x28 to 128 at batch 40 11.1 -> 12.0, and wins else, 32x32 to 320 at batch 12
+    // 15.0 -> 11.1; the 32x64 split-K tile keeps int32 maps, and w1a4's int32 results and low bits: 32x32 to 64 at batch 48
+    // 11.1 -> 12.6, against 128x128 tiles 0.84-0.97 of their time)
+    const long long mid = others(128, 128);
+    const bool w2_full = p.planesB > 1 && !general && other == apnn::MT_128x128 && mid <= cus && 10 * mid >= 9 * cus;
+    const bool split_k = other == apnn::MT_32x64_K4 && (p.resid != nullptr || p.save_acc != nullptr || (p.planesA == 4 && p.epi != APNN_EPI_BN));
+    if (plain && p.C32 == 8 && p.planesA != 3 && !w2_full && !split_k && 2 * n >= 3 * cus && n <= 2 * cus) return t;
     return -1;
   }
   if (tile_pin != 0) {
@@ -419,7 +455,7 @@ int from_hip(hipError_t e) { return e == hipErrorNotSupported ? APNN_EUNSUPPORTE
 // is the one done four times per k-step; then 128x128, 64x64 (128x64 for <= 64 output channels) while every
 // compute unit still gets a work-group; when even 64x64 tiles leave most of the chip idle and the
 // reduction is long, the 32-row tiles whose four waves split K.
-int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, int planes = 3, int planesW = 1) {
+int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, int planes, int planesW) {
   const bool wide = planes > 5 || planes == 2;
   int cus = device_cus();
   if (cus <= 0) cus = 256;

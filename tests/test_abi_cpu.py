@@ -336,6 +336,18 @@ def test_patch_resident_tile_rule(batch, H, C, cout, R, stride, wb, xb, tile):
     (64, 32, 832, 192, 3, 1, 1, 3, "bn", (128, 64)),
     # 5x5 of four planes: the threshold table counts where a unit gets a second tile
     (7, 32, 64, 160, 5, 1, 1, 4, "bn", (128, 64)), (25, 32, 64, 160, 5, 1, 1, 4, "bn", None),
+    # searched codes from one tile per unit, pairs of words from 3/4 against the split-K tile
+    (6, 56, 64, 64, 3, 1, 1, 2, "map", None), (6, 56, 64, 64, 3, 1, 1, 2, "bn", (128, 64)),
+    (20, 16, 64, 416, 3, 1, 1, 2, "avg", (128, 64)), (16, 16, 96, 256, 3, 1, 1, 2, "avg", None),
+    (2, 27, 320, 704, 3, 1, 1, 3, "near", None), (14, 16, 320, 576, 3, 1, 1, 4, "int32", (128, 64)),
+    (32, 7, 320, 704, 3, 1, 1, 4, "near", (128, 64)), (28, 27, 320, 32, 3, 1, 1, 3, "int32", None),
+    # long reductions, full rounds of larger tiles, 256 channels
+    (64, 14, 960, 1024, 3, 1, 1, 2, "bn", (128, 64)), (64, 14, 960, 1024, 3, 1, 1, 3, "bn", None),
+    (64, 14, 960, 1024, 3, 1, 1, 4, "bn", None), (48, 28, 960, 384, 3, 1, 1, 3, "bn", None),
+    (64, 28, 832, 256, 3, 1, 2, 2, "low", None), (7, 28, 928, 320, 3, 1, 2, 2, "avg", None),
+    (20, 56, 64, 224, 3, 1, 1, 3, "bn", None), (40, 28, 256, 128, 3, 1, 2, 2, "bn", None),
+    (12, 32, 256, 320, 3, 1, 2, 2, "bn", (128, 64)), (48, 32, 256, 64, 3, 1, 1, 4, "int32", None),
+    (48, 32, 256, 64, 3, 1, 1, 4, "bn", (128, 64)),
 ])
 def test_patch_resident_tile_rule_by_output(batch, H, C, cout, R, stride, wb, xb, out, tile):
     """The rule where results other than two-bit codes, long reductions or rounds of the other tiles decide.  out: int32, bn,
