@@ -384,16 +384,26 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     const bool tall = p.planesA <= 3 && fits(1) &&
                       (long_w2 || (r256 < r128 && (p.planesA == 2 ? !general || p.C32 >= 20 : !general && p.C32 < 20)));
     const int t = tall ? 1 : 3;
-    // Nowhere against the 32x32 split-K tile, which wins where half of a 64-channel tile is empty: 3x3 on 56x56x192 to 32 at
-    // batch 6, w1a4 8.0 -> 10.1, 5x5 on 28x28x64 to 32 at batch 24 8.5 -> 9.2.
-    if (other == apnn::MT_32x32_K4) return -1;
-    // 5x5 over an even number of channel words, on the tile its unrolled form is built for: one chunk to at most 256 channels
+    // 5x5 over an even number of channel words, on the tile its unrolled form is built for.  One chunk to at most 192 channels
     // from half a tile per unit (28x28x64 to 192 at batch 8 / 16 / 64 7.9 -> 5.9 / 10.9 -> 7.0 / 20.0 -> 16.4, w1a4 at batch 8
-    // 12.1 -> 10.0; level at batch 4 and to 512 channels), several without 128-bit loads from one tile per unit (14x14x192 to
-    // 256 at batch 64 21.5 -> 13.3; with 100 tiles 9.4 -> 10.2)
-    if (taps == 25 && p.S == 5 && p.stride == 1 &&
-        (p.C32 == 2 ? p.rowsB <= 256 && 2 * n >= cus : p.C32 % 4 == 2 && n >= cus))
-      return 3;
+    // 12.1 -> 9.3; level at batch 4), to 256 for general results and while the 128x256 tiles of async_kernel.h leave much of
+    // a round empty (28x28 at batch 64 28.7 -> 23.9 w1a3; 56x56 at batch 28 / 40, 2744 / 3920 tiles, 27.3 -> 29.6 / 34.0 ->
+    // 41.6).  Several chunks without 128-bit loads from one tile per unit (14x14x192 to 256 at batch 64 21.5 -> 13.3; with 100
+    // tiles 9.4 -> 10.2), but not long reductions of two digits a pixel against that tile (w1a3 28x28x960 to 224 at batch 64 223
+    // -> 314).  Two weight planes, whose filter block costs most, on 256x64 tiles of the general form from one per unit, 3/4
+    // beyond 192 channels (28x28x832 to 128 at batch 64 115, 177 on 128x64 tiles, 126 otherwise).
+    // (Nowhere against the 32x32 split-K tile, which wins where half of a 64-channel tile is empty: 3x3 on 56x56x192 to 32 at
+    // batch 6, w1a4 8.0 -> 10.1, 5x5 on 28x28x64 to 32 at batch 24 8.5 -> 9.2.)
+    if (other == apnn::MT_32x32_K4) return -1;
+    if (taps == 25 && p.S == 5 && p.stride == 1 && p.C32 % 4 == 2) {
+      if (p.C32 == 2) return (p.rowsB <= 192 || (p.rowsB <= 256 && (general || n <= 8 * cus))) && 2 * n >= cus ? 3 : -1;
+      if (n < cus) return -1;
+      if (p.planesB > 1) {
+        if (fits(1) && 4 * n256 >= (p.C32 > 6 ? 3 : 4) * cus) return 1;
+        return p.C32 == 6 || p.rowsB <= 32 ? 3 : -1;
+      }
+      return p.planesA == 2 || p.C32 <= 14 || other != apnn::MT_128x256 ? 3 : -1;
+    }
     // 3x3 over one chunk of channels (56x56x64 to 64 at batch 8 5.3 -> 4.6, 196 tiles; 28x28x64 to 192 at batch 64 11.8 -> 9.1;
     // below half a tile per unit 128x64 leaves too much idle: 4.3 -> 4.6 with 98; searched codes from one tile per unit: 56x56x64
     // to 64 at batch 6 with an int32 map 7.0 -> 8.0, averages of 28x28x64 to 640 at batch 4 7.1 -> 7.9, of 16x16x64 to 416 at batch
@@ -419,8 +429,23 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
                           (other == apnn::MT_128x128 && (p.planesA == 3 || (p.planesA == 4 && general))));
       if (enough && !beaten) return t;
     }
-    // Other filter sizes and strides, over a single chunk to few channels or an odd number of words
-    if (((p.rowsB <= 64 && p.C32 <= 2) || (p.C32 & 1)) && !plain && n >= 2 * cus) return t;
+    // Other filter sizes and strides, from two tiles per unit, over a single chunk to few channels or an odd number of words.
+    if (((p.rowsB <= 64 && p.C32 <= 2) || (p.C32 & 1)) && !plain && n >= 2 * cus) {
+      // Strided filters but 3x3 and few taps reuse a patch too little, over long reductions most of all (2x2 on 56x56x864 to 160
+      // at batch 18, w1a4 low bits 74 -> 207, on 56x56x64 to 64 at batch 24 6.1 -> 6.6; 28x28x288 to 288 at batch 42, w2a2
+      // 51.7 -> 27.4; 4x4 of stride 2 on 56x56x96 to 256 at batch 64 31.6 -> 45.2).
+      if (taps != 9 && p.stride > 1) return -1;
+      if (taps < 9) return p.C32 > 9 || (p.C32 == 2 && p.planesA != 3) ? -1 : t;
+      if (taps < 16) return t;
+      // From sixteen taps on the filter block is most of what is staged: 256x64 tiles, which expand it for twice the pixels (4x4
+      // on 32x32x224 to 320 at batch 29, w2a2 34.1, 46.3 on 128x64 tiles, 43.8 otherwise; 5x5 on 32x32x224 to 224 at batch 64
+      // 56, 89, 99), low bits where they save a round.  Searched codes over long reductions, or where they save a round, only
+      // (4x4 on 27x27x480 to 832 at batch 48 160, 219 otherwise; averages of 27x27x224 to 160 at batch 56, w1a3 45.0, 39.7), two digits a pixel not over
+      // one or two words (4x4 on 56x56x32 to 64 at batch 50, w1a4 27.7, 24.7).
+      if (p.planesA > 2 ? searched || p.C32 < 3 : searched && p.C32 < 9 && (r256 >= r128 || p.C32 < 5)) return -1;
+      if (fits(1) && (!general || searched || r256 < r128)) return 1;
+      return p.planesA == 2 || p.C32 >= 5 ? 3 : -1;
+    }
     // 128 channels to at most 128 from 1.5 tiles per unit (28x28 at batch 64 9.9 -> 8.9, 56x56 at batch 64 28.0 -> 22.0; to
     // 256 channels the 128x256 tile of async_kernel.h is ahead, 13.6 -> 14.8)
     if (plain && p.C32 == 4 && p.rowsB <= 128 && 2 * n >= 3 * cus) return t;

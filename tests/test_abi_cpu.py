@@ -348,6 +348,13 @@ def test_patch_resident_tile_rule(batch, H, C, cout, R, stride, wb, xb, tile):
     (20, 56, 64, 224, 3, 1, 1, 3, "bn", None), (40, 28, 256, 128, 3, 1, 2, 2, "bn", None),
     (12, 32, 256, 320, 3, 1, 2, 2, "bn", (128, 64)), (48, 32, 256, 64, 3, 1, 1, 4, "int32", None),
     (48, 32, 256, 64, 3, 1, 1, 4, "bn", (128, 64)),
+    # 5x5 and the other filters
+    (40, 56, 64, 256, 5, 1, 1, 2, "bn", None), (64, 28, 64, 256, 5, 1, 1, 3, "bn", (128, 64)),
+    (64, 14, 448, 576, 5, 1, 2, 2, "bn", (256, 64)), (48, 14, 448, 256, 5, 1, 2, 2, "low", None),
+    (64, 28, 960, 224, 5, 1, 1, 3, "bn", None), (64, 32, 224, 224, 5, 1, 1, 2, "bn", (256, 64)),
+    (29, 32, 224, 320, 4, 1, 2, 2, "int32", (256, 64)), (56, 27, 224, 160, 4, 1, 1, 3, "avg", None),
+    (18, 56, 864, 160, 2, 1, 1, 4, "low", None), (64, 56, 96, 256, 4, 2, 1, 2, "bn", None),
+    (42, 28, 288, 288, 2, 1, 2, 2, "bn", (256, 64)),
 ])
 def test_patch_resident_tile_rule_by_output(batch, H, C, cout, R, stride, wb, xb, out, tile):
     """The rule where results other than two-bit codes, long reductions or rounds of the other tiles decide.  out: int32, bn,
