@@ -466,8 +466,17 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
   }
   const int narrow[3] = {3, 1, 4}, wide[3] = {2, 0, 4};  // 128x64, 256x64, 64x64 / 64x128, 128x128, 64x64
   const int *cand = p.rowsB <= 64 ? narrow : wide;
+  // Without a pin, 128-column tiles only where two digits a pixel would fit: a filter block that fills the rest of the 80 KB is
+  // better cut in two (4x4 on 56x56x96 to 608 at batch 8, unfolded shortcut 80 us on 64x64 tiles, 122 on 64x128; 27x27x224 to 832
+  // at batch 8, averages 34 and 43).
+  auto roomy = [&](int t) {
+    const size_t cap = (size_t)patch_pixels(p, R, apnn::kPatchTileRows[t]);
+    return fits(t) && (apnn::kPatchTileCols[t] < 128 || (cap * 17 + (size_t)taps * 128 * 8) * 4 <= 80 * 1024);
+  };
   for (int i = 0; i < 3; ++i)
-    if (fits(cand[i]) && ntiles(cand[i]) >= cus) return cand[i];
+    if (roomy(cand[i]) && ntiles(cand[i]) >= cus) return cand[i];
+  for (int i = 2; i >= 0; --i)
+    if (roomy(cand[i])) return cand[i];
   for (int i = 2; i >= 0; --i)
     if (fits(cand[i])) return cand[i];
   return -1;

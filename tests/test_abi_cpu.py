@@ -388,6 +388,15 @@ def test_patch_tile_of_auto_can_be_pinned(batch, H, C, cout, R, wb, xb):
         assert rc == 0 and (pinned.tile, pinned.patch_pixels) == (auto.tile, auto.patch_pixels)
 
 
+@pytest.mark.parametrize("batch,H,C,cout,R,tile", [(8, 56, 96, 608, 4, 4), (8, 27, 224, 832, 4, 4), (64, 14, 96, 256, 4, 2),
+                                                  (64, 28, 128, 256, 3, 2), (46, 28, 192, 64, 5, 3)])
+def test_patch_path_without_a_tile(batch, H, C, cout, R, tile):
+    """The tile that the patch path takes by itself: 64x128 where two digits a pixel fit beside the filter block, else 64x64."""
+    rc, plan = _plan_conv(batch=batch, H=H, Wd=H, cin_pad=C, COUT=cout, R=R, S=R, stride=1, pad=(R - 1) // 2, halo=0, wb=1, xb=2,
+                          path=A.PATH_MFMA_PATCH)
+    assert rc == 0 and plan.tile == tile
+
+
 @pytest.mark.parametrize("H", [28, 32, 60, 64, 66, 68, 70, 72, 74])
 @pytest.mark.parametrize("xb,out_bits", [(2, 2), (2, 4), (3, 3), (4, 4), (4, 2)])
 def test_auto_takes_5x5_patches_that_fit_twice(H, xb, out_bits):
