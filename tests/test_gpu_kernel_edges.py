@@ -369,3 +369,59 @@ def test_patch_conv_forms(G, wb, xb, tile, H, Wd, C, cout, R, S, stride, sym):
     got = G.run_conv(W, X, cin_pad=C, sym=sym, epi=epi, path=G.A.PATH_MFMA_PATCH, tile=tile, **kw).view(np.uint32)
     expect = O.lowbits_pack(O.bn_quantize(acc, None, thr, flip, xb), acc.shape[0], cout, xb)
     assert np.array_equal(got.reshape(expect.shape), expect)
+
+
+# Every output of the patch-resident convolution, in each form of its kernel: low bits, pooled averages and maxima, searched and
+# compared codes of one to four bits, flips, a shortcut that the matrix cores add (with one and two digits a pixel, with
+# weight operands of -1 / +1, of 0 / 1 and of two planes) and one that they do not, an int32 map with the sums saved.
+@pytest.mark.parametrize("tile", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("wb,xb,ob,sym", [(1, 2, 2, 1), (1, 2, 3, 0), (1, 3, 3, 1), (1, 4, 4, 1), (1, 4, 2, 0), (2, 2, 1, 0), (2, 2, 2, 1)])
+@pytest.mark.parametrize("batch,H,C,R", [(3, 6, 128, 3), (2, 10, 96, 3), (3, 8, 64, 5), (2, 6, 160, 2)])
+@pytest.mark.parametrize("out", ["low", "low_avg", "low_max", "near", "far", "map", "avg", "max"])
+def test_patch_conv_output_forms(G, tile, wb, xb, ob, sym, batch, H, C, R, out):
+    if R == 5 and tile not in ((1, 3, 4) if xb == 2 else (3, 4)):
+        pytest.skip("the patch and the filter block of 25 taps do not fit")
+    cout, pad, far = 96, R // 2, 1365
+    rng = np.random.default_rng(9300 + 100 * tile + 10 * xb + ob + 3 * C + len(out))
+    Ho = H + 2 * pad - R + 1
+    if out[-3:] in ("avg", "max") and Ho % 2:
+        H, Ho = H + 1, Ho + 1
+    W, X = O.random_planes(rng, wb, cout * R * R, C // 32), O.random_planes(rng, xb, batch * H * H, C // 32)
+    kw = dict(batch=batch, H=H, W=H, cout=cout, R=R, S=R, stride=1, pad=pad, halo=0, wb=wb, xb=xb)
+    v = O.conv(W, X, cwords=C // 32, sym_w=sym, **kw).reshape(-1, cout).astype(np.int64)
+    extra, keep, pool = {}, [], {"avg": 1, "max": 2}.get(out[-3:], 0)
+    if out in ("near", "far"):
+        scale = 12 if out == "near" else far
+        short = rng.integers(0, 4, size=v.shape).astype(np.uint32)
+        v = v + scale * short.astype(np.int64)
+        keep.append(G.to_dev(O.pack_bits(short, v.shape[0], cout, cout, 2)))
+        extra = dict(resid_planes=keep[-1], resid_bits=2, resid_scale=scale)
+    elif out == "map":
+        res = rng.integers(-500, 500, size=v.shape).astype(np.int32)
+        v = v + res
+        keep += [G.to_dev(res), G.dev_empty_i32(v.size, fill=-7)]
+        extra = dict(resid=keep[0], save=keep[1])
+    if pool:  # windows in raster order, four values each
+        v = v.reshape(batch, Ho // 2, 2, Ho // 2, 2, cout).transpose(0, 1, 3, 2, 4, 5).reshape(-1, 4, cout)
+    if pool == 1:
+        s = v.sum(axis=1)
+        v = np.where(s < 0, -(-s // 4), s // 4)[:, None, :]
+    v = v.reshape(-1, cout)
+    if out.startswith("low"):
+        epi = G.epilogue(mode=G.A.EPI_LOWBITS, out_bits=ob, pool=pool)
+        q = v & (2 ** ob - 1)
+    else:
+        thr = np.sort(rng.integers(v.min() - 5, v.max() + 6, size=(cout, 2 ** ob - 1)), axis=1).astype(np.int32)
+        thr[0, :], thr[1, :] = np.iinfo(np.int32).min, np.iinfo(np.int32).max
+        flip = rng.integers(0, 2, size=cout).astype(np.uint8)
+        thr[flip != 0] = np.sort(-thr[flip != 0].astype(np.int64), axis=1).clip(-2 ** 31, 2 ** 31 - 1).astype(np.int32)
+        keep += [G.to_dev(thr), G.to_dev(flip)]
+        epi = G.epilogue(mode=G.A.EPI_BN, out_bits=ob, pool=pool, thr=keep[-2], flip=keep[-1], **extra)
+        q = O.bn_quantize(v.astype(np.int32), None, thr, flip, ob)
+    q = np.asarray(q).astype(np.uint32).reshape(-1, cout)
+    if pool == 2:
+        q = np.ascontiguousarray(q.reshape(-1, 4, cout).max(axis=1))
+    got = G.run_conv(W, X, cin_pad=C, sym=sym, epi=epi, path=G.A.PATH_MFMA_PATCH, tile=tile, **kw).view(np.uint32)
+    assert np.array_equal(got.reshape(ob, -1, cout // 32), O.lowbits_pack(q, q.shape[0], cout, ob))
+    if out == "map":
+        assert np.array_equal(G.to_host(keep[1]).reshape(v.shape), v)
