@@ -379,12 +379,9 @@ inline hipError_t launch_async(const KParams &p, hipStream_t stream) {
   static_assert(most <= 160 * 1024, "LDS of a compute unit");
   auto kern = p.sym ? apnn_async_kernel<PA, PB, FA, FB, WA, WB, CONV, true, OCC> : apnn_async_kernel<PA, PB, FA, FB, WA, WB, CONV, false, OCC>;
   if (most > 64 * 1024) {
-    static bool raised[2] = {false, false};  // a repeated call is harmless
-    if (!raised[p.sym != 0]) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
-      if (e != hipSuccess) return e;
-      raised[p.sym != 0] = true;
-    }
+    static std::atomic<unsigned long long> raised[2];
+    const hipError_t e = raise_lds_limit(raised[p.sym != 0], reinterpret_cast<const void *>(kern), most);
+    if (e != hipSuccess) return e;
   }
   const long long tilesB = (p.rowsB + TB - 1) / TB, tiles = (long long)((p.rowsA + TA - 1) / TA) * tilesB;
   KParams q = p;

@@ -2,9 +2,23 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+
 #include "kparams.h"
 
 namespace apnn {
+
+// Raises the limit of a kernel's dynamic LDS on the current device.  `done` belongs to the kernel and holds a bit per device:
+// the attribute is a device's own, and threads may launch at once (a repeated call is harmless).
+inline hipError_t raise_lds_limit(std::atomic<unsigned long long> &done, const void *kern, size_t bytes) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  const unsigned long long bit = 1ull << (dev & 63);
+  if (e != hipSuccess || (done.load(std::memory_order_relaxed) & bit) != 0) return e;
+  e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  if (e == hipSuccess) done.fetch_or(bit, std::memory_order_relaxed);
+  return e;
+}
 
 #define APNN_DECL_VALU(kind, pa, pb) \
   hipError_t valu_##kind##_##pa##_##pb##_x(int vw, int tile, const KParams &p, hipStream_t s);

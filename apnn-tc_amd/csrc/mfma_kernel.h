@@ -1900,13 +1900,9 @@ inline hipError_t launch_mfma(const KParams &p, hipStream_t stream) {
   const size_t launch_bytes = smem_bytes + (LP ? conv_epilogue_bytes(p, TB) : 0);
   constexpr size_t attr_bytes = smem_bytes + (LP ? (conv_table_words(4, TB) + 4) * 4 : 0);
   if (attr_bytes > 64 * 1024) {
-    static bool raised = false;  // per instantiation; a repeated call is harmless
-    if (!raised) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)attr_bytes);
-      if (e != hipSuccess) return e;
-      raised = true;
-    }
+    static std::atomic<unsigned long long> raised;
+    const hipError_t e = raise_lds_limit(raised, reinterpret_cast<const void *>(kern), attr_bytes);
+    if (e != hipSuccess) return e;
   }
   const long long tiles = (long long)((p.rowsA + TA - 1) / TA) * ((p.rowsB + TB - 1) / TB);
   KParams q = p;

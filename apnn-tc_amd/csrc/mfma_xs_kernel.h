@@ -350,13 +350,9 @@ inline hipError_t launch_mfma_xs(const KParams &p, hipStream_t stream) {
   static_assert(smem_bytes + 2048 <= 160 * 1024, "LDS budget of a gfx950 compute unit");
   auto kern = apnn_mfma_xs_kernel<PA, PB, FA, FB, WA, WB, VW, CONV, OCC>;
   if (smem_bytes > 64 * 1024) {
-    static bool raised = false;
-    if (!raised) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_bytes);
-      if (e != hipSuccess) return e;
-      raised = true;
-    }
+    static std::atomic<unsigned long long> raised;
+    const hipError_t e = raise_lds_limit(raised, reinterpret_cast<const void *>(kern), smem_bytes);
+    if (e != hipSuccess) return e;
   }
   const long long tiles = (long long)((p.rowsA + TA - 1) / TA) * ((p.rowsB + TB - 1) / TB);
   KParams q = p;

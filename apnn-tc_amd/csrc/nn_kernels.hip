@@ -999,14 +999,8 @@ hipError_t launch_conv_i8_bn(const int8_t *X, const int8_t *Wt, const int32_t *t
       int per_cu = 0, cus = 0, dev = 0;
       hipError_t e = hipGetDevice(&dev);
       if (all > 64 * 1024 && e == hipSuccess) {
-        // once per kernel and device (a bit each; a repeated call is harmless)
         static std::atomic<unsigned long long> raised[5];
-        const unsigned long long bit = 1ull << (dev & 63);
-        if ((raised[variant].load(std::memory_order_relaxed) & bit) == 0) {
-          e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  80 * 1024 + kRowsTable);
-          if (e == hipSuccess) raised[variant].fetch_or(bit, std::memory_order_relaxed);
-        }
+        e = raise_lds_limit(raised[variant], reinterpret_cast<const void *>(kern), 80 * 1024 + kRowsTable);
       }
       if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
       if (e == hipSuccess)
@@ -1044,13 +1038,9 @@ hipError_t launch_conv_i8_bn(const int8_t *X, const int8_t *Wt, const int32_t *t
     const size_t lds = (size_t)64 * (R * KR * 32 + 16) + 4 * (size_t)patch_words * 4;
     if (lds <= 160 * 1024) {
       if (lds > 64 * 1024) {
-        static bool raised = false;
-        if (!raised) {
-          const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(conv_i8_c4_kernel),
-                                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-          if (e != hipSuccess) return e;
-          raised = true;
-        }
+        static std::atomic<unsigned long long> raised;
+        const hipError_t e = raise_lds_limit(raised, reinterpret_cast<const void *>(conv_i8_c4_kernel), 160 * 1024);
+        if (e != hipSuccess) return e;
       }
       hipLaunchKernelGGL(conv_i8_c4_kernel, grid, dim3(256), lds, s, X, Wt, thr, codes, acc_out, planes, B, H, W, C,
                          COUT, R, S, stride, pad, Ho, Wo, bits, zero_point, KR, PW, patch_words);

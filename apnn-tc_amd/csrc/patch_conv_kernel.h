@@ -382,13 +382,9 @@ inline hipError_t launch_patch_form(const KParams &p, hipStream_t stream) {
   if (smem_bytes > 160 * 1024 || p.patch_cap > PATCH_NPT * 256) return hipErrorNotSupported;
   auto kern = apnn_patch_conv_kernel<PA, PB, FA, FB, WA, WB, FORM>;
   if (smem_bytes > 64 * 1024) {
-    static bool raised = false;  // a repeated call is harmless
-    if (!raised) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-      if (e != hipSuccess) return e;
-      raised = true;
-    }
+    static std::atomic<unsigned long long> raised;
+    const hipError_t e = raise_lds_limit(raised, reinterpret_cast<const void *>(kern), 160 * 1024);
+    if (e != hipSuccess) return e;
   }
   const long long tiles = (long long)((p.rowsA + TA - 1) / TA) * ((p.rowsB + TB - 1) / TB);
   hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(256), smem_bytes, stream, p);
