@@ -63,6 +63,12 @@ int device_cus() {
 
 uint32_t magic_of(int d) { return d >= 2 ? (uint32_t)(((1ull << 32) + (uint32_t)d - 1) / (uint32_t)d) : 0u; }
 
+// Whether the multiply-high by magic_of(d) is n / d for all n < top: n times its excess over 2^32 / d must stay below 2^32.
+bool exact_below(int d, long long top) {
+  const unsigned long long excess = d >= 2 ? (unsigned long long)magic_of(d) * (unsigned)d - (1ull << 32) : 0;
+  return excess * (unsigned long long)top < (1ull << 32);
+}
+
 // largest tile that still gives every compute unit a work-group, else the smallest one
 int choose_tile(int rowsA, int rowsB, bool packed) {
   static const int ta[apnn::TILE_COUNT] = {64, 32, 16, 16};
@@ -783,6 +789,7 @@ int build_conv_params(const apnn_conv_desc *d, KParams &p, int *vw_out) {
   p.pad = d->halo ? 0 : d->pad;
   p.magicC32 = d->R * d->S == 1 ? 0u : magic_of(C32);  // one tap: every word belongs to tap 0, however many there are
   p.magicS = magic_of(d->S);
+  p.tap_div = !(p.magicC32 == 0 || exact_below(C32, KW)) || !exact_below(d->S, (long long)d->R * d->S);
   p.pool_order = d->epi.pool != APNN_POOL_NONE;
   p.sym = d->weight_mode == APNN_WEIGHT_SYMMETRIC;
   p.wmax = (1 << d->wb) - 1;
@@ -799,7 +806,7 @@ int build_conv_params(const apnn_conv_desc *d, KParams &p, int *vw_out) {
     const long long taps = (long long)d->R * d->S;
     p.c32_shift = pow2 ? sh : -1;
     p.magicS16 = (uint32_t)((65536 + d->S - 1) / d->S);
-    p.addr32 = taps * d->S < 65536 && (long long)p.Ws * d->R < (1 << 24) && C32 < (1 << 24) && KW < (1 << 24) &&
+    p.addr32 = !p.tap_div && taps * d->S < 65536 && (long long)p.Ws * d->R < (1 << 24) && C32 < (1 << 24) && KW < (1 << 24) &&
                (unsigned long long)p.planeA * 4ull < (1ull << 32) && (unsigned long long)p.planeB * 4ull < (1ull << 32);
   }
   p.batch = d->batch;
@@ -841,7 +848,7 @@ int run_conv(const apnn_conv_desc *d, hipStream_t stream, apnn_plan *plan = null
     return APNN_EUNSUPPORTED;
   if (path == APNN_PATH_MFMA_XS) {
     valu_fn fn = mfmaxs_conv_fn(d->xb, d->wb);
-    if (fn == nullptr) return APNN_EUNSUPPORTED;
+    if (fn == nullptr || p.tap_div) return APNN_EUNSUPPORTED;
     tile = tile_pin == 0 ? choose_xs_tile(p.rowsA, p.rowsB, true) : tile_pin - 1;
     if (tile >= apnn::kMfmaTileCount) return APNN_EINVAL;
     if (!apnn::mfma_xs_tile_enabled(true, vw, tile)) return APNN_EUNSUPPORTED;
@@ -867,7 +874,7 @@ int run_conv(const apnn_conv_desc *d, hipStream_t stream, apnn_plan *plan = null
     }
     if (path == APNN_PATH_MFMA_PATCH) return APNN_EUNSUPPORTED;
   }
-  // operand planes of 4 GiB or more, or a filter beyond the kernels' 24-bit index arithmetic: refused
+  // operand planes of 4 GiB or more, or a filter beyond the kernels' index arithmetic (24 bits, exact quotients): refused
   if ((path == APNN_PATH_MFMA || path == APNN_PATH_MFMA_I8) && !p.addr32) return APNN_EUNSUPPORTED;
   if (path == APNN_PATH_MFMA || path == APNN_PATH_MFMA_I8 || (path == APNN_PATH_AUTO && p.addr32 && (auto_prefers_mfma(p) || any_precision_only(d->wb, d->xb, tile_pin)))) {
     const bool i8 = path == APNN_PATH_MFMA_I8 || (path == APNN_PATH_AUTO && !f4ok);
@@ -883,7 +890,7 @@ int run_conv(const apnn_conv_desc *d, hipStream_t stream, apnn_plan *plan = null
     }
     if (path != APNN_PATH_AUTO) return APNN_EUNSUPPORTED;
   }
-  valu_fn fn = valu_conv_fn(d->xb, d->wb);
+  valu_fn fn = p.tap_div ? apnn::valu_conv_any_x : valu_conv_fn(d->xb, d->wb);
   if (fn == nullptr) return APNN_EUNSUPPORTED;
   if ((rc = pick_valu_tile(tile_pin, p, d->epi.mode != APNN_EPI_INT32, &tile))) return rc;
   if (plan != nullptr) return plan_valu(plan, tile, fn == apnn::valu_conv_any_x, p, f4ok);

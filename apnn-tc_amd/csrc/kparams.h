@@ -28,6 +28,7 @@ struct KParams {
   int S;                     // filter width (filter height = KW / (S*C32))
   int stride, pad;
   uint32_t magicC32, magicS; // ceil(2^32/d) for d >= 2 (unused when d == 1; magicC32 is 0 for a single tap)
+  int tap_div;               // 1: these quotients are not exact over the whole filter; the any-precision popcount kernel divides, others refuse
   int pool_order;            // 1: row index enumerates 2x2 output windows (4 consecutive rows each)
 
   // patch-resident convolution kernel only: padded frame (stored frame + pad on every side) and

@@ -48,7 +48,8 @@ __device__ __forceinline__ uint32_t fast_div(uint32_t n, uint32_t d, uint32_t m)
   return d == 1 ? n : __umulhi(n, m);
 }
 
-template <int PA, int PB, int RA, int RB, int VW, bool CONV>
+// DIV: filter taps by division (KParams::tap_div)
+template <int PA, int PB, int RA, int RB, int VW, bool CONV, bool DIV = false>
 __global__ __launch_bounds__(256) void apnn_valu_kernel(const KParams p) {
   // PA == PB == 8 is the any-precision instantiation: the plane counts of the launch (1..8 each) come
   // from KParams and the plane loops skip what is not there.
@@ -145,9 +146,9 @@ __global__ __launch_bounds__(256) void apnn_valu_kernel(const KParams p) {
       bool ok = a_ok[it] && kw0 < p.KW;
       long long off;
       if (CONV) {
-        const uint32_t tap = fast_div((uint32_t)kw0, (uint32_t)p.C32, p.magicC32);
+        const uint32_t tap = DIV ? (uint32_t)kw0 / (uint32_t)p.C32 : fast_div((uint32_t)kw0, (uint32_t)p.C32, p.magicC32);
         const int cw = kw0 - (int)tap * p.C32;
-        const uint32_t r = fast_div(tap, (uint32_t)p.S, p.magicS);
+        const uint32_t r = DIV ? tap / (uint32_t)p.S : fast_div(tap, (uint32_t)p.S, p.magicS);
         const int s = (int)tap - (int)r * p.S;
         const int iy = a_y0[it] + (int)r, ix = a_x0[it] + s;
         ok = ok && iy >= 0 && iy < p.Hs && ix >= 0 && ix < p.Ws;
@@ -317,11 +318,11 @@ __global__ __launch_bounds__(256) void apnn_valu_kernel(const KParams p) {
   }
 }
 
-template <int PA, int PB, int RA, int RB, int VW, bool CONV>
+template <int PA, int PB, int RA, int RB, int VW, bool CONV, bool DIV = false>
 inline hipError_t launch_valu(const KParams &p, hipStream_t stream) {
   constexpr int TA = 16 * RA, TB = 16 * RB;
   const long long tiles = (long long)((p.rowsA + TA - 1) / TA) * ((p.rowsB + TB - 1) / TB);
-  hipLaunchKernelGGL((apnn_valu_kernel<PA, PB, RA, RB, VW, CONV>), dim3((unsigned)tiles), dim3(256), 0, stream, p);
+  hipLaunchKernelGGL((apnn_valu_kernel<PA, PB, RA, RB, VW, CONV, DIV>), dim3((unsigned)tiles), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 

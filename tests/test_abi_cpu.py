@@ -271,6 +271,24 @@ def test_matrix_core_kernels_refuse_operands_beyond_32_bit_offsets():
     assert rc == 0 and plan.kernel == A.KERNEL_MFMA_FP4
 
 
+@pytest.mark.parametrize("words,S,exact", [(92820, 2, False), (66466, 2, False), (46779, 2, False), (46780, 2, True), (65536, 2, True),
+                                           (92816, 2, True), (131072, 1, True), (174760, 1, True), (44196, 9, False)])
+def test_filters_whose_taps_need_a_division(words, S, exact):
+    """A word index becomes a filter tap by a multiply-high.  Where it is not exact over the whole filter the matrix-core
+    kernels refuse and AUTO takes the any-precision popcount kernel, which divides; one tap and powers of two need no quotient."""
+    m = (2 ** 32 + words - 1) // words
+    wrong = any((n * m) >> 32 != n // words for t in range(S) for n in [(t + 1) * words - (4 if words % 4 == 0 else 2 if words % 2 == 0 else 1)])
+    assert S == 1 or not (exact and wrong)
+    geo = dict(batch=1, H=32, Wd=32 + S, COUT=256, cin_pad=32 * words, R=1, S=S, stride=1, pad=0, halo=0, wb=1, xb=2)
+    rc, plan = _plan_conv(path=A.PATH_AUTO, **geo)
+    assert rc == 0 and (plan.kernel == A.KERNEL_VALU_TILE) != exact
+    rc, _ = _plan_conv(path=A.PATH_MFMA_I8, **geo)
+    assert rc == (0 if exact else A.EUNSUPPORTED)
+    for path in (A.PATH_MFMA, A.PATH_MFMA_XS):
+        rc, _ = _plan_conv(path=path, **geo)
+        assert exact or rc == A.EUNSUPPORTED
+
+
 def test_plan_reports_the_dispatchers_choices():
     """Without a device the dispatcher assumes 256 compute units: the choices for the benchmark shapes."""
     rc, plan = _plan_gemm(M=64, N=1024, K=1024, wb=1, xb=2, path=A.PATH_AUTO)

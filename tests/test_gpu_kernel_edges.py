@@ -334,6 +334,18 @@ def test_very_long_single_tap(G, path, tile):
     assert np.all(got == 3 * K)
 
 
+@pytest.mark.parametrize("path,tile", [(0, None), (1, 0), (1, 1), (1, 3)])
+@pytest.mark.parametrize("words", [92820, 66466, 46779])
+def test_taps_of_very_long_filters(G, path, tile, words):
+    """Two taps of 128-, 64- and 32-bit loads over more channels than the multiply-high finds the tap of exactly."""
+    rows, cols = 8, 32
+    rng = np.random.default_rng(words)
+    W, X = O.random_planes(rng, 1, cols * 2, words), O.random_planes(rng, 2, rows + 1, words)
+    kw = dict(batch=1, H=1, W=rows + 1, cout=cols, R=1, S=2, stride=1, pad=0, halo=0, wb=1, xb=2)
+    got = G.run_conv(W, X, cin_pad=32 * words, sym=0, path=path, tile=tile, **kw)
+    assert np.array_equal(got.reshape(rows, cols), O.conv(W, X, cwords=words, sym_w=0, **kw).reshape(rows, cols))
+
+
 # Patch-resident convolution: the forms of its kernel (any filter; 3x3 over an odd and over an even number of channel words; 5x5
 # over an even one, run on the narrow tiles), one chunk of 64 channels and several, rows one past a tile and one short of it, a last column tile that is
 # mostly empty, raw sums and codes with flips.
