@@ -370,36 +370,42 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     // of three and four bits.
     const bool general = p.epi != APNN_EPI_INT32 && !apnn::conv_float_codes(p, p.planesA >= 3 ? 4 : 2);
     const bool searched = general && p.epi == APNN_EPI_BN;
-    // the tile that takes the layer otherwise, and whether its 128x256 tiles would fill one round of the units
+    // the tile that takes the layer otherwise, and how full the rounds of its large tiles are (two per unit at a time)
     const int vw = p.C32 % 4 == 0 ? 4 : p.C32 % 2 == 0 ? 2 : 1;
     const int other = choose_mfma_tile(p.rowsA, p.rowsB, p.KW, true, vw, false, p.planesA + p.planesB, p.planesB);
-    auto others = [&](int ta, int tb) { return (long long)((p.rowsA + ta - 1) / ta) * ((p.rowsB + tb - 1) / tb); };
-    const long long big = others(128, 256);
-    const bool full_round = other == apnn::MT_128x256 && big <= 2 * cus && 10 * big >= 19 * cus;
-    // 3x3: 256x64 tiles (three work-groups per unit at a time, against four of 128x64; LDS holds as many, but three of either
-    // with two digits a pixel) where they save a round: 56x56x96 to 256 channels at batch 64 39.8 against 42.9, 27x27x96 to 256
-    // 12.6 against 14.9, w1a3 level.  Not with four activation planes, whose patch is twice as large (97 against 92), nor for
-    // general results (1.1 to 1.6 times the 128x64 tile's time: 56x56x64 to 64 at batch 62, w1a3 averages 27.6 against 19.2),
-    // unless the reduction is long (27x27x960 to 896 at batch 48 187 against 221; w1a3, the other way round, 832 to 192 at batch
-    // 64 on 32x32 117 against 102).  With two weight planes over many chunks of
-    // channels also at equal rounds, as each tile expands its filter block again (28x28x320 to 256 at batch 64 31.9 against
-    // 39.1), from 9/16 of a tile per unit (14x14x960 to 192 at batch 64, 147 tiles, 31.3 against 39.1; 28x28x320 to 32 at batch
-    // 25, 77 tiles, 14.6 against 9.4), general results from one.
+    auto others = [&](int tb) { return (long long)((p.rowsA + 127) / 128) * ((p.rowsB + tb - 1) / tb); };
+    const long long large = others(other == apnn::MT_128x256 ? 256 : 128);
+    const double full = (double)large / (double)((large + 2 * cus - 1) / (2 * cus) * (2 * cus));
+    const bool full_round = other == apnn::MT_128x256 && large <= 2 * cus && full >= 0.95;
+    // 3x3: 256x64 tiles (three work-groups per unit at a time, against four of 128x64; LDS holds as many, but three of
+    // either with two digits a pixel) where they save a round: 56x56x96 to 256 channels at batch 64 39.8 against 42.9,
+    // 27x27x96 to 256 12.6 against 14.9, w1a3 level.  Not with four activation planes, whose patch is twice as large
+    // (97 against 92), nor for general results (1.1 to 1.6 times the 128x64 tile's time: 56x56x64 to 64 at batch 62,
+    // w1a3 averages 27.6 against 19.2), unless the reduction is long (27x27x960 to 896 at batch 48 187 against 221;
+    // w1a3, the other way round, 832 to 192 at batch 64 on 32x32 117 against 102).  With two weight planes over many
+    // chunks of channels also at equal rounds, as each tile expands its filter block again (28x28x320 to 256 at batch
+    // 64 31.9 against 39.1), from 9/16 of a tile per unit (14x14x960 to 192 at batch 64, 147 tiles, 31.3 against 39.1;
+    // 28x28x320 to 32 at batch 25, 77 tiles, 14.6 against 9.4), general results from one; with one weight plane over
+    // long reductions from one (14x14x832 to 512 at batch 64 31 against 41), below 26 words where no unit gets a larger
+    // share or the other tile is 128x256 (13x13x576 to 384 at batch 64, 258 tiles, 20.1 against 17.7).
     const long long r128 = (n + 4 * cus - 1) / (4 * cus), r256 = (n256 + 3 * cus - 1) / (3 * cus);
     const bool long_w2 = p.planesB > 1 && p.C32 > 8 && r256 <= r128 && 16 * n256 >= (general ? 16 : 9) * cus;
+    const bool long_w1 = p.planesB == 1 && p.planesA == 2 && p.C32 >= 14 && n256 >= cus && !general &&
+                         (p.C32 >= 26 || other == apnn::MT_128x256 || 2 * ((n256 + cus - 1) / cus) <= (n + cus - 1) / cus);
     const bool tall = p.planesA <= 3 && fits(1) &&
-                      (long_w2 || (r256 < r128 && (p.planesA == 2 ? !general || p.C32 >= 20 : !general && p.C32 < 20)));
+                      (long_w2 || long_w1 || (r256 < r128 && (p.planesA == 2 ? !general || p.C32 >= 20 : !general && p.C32 < 20)));
     const int t = tall ? 1 : 3;
-    // 5x5 over an even number of channel words, on the tile its unrolled form is built for.  One chunk to at most 192 channels
-    // from half a tile per unit (28x28x64 to 192 at batch 8 / 16 / 64 7.9 -> 5.9 / 10.9 -> 7.0 / 20.0 -> 16.4, w1a4 at batch 8
-    // 12.1 -> 9.3; level at batch 4), to 256 for general results and while the 128x256 tiles of async_kernel.h leave much of
-    // a round empty (28x28 at batch 64 28.7 -> 23.9 w1a3; 56x56 at batch 28 / 40, 2744 / 3920 tiles, 27.3 -> 29.6 / 34.0 ->
-    // 41.6).  Several chunks without 128-bit loads from one tile per unit (14x14x192 to 256 at batch 64 21.5 -> 13.3; with 100
-    // tiles 9.4 -> 10.2), but not long reductions of two digits a pixel against that tile (w1a3 28x28x960 to 224 at batch 64 223
-    // -> 314).  Two weight planes, whose filter block costs most, on 256x64 tiles of the general form from one per unit, 3/4
-    // beyond 192 channels (28x28x832 to 128 at batch 64 115, 177 on 128x64 tiles, 126 otherwise).
-    // (Nowhere against the 32x32 split-K tile, which wins where half of a 64-channel tile is empty: 3x3 on 56x56x192 to 32 at
-    // batch 6, w1a4 8.0 -> 10.1, 5x5 on 28x28x64 to 32 at batch 24 8.5 -> 9.2.)
+    // 5x5 over an even number of channel words, on the tile its unrolled form is built for.  One chunk to at most 192
+    // channels from half a tile per unit (28x28x64 to 192 at batch 8 / 16 / 64 7.9 -> 5.9 / 10.9 -> 7.0 / 20.0 -> 16.4,
+    // w1a4 at batch 8 12.1 -> 9.3; level at batch 4), to 256 for general results and while the 128x256 tiles of
+    // async_kernel.h leave much of a round empty (28x28 at batch 64 28.7 -> 23.9 w1a3; 56x56 at batch 28 / 40, 2744 /
+    // 3920 tiles, 27.3 -> 29.6 / 34.0 -> 41.6).  Several chunks without 128-bit loads from one tile per unit (14x14x192
+    // to 256 at batch 64 21.5 -> 13.3; with 100 tiles 9.4 -> 10.2), but not long reductions of two digits a pixel
+    // against that tile (w1a3 28x28x960 to 224 at batch 64 223 -> 314).  Two weight planes, whose filter block costs
+    // most, on 256x64 tiles of the general form from one per unit, 3/4 beyond 192 channels (28x28x832 to 128 at batch
+    // 64 115, 177 on 128x64 tiles, 126 otherwise).
+    // (Nowhere against the 32x32 split-K tile, which wins where half of a 64-channel tile is empty: 3x3 on 56x56x192 to
+    // 32 at batch 6, w1a4 8.0 -> 10.1, 5x5 on 28x28x64 to 32 at batch 24 8.5 -> 9.2.)
     if (other == apnn::MT_32x32_K4) return -1;
     if (taps == 25 && p.S == 5 && p.stride == 1 && p.C32 % 4 == 2) {
       if (p.C32 == 2) return (p.rowsB <= 192 || (p.rowsB <= 256 && (general || n <= 8 * cus))) && 2 * n >= cus ? 3 : -1;
@@ -410,44 +416,55 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
       }
       return p.planesA == 2 || p.C32 <= 14 || other != apnn::MT_128x256 ? 3 : -1;
     }
-    // 3x3 over one chunk of channels (56x56x64 to 64 at batch 8 5.3 -> 4.6, 196 tiles; 28x28x64 to 192 at batch 64 11.8 -> 9.1;
-    // below half a tile per unit 128x64 leaves too much idle: 4.3 -> 4.6 with 98; searched codes from one tile per unit: 56x56x64
-    // to 64 at batch 6 with an int32 map 7.0 -> 8.0, averages of 28x28x64 to 640 at batch 4 7.1 -> 7.9, of 16x16x64 to 416 at batch
-    // 20, 280 tiles, 8.7 -> 7.4).  A single channel word fills half a chunk: to many channels it loses (32x32x32 to 1024 at batch
-    // 3 6.3 -> 6.7), and so does a layer whose 128x256 tiles fill one round (56x56x64 to 224 at batch 20, 490 tiles, w1a3
-    // 16.3 -> 20.1, w2a2 to 256 12.2 -> 12.7).
+    // 3x3 over one chunk of channels (56x56x64 to 64 at batch 8 5.3 -> 4.6, 196 tiles; 28x28x64 to 192 at batch 64 11.8
+    // -> 9.1; below half a tile per unit 128x64 leaves too much idle: 4.3 -> 4.6 with 98; searched codes from one tile
+    // per unit: 56x56x64 to 64 at batch 6 with an int32 map 7.0 -> 8.0, averages of 28x28x64 to 640 at batch 4 7.1 ->
+    // 7.9, of 16x16x64 to 416 at batch 20, 280 tiles, 8.7 -> 7.4).  A single channel word fills half a chunk: to many
+    // channels it loses (32x32x32 to 1024 at batch 3 6.3 -> 6.7), and so does a layer whose 128x256 tiles fill one
+    // round (56x56x64 to 224 at batch 20, 490 tiles, w1a3 16.3 -> 20.1, w2a2 to 256 12.2 -> 12.7).
     if (plain && p.C32 <= 2 && (p.C32 > 1 || p.rowsB <= 64) && !full_round && (searched ? n > cus : 2 * n >= cus)) return t;
-    // 3x3 over channel words without 128-bit loads, which leave the others their 32- and 64-bit forms (56x56x96 to 256 at batch
-    // 4 / 64 11.4 -> 7.4 / 68.9 -> 40.6, 14x14x960 to 1024 at batch 16 33.4 -> 27.0, 7x7x480 to 512 at batch 64 18.2 -> 13.4).
-    // An odd number: from half a tile per unit (searched codes: just above it).  Pairs: from half a tile over 192 channels,
-    // whose other kernel is the plain 64x64 tile; from 3/4 where that is the 32x64 split-K tile (27x27x320 to 704 at batch 2, 132
-    // tiles, w1a3 8.9 -> 10.8, 16x16x320 to 576 at batch 14, 252 tiles, w1a4 16.8 -> 13.6), w1a4 from half (7x7x320 to 704 at
-    // batch 32, 143 tiles, 16.5 -> 14.1).  Not long reductions of two digits a pixel against 128x256 tiles (14x14x960 to 1024 at
-    // batch 64 w1a3 / w1a4 86 -> 118 / 98 -> 133) or of w1a3 against 128x128 (28x28x960 to 384 at batch 48 128 -> 141); nor general
-    // results of two weight planes but on 256x64 tiles (28x28x928 to 320 at batch 7 33.2 -> 38.9) and not against 128x256 ones
-    // (low bits of 28x28x832 to 256 at batch 64 82 -> 98).
+    // 3x3 over channel words without 128-bit loads, which leave the others their 32- and 64-bit forms (56x56x96 to 256
+    // at batch 4 / 64 11.4 -> 7.4 / 68.9 -> 40.6, 14x14x960 to 1024 at batch 16 33.4 -> 27.0, 7x7x480 to 512 at batch
+    // 64 18.2 -> 13.4). An odd number: from half a tile per unit (searched codes: just above it).  Pairs: from half a
+    // tile over 192 channels, whose other kernel is the plain 64x64 tile; from 3/4 where that is the 32x64 split-K tile
+    // (27x27x320 to 704 at batch 2, 132 tiles, w1a3 8.9 -> 10.8, 16x16x320 to 576 at batch 14, 252 tiles, w1a4 16.8 ->
+    // 13.6), w1a4 from half (7x7x320 to 704 at batch 32, 143 tiles, 16.5 -> 14.1).  Not long reductions whose other
+    // tiles are large and fill their rounds: against 128x256 with two digits a pixel (14x14x960 to 1024 at batch 64,
+    // 392 tiles on 512 places, w1a3 / w1a4 86 -> 118 / 98 -> 133; 28x28x576 to 832 at batch 12, 296 tiles, w1a3
+    // averages 68 -> 45; from 24 words w1a3 always, 28x28x960 to 768 at batch 32 150 -> 183), two weight planes
+    // (14x14x960 to 1024 85 -> 102; 27x27x960 to 704 at batch 16, 276 tiles, 82 -> 62) and the longest (28x28x832 to
+    // 512 at batch 32 63 -> 68; 28x28x832 to 768 at batch 16, 294 tiles, 61.5 -> 52.7); against 128x128 with w1a3
+    // (28x28x960 to 384 at batch 48 128 -> 141), two weight planes (13x13x960 to 768 at batch 64, 510 tiles, 58 -> 68)
+    // and w1a4's general results (56x56x704 to 128 at batch 16 65 -> 91); nor results of two weight planes but on
+    // 256x64 tiles (28x28x928 to 320 at batch 7, averages, 33.2 -> 38.9; 13x13x832 to 768 at batch 16 25.6 -> 30.9).
     const bool w2_general = p.planesB > 1 && general && p.C32 > 16 && !tall;
     if (plain && (p.C32 & 1) && p.C32 >= 3 && !w2_general && (searched ? 2 * n > cus : 2 * n >= cus)) return t;
     if (plain && p.C32 % 4 == 2 && p.C32 > 2 && !full_round && !w2_general) {
       const bool enough = p.C32 == 6 ? 2 * n >= cus : p.planesA == 4 && !general ? 2 * n > cus : 4 * n > 3 * cus;
-      const bool heavy = p.planesA >= 3 || (p.planesB > 1 && general);
-      const bool beaten = p.C32 >= 20 && heavy && (other == apnn::MT_128x256 ||
-                          (other == apnn::MT_128x128 && (p.planesA == 3 || (p.planesA == 4 && general))));
+      const bool w2 = p.planesB > 1;
+      const bool beaten =
+          other == apnn::MT_128x256 ? (full >= 0.7 && (p.planesA >= 3 ? p.C32 >= 14 : w2 ? p.C32 >= 20 : p.C32 >= 26 && !general)) ||
+                                          (p.planesA == 3 && p.C32 >= 24)
+          : other == apnn::MT_128x128 && p.C32 >= 20 &&
+                (p.planesA == 3 ? full >= 0.8 : p.planesA == 4 ? general && full >= 0.7 : w2 && full >= 0.9);
+      if (w2 && p.C32 >= 20 && !tall) return -1;
       if (enough && !beaten) return t;
     }
-    // Other filter sizes and strides, from two tiles per unit, over a single chunk to few channels or an odd number of words.
+    // Other filter sizes and strides, from two tiles per unit, over a single chunk to few channels or an odd number of
+    // words.
     if (((p.rowsB <= 64 && p.C32 <= 2) || (p.C32 & 1)) && !plain && n >= 2 * cus) {
-      // Strided filters but 3x3 and few taps reuse a patch too little, over long reductions most of all (2x2 on 56x56x864 to 160
-      // at batch 18, w1a4 low bits 74 -> 207, on 56x56x64 to 64 at batch 24 6.1 -> 6.6; 28x28x288 to 288 at batch 42, w2a2
-      // 51.7 -> 27.4; 4x4 of stride 2 on 56x56x96 to 256 at batch 64 31.6 -> 45.2).
+      // Strided filters but 3x3 and few taps reuse a patch too little, over long reductions most of all (2x2 on
+      // 56x56x864 to 160 at batch 18, w1a4 low bits 74 -> 207, on 56x56x64 to 64 at batch 24 6.1 -> 6.6; 28x28x288 to
+      // 288 at batch 42, w2a2 51.7 -> 27.4; 4x4 of stride 2 on 56x56x96 to 256 at batch 64 31.6 -> 45.2).
       if (taps != 9 && p.stride > 1) return -1;
       if (taps < 9) return p.C32 > 9 || (p.C32 == 2 && p.planesA != 3) ? -1 : t;
       if (taps < 16) return t;
-      // From sixteen taps on the filter block is most of what is staged: 256x64 tiles, which expand it for twice the pixels (4x4
-      // on 32x32x224 to 320 at batch 29, w2a2 34.1, 46.3 on 128x64 tiles, 43.8 otherwise; 5x5 on 32x32x224 to 224 at batch 64
-      // 56, 89, 99), low bits where they save a round.  Searched codes over long reductions, or where they save a round, only
-      // (4x4 on 27x27x480 to 832 at batch 48 160, 219 otherwise; averages of 27x27x224 to 160 at batch 56, w1a3 45.0, 39.7), two digits a pixel not over
-      // one or two words (4x4 on 56x56x32 to 64 at batch 50, w1a4 27.7, 24.7).
+      // From sixteen taps on the filter block is most of what is staged: 256x64 tiles, which expand it for twice the
+      // pixels (4x4 on 32x32x224 to 320 at batch 29, w2a2 34.1, 46.3 on 128x64 tiles, 43.8 otherwise; 5x5 on 32x32x224
+      // to 224 at batch 64 56, 89, 99), low bits where they save a round.  Searched codes over long reductions, or
+      // where they save a round, only (4x4 on 27x27x480 to 832 at batch 48 160, 219 otherwise; averages of 27x27x224 to
+      // 160 at batch 56, w1a3 45.0, 39.7), two digits a pixel not over one or two words (4x4 on 56x56x32 to 64 at batch
+      // 50, w1a4 27.7, 24.7).
       if (p.planesA > 2 ? searched || p.C32 < 3 : searched && p.C32 < 9 && (r256 >= r128 || p.C32 < 5)) return -1;
       if (fits(1) && (!general || searched || r256 < r128)) return 1;
       return p.planesA == 2 || p.C32 >= 5 ? 3 : -1;
@@ -455,13 +472,12 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     // 128 channels to at most 128 from 1.5 tiles per unit (28x28 at batch 64 9.9 -> 8.9, 56x56 at batch 64 28.0 -> 22.0; to
     // 256 channels the 128x256 tile of async_kernel.h is ahead, 13.6 -> 14.8)
     if (plain && p.C32 == 4 && p.rowsB <= 128 && 2 * n >= 3 * cus) return t;
-    // 256 channels at 1.5 to 2 tiles per unit, all resident at once (14x14 to 256 at batch 64 9.9 -> 9.3, w1a4 17.4 -> 15.5;
-    // w1a3, whose two FP4 digits cost as much as w1a4's, is level: 13.1 -> 13.4 on 28x28 at batch 16; w2a2 loses where 128x128
-    // tiles fill one round of the units, 28x28 to 128 at batch 40 11.1 -> 12.0, and wins else, 32x32 to 320 at batch 12
-    // 15.0 -> 11.1; the 32x64 split-K tile keeps int32 maps, and w1a4's int32 results and low bits: 32x32 to 64 at batch 48
-    // 11.1 -> 12.6, against 128x128 tiles 0.84-0.97 of their time)
-    const long long mid = others(128, 128);
-    const bool w2_full = p.planesB > 1 && !general && other == apnn::MT_128x128 && mid <= cus && 10 * mid >= 9 * cus;
+    // 256 channels at 1.5 to 2 tiles per unit, all resident at once (14x14 to 256 at batch 64 9.9 -> 9.3, w1a4 17.4 ->
+    // 15.5; w1a3, whose two FP4 digits cost as much as w1a4's, is level: 13.1 -> 13.4 on 28x28 at batch 16; w2a2 loses
+    // where 128x128 tiles fill one round of the units, 28x28 to 128 at batch 40 11.1 -> 12.0, and wins else, 32x32 to
+    // 320 at batch 12 15.0 -> 11.1; the 32x64 split-K tile keeps int32 maps, and w1a4's int32 results and low bits:
+    // 32x32 to 64 at batch 48 11.1 -> 12.6, against 128x128 tiles 0.84-0.97 of their time)
+    const bool w2_full = p.planesB > 1 && !general && other == apnn::MT_128x128 && large <= cus && 10 * large >= 9 * cus;
     const bool split_k = other == apnn::MT_32x64_K4 && (p.resid != nullptr || p.save_acc != nullptr || (p.planesA == 4 && p.epi != APNN_EPI_BN));
     if (plain && p.C32 == 8 && p.planesA != 3 && !w2_full && !split_k && 2 * n >= 3 * cus && n <= 2 * cus) return t;
     return -1;

@@ -360,8 +360,12 @@ def test_patch_resident_tile_rule(batch, H, C, cout, R, stride, wb, xb, tile):
     (2, 27, 320, 704, 3, 1, 1, 3, "near", None), (14, 16, 320, 576, 3, 1, 1, 4, "int32", (128, 64)),
     (32, 7, 320, 704, 3, 1, 1, 4, "near", (128, 64)), (28, 27, 320, 32, 3, 1, 1, 3, "int32", None),
     # long reductions, full rounds of larger tiles, 256 channels
-    (64, 14, 960, 1024, 3, 1, 1, 2, "bn", (128, 64)), (64, 14, 960, 1024, 3, 1, 1, 3, "bn", None),
+    (64, 14, 960, 1024, 3, 1, 1, 2, "bn", None), (64, 14, 960, 1024, 3, 1, 1, 3, "bn", None),
     (64, 14, 960, 1024, 3, 1, 1, 4, "bn", None), (48, 28, 960, 384, 3, 1, 1, 3, "bn", None),
+    (64, 14, 960, 1024, 3, 1, 2, 2, "bn", None), (16, 28, 832, 768, 3, 1, 1, 2, "bn", (256, 64)),
+    (12, 28, 576, 832, 3, 1, 1, 3, "avg", (128, 64)), (64, 14, 832, 512, 3, 1, 1, 2, "bn", (256, 64)),
+    (64, 13, 576, 384, 3, 1, 1, 2, "bn", (128, 64)), (64, 13, 960, 768, 3, 1, 2, 2, "bn", None),
+    (16, 13, 832, 768, 3, 1, 2, 2, "bn", None), (16, 27, 960, 704, 3, 1, 2, 2, "bn", (256, 64)),
     (64, 28, 832, 256, 3, 1, 2, 2, "low", None), (7, 28, 928, 320, 3, 1, 2, 2, "avg", None),
     (20, 56, 64, 224, 3, 1, 1, 3, "bn", None), (40, 28, 256, 128, 3, 1, 2, 2, "bn", None),
     (12, 32, 256, 320, 3, 1, 2, 2, "bn", (128, 64)), (48, 32, 256, 64, 3, 1, 1, 4, "int32", None),
