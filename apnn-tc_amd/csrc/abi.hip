@@ -401,19 +401,21 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     // async_kernel.h leave much of a round empty (28x28 at batch 64 28.7 -> 23.9 w1a3; 56x56 at batch 28 / 40, 2744 /
     // 3920 tiles, 27.3 -> 29.6 / 34.0 -> 41.6).  Several chunks without 128-bit loads from one tile per unit (14x14x192
     // to 256 at batch 64 21.5 -> 13.3; with 100 tiles 9.4 -> 10.2), but not long reductions of two digits a pixel
-    // against that tile (w1a3 28x28x960 to 224 at batch 64 223 -> 314).  Two weight planes, whose filter block costs
-    // most, on 256x64 tiles of the general form from one per unit, 3/4 beyond 192 channels (28x28x832 to 128 at batch
-    // 64 115, 177 on 128x64 tiles, 126 otherwise).
+    // against that tile (w1a3 28x28x960 to 224 at batch 64 223 -> 314), nor w1a3 where its rounds are full (32x32x192
+    // to 960 at batch 32 110 -> 130), nor w1a4 to 256 channels (28x28 at batch 64 32.4 -> 37.8).  Two weight planes,
+    // whose filter block costs most, on 256x64 tiles of the general form from one per unit, 3/4 beyond 192 channels
+    // (28x28x832 to 128 at batch 64 115, 177 on 128x64 tiles, 126 otherwise).
     // (Nowhere against the 32x32 split-K tile, which wins where half of a 64-channel tile is empty: 3x3 on 56x56x192 to
     // 32 at batch 6, w1a4 8.0 -> 10.1, 5x5 on 28x28x64 to 32 at batch 24 8.5 -> 9.2.)
     if (other == apnn::MT_32x32_K4) return -1;
     if (taps == 25 && p.S == 5 && p.stride == 1 && p.C32 % 4 == 2) {
-      if (p.C32 == 2) return (p.rowsB <= 192 || (p.rowsB <= 256 && (general || n <= 8 * cus))) && 2 * n >= cus ? 3 : -1;
+      if (p.C32 == 2) return (p.rowsB <= 192 || (p.rowsB <= 256 && p.planesA < 4 && (general || n <= 8 * cus))) && 2 * n >= cus ? 3 : -1;
       if (n < cus) return -1;
       if (p.planesB > 1) {
         if (fits(1) && 4 * n256 >= (p.C32 > 6 ? 3 : 4) * cus) return 1;
         return p.C32 == 6 || p.rowsB <= 32 ? 3 : -1;
       }
+      if (p.planesA == 3 && (p.C32 >= 26 || (other == apnn::MT_128x256 && full >= 0.7))) return -1;
       return p.planesA == 2 || p.C32 <= 14 || other != apnn::MT_128x256 ? 3 : -1;
     }
     // 3x3 over one chunk of channels (56x56x64 to 64 at batch 8 5.3 -> 4.6, 196 tiles; 28x28x64 to 192 at batch 64 11.8
@@ -436,18 +438,21 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     // 512 at batch 32 63 -> 68; 28x28x832 to 768 at batch 16, 294 tiles, 61.5 -> 52.7); against 128x128 with w1a3
     // (28x28x960 to 384 at batch 48 128 -> 141), two weight planes (13x13x960 to 768 at batch 64, 510 tiles, 58 -> 68)
     // and w1a4's general results (56x56x704 to 128 at batch 16 65 -> 91); nor results of two weight planes but on
-    // 256x64 tiles (28x28x928 to 320 at batch 7, averages, 33.2 -> 38.9; 13x13x832 to 768 at batch 16 25.6 -> 30.9).
+    // 256x64 tiles (28x28x928 to 320 at batch 7, averages, 33.2 -> 38.9; 13x13x832 to 768 at batch 16 25.6 -> 30.9);
+    // and w1a4 over the longest from two tiles per unit (56x56x960 to 96 at batch 24 146 -> 231).
     const bool w2_general = p.planesB > 1 && general && p.C32 > 16 && !tall;
     if (plain && (p.C32 & 1) && p.C32 >= 3 && !w2_general && (searched ? 2 * n > cus : 2 * n >= cus)) return t;
     if (plain && p.C32 % 4 == 2 && p.C32 > 2 && !full_round && !w2_general) {
       const bool enough = p.C32 == 6 ? 2 * n >= cus : p.planesA == 4 && !general ? 2 * n > cus : 4 * n > 3 * cus;
       const bool w2 = p.planesB > 1;
       const bool beaten =
-          other == apnn::MT_128x256 ? (full >= 0.7 && (p.planesA >= 3 ? p.C32 >= 14 : w2 ? p.C32 >= 20 : p.C32 >= 26 && !general)) ||
-                                          (p.planesA == 3 && p.C32 >= 24)
+          other == apnn::MT_128x256
+              ? (full >= 0.7 && (p.planesA >= 3 ? p.C32 >= 14 : w2 ? p.C32 >= 20 : p.C32 >= 26 && !general)) ||
+                    (p.planesA == 3 && p.C32 >= 24)
           : other == apnn::MT_128x128 && p.C32 >= 20 &&
                 (p.planesA == 3 ? full >= 0.8 : p.planesA == 4 ? general && full >= 0.7 : w2 && full >= 0.9);
       if (w2 && p.C32 >= 20 && !tall) return -1;
+      if (p.planesA == 4 && p.C32 >= 26 && n > 2 * cus) return -1;
       if (enough && !beaten) return t;
     }
     // Other filter sizes and strides, from two tiles per unit, over a single chunk to few channels or an odd number of
@@ -466,11 +471,11 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
       // 160 at batch 56, w1a3 45.0, 39.7), two digits a pixel not over one or two words (4x4 on 56x56x32 to 64 at batch
       // 50, w1a4 27.7, 24.7).
       if (p.planesA > 2 ? searched || p.C32 < 3 : searched && p.C32 < 9 && (r256 >= r128 || p.C32 < 5)) return -1;
-      if (fits(1) && (!general || searched || r256 < r128)) return 1;
+      if (fits(1) && (!general || searched || tall)) return 1;
       return p.planesA == 2 || p.C32 >= 5 ? 3 : -1;
     }
-    // 128 channels to at most 128 from 1.5 tiles per unit (28x28 at batch 64 9.9 -> 8.9, 56x56 at batch 64 28.0 -> 22.0; to
-    // 256 channels the 128x256 tile of async_kernel.h is ahead, 13.6 -> 14.8)
+    // 128 channels to at most 128 from 1.5 tiles per unit (28x28 at batch 64 9.9 -> 8.9, 56x56 at batch 64 28.0 ->
+    // 22.0; to 256 channels the 128x256 tile of async_kernel.h is ahead, 13.6 -> 14.8)
     if (plain && p.C32 == 4 && p.rowsB <= 128 && 2 * n >= 3 * cus) return t;
     // 256 channels at 1.5 to 2 tiles per unit, all resident at once (14x14 to 256 at batch 64 9.9 -> 9.3, w1a4 17.4 ->
     // 15.5; w1a3, whose two FP4 digits cost as much as w1a4's, is level: 13.1 -> 13.4 on 28x28 at batch 16; w2a2 loses
@@ -478,7 +483,8 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     // 320 at batch 12 15.0 -> 11.1; the 32x64 split-K tile keeps int32 maps, and w1a4's int32 results and low bits:
     // 32x32 to 64 at batch 48 11.1 -> 12.6, against 128x128 tiles 0.84-0.97 of their time)
     const bool w2_full = p.planesB > 1 && !general && other == apnn::MT_128x128 && large <= cus && 10 * large >= 9 * cus;
-    const bool split_k = other == apnn::MT_32x64_K4 && (p.resid != nullptr || p.save_acc != nullptr || (p.planesA == 4 && p.epi != APNN_EPI_BN));
+    const bool map = p.resid != nullptr || p.save_acc != nullptr;
+    const bool split_k = other == apnn::MT_32x64_K4 && (map || (p.planesA == 4 && p.epi != APNN_EPI_BN));
     if (plain && p.C32 == 8 && p.planesA != 3 && !w2_full && !split_k && 2 * n >= 3 * cus && n <= 2 * cus) return t;
     return -1;
   }

@@ -376,7 +376,8 @@ def test_patch_resident_tile_rule(batch, H, C, cout, R, stride, wb, xb, tile):
     (64, 28, 960, 224, 5, 1, 1, 3, "bn", None), (64, 32, 224, 224, 5, 1, 1, 2, "bn", (256, 64)),
     (29, 32, 224, 320, 4, 1, 2, 2, "int32", (256, 64)), (56, 27, 224, 160, 4, 1, 1, 3, "avg", None),
     (18, 56, 864, 160, 2, 1, 1, 4, "low", None), (64, 56, 96, 256, 4, 2, 1, 2, "bn", None),
-    (42, 28, 288, 288, 2, 1, 2, 2, "bn", (256, 64)),
+    (42, 28, 288, 288, 2, 1, 2, 2, "bn", (256, 64)), (64, 56, 288, 64, 5, 1, 2, 2, "low", (256, 64)),
+    (32, 32, 192, 960, 5, 1, 1, 3, "near", None), (64, 28, 64, 256, 5, 1, 1, 4, "bn", None), (24, 56, 960, 96, 3, 1, 1, 4, "near", None),
 ])
 def test_patch_resident_tile_rule_by_output(batch, H, C, cout, R, stride, wb, xb, out, tile):
     """The rule where results other than two-bit codes, long reductions or rounds of the other tiles decide.  out: int32, bn,
