@@ -26,10 +26,12 @@
 // residency: the staging of one work-group hides behind the products of others, so registers are cut for four
 // work-groups per compute unit (three where a wave has four blocks; what spills is the general output path alone).
 // us before -> without and with the cut, w1a2 with threshold codes in graph replay: 56x56x64 to 64 at batch 64 14.6 -> 11.6 ->
-// 10.6; 56x56x96 to 256 at batch 64 68.9 -> 53.6 -> 40.0 (256x64 tiles); w1a4 there 169 -> 90.  Left: the two LDS reads per
-// matrix instruction pair of a 2x2-block wave are the LDS rate (128 bytes a clock), so long reductions stay level with
-// async_kernel.h (56x56x256 at batch 64 59 against 61 us).  A 256x128 tile of 4x2 blocks reads less, but two of them per
-// unit leave their last round emptier: 62 us there, 68 against 60 on 28x28x512.
+// 10.6; 56x56x96 to 256 at batch 64 68.9 -> 53.6 -> 40.0 (256x64 tiles); w1a4 there 169 -> 90.  Left: no pipe is full.  Of the
+// busy clocks, matrix / vector / LDS: 56x56x64 16 / 46 / 30 %, 56x56x96 to 256 33 / 51 / 32, 14x14x832 to 512 on 256x64 tiles
+// 33 / 19 / 32, waves waiting 35-46 % of their time (profiles/patch_conv_w1a2_counters.md): staging and products of a work-group
+// alternate behind two barriers a chunk, and one and a half to four work-groups on a unit cover that in part.  Long reductions
+// stay level with async_kernel.h (56x56x256 at batch 64 59 against 61 us).  A 256x128 tile of 4x2 blocks reads less, but two of
+// them per unit leave their last round emptier: 62 us there, 68 against 60 on 28x28x512.
 // 5x5 filters in a form of their own, all filter words of a chunk in flight at once: 28x28x64 to 192 at batch 64 21.2 us in
 // the general form, 16.4 in this one (two work-groups per unit, by the LDS).
 #pragma once
