@@ -362,8 +362,9 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
   };
   if (automatic) {
     if (tile_pin != 0) return -1;  // a pinned tile names a tile of the implicit-GEMM families
-    if (taps == 1 || !fits(3)) return -1;
     const long long n = ntiles(3), n256 = ntiles(1);  // 128x64 and 256x64 tiles
+    // no rule below takes one tap, less than half a tile per unit or these channel words
+    if (taps == 1 || 2 * n < cus || (p.C32 % 4 == 0 && p.C32 != 4 && p.C32 != 8) || !fits(3)) return -1;
     const bool plain = taps == 9 && p.S == 3 && p.stride == 1;  // the filters with an unrolled loop, the densest patches
     // Results that leave over the output stage's general path (its values pass LDS, and 2x2 blocks keep part of them in
     // scratch), and those of them that are searched codes: pooled averages, unfolded shortcuts, int32 maps, pooled maxima
