@@ -555,6 +555,24 @@ int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, i
   // the small tiles repeat, 3/4 suffice.  Over at most 128 words the plain tile is ahead of both from 3/4 on
   // (14x14x256 at batch 64: w1a2 9.6 us against 10.4 for the groups and 11.2 for split-K, w1a4 16.7 against 17.1 and
   // 17.2, w2a2 10.9 against 11.6 and 12.5).
+  // GEMM entry points, one round of tiles over at least 1024 bits: eight waves that split K (ksplit_kernel.h).  Below half
+  // a 128x64 tile per unit the 32x64 split-K tile has the better spread, below 1024 bits the meeting of the partial tiles
+  // costs more than the loop saves.  us, other tiles first, 1000x2016 outputs (256 tiles): w1a2 K = 512 / 1024 / 2048 / 8192
+  // 5.3 -> 6.0 / 6.6 -> 6.0 / 9.3 -> 7.3 / 24 -> 13, w1a4 over 2048 bits 12.1 -> 8.4, w1a8 18.6 -> 11.3, w2a2 packed 11.1 -> 8.5;
+  // 1000x1000 (128 tiles) over 2048 bits w1a2 / w1a4 0.94 / 0.86 of the time, w2a2 1.04; w1a8, whose other tiles repeat
+  // sixteen planes' expansion, from 48 tiles (1024x384 over 2048 bits 0.89) and over several rounds (2048x2048 24.5 -> 20.0,
+  // 4096x1536 0.70); the others lose there (2304x1024, 288 tiles: w1a2 1.07, w2a2 1.16).  w2a2 is level at 1024 bits.
+  // w4a4 takes 64x96 tiles where they fill three quarters of a round (half from 4096 bits): 4096x333 over 4096 bits, 256
+  // tiles, 25.5 on 64x64, 18.8 on 128x64, 13.6.
+  if (!conv && !i8 && KW >= 32 && planes > 2 && planes < 10) {
+    const bool w4 = planesW == 4, w1a8 = planes == 9;
+    const long long n10 = ntiles(apnn::MT_128x64_K4), n11 = ntiles(apnn::MT_64x96_K8);
+    if (w4 && KW >= 64 && n11 <= cus && (KW >= 128 ? 2 : 1) * n11 * 4 >= 3 * cus && fill(apnn::MT_64x96_K8) >= 0.75)
+      return apnn::MT_64x96_K8;
+    const long long least = w1a8 ? 3 * cus / 16 : w4 || planesW > 1 ? cus / 2 + 1 : 3 * cus / 8;
+    if (n10 >= least && n10 <= (w1a8 ? 3 : 1) * cus && (planesW != 2 || KW > 32) && fill(apnn::MT_128x64_K4) >= 0.75)
+      return apnn::MT_128x64_K4;
+  }
   if ((!conv || vw == 4) && planes > 2 && KW >= 64 && fill(1) >= 0.8) {
     const long long nt1 = ntiles(1);
     if (!conv || wide) {
@@ -680,7 +698,7 @@ int plan_direct(apnn_plan *plan, const KParams &p, bool f4ok) {
 
 int plan_mfma(apnn_plan *plan, bool i8, int tile, const KParams &p, bool f4ok) {
   const bool split = tile == apnn::MT_32x32_K4 || tile == apnn::MT_32x64_K4 || tile == apnn::MT_32x128_K4;
-  const int ksplit = split ? 4 : (tile == apnn::MT_128x128_G2 ? 2 : 1);
+  const int ksplit = split || tile == apnn::MT_128x64_K4 ? 4 : tile == apnn::MT_64x96_K8 ? 8 : tile == apnn::MT_128x128_G2 ? 2 : 1;
   return fill_plan(plan, i8 ? APNN_PATH_MFMA_I8 : APNN_PATH_MFMA, i8 ? APNN_KERNEL_MFMA_I8 : APNN_KERNEL_MFMA_FP4, tile,
                    apnn::kMfmaTileA[tile], apnn::kMfmaTileB[tile], ksplit, p, 0, f4ok);
 }

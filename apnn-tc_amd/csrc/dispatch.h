@@ -87,14 +87,15 @@ APNN_DECL_PATCH(2, 2)
 enum { CORE_I8 = 0, CORE_F4 = 1 };
 
 // tile shapes of the MFMA kernels, index = enum MfmaTile in mfma_kernel.h
-constexpr int kMfmaTileCount = 10;
-constexpr int kMfmaTileA[kMfmaTileCount] = {256, 128, 64, 128, 32, 32, 256, 128, 32, 128};
-constexpr int kMfmaTileB[kMfmaTileCount] = {256, 128, 64, 64, 32, 64, 128, 256, 128, 128};
+constexpr int kMfmaTileCount = 12;
+constexpr int kMfmaTileA[kMfmaTileCount] = {256, 128, 64, 128, 32, 32, 256, 128, 32, 128, 128, 64};
+constexpr int kMfmaTileB[kMfmaTileCount] = {256, 128, 64, 64, 32, 64, 128, 256, 128, 128, 64, 96};
 
 // MT_128x128_G2: the 128x128 tile computed by two groups of four waves that share its k-steps (work-groups
-// of 512 threads)
+// of 512 threads).  MT_128x64_K4, MT_64x96_K8: eight waves that split K by four and eight (ksplit_kernel.h)
 enum MfmaTile { MT_256x256 = 0, MT_128x128 = 1, MT_64x64 = 2, MT_128x64 = 3, MT_32x32_K4 = 4, MT_32x64_K4 = 5,
-                MT_256x128 = 6, MT_128x256 = 7, MT_32x128_K4 = 8, MT_128x128_G2 = 9, MT_COUNT = 10 };
+                MT_256x128 = 6, MT_128x256 = 7, MT_32x128_K4 = 8, MT_128x128_G2 = 9, MT_128x64_K4 = 10, MT_64x96_K8 = 11,
+                MT_COUNT = 12 };
 
 // Which (core, family, load width, tile, plane counts) combinations are built.  Every kernel
 // instantiation costs seconds of compile time, so only the shapes the dispatcher can choose are kept:
@@ -105,8 +106,15 @@ enum MfmaTile { MT_256x256 = 0, MT_128x128 = 1, MT_64x64 = 2, MT_128x64 = 3, MT_
 //               plus, for convolution with 128-bit loads, the 32x128 split-K tile;
 //               precisions with more than five planes in all (w4a4, w1a8, w2a8, ...) and w1a1: FP4 / FP6 operands
 //               only, and for convolution with narrower loads the 64x64 tile only.
+// MT_128x64_K4: where AUTO can take it (w2a8's operands spill there, 1.0 to 1.8 times the other tiles' time; w1a1 is level
+// with its 64x64 tile);  MT_64x96_K8: w4a4, 22 operations a block on either side
+constexpr bool ksplit_built(int core, bool conv, int tile, int pa, int pb) {
+  if (core != CORE_F4 || conv || pa + pb == 2) return false;
+  return tile == MT_128x64_K4 ? pa + pb < 10 : pa == 4 && pb == 4;
+}
 constexpr bool mfma_tile_enabled(int core, bool conv, int vw, int tile, int pa, int pb) {
   const bool wide = pa + pb > 5 || pa + pb == 2;
+  if (tile == MT_128x64_K4 || tile == MT_64x96_K8) return ksplit_built(core, conv, tile, pa, pb);
   if (wide && core == CORE_I8) return false;
   if (wide && conv && vw != 4) return tile == MT_64x64;
   if (tile == MT_128x128_G2) return core == CORE_F4 && (!conv || vw == 4);  // two wave groups: 128-bit loads
