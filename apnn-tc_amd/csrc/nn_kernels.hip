@@ -359,36 +359,43 @@ __device__ __forceinline__ void append_int_codes(int v0, int v1, int v2, int v3,
 // In NHWC memory the S pixels x C channels under one filter row are S*C consecutive bytes, so K is laid
 // out per filter row as that byte run, padded with zero weights to whole 16-byte halves (HPR halves per
 // row); the halves of all R rows are numbered consecutively and k-step ks consumes halves 2ks (lane
-// half 0) and 2ks+1 (lane half 1).  The patch of a pixel group (32 consecutive output pixels of one
-// output row) is R image-row segments copied to LDS as aligned dwords -- no per-pixel repacking -- with
+// half 0) and 2ks+1 (lane half 1).  A wave works on a block of NSETS * 32 output pixels, 2^LW wide: its patch is
+// the image-row segments under the block, copied to LDS as aligned dwords -- no per-pixel repacking -- with
 // the zero point removed by an XOR (x - 128 == x ^ 0x80 as int8) and out-of-image dwords set to zero.
 // A lane's 16 operand bytes start at byte lead + pixel*stride*C + 16*half of its row segment: five
-// aligned dword reads and four v_alignbyte.  NKS > 0: the number of k-steps is known, the loop is unrolled and a
-// lane keeps the patch offset of each step; with WREG the wave also keeps its 64 x (NKS*32) weight block in
-// registers for the whole (persistent) kernel, otherwise weights are read from LDS.
+// aligned dword reads and four v_alignbyte (one 16-byte read that is not aligned takes 48 clocks of the LDS, these
+// about 20).  NKS > 0: the number of k-steps is known, the loop is unrolled and a lane keeps the patch address of each step.
 // Weights are the first operand, so a lane of the accumulator owns one output pixel and its registers hold
 // channels: code bits are appended to the lane's own words, thresholds come from a table in LDS.  Filter row
 // 8q + 4h + j of a block of 32 holds channel 16h + 4q + j, which gives lane half h the channels 16h .. 16h + 15 in
 // order; one half-wave swap joins the two halves of both planes' words.
-// What bounds it: vector issue and LDS reads share the time of a group of 32 pixels about evenly.  Five vector
-// operations per value (compare, select, compare, two appends) instead of eight with lane writes alone gain little,
-// because the table adds 24 LDS reads (11x11 filter at batch 8 15.1 -> 14.8 us); with the unrolled loop, which drops
-// the decode of every k-step, 7x7 stride 2 on 224x224x3 at batch 64 39.7 -> 36.0 us, 3x3 to 96 channels 53.0 -> 48.1.
+// What bounds it: LDS reads, then vector issue (five operations per value: compare, select, compare, two appends).  Blocks
+// instead of 32 pixels of a row (maps of 112 and 56 pixels left the fourth and second part of a row half empty, and a
+// patch of R rows is loaded for 32 pixels), 64 pixels to every read of the filter and of the thresholds, patches of as many
+// slots as they have, and a filter staged without vector work (a lane per channel: half, filter row and mask are scalar, all
+// loads of a wave at once): us in graph replay at batch 8 / 64, 224x224x3, 7x7 stride 2 to 64 channels 10.4 -> 8.8 / 31.6
+// -> 25.1, 3x3 stride 2 to 96 12.0 -> 7.7 / 41.9 -> 28.0, 11x11 stride 4 to 64 12.9 -> 9.8 / 25.9 -> 19.4.
+// Two sets of 32 pixels from two blocks per unit (7x7 at batch 8 9.8 with one, 9.5 with two; 3x3 to 128 channels on 32x32 maps
+// at batch 64 9.0 and 7.2), below that one, with the filter block in registers (7x7 at batch 8 10.6 without).
 // Requires C <= 4, (W*C) % 4 == 0, X 4-byte aligned, bits <= 2, COUT % 32 == 0.
 // NWAV waves per work-group share one filter block in LDS (each wave has its own patch and walks its
-// own pixel groups): eight waves where the filter block is large, so that its LDS cost per wave halves
+// own pixel blocks): eight waves where the filter block is large, so that its LDS cost per wave halves
 // and four waves per SIMD stay resident (two work-groups per compute unit: the register budget of that
 // variant is held to 128 by its launch bounds).
 constexpr int kRowsTable = 3 * 64 * 4;  // bytes of thresholds in LDS, [3][64]
+// bytes of a wave's patch of `dwords` dwords: the last pixel's last half may end 20 bytes past the segment
+__host__ __device__ inline int rows_patch_bytes(int dwords) { return (4 * dwords + 32 + 15) & ~15; }
 
-template <int NKS, bool WREG, int NSLOT, int NWAV>
+typedef v4i_t v4i_bytes __attribute__((aligned(1)));
+
+template <int NKS, int NSETS, bool WREG, int NSLOT, int NWAV>
 __global__ __launch_bounds__(64 * NWAV, WREG ? 3 : 4) void conv_i8_rows_kernel(const uint8_t *__restrict__ X, const int8_t *__restrict__ Wt,
                                                            const int32_t *__restrict__ thr,
                                                            uint32_t *__restrict__ planes, int B, int H, int W, int C,
                                                            int COUT, int R, int S, int stride, int pad, int Ho, int Wo,
-                                                           int bits, uint32_t xor_mask, int HPR, int NDW, int PWD,
-                                                           uint32_t magic_gpr, uint32_t magic_ho, uint32_t magic_ndw,
-                                                           uint32_t magic_nh2, uint32_t magic_hpr, int wt_dwords) {
+                                                           int bits, uint32_t xor_mask, int HPR, int PR, int NDW, int LW,
+                                                           uint32_t magic_gpr, uint32_t magic_gpc, uint32_t magic_ndw,
+                                                           uint32_t magic_hpr) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   // n / d by multiply-high with ceil(2^32 / d) where the launcher found it exact (magic != 0)
   auto quot = [](uint32_t n, uint32_t d, uint32_t magic) { return magic != 0 ? __umulhi(n, magic) : (d == 1 ? n : n / d); };
@@ -397,58 +404,61 @@ __global__ __launch_bounds__(64 * NWAV, WREG ? 3 : 4) void conv_i8_rows_kernel(c
   const int KB = nks * 32, KPL = KB + 16;
   int *table = reinterpret_cast<int *>(lds);                  // [3][64]
   int8_t *wl = reinterpret_cast<int8_t *>(lds + kRowsTable);  // [64][KPL]
-  // the wave index is the same in all 64 lanes: as a scalar it keeps the pixel-group arithmetic below
-  // (group -> image, output row, image row addresses) on the scalar unit
+  // the wave index is the same in all 64 lanes: as a scalar it keeps the pixel-block arithmetic below
+  // (block -> image, output row, image row addresses) on the scalar unit
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 31, g = lane >> 5;
-  uint32_t *patch = reinterpret_cast<uint32_t *>(lds + kRowsTable + 64 * KPL) + wave * (R * PWD);
+  const int npatch = PR * NDW;
+  uint8_t *patch = lds + kRowsTable + 64 * KPL + wave * rows_patch_bytes(npatch);
   const int co0 = blockIdx.y * 64;
   const int SC = S * C;
 
-  // filter block -> LDS, one 16-byte half per task.  Four tasks per thread are in flight at a time:
-  // all their byte loads are issued before the first LDS store, so the block costs one or two memory
-  // round trips instead of one per task.
-  const int ntasks = 64 * nks * 2;
-  for (int t0 = 0; t0 < ntasks; t0 += 4 * 64 * NWAV) {
-    uint32_t w[4][4];
-    int dst_off[4];
+  const int PX = 1 << LW, PY = 32 >> LW;  // of a set
+  // filter block -> LDS: a lane per channel, a wave per 16-byte half, so that the half's place in the filter and the bytes
+  // of it that hold weights are scalar.  The halves of a wave are requested before the first LDS store (all of them where
+  // the number of k-steps is known).  Loads are unaligned; the filter's last 16 bytes are loaded instead of bytes past it.
+  constexpr int NT = NKS > 0 ? (NKS * 2 + NWAV - 1) / NWAV : 4;
+  {
+    const int co = co0 + lane;
+    const uint32_t live = co < COUT ? 0xffffffffu : 0u;
+    const uint32_t top = (uint32_t)(COUT * R * SC) - 16u, base = (uint32_t)(min(co, COUT - 1) * R * SC);
+    const int row = (lane & 0x23) | ((lane & 0xc) << 1) | ((lane & 0x10) >> 2);
+    for (int h0 = wave; h0 < 2 * nks; h0 += NT * NWAV) {
+      v4i_t w[NT];
+      uint32_t past[NT];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int task = t0 + u * 64 * NWAV + tid;
-      const int col = (int)quot((uint32_t)task, (uint32_t)(nks * 2), magic_nh2), hh = task - col * (nks * 2);
-      const int r = (int)quot((uint32_t)hh, (uint32_t)HPR, magic_hpr), hq = hh - r * HPR;
-      const int row = (col & 0x23) | ((col & 0xc) << 1) | ((col & 0x10) >> 2);
-      dst_off[u] = row * KPL + hh * 16;
-      const int co = co0 + col;
-      const int nvalid = (task < ntasks && co < COUT && r < R) ? min(max(SC - hq * 16, 0), 16) : 0;
-      const int8_t *src = Wt + ((long long)co * R + r) * SC + hq * 16;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) w[u][q] = 0;
-      if (wt_dwords) {
-        // filter array readable as whole aligned dwords: five dword loads cover the 16 bytes at any
-        // byte offset, v_alignbyte shifts them into place, bytes past the row's end are masked off
-        const long long boff = src - Wt;
-        const uint32_t *wp = reinterpret_cast<const uint32_t *>(Wt) + (boff >> 2);
-        const uint32_t sh = (uint32_t)boff & 3u;
-        uint32_t d[5];
-#pragma unroll
-        for (int k = 0; k < 5; ++k) d[k] = (nvalid > 0 && 4 * k < (int)sh + nvalid) ? wp[k] : 0u;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int nb = min(max(nvalid - 4 * q, 0), 4);
-          const uint32_t mask = nb == 4 ? 0xffffffffu : ((1u << (8 * nb)) - 1u);
-          w[u][q] = __builtin_amdgcn_alignbyte(d[q + 1], d[q], sh) & mask;
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (i < nvalid) w[u][i >> 2] |= (uint32_t)(uint8_t)src[i] << (8 * (i & 3));
+      for (int u = 0; u < NT; ++u) {
+        const int hh = h0 + u * NWAV;
+        const int r = min((int)quot((uint32_t)hh, (uint32_t)HPR, magic_hpr), R - 1);
+        const uint32_t off = min(base + (uint32_t)(r * SC + min(hh - r * HPR, HPR - 1) * 16), top + 15u), at = min(off, top);
+        past[u] = off - at;
+        w[u] = *reinterpret_cast<const v4i_bytes *>(Wt + at);
       }
-    }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int task = t0 + u * 64 * NWAV + tid;
-      if (task < ntasks) *reinterpret_cast<uint4 *>(wl + dst_off[u]) = make_uint4(w[u][0], w[u][1], w[u][2], w[u][3]);
+      for (int u = 0; u < NT; ++u) {
+        const int hh = h0 + u * NWAV;
+        if (hh < 2 * nks) {
+          const int r = (int)quot((uint32_t)hh, (uint32_t)HPR, magic_hpr);
+          const int nvalid = r < R ? min(SC - (hh - r * HPR) * 16, 16) : 0;
+          uint32_t v[5] = {(uint32_t)w[u][0], (uint32_t)w[u][1], (uint32_t)w[u][2], (uint32_t)w[u][3], 0u};
+          if (__any(past[u] != 0)) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+              const bool drop = (past[u] >> 2) > (uint32_t)i;
+#pragma unroll
+              for (int q = 0; q < 4; ++q) v[q] = drop ? v[q + 1] : v[q];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = __builtin_amdgcn_alignbyte(v[q + 1], v[q], past[u] & 3u);
+          }
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int nb = min(max(nvalid - 4 * q, 0), 4);
+            v[q] &= live & (nb == 4 ? 0xffffffffu : (1u << (8 * nb)) - 1u);
+          }
+          *reinterpret_cast<uint4 *>(wl + row * KPL + hh * 16) = make_uint4(v[0], v[1], v[2], v[3]);
+        }
+      }
     }
   }
   const int nt = (1 << bits) - 1;
@@ -458,9 +468,17 @@ __global__ __launch_bounds__(64 * NWAV, WREG ? 3 : 4) void conv_i8_rows_kernel(c
   }
   __syncthreads();
 
+  // this lane's pixel of set 0 (bytes into the patch) and the distance to the pixels of the next set
+  const int px = li & (PX - 1), py = li >> LW;
+  const int lead = (-pad * C) & 3;  // (a block's first byte is a multiple of 8 * stride * C beyond the padding)
+  const int rowpitch = NDW * 4;
+  const int first = lead + px * stride * C + py * stride * rowpitch;
+  const uint32_t *mine = reinterpret_cast<const uint32_t *>(patch) + (first >> 2);
+  const uint32_t sh = (uint32_t)first & 3u;
+  const int set_bytes = PY * stride * rowpitch;
   constexpr int NW = NKS > 0 ? NKS : 1;
   v4i_t wreg[2][WREG ? NW : 1];
-  int koff[NW];  // byte offset of this lane's half of k-step ks inside the patch
+  int koff[NW];  // byte offset of this lane's half of k-step ks
   if (NKS > 0) {
 #pragma unroll
     for (int ks = 0; ks < NW; ++ks) {
@@ -468,26 +486,22 @@ __global__ __launch_bounds__(64 * NWAV, WREG ? 3 : 4) void conv_i8_rows_kernel(c
       for (int nb = 0; nb < (WREG ? 2 : 0); ++nb)
         wreg[nb][WREG ? ks : 0] = *reinterpret_cast<const v4i_t *>(wl + (nb * 32 + li) * KPL + ks * 32 + g * 16);
       const int hh = 2 * ks + g;
-      const int r = min(hh / HPR, R - 1);
-      koff[ks] = r * PWD * 4 + (hh % HPR) * 16;
+      const int r = min((int)quot((uint32_t)hh, (uint32_t)HPR, magic_hpr), R - 1);
+      koff[ks] = r * rowpitch + (hh - (int)quot((uint32_t)hh, (uint32_t)HPR, magic_hpr) * HPR) * 16;
     }
   }
 
-  const int gpr = (Wo + 31) / 32;
-  const long long ngroups = (long long)B * Ho * gpr;
+  const int gpr = (Wo + PX - 1) >> LW, gpc = (Ho + NSETS * PY - 1) / (NSETS * PY);
   const long long rows_total = (long long)B * Ho * Wo;
   const int cw32 = COUT >> 5;
   const int rowbytes = W * C;
-  const int npatch = R * NDW;
-  const int lane_bytes = li * stride * C;
 
-  // Patch element idx = slot * 64 + lane is dword d of row segment r, the same for every group:
-  // (r, d) is decoded once.  The raw dwords of the next group are requested before the current
-  // group is computed (patches of up to 64 * NSLOT dwords: NSLOT = 8 covers a 7x7 stride-2 filter on
-  // three channels, 18 an 11x11 stride-4 one; larger patches are staged in place, chunk by chunk).
+  // Patch element idx = slot * 64 + lane is dword d of row segment r, the same for every block:
+  // (r, d) is decoded once.  The raw dwords of the next block are requested before the current
+  // one is computed (patches of up to 64 * NSLOT dwords; larger ones are staged in place, chunk by chunk).
   const bool prefetch = npatch <= 64 * NSLOT;
   // rd[j]: row segment r in the upper half-word, byte offset 4*d in the lower one; r = NO_ROW marks a
-  // slot past the end of the patch (it then fails the row test of every group)
+  // slot past the end of the patch (it then fails the row test of every block)
   constexpr int NO_ROW = 0x7fff;
   auto slot_code = [&](int idx) {
     const int r = (int)quot((uint32_t)idx, (uint32_t)NDW, magic_ndw);
@@ -496,164 +510,161 @@ __global__ __launch_bounds__(64 * NWAV, WREG ? 3 : 4) void conv_i8_rows_kernel(c
   int rd[NSLOT];
 #pragma unroll
   for (int j = 0; j < NSLOT; ++j) rd[j] = slot_code(j * 64 + lane);
-  // Loads are unconditional (addresses clamped into the image) and leave the registers untouched until
-  // publish(): a load whose value is used inside a branch on its predicate makes the compiler wait
-  // for it there, one memory round trip per slot.  raw_ok[j]: slot j lies inside the image.  The address
-  // is the image's base (uniform) plus a 32-bit byte offset, seven vector operations per slot: row and
-  // byte position, two range tests, two clamps, one multiply-add (the launcher checks H * W * C < 2^31,
-  // W * C < 2^24 and H + pad < NO_ROW).
+  // Loads go through a descriptor of the image (the launcher checks H * W * C < 2^31, W * C < 2^24 and H + pad < NO_ROW),
+  // a dword outside the image has the offset 0xffffffff; raw_ok[j]: slot j lies inside.  A load whose value is used inside
+  // a branch on its predicate would make the compiler wait for it there, one memory round trip per slot.
   uint32_t raw[NSLOT];
   bool raw_ok[NSLOT];
-  // one patch dword of pixel group grp: image dword and whether it lies inside the image
-  auto load_slot = [&](const uint8_t *img, int ybase, int sbase, int code, uint32_t &word, bool &inside) {
+  struct Origin {
+    int b, oy0, ox0;
+  };
+  auto origin = [&](uint32_t blk) {
+    const uint32_t t = quot(blk, (uint32_t)gpr, magic_gpr);
+    Origin o;
+    o.ox0 = (int)(blk - t * (uint32_t)gpr) << LW;
+    o.b = (int)quot(t, (uint32_t)gpc, magic_gpc);
+    o.oy0 = (int)(t - (uint32_t)o.b * (uint32_t)gpc) * (NSETS * PY);
+    return o;
+  };
+  auto image = [&](const Origin &o) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(X + (long long)o.b * H * rowbytes), 0, H * rowbytes, 0x00020000);
+  };
+  auto load_slot = [&](__amdgpu_buffer_rsrc_t img, int ybase, int sbase, int code, uint32_t &word, bool &inside) {
     const int iy = ybase + (code >> 16);
     const int sb = sbase + (code & 0xffff);
     inside = (uint32_t)iy < (uint32_t)H && (uint32_t)sb < (uint32_t)rowbytes;
-    const int iyc = min(max(iy, 0), H - 1), sbc = min(max(sb, 0), rowbytes - 4);
-    const uint32_t off = __umul24((uint32_t)iyc, (uint32_t)rowbytes) + (uint32_t)sbc;
-    word = *reinterpret_cast<const uint32_t *>(img + off);
+    const int off = iy * rowbytes + sb;
+    word = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(img, inside ? off : -1, 0, 0);
   };
-  auto group_origin = [&](uint32_t grp, const uint8_t *&img, int &ybase, int &sbase) {
-    const uint32_t trow = quot(grp, (uint32_t)gpr, magic_gpr);
-    const int gx = (int)(grp - trow * (uint32_t)gpr);
-    const int b = (int)quot(trow, (uint32_t)Ho, magic_ho);
-    const int oy = (int)(trow - (uint32_t)b * (uint32_t)Ho);
-    sbase = ((gx * 32 * stride - pad) * C) & ~3;  // two's complement: rounds towards minus infinity
-    ybase = oy * stride - pad;
-    img = X + (long long)b * H * rowbytes;
-  };
-  auto request = [&](uint32_t grp) {
-    const uint8_t *img;
-    int ybase, sbase;
-    group_origin(grp, img, ybase, sbase);
+  auto request = [&](uint32_t blk) {
+    const Origin o = origin(blk);
+    const auto img = image(o);
+    const int sbase = ((o.ox0 * stride - pad) * C) & ~3;  // two's complement: rounds towards minus infinity
+    const int ybase = o.oy0 * stride - pad;
 #pragma unroll
     for (int j = 0; j < NSLOT; ++j) load_slot(img, ybase, sbase, rd[j], raw[j], raw_ok[j]);
   };
+  uint32_t *pdw = reinterpret_cast<uint32_t *>(patch) + lane;
   auto publish = [&]() {
 #pragma unroll
-    for (int j = 0; j < NSLOT; ++j) {
-      const uint32_t val = raw_ok[j] ? raw[j] ^ xor_mask : 0u;
-      if (rd[j] < (NO_ROW << 16)) patch[(rd[j] >> 16) * PWD + ((rd[j] & 0xffff) >> 2)] = val;
-    }
+    for (int j = 0; j < NSLOT; ++j)
+      if (j * 64 + 64 <= npatch || j * 64 + lane < npatch) pdw[j * 64] = raw_ok[j] ? raw[j] ^ xor_mask : 0u;
   };
   // patches larger than the slots: staged in place, one dword per lane and round trip
-  auto stage_in_place = [&](uint32_t grp) {
-    const uint8_t *img;
-    int ybase, sbase;
-    group_origin(grp, img, ybase, sbase);
+  auto stage_in_place = [&](uint32_t blk) {
+    const Origin o = origin(blk);
+    const auto img = image(o);
+    const int sbase = ((o.ox0 * stride - pad) * C) & ~3, ybase = o.oy0 * stride - pad;
 #pragma unroll 1
     for (int idx = lane; idx < npatch; idx += 64) {
-      const int code = slot_code(idx);
       uint32_t word;
       bool inside;
-      load_slot(img, ybase, sbase, code, word, inside);
-      patch[(code >> 16) * PWD + ((code & 0xffff) >> 2)] = inside ? word ^ xor_mask : 0u;
+      load_slot(img, ybase, sbase, slot_code(idx), word, inside);
+      reinterpret_cast<uint32_t *>(patch)[idx] = inside ? word ^ xor_mask : 0u;
     }
   };
 
-  // (the launcher keeps the number of groups below 2^31: 32-bit index arithmetic)
-  const uint32_t gstep = gridDim.x * (uint32_t)NWAV, ng = (uint32_t)ngroups;
-  uint32_t group = blockIdx.x * (uint32_t)NWAV + (uint32_t)wave;
-  if (prefetch && group < ng) request(group);
-  for (; group < ng; group += gstep) {
-    const uint32_t trow = quot(group, (uint32_t)gpr, magic_gpr);
-    const int gx = (int)(group - trow * (uint32_t)gpr);
-    const int b = (int)quot(trow, (uint32_t)Ho, magic_ho);
-    const int oy = (int)(trow - (uint32_t)b * (uint32_t)Ho);
-    const int ox0 = gx * 32;
-    const int s0 = (ox0 * stride - pad) * C;
-    const int lead = s0 - (s0 & ~3);
+  // (the launcher keeps the number of blocks below 2^31: 32-bit index arithmetic)
+  const uint32_t gstep = gridDim.x * (uint32_t)NWAV, ng = (uint32_t)B * (uint32_t)(gpr * gpc);
+  uint32_t block = blockIdx.x * (uint32_t)NWAV + (uint32_t)wave;
+  if (prefetch && block < ng) request(block);
+  for (; block < ng; block += gstep) {
     if (prefetch) {
       publish();
-      if (group + gstep < ng) request(group + gstep);
+      if (block + gstep < ng) request(block + gstep);
     } else {
-      stage_in_place(group);
+      stage_in_place(block);
     }
 
-    v16i_t acc[2];
+    v16i_t acc[NSETS][2];
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
+    for (int st = 0; st < NSETS; ++st)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[nb][r] = 0;
-    const int a0 = lead + lane_bytes;
-    auto operand = [&](int byte_off) {
-      const int a = a0 + byte_off;
-      const uint32_t *wp = patch + (a >> 2);
-      const uint32_t sh = (uint32_t)a & 3u;
-      const uint32_t w0 = wp[0], w1 = wp[1], w2 = wp[2], w3 = wp[3], w4 = wp[4];
-      v4i_t af;
-      af[0] = (int)__builtin_amdgcn_alignbyte(w1, w0, sh);
-      af[1] = (int)__builtin_amdgcn_alignbyte(w2, w1, sh);
-      af[2] = (int)__builtin_amdgcn_alignbyte(w3, w2, sh);
-      af[3] = (int)__builtin_amdgcn_alignbyte(w4, w3, sh);
-      return af;
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[st][nb][r] = 0;
+    auto k_step = [&](int ks, int off, int rs) {
+      v4i_t w[2], af[NSETS];
+#pragma unroll
+      for (int st = 0; st < NSETS; ++st) {
+        const uint32_t *wp = mine + ((off + st * set_bytes) >> 2);
+        const uint32_t w0 = wp[0], w1 = wp[1], w2 = wp[2], w3 = wp[3], w4 = wp[4];
+        af[st][0] = (int)__builtin_amdgcn_alignbyte(w1, w0, sh);
+        af[st][1] = (int)__builtin_amdgcn_alignbyte(w2, w1, sh);
+        af[st][2] = (int)__builtin_amdgcn_alignbyte(w3, w2, sh);
+        af[st][3] = (int)__builtin_amdgcn_alignbyte(w4, w3, sh);
+      }
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) {
+        if constexpr (WREG) w[nb] = wreg[nb][rs];
+        else w[nb] = *reinterpret_cast<const v4i_t *>(wl + (nb * 32 + li) * KPL + ks * 32 + g * 16);
+      }
+#pragma unroll
+      for (int st = 0; st < NSETS; ++st)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) acc[st][nb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[nb], af[st], acc[st][nb], 0, 0, 0);
     };
     if (NKS > 0) {
 #pragma unroll
-      for (int ks = 0; ks < NW; ++ks) {
-        const v4i_t af = operand(koff[ks]);
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-          v4i_t w;
-          if constexpr (WREG) w = wreg[nb][ks];
-          else w = *reinterpret_cast<const v4i_t *>(wl + (nb * 32 + li) * KPL + ks * 32 + g * 16);
-          acc[nb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w, af, acc[nb], 0, 0, 0);
-        }
-      }
+      for (int ks = 0; ks < NW; ++ks) k_step(ks, koff[ks], ks);
     } else {
       int r = 0, h = g;  // half index 2ks + g = r * HPR + h
-      while (h >= HPR) {
-        h -= HPR;
-        ++r;
-      }
-      // k-step 0 is peeled: its matrix instructions take the constant zero as their addend, which saves
-      // clearing 32 accumulator registers per pixel group (this loop's trip count is a run-time value)
-      auto k_step = [&](int ks, const v16i_t &c0, const v16i_t &c1) {
-        const v4i_t af = operand(min(r, R - 1) * PWD * 4 + h * 16);
-        const v4i_t b0 = *reinterpret_cast<const v4i_t *>(wl + li * KPL + ks * 32 + g * 16);
-        const v4i_t b1 = *reinterpret_cast<const v4i_t *>(wl + (32 + li) * KPL + ks * 32 + g * 16);
-        acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b0, af, c0, 0, 0, 0);
-        acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b1, af, c1, 0, 0, 0);
-        h += 2;
+      for (int ks = 0; ks < nks; ++ks) {
         while (h >= HPR) {
           h -= HPR;
           ++r;
         }
-      };
-      const v16i_t zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-      k_step(0, zero, zero);
-      for (int ks = 1; ks < nks; ++ks) k_step(ks, acc[0], acc[1]);
+        k_step(ks, min(r, R - 1) * rowpitch + h * 16, 0);
+        h += 2;
+      }
     }
 
     // ---- thresholds -> bit-plane words: lane half 0 ends with the pixel's word of plane 0, half 1 of plane 1 ----
     // wait states between the last matrix instruction and a vector instruction that reads its result (19 for sixteen
     // passes): the compiler adds them for instructions it can see, not for the assembly of append_int_codes
-    asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]), "+v"(acc[1]));
+#pragma unroll
+    for (int st = 0; st < NSETS; ++st) asm volatile("" : "+v"(acc[st][0]), "+v"(acc[st][1]));
+    asm volatile("s_nop 15\n\ts_nop 7");
+#pragma unroll
+    for (int st = 0; st < NSETS; ++st) asm volatile("" : "+v"(acc[st][0]), "+v"(acc[st][1]));
     __builtin_amdgcn_sched_barrier(0);  // (keeps the threshold reads from piling up in registers)
     const int *tab = table + 16 * g;
-    uint32_t word[2];
+    uint32_t word[NSETS][2];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
-      uint32_t w0 = 0, w1 = 0;
+      uint32_t w0[NSETS], w1[NSETS];
+#pragma unroll
+      for (int st = 0; st < NSETS; ++st) w0[st] = w1[st] = 0;
       static_for_n<0, 4>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         const v4i_t a = *reinterpret_cast<const v4i_t *>(tab + nb * 32 + 4 * q);
         const v4i_t b1 = *reinterpret_cast<const v4i_t *>(tab + 64 + nb * 32 + 4 * q);
         const v4i_t c2 = *reinterpret_cast<const v4i_t *>(tab + 128 + nb * 32 + 4 * q);
-        append_int_codes(acc[nb][4 * q], acc[nb][4 * q + 1], acc[nb][4 * q + 2], acc[nb][4 * q + 3], a, b1, c2, w1, w0);
+#pragma unroll
+        for (int st = 0; st < NSETS; ++st)
+          append_int_codes(acc[st][nb][4 * q], acc[st][nb][4 * q + 1], acc[st][nb][4 * q + 2], acc[st][nb][4 * q + 3], a, b1, c2,
+                           w1[st], w0[st]);
         __builtin_amdgcn_sched_barrier(0);
       });
-      const auto s = __builtin_amdgcn_permlane32_swap(w0, w1, false, false);
-      word[nb] = (s[0] << 16) | s[1];
+#pragma unroll
+      for (int st = 0; st < NSETS; ++st) {
+        const auto s = __builtin_amdgcn_permlane32_swap(w0[st], w1[st], false, false);
+        word[st][nb] = (s[0] << 16) | s[1];
+      }
     }
-    const int ox = ox0 + li, plane = g;
-    if (ox < Wo && plane < bits) {
-      uint32_t *dst = planes + plane * rows_total * cw32 + (((long long)b * Ho + oy) * Wo + ox) * cw32 + (co0 >> 5);
-      if ((cw32 & 1) == 0) {
-        *reinterpret_cast<uint2 *>(dst) = make_uint2(word[0], word[1]);
-      } else {
-        dst[0] = word[0];
-        if (co0 + 32 < COUT) dst[1] = word[1];
+    const Origin o = origin(block);
+    const int plane = g;
+#pragma unroll
+    for (int st = 0; st < NSETS; ++st) {
+      const int ox = o.ox0 + px, oy = o.oy0 + st * PY + py;
+      if (ox < Wo && oy < Ho && plane < bits) {
+        uint32_t *dst = planes + plane * rows_total * cw32 + (((long long)o.b * Ho + oy) * Wo + ox) * cw32 + (co0 >> 5);
+        if ((cw32 & 1) == 0) {
+          *reinterpret_cast<uint2 *>(dst) = make_uint2(word[st][0], word[st][1]);
+        } else {
+          dst[0] = word[st][0];
+          if (co0 + 32 < COUT) dst[1] = word[st][1];
+        }
       }
     }
   }
@@ -967,64 +978,73 @@ hipError_t launch_conv_i8_bn(const int8_t *X, const int8_t *Wt, const int32_t *t
   dim3 grid((unsigned)((groups + 3) / 4), (unsigned)((COUT + 63) / 64));
   if (C <= 4 && planes != nullptr && codes == nullptr && acc_out == nullptr && bits <= 2 && (COUT % 32) == 0 &&
       groups < 0x7fffffffLL && (long long)H * W * C < 0x7fffffffLL && (long long)W * C < (1 << 24) &&
-      (long long)H + pad < 0x7fff && ((W * C) % 4) == 0 && (reinterpret_cast<uintptr_t>(X) & 3u) == 0 && (zero_point == 0 || zero_point == 128) &&
+      (long long)H + pad < 0x7fff && (long long)COUT * R * S * C < 0x7fffffffLL && ((W * C) % 4) == 0 && (reinterpret_cast<uintptr_t>(X) & 3u) == 0 && (zero_point == 0 || zero_point == 128) &&
       thr != nullptr) {
     // image rows consumed as bytes (no repacking): see conv_i8_rows_kernel
     const int HPR = (S * C + 15) / 16;
     const int nks = (R * HPR + 1) / 2;
-    const int NDW = (3 + (31 * stride + S) * C + 3) / 4;
-    const int need = (3 + 31 * stride * C + 16 * (HPR - 1) + 20 + 3) / 4;
-    const int PWD = (need > NDW ? need : NDW) | 1;  // odd pitch
-    // slots of image dwords a lane keeps in flight: 8 where that covers the patch, else 18 together with
-    // eight waves per work-group (large filters: 11x11)
-    const bool wide_patch = R * NDW > 64 * 8;
+    int cus = 0, dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return e;
+    if (cus <= 0) cus = 256;
+    // pixel blocks 16 or 8 wide, whichever needs fewer of them, then the smaller patch
+    struct Shape {
+      int lw, pr, ndw, gpr, gpc;
+    };
+    auto shape = [&](int sets, int lw) {
+      const int px = 1 << lw, py = sets * (32 >> lw);
+      return Shape{lw, (py - 1) * stride + R, (3 + ((px - 1) * stride + S) * C + 3) / 4, (Wo + px - 1) / px, (Ho + py - 1) / py};
+    };
+    auto best = [&](int sets) {
+      const Shape w = shape(sets, 4), n = shape(sets, 3);
+      const long long bw = (long long)w.gpr * w.gpc, bn = (long long)n.gpr * n.gpc;
+      return bw < bn || (bw == bn && w.pr * w.ndw <= n.pr * n.ndw) ? w : n;
+    };
+    const bool wide_patch = nks > 8;
     const int nwav = wide_patch ? 8 : 4;
-    const size_t lds = (size_t)64 * (nks * 32 + 16) + (size_t)nwav * R * PWD * 4;
-    if (lds <= (wide_patch ? 80 * 1024 : 64 * 1024)) {
-      const size_t all = lds + kRowsTable;
+    Shape sh = best(2);
+    const bool two = !wide_patch && sh.pr * sh.ndw <= 64 * (nks == 2 ? 4 : 6) && (long long)B * sh.gpr * sh.gpc >= 2 * cus;
+    if (!two) sh = best(1);
+    const int npatch = sh.pr * sh.ndw;
+    const long long blocks = (long long)B * sh.gpr * sh.gpc;
+    const size_t all = kRowsTable + (size_t)64 * (nks * 32 + 16) + (size_t)nwav * rows_patch_bytes(npatch);
+    if (all <= (wide_patch ? 80 * 1024 : 64 * 1024) && blocks < 0x7fffffffLL) {
+      auto kern = wide_patch && nks == 17 ? conv_i8_rows_kernel<17, 1, false, 12, 8>
+                  : wide_patch ? conv_i8_rows_kernel<0, 1, false, 12, 8>
+                  : two && nks == 7 ? conv_i8_rows_kernel<7, 2, false, 6, 4>
+                  : two && nks == 2 ? conv_i8_rows_kernel<2, 2, false, 4, 4>
+                  : two             ? conv_i8_rows_kernel<0, 2, false, 6, 4>
+                  : nks == 7        ? conv_i8_rows_kernel<7, 1, true, 6, 4>
+                  : nks == 2        ? conv_i8_rows_kernel<2, 1, true, 6, 4>
+                                    : conv_i8_rows_kernel<0, 1, false, 8, 4>;
+      const int variant = wide_patch ? (nks == 17 ? 0 : 1) : two ? (nks == 7 ? 2 : nks == 2 ? 3 : 4) : nks == 7 ? 5 : nks == 2 ? 6 : 7;
       // persistent grid: exactly as many work-groups as the device holds at once
-      // Filter block in registers (two work-groups per compute unit fit) while one or two rounds of
-      // work-groups cover all pixel groups; beyond that the variant that re-reads the filter from LDS
-      // wins through its higher occupancy (four per compute unit).
-      // Unrolled loops for the k-steps of 7x7x3 and 3x3x3 filters (see the kernel); any other number runs the loop with a
-      // decode per step, the 11x11 one because its 17 offsets do not fit the 128 registers of four waves per SIMD.
-      const bool wreg = nks == 7 && grid.x <= 1024 && !wide_patch;
-      auto kern = wreg ? conv_i8_rows_kernel<7, true, 8, 4>
-                  : wide_patch ? conv_i8_rows_kernel<0, false, 18, 8>
-                  : nks == 7   ? conv_i8_rows_kernel<7, false, 8, 4>
-                  : nks == 2   ? conv_i8_rows_kernel<2, false, 8, 4>
-                               : conv_i8_rows_kernel<0, false, 8, 4>;
-      const int variant = wreg ? 0 : wide_patch ? 1 : nks == 7 ? 2 : nks == 2 ? 3 : 4;
-      if (wide_patch) grid.x = (unsigned)((groups + 7) / 8);
-      int per_cu = 0, cus = 0, dev = 0;
-      hipError_t e = hipGetDevice(&dev);
-      if (all > 64 * 1024 && e == hipSuccess) {
-        static std::atomic<unsigned long long> raised[5];
-        e = raise_lds_limit(raised[variant], reinterpret_cast<const void *>(kern), 80 * 1024 + kRowsTable);
+      int per_cu = 0;
+      if (wide_patch) {  // up to 80 KB
+        static std::atomic<unsigned long long> raised[8];
+        e = raise_lds_limit(raised[variant], reinterpret_cast<const void *>(kern), 80 * 1024);
       }
-      if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
       if (e == hipSuccess)
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kern), 64 * nwav, all);
       if (e != hipSuccess) return e;
-      unsigned resident = (unsigned)(per_cu > 0 ? per_cu : 1) * (unsigned)(cus > 0 ? cus : 256);
-      const unsigned slices = grid.y > 0 ? grid.y : 1;
+      unsigned resident = (unsigned)(per_cu > 0 ? per_cu : 1) * (unsigned)cus;
+      const unsigned slices = (unsigned)((COUT + 63) / 64);
       resident = resident / slices > 0 ? resident / slices : 1;
-      dim3 g2(grid.x > resident ? resident : grid.x, grid.y);
+      const unsigned want = (unsigned)((blocks + nwav - 1) / nwav);
+      dim3 g2(want > resident ? resident : want, slices);
       const uint32_t xm = zero_point == 128 ? 0x80808080u : 0u;
       const uint8_t *Xu = reinterpret_cast<const uint8_t *>(X);
-      // multiply-high quotients for the pixel-group decode, where they are exact (n * d < 2^32)
-      const unsigned long long gpr = (unsigned long long)(Wo + 31) / 32, ngr = (unsigned long long)B * Ho * gpr;
+      // multiply-high quotients for the block decode, where they are exact (n * d < 2^32)
       auto magic = [&](unsigned long long d) {
-        return (d >= 2 && ngr * d < (1ull << 32)) ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u;
+        return (d >= 2 && (unsigned long long)blocks * d < (1ull << 32)) ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u;
       };
-      const uint32_t mg = magic(gpr), mh = magic((unsigned long long)Ho);
-      // small dividends (patch slots below 1152, filter tasks below 2^16): always exact
+      const uint32_t mg = magic((unsigned long long)sh.gpr), mh = magic((unsigned long long)sh.gpc);
+      // small dividends (patch slots, filter tasks below 2^16): always exact
       auto small_magic = [](int d) { return d >= 2 ? (uint32_t)(((1ull << 32) + (unsigned)d - 1) / (unsigned)d) : 0u; };
-      const uint32_t mn = small_magic(NDW), mt = small_magic(nks * 2), mp = small_magic(HPR);
-      // the filter array as aligned dwords: base 4-byte aligned and a whole number of dwords long
-      const int wt_dwords = (reinterpret_cast<uintptr_t>(Wt) & 3u) == 0 && ((long long)COUT * R * S * C) % 4 == 0;
+      const uint32_t mn = small_magic(sh.ndw), mp = small_magic(HPR);
       hipLaunchKernelGGL(kern, g2, dim3(64 * nwav), all, s, Xu, Wt, thr, planes, B, H, W, C, COUT, R, S, stride, pad, Ho,
-                         Wo, bits, xm, HPR, NDW, PWD, mg, mh, mn, mt, mp, wt_dwords);
+                         Wo, bits, xm, HPR, sh.pr, sh.ndw, sh.lw, mg, mh, mn, mp);
       return hipGetLastError();
     }
   }
