@@ -14,9 +14,9 @@
 //     (wider symmetric weights: activation sums, as in mfma_kernel.h);
 //   - the last k-step of a chunk carries the barrier, and expands the first operands of the next chunk.
 // w1a2: 6.1 vector operations per matrix instruction in the loop instead of 6.75 plus staging, 212 registers.  8192^3 w1a2
-// 226 -> 220 us.  Counters there: matrix pipes 64 % busy, vector pipes 63 %, waves waiting 14 % of their lifetime, 1.89
+// 226 -> 220 us, 206 in graph replay (212 with LDS rows permuted for 32 banks).  Counters there: matrix pipes 64 % busy, vector pipes 63 %, waves waiting 14 % of their lifetime, 1.89
 // GHz.  The loop alone would leave the matrix pipes above 90 % busy; what takes the rest (a chunk's wait and barrier, the
-// output stage, 268 MB of results) has not been separated.  4096^3 w1a4 58.2 -> 45.2 us (48.0 with FP6 digits alone):
+// output stage, 268 MB of results) has not been separated.  4096^3 w1a4 58.2 -> 45.2 us (48.0 with FP6 digits alone), over 8192 bits 81.6 (83 with the other order):
 // one round of tiles, whose 67 MB of results leave the chip after the last product.
 // Convolution: a load's lane decodes the tap of its 16 bytes once per chunk; padding pixels are disabled loads, which
 // write zeros.  Two tiles of 128x256 per compute unit, three of 128x128.  3x3 convolutions at batch
@@ -25,7 +25,8 @@
 // batch 64 541 -> 489 us.
 //
 // LDS rows are KC words (64 or 32 bytes) without padding, as the loads fill them in lane order; the 16-byte units of a
-// row are permuted by its index so that any eight consecutive rows read from eight different bank groups.
+// row are permuted by its index so that any sixteen consecutive rows read from the sixteen groups of four banks (64 banks: a
+// 16-byte read takes 2.7 ns of a unit's LDS, 3.7 with eight rows in eight groups).
 #pragma once
 #include "mfma_kernel.h"
 
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
 
   // lane l of a load instruction fills the 16 bytes at 16 * l of a row group: row l / UPR, unit place l % UPR
   const int lrow = lane / UPR;
-  const int unit = (lane % UPR) ^ (UPR == 4 ? (lrow >> 1) & 3 : (lrow >> 2) & 1);
+  const int unit = (lane % UPR) ^ (UPR == 4 ? (lrow >> 2) & 3 : (lrow >> 3) & 1);
   uint32_t voA[NA], voB[NB];  // byte offset of the row's unit (convolution: word offset of the pixel's tap (0, 0), mod 2^32)
   int y0[NA], x0[NA];
 #pragma unroll
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(256, OCC) void apnn_async_kernel(const KParams pk) 
   // four k-steps of words of this lane's rows (lower lane half: the first four words of a group, upper: the last four)
   uint4 qA[FA][PA], qB[FB][PB];
   const int rowA = wa * FA * 32 + li, rowB = wb * FB * 32 + li;
-  const int swz = UPR == 4 ? (li >> 1) & 3 : (li >> 2) & 1;
+  const int swz = UPR == 4 ? (li >> 2) & 3 : (li >> 3) & 1;
   auto read_group = [&](const uint32_t *buf, auto jc) {
     constexpr int j = decltype(jc)::value;
     const int place = ((2 * j + g) ^ swz) * 4;

@@ -8,7 +8,8 @@
 //   - a wave's tile is as large as its registers allow (FA x FB blocks), because expansion work goes with its circumference;
 //   - a chunk is 32 words of every row, one cache line: eight lanes load a row's 128 bytes.  (Loaded row by row straight into
 //     registers, 32 bytes of a line at a time, the lines' way through L1 took three times as long as the expansion.)  The
-//     16-byte units of a row are permuted by its index in LDS, so that eight rows are written and read without a bank met twice;
+//     16-byte units of a row are permuted by its index in LDS, so that sixteen rows are read without one of the 64 banks met
+//     twice (by half the index; the whole index, which repeats after eight rows, was 2 to 3 % slower);
 //   - the eight units of a row go to the KS waves: two to each of four, whose lane halves take one each (four k-steps a
 //     chunk), or one to each of eight, whose lane halves take half of it (two k-steps).  Both operands alike: a permutation
 //     of the terms of each dot product.
@@ -16,8 +17,8 @@
 // group sums block k over the KS shares and finishes it like a wave of the other kernels (epi_finish).
 //
 // us in graph replay, the tiles these products took before first: w4a4 4096x333x4096 (64x64 tiles, 384 on 256 units) 25.5 ->
-// 13.6, over 8192 bits 43.9 -> 20.4; w2a2 1000x2016x2048 packed (128x64) 11.1 -> 8.5, over 8192 bits 27.5 -> 16.0; w1a4 and
-// w1a8 there 12.1 -> 8.4 and 18.6 -> 11.3.  Left: a chunk of 1024 bits takes 1.2 us (w2a2) where its vector and matrix work
+// 13.6, over 8192 bits 43.9 -> 20.4; w2a2 1000x2016x2048 packed (128x64) 11.1 -> 8.3, over 8192 bits 27.5 -> 15.6; w1a4 and
+// w1a8 there 12.1 -> 8.3 and 18.6 -> 11.3.  Left: a chunk of 1024 bits takes 1.2 us (w2a2) where its vector and matrix work
 // is 0.65; about 6 us are spent outside the loop, the meeting of the partial tiles and the first fetch the most of it.  Words
 // of the next chunk held in a second register set gained 2 % and spilled with four activation planes: taken out.
 #pragma once
@@ -95,9 +96,10 @@ __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KPar
       st[it] = make_uint4(v[0], v[1], v[2], v[3]);
     }
   };
-  // Units are permuted by the row; for eight waves, which read half units, the halves are too.
+  // Units are permuted by the row; for eight waves, which read half units, the halves are too (by the whole index: by half of
+  // it 4096x333 over 4096 and 8192 bits took 15.1 and 22.6 us instead of 14.6 and 22.1).
   const int wrow = wave * 8 + sr;
-  const uint32_t swr = (uint32_t)(wrow * 32 + (KS == 8 ? (2 * su ^ (wrow & 15)) * 2 : (su ^ sr) * 4));
+  const uint32_t swr = (uint32_t)(wrow * 32 + (KS == 8 ? (2 * su ^ (wrow & 15)) * 2 : (su ^ ((wrow >> 1) & 7)) * 4));
   auto stage = [&](uint32_t *buf) {
 #pragma unroll
     for (int it = 0; it < NI; ++it) {
@@ -128,7 +130,7 @@ __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KPar
   // this wave's words of a chunk
   constexpr int NW = KS == 8 ? 2 : 4;  // per row: k-steps of the wave
   uint32_t qA[FA][PA][NW], qB[FB][PB][NW];
-  const int place = KS == 8 ? ((2 * ks + g) ^ (li & 15)) * 2 : ((2 * ks + g) ^ (li & 7)) * 4;
+  const int place = KS == 8 ? ((2 * ks + g) ^ (li & 15)) * 2 : ((2 * ks + g) ^ ((li >> 1) & 7)) * 4;
   auto read = [&](const uint32_t *buf) {
     auto get = [&](int row, uint32_t (&q)[NW]) {
       const uint32_t *at = buf + (row + li) * 32 + place;
