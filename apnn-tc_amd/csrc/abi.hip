@@ -9,6 +9,7 @@
 #include "../../include/apnn_tc.h"
 #include "conv_epilogue.h"
 #include "dispatch.h"
+#include "wide_patch.h"
 
 // One error word per device (each device holds its own copy of a __device__ variable).
 __device__ int g_kernel_error_word;
@@ -863,6 +864,53 @@ int build_conv_params(const apnn_conv_desc *d, KParams &p, int *vw_out) {
   return APNN_OK;
 }
 
+typedef hipError_t (*wide_fn)(const KParams &, hipStream_t);
+wide_fn wide_patch_fn(int xb, int wb) {
+  if (xb == 2 && wb == 1) return apnn::wide_patch_2_1_x;
+  if (xb == 3 && wb == 1) return apnn::wide_patch_3_1_x;
+  if (xb == 4 && wb == 1) return apnn::wide_patch_4_1_x;
+  if (xb == 2 && wb == 2) return apnn::wide_patch_2_2_x;
+  return nullptr;
+}
+
+// The padded frame of wide_patch_kernel.h.  The zeros after a row are those before the next one, the zeros below an image
+// those above the next: half the padding of the frame is stored, a patch of 28x28 pixels shrinks from 260 to 222.  Needs
+// padding narrower than the filter, so that output pixels follow each other in the frame in their own order.
+bool wide_patch_frame(KParams &p, int R) {
+  const int pad = (p.PHs - p.Hs) / 2;
+  if (pad >= R || pad >= p.S) return false;
+  p.PHs = p.Hs + pad;
+  p.PWs = p.Ws + pad;
+  return true;
+}
+
+// Whether the tile of wide_patch_kernel.h holds the layer: passes of 256 channels, a patch of at most `pixels`, everything in
+// the LDS of `per_unit` work-groups a compute unit.
+bool wide_patch_fits(const KParams &q, int R, int per_unit, int pixels = apnn::kWidePatchPixels) {
+  KParams p = q;
+  if (wide_patch_fn(p.planesA, p.planesB) == nullptr || (p.C32 & 7) != 0 || !wide_patch_frame(p, R)) return false;
+  const int cap = patch_pixels(p, R, apnn::kMfmaTileA[apnn::MT_128x128_P]), tb = apnn::kMfmaTileB[apnn::MT_128x128_P];
+  return cap <= apnn::kWidePatchPixels && cap <= pixels && (apnn::wide_stage_words(p.planesA, p.planesB, tb, cap) * 4 +
+                                           apnn::conv_epilogue_bytes(p, tb)) * per_unit <= 160 * 1024;
+}
+
+// The tile AUTO takes instead of the implicit-GEMM tiles 128x128 and 128x256: the one over a patch, where it keeps all its
+// work-groups on a compute unit.  Graph replay, implicit GEMM = 1, over 24 layers of 256 to 1024 channels, 3x3 and 5x5:
+// w1a2 .85 to .97, w2a2 .77 to .96, w1a3 .78 to .98, w1a4 .69 to .95; 56x56x256 w1a2 .94 to .96 and, where they lose a
+// work-group or stage 304 pixels of 24 bytes for nine taps, w2a2 1.0, w1a3 1.03, w1a4 1.0.
+// Not for 1x1 filters (every pixel is read once: 1.03 to 1.33), nor where 128x256 tiles, two a unit, need one round and
+// these, three a unit, a second (784 and 980 tiles on 256 units: w1a2 1.09 to 1.12, w2a2 .98 to 1.02, w1a3 1.02 to 1.07, w1a4
+// .99; 1029 tiles .89, .78, .86, .84).
+int prefer_wide_patch(const KParams &p, int R, int tile) {
+  if ((tile != apnn::MT_128x128 && tile != apnn::MT_128x256) || R < 3 ||
+      !wide_patch_fits(p, R, apnn::wide_patch_units(p.planesA), p.planesA > 2 ? 32 * (p.KW / p.C32) : apnn::kWidePatchPixels))
+    return tile;
+  const long long cus = device_cus() > 0 ? device_cus() : 256;
+  const long long rows = (p.rowsA + 127) / 128, n = rows * ((p.rowsB + 127) / 128), n256 = rows * ((p.rowsB + 255) / 256);
+  if (tile == apnn::MT_128x256 && n > 3 * cus && n256 <= 2 * cus) return tile;
+  return apnn::MT_128x128_P;
+}
+
 int run_conv(const apnn_conv_desc *d, hipStream_t stream, apnn_plan *plan = nullptr) {
   KParams p{};
   int vw = 1, rc, tile;
@@ -922,6 +970,21 @@ int run_conv(const apnn_conv_desc *d, hipStream_t stream, apnn_plan *plan = null
     valu_fn fn = mfma_conv_fn(d->xb, d->wb, i8);
     if (fn != nullptr) {
       if ((rc = pick_mfma_tile(tile_pin, p, true, vw, i8, &tile))) return rc;
+      if (tile_pin == 0 && !i8) tile = prefer_wide_patch(p, d->R, tile);
+      if (!i8 && tile == apnn::MT_128x128_P) {
+        if (!wide_patch_fits(p, d->R, 1)) return APNN_EUNSUPPORTED;
+        wide_patch_frame(p, d->R);
+        p.patch_cap = patch_pixels(p, d->R, apnn::kMfmaTileA[tile]);
+        if (plan != nullptr) {
+          plan_mfma(plan, false, tile, p, f4ok);
+          plan->patch_pixels = p.patch_cap;
+          return APNN_OK;
+        }
+        p.err = kernel_error_word();
+        p.magicPW = magic_of(p.PWs);
+        p.magicPH = magic_of(p.PHs);
+        return from_hip(wide_patch_fn(d->xb, d->wb)(p, stream));
+      }
       if (plan != nullptr) {
         return apnn::mfma_tile_enabled(i8 ? apnn::CORE_I8 : apnn::CORE_F4, true, vw, tile, d->xb, d->wb)
                    ? plan_mfma(plan, i8, tile, p, f4ok)

@@ -75,6 +75,12 @@ APNN_DECL_MFMAXS(conv, 3, 1)
 APNN_DECL_MFMAXS(conv, 4, 1)
 APNN_DECL_MFMAXS(conv, 2, 2)
 #undef APNN_DECL_MFMAXS
+#define APNN_DECL_WIDE(pa, pb) hipError_t wide_patch_##pa##_##pb##_x(const KParams &p, hipStream_t s);
+APNN_DECL_WIDE(2, 1)
+APNN_DECL_WIDE(3, 1)
+APNN_DECL_WIDE(4, 1)
+APNN_DECL_WIDE(2, 2)
+#undef APNN_DECL_WIDE
 #define APNN_DECL_PATCH(pa, pb) hipError_t patch_conv_##pa##_##pb##_x(int tile, const KParams &p, hipStream_t s);
 APNN_DECL_PATCH(2, 1)
 APNN_DECL_PATCH(3, 1)
@@ -87,15 +93,16 @@ APNN_DECL_PATCH(2, 2)
 enum { CORE_I8 = 0, CORE_F4 = 1 };
 
 // tile shapes of the MFMA kernels, index = enum MfmaTile in mfma_kernel.h
-constexpr int kMfmaTileCount = 12;
-constexpr int kMfmaTileA[kMfmaTileCount] = {256, 128, 64, 128, 32, 32, 256, 128, 32, 128, 128, 64};
-constexpr int kMfmaTileB[kMfmaTileCount] = {256, 128, 64, 64, 32, 64, 128, 256, 128, 128, 64, 96};
+constexpr int kMfmaTileCount = 13;
+constexpr int kMfmaTileA[kMfmaTileCount] = {256, 128, 64, 128, 32, 32, 256, 128, 32, 128, 128, 64, 128};
+constexpr int kMfmaTileB[kMfmaTileCount] = {256, 128, 64, 64, 32, 64, 128, 256, 128, 128, 64, 96, 128};
 
 // MT_128x128_G2: the 128x128 tile computed by two groups of four waves that share its k-steps (work-groups
-// of 512 threads).  MT_128x64_K4, MT_64x96_K8: eight waves that split K by four and eight (ksplit_kernel.h)
+// of 512 threads).  MT_128x64_K4, MT_64x96_K8: eight waves that split K by four and eight (ksplit_kernel.h).
+// MT_128x128_P: a convolution over a patch of expanded activations, packed weights (wide_patch_kernel.h)
 enum MfmaTile { MT_256x256 = 0, MT_128x128 = 1, MT_64x64 = 2, MT_128x64 = 3, MT_32x32_K4 = 4, MT_32x64_K4 = 5,
                 MT_256x128 = 6, MT_128x256 = 7, MT_32x128_K4 = 8, MT_128x128_G2 = 9, MT_128x64_K4 = 10, MT_64x96_K8 = 11,
-                MT_COUNT = 12 };
+                MT_128x128_P = 12, MT_COUNT = 13 };
 
 // Which (core, family, load width, tile, plane counts) combinations are built.  Every kernel
 // instantiation costs seconds of compile time, so only the shapes the dispatcher can choose are kept:
@@ -112,8 +119,11 @@ constexpr bool ksplit_built(int core, bool conv, int tile, int pa, int pb) {
   if (core != CORE_F4 || conv || pa + pb == 2) return false;
   return tile == MT_128x64_K4 ? pa + pb < 10 : pa == 4 && pb == 4;
 }
+// planes of activations, of weights that wide_patch_kernel.h is built for
+constexpr bool wide_patch_built(int pa, int pb) { return pa >= 2 && pa <= 4 && pa + pb <= 5 && !(pa == 3 && pb == 2); }
 constexpr bool mfma_tile_enabled(int core, bool conv, int vw, int tile, int pa, int pb) {
   const bool wide = pa + pb > 5 || pa + pb == 2;
+  if (tile == MT_128x128_P) return core == CORE_F4 && conv && vw == 4 && wide_patch_built(pa, pb);
   if (tile == MT_128x64_K4 || tile == MT_64x96_K8) return ksplit_built(core, conv, tile, pa, pb);
   if (wide && core == CORE_I8) return false;
   if (wide && conv && vw != 4) return tile == MT_64x64;
