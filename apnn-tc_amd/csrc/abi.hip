@@ -900,13 +900,17 @@ bool wide_patch_fits(const KParams &q, int R, int per_unit, int pixels = apnn::k
 // work-group or stage 304 pixels of 24 bytes for nine taps, w2a2 1.0, w1a3 1.03, w1a4 1.0.
 // Not for 1x1 filters (every pixel is read once: 1.03 to 1.33), nor where 128x256 tiles, two a unit, need one round and
 // these, three a unit, a second (784 and 980 tiles on 256 units: w1a2 1.09 to 1.12, w2a2 .98 to 1.02, w1a3 1.02 to 1.07, w1a4
-// .99; 1029 tiles .89, .78, .86, .84).
+// .99; 1029 tiles .89, .78, .86, .84).  Instead of the tiles that split K beyond three of them to four units: 14x14x512 at
+// batch 32, 28x28x512 at batch 8 and 7x7 of 512 to 1024 at batch 64 (196 to 200 tiles) w1a2 .82 to .85, w1a3 .89 to .92, w1a4
+// .88 to .91, w2a2 .93 to .95; 192 tiles w1a2 .98, w1a3 1.02; 148 tiles 1.04 to 1.15, 100 tiles 1.2 to 1.4.
 int prefer_wide_patch(const KParams &p, int R, int tile) {
-  if ((tile != apnn::MT_128x128 && tile != apnn::MT_128x256) || R < 3 ||
+  const bool split = tile == apnn::MT_32x64_K4 || tile == apnn::MT_32x128_K4 || tile == apnn::MT_128x128_G2;
+  if ((tile != apnn::MT_128x128 && tile != apnn::MT_128x256 && !split) || R < 3 ||
       !wide_patch_fits(p, R, apnn::wide_patch_units(p.planesA), p.planesA > 2 ? 32 * (p.KW / p.C32) : apnn::kWidePatchPixels))
     return tile;
   const long long cus = device_cus() > 0 ? device_cus() : 256;
   const long long rows = (p.rowsA + 127) / 128, n = rows * ((p.rowsB + 127) / 128), n256 = rows * ((p.rowsB + 255) / 256);
+  if (split && (4 * n <= 3 * cus || n >= cus)) return tile;
   if (tile == apnn::MT_128x256 && n > 3 * cus && n256 <= 2 * cus) return tile;
   return apnn::MT_128x128_P;
 }

@@ -124,7 +124,8 @@ def _plan(batch, H, W, C, cout, R, S, stride, pad, wb, xb, path=A.PATH_AUTO, poo
     (64, 14, 512, 1024, 3, 1, []), (40, 28, 512, 512, 3, 1, []),    # 784, 980 tiles: a second round
     (64, 28, 512, 512, 1, 1, []), (64, 28, 512, 512, 3, 2, []),     # nothing to keep; a patch of 636 pixels and more
     (64, 56, 256, 256, 3, 1, [(1, 2)]), (64, 14, 384, 512, 3, 1, []),   # two work-groups a unit or a large patch; a pass and a half
-    (16, 16, 1024, 1024, 3, 1, []), (8, 28, 512, 512, 3, 1, []),    # split and patch-resident tiles keep theirs
+    (32, 14, 512, 512, 3, 1, COMBOS), (8, 28, 512, 512, 3, 1, COMBOS), (64, 7, 512, 1024, 3, 1, COMBOS),  # three tiles to four units
+    (31, 14, 512, 512, 3, 1, []), (16, 16, 1024, 1024, 3, 1, []), (64, 7, 512, 512, 3, 1, []),    # the split tiles keep theirs
 ])
 def test_wide_patch_rule(B, H, C, cout, R, stride, combos):
     for wb, xb in COMBOS + [(1, 8), (2, 8), (1, 1), (4, 4)]:
