@@ -407,9 +407,10 @@ int choose_patch_tile(const KParams &p, int R, int tile_pin, bool automatic) {
     // to 960 at batch 32 110 -> 130), nor w1a4 to 256 channels (28x28 at batch 64 32.4 -> 37.8).  Two weight planes,
     // whose filter block costs most, on 256x64 tiles of the general form from one per unit, 3/4 beyond 192 channels
     // (28x28x832 to 128 at batch 64 115, 177 on 128x64 tiles, 126 otherwise).
-    // (Nowhere against the 32x32 split-K tile, which wins where half of a 64-channel tile is empty: 3x3 on 56x56x192 to
+    // (Nowhere against the 32x32 split-K tile nor the 32x64 one that serves up to 640 blocks of 32x32 in its place, which win where half of a 64-channel tile is empty: 3x3 on 56x56x192 to
     // 32 at batch 6, w1a4 8.0 -> 10.1, 5x5 on 28x28x64 to 32 at batch 24 8.5 -> 9.2.)
-    if (other == apnn::MT_32x32_K4) return -1;
+    const long long blocks = (long long)((p.rowsA + 31) / 32) * ((p.rowsB + 31) / 32);
+    if (other == apnn::MT_32x32_K4 || (other == apnn::MT_32x64_K4 && p.planesA + p.planesB > 3 && blocks <= 640)) return -1;
     if (taps == 25 && p.S == 5 && p.stride == 1 && p.C32 % 4 == 2) {
       if (p.C32 == 2) return (p.rowsB <= 192 || (p.rowsB <= 256 && p.planesA < 4 && (general || n <= 8 * cus))) && 2 * n >= cus ? 3 : -1;
       if (n < cus) return -1;
@@ -599,12 +600,13 @@ int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, i
     if (vw == 4 && planes >= 5 && planesW == 1 && KW >= 128 && rowsB >= 512 && 2 * ntiles(8) >= 3 * cus &&
         ntiles(8) <= 2 * cus)
       return 8;
-    // 32x32 blocks, one work-group each: with three planes in all while every compute unit gets at most one
-    // (from 296 blocks the 32x64 tile, whose wave expands an activation block once for two channel blocks,
-    // is 5-9 % ahead with quantized output and level with int32 output); with four or more planes up to 2.5
-    // per compute unit (the second operand's expansion dominates and is not shared: 32x32 stays 2-12 %
-    // ahead up to 592 blocks, 32x64 takes over at 784).  Measured on 14x14x256 maps at batch 4..16.
-    if (KW >= 32 && nb32 <= (planes <= 3 ? 256 : 640)) return 4;
+    // 32x32 blocks, one work-group each, while every compute unit gets at most one (256 blocks: 32x64 takes 1.04 to 1.18 of
+    // it); beyond, the 32x64 tile, whose wave expands an activation block once for two channel blocks and loads it once.
+    // With four and five planes, 296 to 640 blocks of 13x13, 14x14, 16x16, 28x28 and 7x7 maps over 72 to 180 words, quantized:
+    // w1a3 .90 to .98, w1a4 .89 to .98, w2a2 .89 to 1.01 of 32x32 (13x13x384 to 256 at batch 8 6.9 -> 6.2, 8.0 -> 7.1, 6.5 -> 5.8
+    // us), int32 .85 to .98; wider precisions, shorter reductions and narrower
+    // loads keep 32x32 up to 2.5 per unit.
+    if (KW >= 32 && nb32 <= (planes <= 3 || (planes <= 5 && vw == 4 && KW >= 72) ? 256 : 640)) return 4;
     if (KW >= 32 && nb32 <= 640) return 5;
     if (KW >= 64 && nb32 <= 14 * cus) return 5;  // up to 3584 blocks: 16x16 maps at batch 16, 896 channels
   }
