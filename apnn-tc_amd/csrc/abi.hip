@@ -9,6 +9,7 @@
 #include "../../include/apnn_tc.h"
 #include "conv_epilogue.h"
 #include "dispatch.h"
+#include "quotient.h"
 #include "wide_patch.h"
 
 // One error word per device (each device holds its own copy of a __device__ variable).
@@ -866,6 +867,14 @@ int build_conv_params(const apnn_conv_desc *d, KParams &p, int *vw_out) {
   return APNN_OK;
 }
 
+// The quotients of a patch-resident kernel: a tile's pixels over the row grid, its patch's over the padded frame.
+void patch_quotients(KParams &p) {
+  p.magicGW = apnn::quotient_magic((uint32_t)(p.pool_order ? p.Wo / 2 : p.Wo));
+  p.magicGH = apnn::quotient_magic((uint32_t)(p.pool_order ? p.Ho / 2 : p.Ho));
+  p.magicPW = apnn::quotient_magic((uint32_t)p.PWs);
+  p.magicPH = apnn::quotient_magic((uint32_t)p.PHs);
+}
+
 typedef hipError_t (*wide_fn)(const KParams &, hipStream_t);
 wide_fn wide_patch_fn(int xb, int wb) {
   if (xb == 2 && wb == 1) return apnn::wide_patch_2_1_x;
@@ -987,8 +996,7 @@ int run_conv(const apnn_conv_desc *d, hipStream_t stream, apnn_plan *plan = null
           return APNN_OK;
         }
         p.err = kernel_error_word();
-        p.magicPW = magic_of(p.PWs);
-        p.magicPH = magic_of(p.PHs);
+        patch_quotients(p);
         return from_hip(wide_patch_fn(d->xb, d->wb)(p, stream));
       }
       if (plan != nullptr) {

@@ -20,6 +20,7 @@
 // 78.7 -> 72.4, w1a4 94.3 -> 84.5, w2a2 73.8 -> 62.4.
 #pragma once
 #include "async_kernel.h"
+#include "quotient.h"
 #include "wide_patch.h"
 
 namespace apnn {
@@ -81,16 +82,17 @@ __global__ __launch_bounds__(256, wide_patch_units(PA)) void apnn_wide_patch_ker
   const int gst = pooled ? 2 * p.stride : p.stride;
   const uint32_t u0 = (uint32_t)(pooled ? a0 >> 2 : a0);
   const uint32_t t0 = u0 / (uint32_t)gw;
+  const int shift_gw = quotient_shift((uint32_t)gw), shift_gh = quotient_shift((uint32_t)gh);
   const int gx0 = (int)(u0 - t0 * (uint32_t)gw);
   const int b0i = (int)(t0 / (uint32_t)gh);
   const int gy0 = (int)(t0 - (uint32_t)b0i * (uint32_t)gh);
   auto row_base = [&](int k) {
     const int u = pooled ? k >> 2 : k, sub = pooled ? k & 3 : 0;
     int gx = gx0 + u;
-    const int cy = (int)fast_div((uint32_t)gx, (uint32_t)gw, p.magicGW);
+    const int cy = (int)quotient((uint32_t)gx, (uint32_t)gw, p.magicGW, shift_gw);
     gx -= cy * gw;
     int gy = gy0 + cy;
-    const int cb = (int)fast_div((uint32_t)gy, (uint32_t)gh, p.magicGH);
+    const int cb = (int)quotient((uint32_t)gy, (uint32_t)gh, p.magicGH, shift_gh);
     gy -= cb * gh;
     return (cb * p.PHs + gy * gst + (sub >> 1) * p.stride) * p.PWs + gx * gst + (sub & 1) * p.stride;
   };
@@ -113,16 +115,17 @@ __global__ __launch_bounds__(256, wide_patch_units(PA)) void apnn_wide_patch_ker
   uint32_t poff[WIDE_NPT];
   const int pad_v = p.PHs - p.Hs;  // (the frame ends with its last stored row and pixel, see wide_patch_frame)
   const int yp0 = gy0 * gst, xp0 = gx0 * gst;
+  const int shift_pw = quotient_shift((uint32_t)p.PWs), shift_ph = quotient_shift((uint32_t)p.PHs);
 #pragma unroll
   for (int j = 0; j < WIDE_NPT; ++j) {
     const int q = (tid + j * 256) >> 1;
     poff[j] = 0xffffffffu;
     if (q < npp) {
       int xp = xp0 + q;
-      const int cy = (int)fast_div((uint32_t)xp, (uint32_t)p.PWs, p.magicPW);
+      const int cy = (int)quotient((uint32_t)xp, (uint32_t)p.PWs, p.magicPW, shift_pw);
       xp -= cy * p.PWs;
       int yp = yp0 + cy;
-      const int ci = (int)fast_div((uint32_t)yp, (uint32_t)p.PHs, p.magicPH);
+      const int ci = (int)quotient((uint32_t)yp, (uint32_t)p.PHs, p.magicPH, shift_ph);
       yp -= ci * p.PHs;
       const int img = b0i + ci;
       const int iy = yp - pad_v, ix = xp - pad_v;
