@@ -304,6 +304,17 @@ bool direct_kernel_serves(const KParams &p) {
          p.resid_planes == nullptr;
 }
 
+// The quotients of a patch-resident kernel: a tile's pixels over the row grid, its patch's over the padded frame.
+void patch_quotients(KParams &p) {
+  const uint32_t gw = p.pool_order ? p.Wo / 2 : p.Wo, gh = p.pool_order ? p.Ho / 2 : p.Ho, pw = p.PWs, ph = p.PHs;
+  const uint32_t top = apnn::kShortDivisor;
+  p.geo_fast = gw <= top && gh <= top && pw <= top && ph <= top;
+  p.magicGW = apnn::quotient_magic(gw, p.geo_fast);
+  p.magicGH = apnn::quotient_magic(gh, p.geo_fast);
+  p.magicPW = apnn::quotient_magic(pw, p.geo_fast);
+  p.magicPH = apnn::quotient_magic(ph, p.geo_fast);
+}
+
 typedef hipError_t (*patch_fn)(int, const KParams &, hipStream_t);
 patch_fn patch_conv_fn(int xb, int wb) {
   if (xb == 2 && wb == 1) return apnn::patch_conv_2_1_x;
@@ -867,14 +878,6 @@ int build_conv_params(const apnn_conv_desc *d, KParams &p, int *vw_out) {
   return APNN_OK;
 }
 
-// The quotients of a patch-resident kernel: a tile's pixels over the row grid, its patch's over the padded frame.
-void patch_quotients(KParams &p) {
-  p.magicGW = apnn::quotient_magic((uint32_t)(p.pool_order ? p.Wo / 2 : p.Wo));
-  p.magicGH = apnn::quotient_magic((uint32_t)(p.pool_order ? p.Ho / 2 : p.Ho));
-  p.magicPW = apnn::quotient_magic((uint32_t)p.PWs);
-  p.magicPH = apnn::quotient_magic((uint32_t)p.PHs);
-}
-
 typedef hipError_t (*wide_fn)(const KParams &, hipStream_t);
 wide_fn wide_patch_fn(int xb, int wb) {
   if (xb == 2 && wb == 1) return apnn::wide_patch_2_1_x;
@@ -969,11 +972,10 @@ int run_conv(const apnn_conv_desc *d, hipStream_t stream, apnn_plan *plan = null
     if (pt >= 0) {
       p.patch_cap = patch_pixels(p, d->R, apnn::kPatchTileRows[pt]);
       if (plan == nullptr) p.err = kernel_error_word();
-      p.magicPW = magic_of(p.PWs);
-      p.magicPH = magic_of(p.PHs);
       if (plan != nullptr)
         return fill_plan(plan, APNN_PATH_MFMA_PATCH, APNN_KERNEL_PATCH_FP4, pt, apnn::kPatchTileRows[pt],
                          apnn::kPatchTileCols[pt], 1, p, p.patch_cap, f4ok);
+      patch_quotients(p);
       return from_hip(pf(pt, p, stream));
     }
     if (path == APNN_PATH_MFMA_PATCH) return APNN_EUNSUPPORTED;

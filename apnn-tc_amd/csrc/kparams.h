@@ -35,11 +35,11 @@ struct KParams {
   // the capacity of the LDS patch in pixels
   int batch, PHs, PWs, patch_cap;
   // ceil(2^32/d) for the row grid (Wo, Ho; in pool order Wo/2, Ho/2), which is exact under geo_fast.  Patch-resident
-  // kernels with packed weights: quotient_magic(d) of quotient.h, also for the padded frame (PWs, PHs), exact for all maps;
-  // the others ceil(2^32/d), exact for dividends below d + 1024 while d is at most 65536
+  // kernels: quotient_magic(d) of quotient.h, also for the padded frame (PWs, PHs)
   uint32_t magicGW, magicGH, magicPW, magicPH;
   // 1: every output row index times the larger of the row grid's sides stays below 2^32, so the
-  // matrix-core kernels may decode a row index into (image, y, x) with magicGW / magicGH
+  // matrix-core kernels may decode a row index into (image, y, x) with magicGW / magicGH.  Patch-resident kernels: the
+  // four quotients are the short ones
   int geo_fast;
   // 1: the matrix-core kernels of mfma_kernel.h may run: every operand plane spans less than 2^32 bytes
   // (rows are addressed with 32-bit word offsets through buffer descriptors) and, for a convolution, the

@@ -36,6 +36,7 @@
 // the general form, 16.4 in this one (two work-groups per unit, by the LDS).
 #pragma once
 #include "mfma_kernel.h"
+#include "quotient.h"
 
 namespace apnn {
 
@@ -63,7 +64,9 @@ constexpr int patch_occupancy(int blocks, int form, int planes) {
 
 constexpr int PATCH_NPT = 4;  // patch pixels per thread (patch capacity = 4 * 256 pixels)
 
-template <int PA, int PB, int FA, int FB, int WA, int WB, int FORM>
+// SHORT: maps of at most 65536 rows and columns (quotient.h); others have PF_ANY alone.  With shifts for all 56x56x64 to 64 at
+// batch 64 took 10.7 us instead of 10.4, 56x56x96 to 256 w2a2 44.5 instead of 42.6.
+template <int PA, int PB, int FA, int FB, int WA, int WB, int FORM, bool SHORT>
 __global__ __launch_bounds__(256, patch_occupancy(FA * FB, FORM, PA)) void apnn_patch_conv_kernel(const KParams p) {
   static_assert(WA * WB == 4, "four waves tile the output");
   constexpr int DA = (PA + 1) / 2, DB = (PB + 1) / 2;
@@ -96,8 +99,7 @@ __global__ __launch_bounds__(256, patch_occupancy(FA * FB, FORM, PA)) void apnn_
   table.load(p, b0);
 
   // ---- tile geometry.  Only the tile's first row is decoded with full divisions (uniform); every
-  // other row and patch pixel is a small offset from it, for which the multiply-high quotients are
-  // exact. -----------------------------------------------------------------------------------------
+  // other row and patch pixel is a small offset from it, decoded with the quotients of quotient.h ----------------
   const int last_row = min(a0 + TA, p.rowsA) - 1;
   const int R = FORM != PF_ANY ? SIDE : taps / p.S;
   const bool pooled = p.pool_order != 0;
@@ -112,10 +114,10 @@ __global__ __launch_bounds__(256, patch_occupancy(FA * FB, FORM, PA)) void apnn_
   auto row_base = [&](int k) {
     const int u = pooled ? k >> 2 : k, sub = pooled ? k & 3 : 0;
     int gx = gx0 + u;
-    const int cy = (int)fast_div((uint32_t)gx, (uint32_t)gw, p.magicGW);
+    const int cy = (int)quotient<SHORT>((uint32_t)gx, (uint32_t)gw, p.magicGW);
     gx -= cy * gw;
     int gy = gy0 + cy;
-    const int cb = (int)fast_div((uint32_t)gy, (uint32_t)gh, p.magicGH);
+    const int cb = (int)quotient<SHORT>((uint32_t)gy, (uint32_t)gh, p.magicGH);
     gy -= cb * gh;
     return (cb * p.PHs + gy * gst + (sub >> 1) * p.stride) * p.PWs + gx * gst + (sub & 1) * p.stride;
   };
@@ -172,10 +174,10 @@ __global__ __launch_bounds__(256, patch_occupancy(FA * FB, FORM, PA)) void apnn_
     poff[j] = kOff;
     if (j * NT < npp && q < npp) {
       int xp = xp0 + q;
-      const int cy = (int)fast_div((uint32_t)xp, (uint32_t)p.PWs, p.magicPW);
+      const int cy = (int)quotient<SHORT>((uint32_t)xp, (uint32_t)p.PWs, p.magicPW);
       xp -= cy * p.PWs;
       int yp = yp0 + cy;
-      const int ci = (int)fast_div((uint32_t)yp, (uint32_t)p.PHs, p.magicPH);
+      const int ci = (int)quotient<SHORT>((uint32_t)yp, (uint32_t)p.PHs, p.magicPH);
       yp -= ci * p.PHs;
       const int img = b0i + ci;
       const int iy = yp - pad_v, ix = xp - pad_v;
@@ -377,12 +379,12 @@ __global__ __launch_bounds__(256, patch_occupancy(FA * FB, FORM, PA)) void apnn_
 enum PatchTile { PT_128x128 = 0, PT_256x64 = 1, PT_64x128 = 2, PT_128x64 = 3, PT_64x64 = 4, PT_COUNT = 5 };
 static_assert(PT_COUNT == kPatchTileCount, "tile tables of dispatch.h");
 
-template <int PA, int PB, int FA, int FB, int WA, int WB, int FORM>
+template <int PA, int PB, int FA, int FB, int WA, int WB, int FORM, bool SHORT = true>
 inline hipError_t launch_patch_form(const KParams &p, hipStream_t stream) {
   constexpr int TA = WA * FA * 32, TB = WB * FB * 32;
   const size_t smem_bytes = patch_stage_words(PA, PB, TB, p.KW / p.C32, p.patch_cap) * 4 + conv_epilogue_bytes(p, TB);
   if (smem_bytes > 160 * 1024 || p.patch_cap > PATCH_NPT * 256) return hipErrorNotSupported;
-  auto kern = apnn_patch_conv_kernel<PA, PB, FA, FB, WA, WB, FORM>;
+  auto kern = apnn_patch_conv_kernel<PA, PB, FA, FB, WA, WB, FORM, SHORT>;
   if (smem_bytes > 64 * 1024) {
     static std::atomic<unsigned long long> raised;
     const hipError_t e = raise_lds_limit(raised, reinterpret_cast<const void *>(kern), 160 * 1024);
@@ -396,6 +398,7 @@ inline hipError_t launch_patch_form(const KParams &p, hipStream_t stream) {
 // ODD, BIG: whether the forms for odd channel words and for 5x5 filters are built
 template <int PA, int PB, int FA, int FB, int WA, int WB, bool ODD = false, bool BIG = false>
 inline hipError_t launch_patch(const KParams &p, hipStream_t stream) {
+  if (!p.geo_fast) return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_ANY, false>(p, stream);
   if (p.KW == 9 * p.C32 && p.S == 3) {
     if ((p.C32 & 1) == 0) return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_3x3_PAIRS>(p, stream);
     if constexpr (ODD) return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_3x3_ODD>(p, stream);

@@ -27,7 +27,8 @@ namespace apnn {
 
 constexpr int WIDE_NPT = kWidePatchPixels * 2 / 256;  // half pixels (four words) a thread stages
 
-template <int PA, int PB, bool SYM>
+// SHORT: maps of at most 65536 rows and columns (quotient.h; with shifts 13.2 -> 13.4 us at one tile per unit)
+template <int PA, int PB, bool SYM, bool SHORT>
 __global__ __launch_bounds__(256, wide_patch_units(PA)) void apnn_wide_patch_kernel(const KParams pk) {
   KParams p = pk;
   constexpr int FA = 2, FB = 2, WA = 2, WB = 2;  // four waves of two by two 32x32 accumulators
@@ -82,17 +83,16 @@ __global__ __launch_bounds__(256, wide_patch_units(PA)) void apnn_wide_patch_ker
   const int gst = pooled ? 2 * p.stride : p.stride;
   const uint32_t u0 = (uint32_t)(pooled ? a0 >> 2 : a0);
   const uint32_t t0 = u0 / (uint32_t)gw;
-  const int shift_gw = quotient_shift((uint32_t)gw), shift_gh = quotient_shift((uint32_t)gh);
   const int gx0 = (int)(u0 - t0 * (uint32_t)gw);
   const int b0i = (int)(t0 / (uint32_t)gh);
   const int gy0 = (int)(t0 - (uint32_t)b0i * (uint32_t)gh);
   auto row_base = [&](int k) {
     const int u = pooled ? k >> 2 : k, sub = pooled ? k & 3 : 0;
     int gx = gx0 + u;
-    const int cy = (int)quotient((uint32_t)gx, (uint32_t)gw, p.magicGW, shift_gw);
+    const int cy = (int)quotient<SHORT>((uint32_t)gx, (uint32_t)gw, p.magicGW);
     gx -= cy * gw;
     int gy = gy0 + cy;
-    const int cb = (int)quotient((uint32_t)gy, (uint32_t)gh, p.magicGH, shift_gh);
+    const int cb = (int)quotient<SHORT>((uint32_t)gy, (uint32_t)gh, p.magicGH);
     gy -= cb * gh;
     return (cb * p.PHs + gy * gst + (sub >> 1) * p.stride) * p.PWs + gx * gst + (sub & 1) * p.stride;
   };
@@ -115,17 +115,16 @@ __global__ __launch_bounds__(256, wide_patch_units(PA)) void apnn_wide_patch_ker
   uint32_t poff[WIDE_NPT];
   const int pad_v = p.PHs - p.Hs;  // (the frame ends with its last stored row and pixel, see wide_patch_frame)
   const int yp0 = gy0 * gst, xp0 = gx0 * gst;
-  const int shift_pw = quotient_shift((uint32_t)p.PWs), shift_ph = quotient_shift((uint32_t)p.PHs);
 #pragma unroll
   for (int j = 0; j < WIDE_NPT; ++j) {
     const int q = (tid + j * 256) >> 1;
     poff[j] = 0xffffffffu;
     if (q < npp) {
       int xp = xp0 + q;
-      const int cy = (int)quotient((uint32_t)xp, (uint32_t)p.PWs, p.magicPW, shift_pw);
+      const int cy = (int)quotient<SHORT>((uint32_t)xp, (uint32_t)p.PWs, p.magicPW);
       xp -= cy * p.PWs;
       int yp = yp0 + cy;
-      const int ci = (int)quotient((uint32_t)yp, (uint32_t)p.PHs, p.magicPH, shift_ph);
+      const int ci = (int)quotient<SHORT>((uint32_t)yp, (uint32_t)p.PHs, p.magicPH);
       yp -= ci * p.PHs;
       const int img = b0i + ci;
       const int iy = yp - pad_v, ix = xp - pad_v;
@@ -391,10 +390,11 @@ inline hipError_t launch_wide_patch(const KParams &p, hipStream_t stream) {
   static_assert(2 * PB * TB * 8 * 4 <= 64 * 1024, "LDS addresses of the loads fit 16 bits");
   const size_t bytes = wide_stage_words(PA, PB, TB, p.patch_cap) * 4 + conv_epilogue_bytes(p, TB);
   if (bytes > 160 * 1024) return hipErrorNotSupported;
-  auto kern = p.sym ? apnn_wide_patch_kernel<PA, PB, true> : apnn_wide_patch_kernel<PA, PB, false>;
+  auto kern = p.sym ? (p.geo_fast ? apnn_wide_patch_kernel<PA, PB, true, true> : apnn_wide_patch_kernel<PA, PB, true, false>)
+                    : (p.geo_fast ? apnn_wide_patch_kernel<PA, PB, false, true> : apnn_wide_patch_kernel<PA, PB, false, false>);
   if (bytes > 64 * 1024) {
-    static std::atomic<unsigned long long> raised[2];
-    const hipError_t e = raise_lds_limit(raised[p.sym != 0], reinterpret_cast<const void *>(kern), 160 * 1024);
+    static std::atomic<unsigned long long> raised[4];
+    const hipError_t e = raise_lds_limit(raised[2 * (p.sym != 0) + (p.geo_fast != 0)], reinterpret_cast<const void *>(kern), 160 * 1024);
     if (e != hipSuccess) return e;
   }
   const long long tilesB = (p.rowsB + TB - 1) / TB, tiles = (long long)((p.rowsA + TA - 1) / TA) * tilesB;

@@ -1,4 +1,4 @@
-"""Quotients of the patch-resident convolutions: exact for every dividend up to 2^31, on maps of any height and width."""
+"""Quotients of the patch-resident convolutions: exact on maps of any height and width."""
 import ctypes
 import os
 import subprocess
@@ -16,28 +16,28 @@ CHECK = r"""
 #include "quotient.h"
 #include <cstdio>
 using namespace apnn;
-static bool bad(uint32_t d, uint32_t m, int s, uint32_t n) {
-  if (quotient(n, d, m, s) == n / d) return false;
+template <bool SHORT> static bool bad(uint32_t d, uint32_t m, uint32_t n) {
+  if (quotient<SHORT>(n, d, m) == n / d) return false;
   printf("%u / %u\n", n, d);
   return true;
 }
 // a quotient a little above n / d is wrong first for the largest n of a remainder d - 1, and at whole multiples where it is below
-static bool bad(uint32_t d) {
-  const uint32_t m = quotient_magic(d), top = 0x80000000u;
-  const int s = quotient_shift(d);
-  const uint32_t last = top / d * d;
+template <bool SHORT> static bool bad(uint32_t d) {
+  const uint32_t m = quotient_magic(d, SHORT), top = SHORT ? d + 1024 : 0x80000000u, last = top / d * d;
   for (uint32_t k = 1; k <= 1024 / d + 2 && (unsigned long long)k * d <= top; ++k)
-    if (bad(d, m, s, k * d - 1) || bad(d, m, s, k * d)) return true;
-  return bad(d, m, s, 0) || bad(d, m, s, last) || bad(d, m, s, last - 1) || bad(d, m, s, top);
+    if (bad<SHORT>(d, m, k * d - 1) || bad<SHORT>(d, m, k * d)) return true;
+  return bad<SHORT>(d, m, 0) || bad<SHORT>(d, m, last) || bad<SHORT>(d, m, last - 1) || bad<SHORT>(d, m, top);
 }
 int main() {
+  for (uint32_t d = 1; d <= kShortDivisor; ++d)
+    if (bad<true>(d)) return 1;
   for (uint32_t d = 1; d < (1u << 22); ++d)
-    if (bad(d)) return 1;
+    if (bad<false>(d)) return 1;
   for (int b = 22; b < 31; ++b)
     for (int k = -300; k <= 300; ++k)
-      if (bad((1u << b) + k)) return 1;
+      if (bad<false>((1u << b) + k)) return 1;
   for (uint32_t d = 4194319, i = 0; i < 2000000; ++i, d = (d * 1664525u + 1013904223u) & 0x7fffffffu)
-    if (d > 0 && bad(d)) return 1;
+    if (d > 0 && bad<false>(d)) return 1;
   return 0;
 }
 """
@@ -71,6 +71,15 @@ def _tall(G, path, tile, wb, xb, B, H, W, C, cout, R, S, pad):
 def test_packed_weights_patch_on_tall_and_wide_maps(B, H, W, R, S, pad, wb, xb):
     import gpu_util as G
     assert _tall(G, A.PATH_MFMA, 12, wb, xb, B, H, W, 256, 32, R, S, pad)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wb,xb", [(1, 2), (1, 4), (2, 2)])
+@pytest.mark.parametrize("tile,C", [(1, 64), (3, 96), (4, 64)])
+@pytest.mark.parametrize("B,H,W,R,S,pad", WIDE_MAPS)
+def test_expanded_patch_on_tall_and_wide_maps(B, H, W, R, S, pad, tile, C, wb, xb):
+    import gpu_util as G
+    assert _tall(G, A.PATH_MFMA_PATCH, tile, wb, xb, B, H, W, C, 32, R, S, pad)
 
 
 @pytest.mark.gpu
