@@ -12,7 +12,8 @@
 //     twice (by half the index; the whole index, which repeats after eight rows, was 2 to 3 % slower);
 //   - the eight units of a row go to the KS waves: two to each of four, whose lane halves take one each (four k-steps a
 //     chunk), or one to each of eight, whose lane halves take half of it (two k-steps).  Both operands alike: a permutation
-//     of the terms of each dot product.
+//     of the terms of each dot product.  A last chunk of up to half its words is spread over the waves word by word instead
+//     (1152 bits, us: 2048x2048 w1a8 20.2 -> 17.9, 1000x2016 w2a2 8.05 -> 7.70, w4a4 11.5 -> 10.6; beyond half the reads word by word cost 1 to 2 %).
 // The partial tiles meet in LDS in the accumulator's register layout, RB blocks of every wave at a time; wave k of a row
 // group sums block k over the KS shares and finishes it like a wave of the other kernels (epi_finish).
 //
@@ -111,7 +112,11 @@ __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KPar
       }
     }
   };
-  const int nchunks = (p.KW + 31) >> 5;
+  // A last chunk of up to half its words gives them to the waves evenly (below): a k-step of all takes 2 KS of a row's.
+  constexpr int NW = KS == 8 ? 2 : 4;  // words of a row in a wave's lane half, k-steps of a full chunk
+  const int nchunks = (p.KW + 31) >> 5, rest = p.KW & 31;
+  const bool tail = rest > 0 && rest <= KS * NW;
+  const int nfull = tail ? nchunks - 1 : nchunks;
   fetch(0);
 
   v16f acc[FA][FB];
@@ -128,7 +133,6 @@ __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KPar
     for (int pl = 0; pl < PB; ++pl) psum[y][pl] = 0;
 
   // this wave's words of a chunk
-  constexpr int NW = KS == 8 ? 2 : 4;  // per row: k-steps of the wave
   uint32_t qA[FA][PA][NW], qB[FB][PB][NW];
   const int place = KS == 8 ? ((2 * ks + g) ^ (li & 15)) * 2 : ((2 * ks + g) ^ ((li >> 1) & 7)) * 4;
   auto read = [&](const uint32_t *buf) {
@@ -229,7 +233,7 @@ __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KPar
   if (nchunks > 1) fetch(1);
   __syncthreads();
 #pragma unroll 1
-  for (int ch = 0; ch < nchunks; ++ch) {
+  for (int ch = 0; ch < nfull; ++ch) {
     read(buffer(ch));
     if constexpr (NBUF == 1) __syncthreads();  // every wave holds its words
     if (ch + 1 < nchunks) {
@@ -250,6 +254,26 @@ __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KPar
           __builtin_amdgcn_sched_barrier(0);
         }
       });
+    }
+    __syncthreads();
+  }
+  if (tail) {
+    const uint32_t *buf = buffer(nfull);
+    const int n = (rest + 2 * KS - 1) / (2 * KS);
+#pragma unroll 1
+    for (int i = 0; i < n; ++i) {
+      const int w = (2 * ks + g) * n + i;
+      const uint32_t *at = buf + li * 32 + (KS == 8 ? ((w >> 1) ^ (li & 15)) * 2 + (w & 1) : ((w >> 2) ^ ((li >> 1) & 7)) * 4 + (w & 3));
+#pragma unroll
+      for (int x = 0; x < FA; ++x)
+#pragma unroll
+        for (int pl = 0; pl < PA; ++pl) qA[x][pl][0] = at[(pl * TA + (wa * FA + x) * 32) * 32];
+#pragma unroll
+      for (int y = 0; y < FB; ++y)
+#pragma unroll
+        for (int pl = 0; pl < PB; ++pl) qB[y][pl][0] = at[(PA * TA + pl * TB + y * 32) * 32];
+      expand(std::integral_constant<int, 0>{}, af, bf);
+      mfma_all();
     }
     __syncthreads();
   }

@@ -32,6 +32,25 @@ def test_ksplit_int32(G, tile, wb, xb, M, N, K, sym):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("sym", [0, 1])
+@pytest.mark.parametrize("K", list(range(128, 1025, 128)) + list(range(1152, 3073, 128)))
+@pytest.mark.parametrize("tile,wb,xb", BUILT)
+def test_ksplit_last_chunk(G, tile, wb, xb, K, sym):
+    """Every number of words in the last chunk, which up to half of them are spread over the waves, alone and behind one and two
+    full ones; all-ones operands and ones with a single word set show a word that is counted twice or left out."""
+    M, N = 97, 70
+    rng = np.random.default_rng(9750 + K + 10 * wb + xb + tile)
+    W, X = O.random_planes(rng, wb, M, K // 32), O.random_planes(rng, xb, N, K // 32)
+    W[:, :4], X[:, :3] = 0xFFFFFFFF, 0xFFFFFFFF
+    for n in range(K // 32):
+        if 8 + n < M:
+            W[:, 8 + n] = 0
+            W[:, 8 + n, n] = 0xFFFFFFFF
+    got = G.run_gemm(W, X, M, N, K, wb, xb, sym=sym, path=A.PATH_MFMA, tile=tile).reshape(M, N)
+    assert np.array_equal(got, O.gemm(W, X, M, N, K, wb, xb, sym_w=sym))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("tile,wb,xb", BUILT)
 @pytest.mark.parametrize("bits,form", [(2, "low"), (1, "bn"), (2, "bn"), (4, "bn"), (5, "bn"), (2, "near"), (2, "far"), (2, "map")])
 def test_ksplit_packed(G, tile, wb, xb, bits, form):
@@ -71,6 +90,10 @@ def test_ksplit_packed(G, tile, wb, xb, bits, form):
     (2048, 2048, 2048, 1, 8, K4), (4096, 4096, 2048, 1, 8, None), (1000, 2016, 2048, 2, 8, None), (1000, 2016, 2048, 1, 1, None),
     (4096, 333, 4096, 4, 4, K8), (4096, 333, 1024, 4, 4, K4), (1000, 1000, 4096, 4, 4, K8), (1000, 2016, 4096, 4, 4, K4),
     (8192, 16, 2048, 1, 2, None), (16, 8192, 2048, 1, 2, None),
+    # up to half a tile per unit a begun chunk costs w1a2 and w1a3 more than it gains
+    (1024, 768, 1024, 1, 2, K4), (1024, 768, 1152, 1, 2, None), (1000, 1000, 1920, 1, 2, None), (1000, 1000, 4224, 1, 2, None),
+    (1024, 768, 2048, 1, 3, K4), (1024, 768, 1152, 1, 3, None), (1000, 1000, 3328, 1, 3, None), (1000, 1000, 3456, 1, 3, K4),
+    (1000, 1000, 1152, 1, 4, K4), (768, 1536, 1152, 1, 2, K4), (768, 1536, 1152, 1, 3, K4),
 ])
 def test_ksplit_rule(M, N, K, wb, xb, tile):
     """Where AUTO takes these tiles: one round of at least 3/8 (1/2) of the units, 1024 bits, tiles mostly filled."""
