@@ -3,6 +3,7 @@
 // of packed codes, code unpacking and the int8 classifier.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -1003,14 +1004,31 @@ hipError_t launch_conv_i8_bn(const int8_t *X, const int8_t *Wt, const int32_t *t
     };
     const bool wide_patch = nks > 8;
     const int nwav = wide_patch ? 8 : 4;
+    auto patch_of = [](const Shape &c) { return c.pr * c.ndw; };
+    auto blocks_of = [&](const Shape &c) { return (long long)B * c.gpr * c.gpc; };
+    auto lds_of = [&](const Shape &c) { return kRowsTable + (size_t)64 * (nks * 32 + 16) + (size_t)nwav * rows_patch_bytes(patch_of(c)); };
+    const size_t lds_limit = wide_patch ? 82 * 1024 : 64 * 1024;
     Shape sh = best(2);
-    const bool two = !wide_patch && sh.pr * sh.ndw <= 64 * (nks == 2 ? 4 : 6) && (long long)B * sh.gpr * sh.gpc >= 2 * cus;
+    const bool two = !wide_patch && patch_of(sh) <= 64 * (nks == 2 ? 4 : 6) && blocks_of(sh) >= 2 * cus;
     if (!two) sh = best(1);
-    const int npatch = sh.pr * sh.ndw;
-    const long long blocks = (long long)B * sh.gpr * sh.gpc;
-    const size_t all = kRowsTable + (size_t)64 * (nks * 32 + 16) + (size_t)nwav * rows_patch_bytes(npatch);
-    if (all <= (wide_patch ? 80 * 1024 : 64 * 1024) && blocks < 0x7fffffffLL) {
-      auto kern = wide_patch && nks == 17 ? conv_i8_rows_kernel<17, 1, false, 12, 8>
+    // A patch beyond the slots of the form for the number of k-steps: strides beyond the filter put rows and pixels that no
+    // output reads between those of a block.  The shape that stages least, 32 pixels of a row among them, a wave's patch counting
+    // alone while the chip holds all blocks at once, and a form of 8 or 18 slots (7x7 stride 32 on one channel, 96x96 at
+    // batch 64: 54 us in blocks of 16x2 pixels, 12 in rows; 11x11 stride 24 fits the LDS only so).
+    const int own_slots = 64 * (wide_patch ? 12 : nks == 7 || nks == 2 ? 6 : 8);
+    if (!two && patch_of(sh) > own_slots) {
+      auto cost = [&](const Shape &c) { return std::max(blocks_of(c), 16LL * cus) * patch_of(c); };
+      for (const Shape &c : {shape(1, 3), shape(1, 4), shape(1, 5)})
+        if (lds_of(c) <= lds_limit && (lds_of(sh) > lds_limit || cost(c) < cost(sh))) sh = c;
+    }
+    const bool more = !two && patch_of(sh) > own_slots;
+    const long long blocks = blocks_of(sh);
+    const size_t all = lds_of(sh);
+    if (all <= lds_limit && blocks < 0x7fffffffLL) {
+      auto kern = more && wide_patch ? conv_i8_rows_kernel<0, 1, false, 18, 8>
+                  : more && patch_of(sh) <= 8 * 64 ? conv_i8_rows_kernel<0, 1, false, 8, 4>
+                  : more ? conv_i8_rows_kernel<0, 1, false, 18, 4>
+                  : wide_patch && nks == 17 ? conv_i8_rows_kernel<17, 1, false, 12, 8>
                   : wide_patch ? conv_i8_rows_kernel<0, 1, false, 12, 8>
                   : two && nks == 7 ? conv_i8_rows_kernel<7, 2, false, 6, 4>
                   : two && nks == 2 ? conv_i8_rows_kernel<2, 2, false, 4, 4>
@@ -1018,12 +1036,11 @@ hipError_t launch_conv_i8_bn(const int8_t *X, const int8_t *Wt, const int32_t *t
                   : nks == 7        ? conv_i8_rows_kernel<7, 1, true, 6, 4>
                   : nks == 2        ? conv_i8_rows_kernel<2, 1, true, 6, 4>
                                     : conv_i8_rows_kernel<0, 1, false, 8, 4>;
-      const int variant = wide_patch ? (nks == 17 ? 0 : 1) : two ? (nks == 7 ? 2 : nks == 2 ? 3 : 4) : nks == 7 ? 5 : nks == 2 ? 6 : 7;
       // persistent grid: exactly as many work-groups as the device holds at once
       int per_cu = 0;
-      if (wide_patch) {  // up to 80 KB
-        static std::atomic<unsigned long long> raised[8];
-        e = raise_lds_limit(raised[variant], reinterpret_cast<const void *>(kern), 80 * 1024);
+      if (wide_patch) {
+        static std::atomic<unsigned long long> raised[3];
+        e = raise_lds_limit(raised[more ? 2 : nks == 17], reinterpret_cast<const void *>(kern), lds_limit);
       }
       if (e == hipSuccess)
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kern), 64 * nwav, all);

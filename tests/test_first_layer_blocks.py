@@ -1,4 +1,4 @@
-"""First layer on blocks of pixels: one and two sets of 32, blocks 8 and 16 wide, maps that end inside a block, every number of
+"""First layer on blocks of pixels: one and two sets of 32, blocks 8, 16 and 32 wide, maps that end inside a block, every number of
 k-steps with a form of its own, half a block of channels, filters whose last 16 bytes are loaded from before their place."""
 import numpy as np
 import pytest
@@ -21,6 +21,9 @@ def G():
     (2, 37, 40, 3, 64, 11, 4, 5), (30, 63, 64, 3, 32, 11, 4, 0),                                  # 17, eight waves
     (3, 20, 16, 1, 64, 7, 2, 3), (60, 40, 44, 1, 32, 7, 1, 3), (50, 31, 32, 4, 96, 5, 1, 2), (2, 40, 40, 3, 32, 9, 3, 4),  # other numbers
     (3, 40, 44, 4, 64, 11, 2, 5), (1, 8, 8, 2, 32, 1, 1, 0),
+    # strides beyond the filter: 32 pixels of a row, also where no other block fits the LDS
+    (2, 64, 64, 1, 64, 16, 16, 0), (1, 96, 96, 1, 32, 11, 24, 5), (3, 100, 100, 3, 64, 4, 32, 2), (40, 69, 72, 3, 96, 5, 16, 2),
+    (1, 9, 1100, 1, 64, 7, 32, 3), (2, 40, 700, 4, 32, 2, 8, 1), (1, 16, 1056, 3, 64, 3, 16, 1),
 ])
 @pytest.mark.parametrize("bits,zero", [(2, 128), (1, 128), (2, 0)])
 def test_first_layer_blocks(G, B, H, W, C, cout, R, stride, pad, bits, zero):
