@@ -922,7 +922,10 @@ bool wide_patch_fits(const KParams &q, int R, int per_unit, int pixels = apnn::k
 // these, three a unit, a second (784 and 980 tiles on 256 units: w1a2 1.09 to 1.12, w2a2 .98 to 1.02, w1a3 1.02 to 1.07, w1a4
 // .99; 1029 tiles .89, .78, .86, .84).  Instead of the tiles that split K beyond three of them to four units: 14x14x512 at
 // batch 32, 28x28x512 at batch 8 and 7x7 of 512 to 1024 at batch 64 (196 to 200 tiles) w1a2 .82 to .85, w1a3 .89 to .92, w1a4
-// .88 to .91, w2a2 .93 to .95; 192 tiles w1a2 .98, w1a3 1.02; 148 tiles 1.04 to 1.15, 100 tiles 1.2 to 1.4.
+// .88 to .91, w2a2 .93 to .95; 192 tiles w1a2 .98, w1a3 1.02; 148 tiles 1.04 to 1.15, 100 tiles 1.2 to 1.4.  Of the 32x64 tile
+// its own blocks count, eight to a tile: from 6 a unit on 453 layers of all results w1a2 to 1.00, w1a4 1.02, w2a2 .96, where
+// the last column of 128 channels is mostly empty (32, 64, 160 channels) 1.1 to 1.6; w1a3's general results (the output
+// stage's path over LDS) 1.05 to 1.09 over 144 words, .95 to 1.05 over 216, .80 to .85 over 288.
 int prefer_wide_patch(const KParams &p, int R, int tile) {
   const bool split = tile == apnn::MT_32x64_K4 || tile == apnn::MT_32x128_K4 || tile == apnn::MT_128x128_G2;
   if ((tile != apnn::MT_128x128 && tile != apnn::MT_128x256 && !split) || R < 3 ||
@@ -930,7 +933,12 @@ int prefer_wide_patch(const KParams &p, int R, int tile) {
     return tile;
   const long long cus = device_cus() > 0 ? device_cus() : 256;
   const long long rows = (p.rowsA + 127) / 128, n = rows * ((p.rowsB + 127) / 128), n256 = rows * ((p.rowsB + 255) / 256);
-  if (split && (4 * n <= 3 * cus || n >= cus)) return tile;
+  if (split) {
+    // counted in the blocks of the 32x64 tile: what is empty of the last column of 128 channels, that tile does not compute
+    const long long used = tile == apnn::MT_128x128_G2 ? 8 * n : (long long)((p.rowsA + 31) / 32) * ((p.rowsB + 63) / 64);
+    const bool general = p.epi != APNN_EPI_INT32 && !apnn::conv_float_codes(p, p.planesA >= 3 ? 4 : 2);
+    if (used <= 6 * cus || n >= cus || (p.planesA == 3 && general && p.KW <= 216 && tile != apnn::MT_128x128_G2)) return tile;
+  }
   if (tile == apnn::MT_128x256 && n > 3 * cus && n256 <= 2 * cus) return tile;
   return apnn::MT_128x128_P;
 }

@@ -126,6 +126,8 @@ def _plan(batch, H, W, C, cout, R, S, stride, pad, wb, xb, path=A.PATH_AUTO, poo
     (64, 56, 256, 256, 3, 1, [(1, 2)]), (64, 14, 384, 512, 3, 1, []),   # two work-groups a unit or a large patch; a pass and a half
     (32, 14, 512, 512, 3, 1, COMBOS), (8, 28, 512, 512, 3, 1, COMBOS), (64, 7, 512, 1024, 3, 1, COMBOS),  # three tiles to four units
     (31, 14, 512, 512, 3, 1, []), (16, 16, 1024, 1024, 3, 1, []), (64, 7, 512, 512, 3, 1, []),    # the split tiles keep theirs
+    (35, 28, 768, 32, 3, 1, []), (33, 28, 256, 64, 3, 1, []), (50, 16, 512, 160, 3, 1, []),       # columns mostly empty
+    (31, 28, 512, 96, 3, 1, []), (40, 28, 512, 96, 3, 1, COMBOS),                                 # three quarters full, below and above
 ])
 def test_wide_patch_rule(B, H, C, cout, R, stride, combos):
     for wb, xb in COMBOS + [(1, 8), (2, 8), (1, 1), (4, 4)]:
@@ -135,6 +137,16 @@ def test_wide_patch_rule(B, H, C, cout, R, stride, combos):
             assert 0 < plan.patch_pixels <= 384 and (plan.tile_rows, plan.tile_cols, plan.split_k) == (128, 128, 1)
             rc, pinned = _plan(B, H, H, C, cout, R, R, stride, R // 2, wb, xb, path=plan.path | ((TILE + 1) << 8))
             assert rc == 0 and (pinned.tile, pinned.patch_pixels) == (TILE, plan.patch_pixels)
+
+
+@pytest.mark.parametrize("C,xb,tile", [(512, 3, 5), (768, 3, 5), (1024, 3, TILE), (512, 2, TILE), (512, 4, TILE)])
+def test_wide_patch_rule_general_results(C, xb, tile):
+    """w1a3 maxima of three-bit codes stay on the 32x64 split-K tile over up to 216 words (33x28x28, 203 tiles)."""
+    plan, epi = A.Plan(), A.Epilogue()
+    epi.mode, epi.out_bits, epi.pool, epi.thresholds = A.EPI_BN, xb, A.POOL_MAX2X2, 0x1000
+    d = A.ConvDesc(W=0x1000, X=0x1000, O=0x1000, batch=33, H=28, Wd=28, cin_pad=C, COUT=128, R=3, S=3, stride=1, pad=1, halo=0, wb=1,
+                   xb=xb, epi=epi, path=A.PATH_AUTO)
+    assert A.lib().apnn_conv_plan(ctypes.byref(d), ctypes.byref(plan)) == 0 and plan.kernel == A.KERNEL_MFMA_FP4 and plan.tile == tile
 
 
 @pytest.mark.parametrize("B,H,W,R,S,stride,pad,pool", [
