@@ -620,11 +620,16 @@ int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, i
       return 8;
     // 32x32 blocks, one work-group each, while every compute unit gets at most one (256 blocks: 32x64 takes 1.04 to 1.18 of
     // it); beyond, the 32x64 tile, whose wave expands an activation block once for two channel blocks and loads it once.
-    // With four and five planes, 296 to 640 blocks of 13x13, 14x14, 16x16, 28x28 and 7x7 maps over 72 to 180 words, quantized:
-    // w1a3 .90 to .98, w1a4 .89 to .98, w2a2 .89 to 1.01 of 32x32 (13x13x384 to 256 at batch 8 6.9 -> 6.2, 8.0 -> 7.1, 6.5 -> 5.8
-    // us), int32 .85 to .98; wider precisions, shorter reductions and narrower
-    // loads keep 32x32 up to 2.5 per unit.
-    if (KW >= 32 && nb32 <= (planes <= 3 || (planes <= 5 && vw == 4 && KW >= 72) ? 256 : 640)) return 4;
+    // With four and five planes over more than 72 words: while that tile still gives no unit two, up to two 32x32 blocks a
+    // unit (1239 layers, all results: median w1a3 .89, w1a4 .88, w2a2 .95, five above 1.03; 13x13x384 to 256 at batch 8 6.9 -> 6.2,
+    // 8.0 -> 7.1, 6.5 -> 5.8 us), where it would 1.0 to 1.4 of 32x32; up to 2.5 while little of the last 64 channels is
+    // empty (293 layers with one weight plane .90 to .97, 1.00 at most; with one block of 32 channels 1.1 to 1.2), w2a2 none of
+    // it and up to 216 words (.99; 1.03 beyond, to 1.14).
+    // 72 words are level; wider precisions, shorter reductions and narrower loads keep 32x32 up to 2.5 per unit.
+    const long long nb64 = ntiles(5);
+    const bool shared = planes <= 5 && vw == 4 && KW > 72 &&
+                        (nb32 <= 2 * cus ? nb64 <= cus : planesW == 1 ? 20 * nb64 < 13 * nb32 : KW <= 216 && 25 * nb64 < 13 * nb32);
+    if (KW >= 32 && nb32 <= (planes <= 3 ? 256 : 640) && !(planes > 3 && nb32 > 256 && shared)) return 4;
     if (KW >= 32 && nb32 <= 640) return 5;
     if (KW >= 64 && nb32 <= 14 * cus) return 5;  // up to 3584 blocks: 16x16 maps at batch 16, 896 channels
   }
