@@ -925,7 +925,8 @@ bool wide_patch_fits(const KParams &q, int R, int per_unit, int pixels = apnn::k
 // work-group or stage 304 pixels of 24 bytes for nine taps, w2a2 1.0, w1a3 1.03, w1a4 1.0.
 // Not for 1x1 filters (every pixel is read once: 1.03 to 1.33), nor where 128x256 tiles, two a unit, need one round and
 // these, three a unit, a second (784 and 980 tiles on 256 units: w1a2 1.09 to 1.12, w2a2 .98 to 1.02, w1a3 1.02 to 1.07, w1a4
-// .99; 1029 tiles .89, .78, .86, .84).  Instead of the tiles that split K beyond three of them to four units: 14x14x512 at
+// .99; 1029 tiles .89, .78, .86, .84), nor, w1a2 and w1a3, where further rounds of filled 128x256 tiles leave less than half a
+// unit's tile idle (79 layers 1.02, to 1.11; of the other 1042 three beyond 1.03).  Instead of the tiles that split K beyond three of them to four units: 14x14x512 at
 // batch 32, 28x28x512 at batch 8 and 7x7 of 512 to 1024 at batch 64 (196 to 200 tiles) w1a2 .82 to .85, w1a3 .89 to .92, w1a4
 // .88 to .91, w2a2 .93 to .95; 192 tiles w1a2 .98, w1a3 1.02; 148 tiles 1.04 to 1.15, 100 tiles 1.2 to 1.4.  Of the 32x64 tile
 // its own blocks count, eight to a tile: from 6 a unit on 453 layers of all results w1a2 to 1.00, w1a4 1.02, w2a2 .96, where
@@ -945,6 +946,8 @@ int prefer_wide_patch(const KParams &p, int R, int tile) {
     if (used <= 6 * cus || n >= cus || (p.planesA == 3 && general && p.KW <= 216 && tile != apnn::MT_128x128_G2)) return tile;
   }
   if (tile == apnn::MT_128x256 && n > 3 * cus && n256 <= 2 * cus) return tile;
+  const bool filled = 25 * (2 * n256 - n) <= n;  // columns of 256
+  if (tile == apnn::MT_128x256 && p.planesB == 1 && p.planesA <= 3 && n256 > 2 * cus && filled && n256 % cus >= cus / 2) return tile;
   return apnn::MT_128x128_P;
 }
 

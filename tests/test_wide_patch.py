@@ -122,6 +122,8 @@ def _plan(batch, H, W, C, cout, R, S, stride, pad, wb, xb, path=A.PATH_AUTO, poo
     (64, 14, 512, 512, 3, 1, COMBOS), (64, 28, 512, 512, 3, 1, COMBOS), (12, 28, 512, 512, 3, 1, COMBOS), (64, 14, 512, 512, 5, 1, COMBOS),
     (48, 28, 512, 512, 3, 1, COMBOS),
     (64, 14, 512, 1024, 3, 1, []), (40, 28, 512, 512, 3, 1, []),    # 784, 980 tiles: a second round
+    (56, 28, 512, 512, 3, 1, [(1, 4), (2, 2)]), (30, 56, 512, 256, 3, 1, []),      # 686, 735 tiles of 128x256: most of a round
+    (56, 28, 512, 416, 3, 1, [(1, 4), (2, 2)]), (56, 28, 512, 384, 3, 1, COMBOS),           # their columns mostly and half filled
     (64, 28, 512, 512, 1, 1, []), (64, 28, 512, 512, 3, 2, []),     # nothing to keep; a patch of 636 pixels and more
     (64, 56, 256, 256, 3, 1, [(1, 2)]), (64, 14, 384, 512, 3, 1, []),   # two work-groups a unit or a large patch; a pass and a half
     (32, 14, 512, 512, 3, 1, COMBOS), (8, 28, 512, 512, 3, 1, COMBOS), (64, 7, 512, 1024, 3, 1, COMBOS),  # three tiles to four units
