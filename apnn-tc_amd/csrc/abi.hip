@@ -576,10 +576,12 @@ int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, i
   // 1000x1000 (128 tiles) over 2048 bits w1a2 / w1a4 0.94 / 0.86 of the time, w2a2 1.04; w1a8, whose other tiles repeat
   // sixteen planes' expansion, from 48 tiles (1024x384 over 2048 bits 0.89) and over several rounds (2048x2048 24.5 -> 20.0,
   // 4096x1536 0.70; 512 tiles of 128x64 at 1152 bits, where the 128x128 ones are one full round, 1.02 to 1.03); the others
-  // lose there (2304x1024, 288 tiles: w1a2 1.07, w2a2 1.16).  w2a2 is level at 1024 bits.  Up to half a tile per unit, where
-  // the 32x64 split-K tile is the other one, a chunk that is begun costs w1a2 and w1a3 more than it gains (96 to 128 tiles: w1a2
-  // 1024 / 2048 / 4096 bits 0.97 / 0.96 / 0.91, all lengths between and up to 5248 1.02 to 1.11, w1a3 1.00 to 1.07 up to
-  // 1920 and 0.95 to 1.02 up to 3328, 0.93 to 0.98 beyond; w1a4 0.71 to 0.98 at all lengths).
+  // lose there (2304x1024, 288 tiles: w1a2 1.07, w2a2 1.16).  w2a2 is level at 1024 bits.  Where
+  // the 32x64 split-K tile is the other one, up to half a tile per unit and a little beyond with tiles partly empty, w2a2 stays
+  // there (408x2272, 144 tiles, 1.19), w4a4 up to 2400 bits (898x1044 over 1152 1.16, 782x1216 over 3072 0.92), and a chunk
+  // that is begun costs w1a2 and w1a3 more than it gains (96 to 140 tiles: w1a2 1024 / 2048 / 4096 bits 0.97 / 0.96 / 0.91, all
+  // lengths between and up to 5248 1.02 to 1.14, w1a3 1.00 to 1.08 up to 1920 and 0.95 to 1.02 up to 3328, 0.93 to 0.98
+  // beyond; w1a4 0.71 to 0.98).
   // w4a4 takes 64x96 tiles where they fill three quarters of a round (half from 4096 bits): 4096x333 over 4096 bits, 256
   // tiles, 25.5 on 64x64, 18.8 on 128x64, 13.6.
   if (!conv && !i8 && KW >= 32 && planes > 2 && planes < 10) {
@@ -587,10 +589,13 @@ int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, i
     const long long n10 = ntiles(apnn::MT_128x64_K4), n11 = ntiles(apnn::MT_64x96_K8);
     if (w4 && KW >= 64 && n11 <= cus && (KW >= 128 ? 2 : 1) * n11 * 4 >= 3 * cus && fill(apnn::MT_64x96_K8) >= 0.75)
       return apnn::MT_64x96_K8;
-    const long long least = w1a8 ? 3 * cus / 16 : w4 || planesW > 1 ? cus / 2 + 1 : 3 * cus / 8;
-    // whole chunks of 32 words, or longer than a chunk's cost shows
-    const bool length = (KW & 31) == 0 || planes > 4 || 2 * n10 > cus || (planes == 4 && KW >= 108);
-    if (n10 >= least && n10 <= (w1a8 ? 3 : 1) * cus && (planesW != 2 || KW > 32) && length && fill(apnn::MT_128x64_K4) >= 0.75)
+    const bool few = ntiles(apnn::MT_32x64_K4) <= 2 * cus;  // that tile is the other one (below)
+    // there: whole chunks of 32 words, or more words than a chunk's cost shows in
+    const bool half = 2 * n10 > cus;
+    const bool length = planesW == 1 ? (KW & 31) == 0 || planes > 4 || (planes == 4 ? KW >= 108 : half && KW >= 92)
+                                     : w4 && half && KW >= 76;
+    if (16 * n10 >= (w1a8 ? 3 : 6) * cus && n10 <= (w1a8 ? 3 : 1) * cus && (planesW != 2 || KW > 32) &&
+        (!few || length) && fill(apnn::MT_128x64_K4) >= 0.75)
       return apnn::MT_128x64_K4;
   }
   if ((!conv || vw == 4) && planes > 2 && KW >= 64 && fill(1) >= 0.8) {
