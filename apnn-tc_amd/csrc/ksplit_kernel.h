@@ -156,7 +156,7 @@ __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KPar
       for (int pl = 0; pl < PB; ++pl) get(PA * TA + pl * TB + y * 32, qB[y][pl]);
   };
   v8i af[FA][DA], bf[FB][DB];
-  auto expand_a = [&](auto ic, v8i (&a)[FA][DA]) {
+  auto expand = [&](auto ic, v8i (&a)[FA][DA], v8i (&b)[FB][DB]) {
     constexpr int i = decltype(ic)::value;
 #pragma unroll
     for (int x = 0; x < FA; ++x) {
@@ -169,43 +169,36 @@ __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KPar
         static_for<0, DA>([&](auto dc) { a[x][decltype(dc)::value] = expand_digit<DIG, PA, decltype(dc)::value>(w); });
       }
     }
-  };
-  auto expand_b = [&](auto ic, int y, v8i (&b)[DB]) {
-    constexpr int i = decltype(ic)::value;
-    uint32_t w[PB];
 #pragma unroll
-    for (int pl = 0; pl < PB; ++pl) {
-      w[pl] = qB[y][pl][i];
-      if constexpr (SUM) psum[y][pl] += __popc(w[pl]);
+    for (int y = 0; y < FB; ++y) {
+      uint32_t w[PB];
+#pragma unroll
+      for (int pl = 0; pl < PB; ++pl) {
+        w[pl] = qB[y][pl][i];
+        if constexpr (SUM) psum[y][pl] += __popc(w[pl]);
+      }
+      static_for<0, DB>([&](auto dc) { b[y][decltype(dc)::value] = expand_digit<DIG, PB, decltype(dc)::value>(w); });
     }
-    static_for<0, DB>([&](auto dc) { b[decltype(dc)::value] = expand_digit<DIG, PB, decltype(dc)::value>(w); });
-  };
-  auto expand = [&](auto ic, v8i (&a)[FA][DA], v8i (&b)[FB][DB]) {
-    expand_a(ic, a);
-#pragma unroll
-    for (int y = 0; y < FB; ++y) expand_b(ic, y, b[y]);
-  };
-  auto mfma_column = [&](int y, const v8i (&b)[DB]) {
-#pragma unroll
-    for (int x = 0; x < FA; ++x)
-      static_for<0, DA>([&](auto dac) {
-        static_for<0, DB>([&](auto dbc) {
-          constexpr int da = decltype(dac)::value, db = decltype(dbc)::value;
-          acc[x][y] = mfma_digits<DIG, da + db>(af[x][da], b[db], acc[x][y]);
-        });
-      });
   };
   auto mfma_all = [&]() {
 #pragma unroll
-    for (int y = 0; y < FB; ++y) mfma_column(y, bf[y]);
+    for (int y = 0; y < FB; ++y)
+#pragma unroll
+      for (int x = 0; x < FA; ++x)
+        static_for<0, DA>([&](auto dac) {
+          static_for<0, DB>([&](auto dbc) {
+            constexpr int da = decltype(dac)::value, db = decltype(dbc)::value;
+            acc[x][y] = mfma_digits<DIG, da + db>(af[x][da], bf[y][db], acc[x][y]);
+          });
+        });
   };
   constexpr int N_MFMA = FA * FB * DA * DB;
   constexpr int XDIG[5] = {0, 7, 10, 18, 22};
   constexpr int XA = XDIG[DIG] * (PA / DIG) + XDIG[PA % DIG], XB = XDIG[DIG] * (PB / DIG) + XDIG[PB % DIG];
   constexpr int N_VALU = FA * XA + FB * XB + (SUM ? FB * PB : 0);
   constexpr int VALU_PER_MFMA = (N_VALU + N_MFMA - 1) / N_MFMA;
-  // (w2a8 has no registers for the operands of two k-steps)
-  constexpr bool PIPE = NBLK * 16 + NW * (FA * PA + FB * PB) + 4 * NI + 2 * (FA * DA + FB * DB) * (DIG == 4 ? 6 : 4) <= 280;
+  // words, staged words and the operands of two k-steps beside the accumulators (w2a8, 264, spills)
+  static_assert(NBLK * 16 + NW * (FA * PA + FB * PB) + 4 * NI + 2 * (FA * DA + FB * DB) * (DIG == 4 ? 6 : 4) <= 256, "registers");
   // Matrix products of one k-step and, between them, the expansion of the next.  Two waves that expand and multiply in
   // turns get in each other's way: while one waits for the matrix pipe the other issues a vector operation every eight
   // clocks only (1000x2016x2048 w2a2 packed 8.8 -> 8.5 us, w1a8 11.9 -> 11.3, w4a4 4096x333x4096 14.1 -> 13.6).
@@ -240,21 +233,9 @@ __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KPar
       stage(buffer(ch + 1));
       if (ch + 2 < nchunks) fetch(ch + 2);
     }
-    if constexpr (PIPE) {
-      expand(std::integral_constant<int, 0>{}, af, bf);
-      static_for<1, NW>([&](auto ic) { step(ic); });
-      mfma_all();
-    } else {
-      static_for<0, NW>([&](auto ic) {
-        expand_a(ic, af);
-#pragma unroll
-        for (int y = 0; y < FB; ++y) {
-          expand_b(ic, y, bf[0]);
-          mfma_column(y, bf[0]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      });
-    }
+    expand(std::integral_constant<int, 0>{}, af, bf);
+    static_for<1, NW>([&](auto ic) { step(ic); });
+    mfma_all();
     __syncthreads();
   }
   if (tail) {
