@@ -42,8 +42,9 @@ def _quantized(G, rng, acc2d, channels, mode, ob, keep):
     return dict(mode=G.A.EPI_LOWBITS, out_bits=ob), lambda a: a & ((1 << ob) - 1)
 
 
-@pytest.mark.parametrize("block", range(8))
+@pytest.mark.parametrize("block", range(10))
 def test_conv_random_shapes(G, block):
+    """Blocks 8 and 9: the 128x128 tile over a patch with packed weights, which takes 256 n channels and patches of 384 pixels."""
     ran = 0
     for i in range(60):
         rng = np.random.default_rng(710000 + 1000 * block + i)
@@ -63,6 +64,11 @@ def test_conv_random_shapes(G, block):
         pool = int(rng.choice([0, 0, 1, 2])) if mode else 0
         ob = int(rng.integers(1, 5)) if mode else 0
         path, tile = CONV_CHOICES[rng.integers(0, len(CONV_CHOICES))]
+        if block >= 8:
+            path, tile, cin_pad = 2, 12, 256 * (1 + i % 3)
+            R, S, stride = min(R, 5), min(S, 5), 1 if i % 4 else stride
+            pad = min(pad, R - 1, S - 1)
+            halo = halo if pad else 0
         if H + 2 * pad < R or Wd + 2 * pad < S:
             continue
         Ho, Wo = (H + 2 * pad - R) // stride + 1, (Wd + 2 * pad - S) // stride + 1
@@ -99,8 +105,9 @@ def test_conv_random_shapes(G, block):
     assert ran >= 25
 
 
-@pytest.mark.parametrize("block", range(6))
+@pytest.mark.parametrize("block", range(8))
 def test_gemm_random_shapes(G, block):
+    """Blocks 6 and 7: the tiles whose eight waves split K."""
     ran = 0
     for i in range(80):
         rng = np.random.default_rng(810000 + 1000 * block + i)
@@ -113,6 +120,10 @@ def test_gemm_random_shapes(G, block):
         if mode:
             N = (N + 31) // 32 * 32
         path, tile = GEMM_CHOICES[rng.integers(0, len(GEMM_CHOICES))]
+        if block >= 6:
+            path, tile = 2, 10 + i % 2
+            if tile == 11:
+                wb, xb = 4, 4
         case = dict(block=block, i=i, wb=wb, xb=xb, M=M, N=N, K=K, mode=mode, sym=sym, ob=ob, path=path, tile=tile)
         W = O.random_planes(rng, wb, M, K // 32)
         X = O.random_planes(rng, xb, N, K // 32)

@@ -32,6 +32,20 @@ def test_ksplit_int32(G, tile, wb, xb, M, N, K, sym):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tile,wb,xb", BUILT)
+@pytest.mark.parametrize("columns", [2, 24])
+def test_ksplit_bands(G, tile, wb, xb, columns):
+    """At least 256 tiles, a multiple of eight, in two columns and more: the order of the bands of an XCD, with a last band that is
+    not full (132 rows of tiles; 11)."""
+    ta, tb = (128, 64) if tile == K4 else (64, 96)
+    M, N, K = (132 if columns == 2 else 11) * ta - 5, columns * tb - 7, 128
+    rng = np.random.default_rng(9770 + 10 * wb + xb + tile)
+    W, X = O.random_planes(rng, wb, M, K // 32), O.random_planes(rng, xb, N, K // 32)
+    got = G.run_gemm(W, X, M, N, K, wb, xb, sym=1, path=A.PATH_MFMA, tile=tile).reshape(M, N)
+    assert np.array_equal(got, O.gemm(W, X, M, N, K, wb, xb, sym_w=1))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("sym", [0, 1])
 @pytest.mark.parametrize("K", list(range(128, 1025, 128)) + list(range(1152, 3073, 128)))
 @pytest.mark.parametrize("tile,wb,xb", BUILT)

@@ -19,8 +19,8 @@ def G():
     return gpu_util
 
 
-# images smaller than a tile and several tiles long, one to three passes, an odd number of taps (half a chunk of weights is
-# left over at the end), rectangular frames and filters, no padding, a stored halo, channels that end inside a tile
+# images smaller than a tile and several tiles long, one to three passes, one tap to 25, rectangular frames and filters, no
+# padding, a stored halo, channels that end inside a tile
 GEOMS = [(1, 5, 5, 256, 32, 3, 3, 1, 0), (2, 9, 9, 512, 160, 3, 3, 1, 0), (3, 14, 14, 768, 128, 3, 3, 1, 0), (2, 8, 8, 256, 96, 5, 5, 2, 0),
          (2, 7, 11, 512, 256, 3, 2, 1, 0), (40, 3, 3, 256, 32, 3, 3, 1, 0), (1, 20, 30, 256, 288, 3, 3, 0, 0), (2, 16, 12, 512, 96, 3, 3, 1, 1),
          (1, 16, 9, 768, 64, 1, 1, 0, 0), (1, 6, 25, 256, 32, 2, 2, 0, 0)]
@@ -51,6 +51,35 @@ def test_wide_patch_geometry(G, wb, xb, B, H, Wd, C, cout, R, S, pad, halo, sym,
     epi = G.epilogue(mode=A.EPI_BN, out_bits=xb, thr=keep[0], **extra)
     got = G.run_conv(Wt, X, cin_pad=C, sym=sym, epi=epi, path=2, tile=TILE, **kw).view(np.uint32).reshape(xb, rows, cout // 32)
     assert np.array_equal(got, O.lowbits_pack(O.bn_quantize(value, None, thr, None, xb), rows, cout, xb))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wb,xb", COMBOS)
+@pytest.mark.parametrize("B,H,Wd,R,S,stride", [(90, 3, 1, 3, 1, 2), (40, 12, 1, 4, 1, 2), (90, 2, 3, 1, 1, 2), (60, 9, 1, 3, 1, 3), (9, 39, 3, 1, 1, 2)])
+def test_wide_patch_strides(G, wb, xb, B, H, Wd, R, S, stride):
+    """A tile's patch is sized for 128 pixels anywhere: only maps a few pixels wide fit one of stride 2 or 3."""
+    rng = np.random.default_rng(9920 + H + 10 * wb + xb)
+    C, cout = 512, 96
+    X, Wt = O.random_planes(rng, xb, B * H * Wd, C // 32), O.random_planes(rng, wb, cout * R * S, C // 32)
+    kw = dict(batch=B, H=H, W=Wd, cout=cout, R=R, S=S, stride=stride, pad=0, halo=0, wb=wb, xb=xb)
+    acc = O.conv(Wt, X, cwords=C // 32, sym_w=1, nthreads=8, **kw).reshape(-1)
+    assert np.array_equal(G.run_conv(Wt, X, cin_pad=C, sym=1, path=2, tile=TILE, **kw), acc)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wb,xb", COMBOS)
+@pytest.mark.parametrize("B,H,cout", [(20, 30, 160), (6, 28, 1000)])
+def test_wide_patch_bands(G, wb, xb, B, H, cout):
+    """At least 256 tiles, a multiple of eight, in two columns and more: the order of the bands of an XCD, with a last band
+    that is not full (132 rows of tiles; 35)."""
+    rows = B * (H - 1) ** 2
+    assert (-(-rows // 128) * -(-cout // 128)) % 8 == 0 and -(-rows // 128) * -(-cout // 128) >= 256
+    rng = np.random.default_rng(9940 + H + 10 * wb + xb)
+    C, R = 256, 2
+    X, Wt = O.random_planes(rng, xb, B * H * H, C // 32), O.random_planes(rng, wb, cout * R * R, C // 32)
+    kw = dict(batch=B, H=H, W=H, cout=cout, R=R, S=R, stride=1, pad=0, halo=0, wb=wb, xb=xb)
+    acc = O.conv(Wt, X, cwords=C // 32, sym_w=1, nthreads=8, **kw).reshape(-1)
+    assert np.array_equal(G.run_conv(Wt, X, cin_pad=C, sym=1, path=2, tile=TILE, **kw), acc)
 
 
 @pytest.mark.gpu
