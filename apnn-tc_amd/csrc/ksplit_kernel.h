@@ -36,7 +36,14 @@ constexpr size_t ksplit_part_words(int FA, int FB, int WA, int KS) {
 constexpr int ksplit_rows(int PA, int PB, int FA, int FB, int WA) { return PA * WA * FA * 32 + PB * FB * 32; }
 constexpr int ksplit_buffers(int rows) { return 2 * rows * 128 <= 160 * 1024 ? 2 : 1; }
 
-template <int PA, int PB, int FA, int FB, int WA, int KS, bool SYM>
+// k-steps of a wave in a full chunk, words of a row in its lane half
+constexpr int ksplit_steps(int KS) { return KS == 8 ? 2 : 4; }
+// whether the last chunk holds at most half its words
+constexpr bool ksplit_tail(int KW, int KS) { return (KW & 31) > 0 && (KW & 31) <= KS * ksplit_steps(KS); }
+
+// TAIL: ksplit_tail; a kernel of its own, as its code behind the loop took products of whole chunks 0.07 us on their way to the
+// output stage (0.14 in front of it)
+template <int PA, int PB, int FA, int FB, int WA, int KS, bool SYM, bool TAIL>
 __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KParams pk) {
   KParams p = pk;
   static_assert(WA * KS == 8, "eight waves");
@@ -112,11 +119,8 @@ __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KPar
       }
     }
   };
-  // A last chunk of up to half its words gives them to the waves evenly (below): a k-step of all takes 2 KS of a row's.
-  constexpr int NW = KS == 8 ? 2 : 4;  // words of a row in a wave's lane half, k-steps of a full chunk
-  const int nchunks = (p.KW + 31) >> 5, rest = p.KW & 31;
-  const bool tail = rest > 0 && rest <= KS * NW;
-  const int nfull = tail ? nchunks - 1 : nchunks;
+  constexpr int NW = ksplit_steps(KS);
+  const int nchunks = (p.KW + 31) >> 5, nfull = TAIL ? nchunks - 1 : nchunks;
   fetch(0);
 
   v16f acc[FA][FB];
@@ -238,9 +242,9 @@ __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KPar
     mfma_all();
     __syncthreads();
   }
-  if (tail) {
+  if constexpr (TAIL) {  // the words evenly: a k-step of all waves takes 2 KS of a row's
     const uint32_t *buf = buffer(nfull);
-    const int n = (rest + 2 * KS - 1) / (2 * KS);
+    const int n = ((p.KW & 31) + 2 * KS - 1) / (2 * KS);
 #pragma unroll 1
     for (int i = 0; i < n; ++i) {
       const int w = (2 * ks + g) * n + i;
@@ -332,9 +336,11 @@ inline hipError_t launch_ksplit(const KParams &p, hipStream_t stream) {
   constexpr size_t chunk = (size_t)ksplit_buffers(rows) * rows * 128;
   constexpr size_t need = part > chunk ? part : chunk, bytes = need > slab ? need : slab;
   static_assert(bytes <= 160 * 1024, "LDS of a compute unit");
-  auto kern = p.sym ? apnn_ksplit_kernel<PA, PB, FA, FB, WA, KS, true> : apnn_ksplit_kernel<PA, PB, FA, FB, WA, KS, false>;
-  static std::atomic<unsigned long long> raised[2];
-  const hipError_t e = raise_lds_limit(raised[p.sym != 0], reinterpret_cast<const void *>(kern), bytes);
+  const bool tail = ksplit_tail(p.KW, KS);
+  auto kern = p.sym ? (!tail ? apnn_ksplit_kernel<PA, PB, FA, FB, WA, KS, true, false> : apnn_ksplit_kernel<PA, PB, FA, FB, WA, KS, true, true>)
+                    : (!tail ? apnn_ksplit_kernel<PA, PB, FA, FB, WA, KS, false, false> : apnn_ksplit_kernel<PA, PB, FA, FB, WA, KS, false, true>);
+  static std::atomic<unsigned long long> raised[4];
+  const hipError_t e = raise_lds_limit(raised[2 * (p.sym != 0) + tail], reinterpret_cast<const void *>(kern), bytes);
   if (e != hipSuccess) return e;
   const long long tilesB = (p.rowsB + TB - 1) / TB, tiles = (long long)((p.rowsA + TA - 1) / TA) * tilesB;
   KParams q = p;
