@@ -1025,17 +1025,17 @@ hipError_t launch_conv_i8_bn(const int8_t *X, const int8_t *Wt, const int32_t *t
     const long long blocks = blocks_of(sh);
     const size_t all = lds_of(sh);
     if (all <= lds_limit && blocks < 0x7fffffffLL) {
-      auto kern = more && wide_patch ? conv_i8_rows_kernel<0, 1, false, 18, 8>
-                  : more && patch_of(sh) <= 8 * 64 ? conv_i8_rows_kernel<0, 1, false, 8, 4>
-                  : more ? conv_i8_rows_kernel<0, 1, false, 18, 4>
-                  : wide_patch && nks == 17 ? conv_i8_rows_kernel<17, 1, false, 12, 8>
-                  : wide_patch ? conv_i8_rows_kernel<0, 1, false, 12, 8>
-                  : two && nks == 7 ? conv_i8_rows_kernel<7, 2, false, 6, 4>
-                  : two && nks == 2 ? conv_i8_rows_kernel<2, 2, false, 4, 4>
-                  : two             ? conv_i8_rows_kernel<0, 2, false, 6, 4>
-                  : nks == 7        ? conv_i8_rows_kernel<7, 1, true, 6, 4>
-                  : nks == 2        ? conv_i8_rows_kernel<2, 1, true, 6, 4>
-                                    : conv_i8_rows_kernel<0, 1, false, 8, 4>;
+      auto kern = !more ? (wide_patch && nks == 17 ? conv_i8_rows_kernel<17, 1, false, 12, 8>
+                           : wide_patch ? conv_i8_rows_kernel<0, 1, false, 12, 8>
+                           : two && nks == 7 ? conv_i8_rows_kernel<7, 2, false, 6, 4>
+                           : two && nks == 2 ? conv_i8_rows_kernel<2, 2, false, 4, 4>
+                           : two             ? conv_i8_rows_kernel<0, 2, false, 6, 4>
+                           : nks == 7        ? conv_i8_rows_kernel<7, 1, true, 6, 4>
+                           : nks == 2        ? conv_i8_rows_kernel<2, 1, true, 6, 4>
+                                             : conv_i8_rows_kernel<0, 1, false, 8, 4>)
+                  : wide_patch                ? conv_i8_rows_kernel<0, 1, false, 18, 8>
+                  : patch_of(sh) <= 8 * 64    ? conv_i8_rows_kernel<0, 1, false, 8, 4>
+                                              : conv_i8_rows_kernel<0, 1, false, 18, 4>;
       // persistent grid: exactly as many work-groups as the device holds at once
       int per_cu = 0;
       if (wide_patch) {

@@ -398,7 +398,6 @@ inline hipError_t launch_patch_form(const KParams &p, hipStream_t stream) {
 // ODD, BIG: whether the forms for odd channel words and for 5x5 filters are built
 template <int PA, int PB, int FA, int FB, int WA, int WB, bool ODD = false, bool BIG = false>
 inline hipError_t launch_patch(const KParams &p, hipStream_t stream) {
-  if (!p.geo_fast) return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_ANY, false>(p, stream);
   if (p.KW == 9 * p.C32 && p.S == 3) {
     if ((p.C32 & 1) == 0) return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_3x3_PAIRS>(p, stream);
     if constexpr (ODD) return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_3x3_ODD>(p, stream);
@@ -409,16 +408,32 @@ inline hipError_t launch_patch(const KParams &p, hipStream_t stream) {
   return launch_patch_form<PA, PB, FA, FB, WA, WB, PF_ANY>(p, stream);
 }
 
+// Maps beyond the short quotients
 template <int PA, int PB>
-inline hipError_t launch_patch_tile(int tile, const KParams &p, hipStream_t stream) {
+inline hipError_t launch_patch_long(int tile, const KParams &p, hipStream_t stream) {
   switch (tile) {
-    case PT_128x128: return launch_patch<PA, PB, 2, 2, 2, 2>(p, stream);
-    case PT_256x64: return launch_patch<PA, PB, 2, 2, 4, 1, true>(p, stream);
-    case PT_64x128: return launch_patch<PA, PB, 1, 2, 2, 2>(p, stream);
-    case PT_128x64: return launch_patch<PA, PB, 1, 2, 4, 1, true, true>(p, stream);
-    case PT_64x64: return launch_patch<PA, PB, 1, 1, 2, 2>(p, stream);
+    case PT_128x128: return launch_patch_form<PA, PB, 2, 2, 2, 2, PF_ANY, false>(p, stream);
+    case PT_256x64: return launch_patch_form<PA, PB, 2, 2, 4, 1, PF_ANY, false>(p, stream);
+    case PT_64x128: return launch_patch_form<PA, PB, 1, 2, 2, 2, PF_ANY, false>(p, stream);
+    case PT_128x64: return launch_patch_form<PA, PB, 1, 2, 4, 1, PF_ANY, false>(p, stream);
+    case PT_64x64: return launch_patch_form<PA, PB, 1, 1, 2, 2, PF_ANY, false>(p, stream);
     default: return hipErrorNotSupported;
   }
+}
+
+template <int PA, int PB>
+inline hipError_t launch_patch_tile(int tile, const KParams &p, hipStream_t stream) {
+  if (p.geo_fast) {
+    switch (tile) {
+      case PT_128x128: return launch_patch<PA, PB, 2, 2, 2, 2>(p, stream);
+      case PT_256x64: return launch_patch<PA, PB, 2, 2, 4, 1, true>(p, stream);
+      case PT_64x128: return launch_patch<PA, PB, 1, 2, 2, 2>(p, stream);
+      case PT_128x64: return launch_patch<PA, PB, 1, 2, 4, 1, true, true>(p, stream);
+      case PT_64x64: return launch_patch<PA, PB, 1, 1, 2, 2>(p, stream);
+      default: return hipErrorNotSupported;
+    }
+  }
+  return launch_patch_long<PA, PB>(tile, p, stream);
 }
 
 }  // namespace apnn
