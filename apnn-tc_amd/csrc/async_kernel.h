@@ -14,10 +14,12 @@
 //     (wider symmetric weights: activation sums, as in mfma_kernel.h);
 //   - the last k-step of a chunk carries the barrier, and expands the first operands of the next chunk.
 // w1a2: 6.1 vector operations per matrix instruction in the loop instead of 6.75 plus staging, 212 registers.  8192^3 w1a2
-// 226 -> 220 us, 206 in graph replay (212 with LDS rows permuted for 32 banks).  Counters there: matrix pipes 64 % busy, vector pipes 63 %, waves waiting 14 % of their lifetime, 1.89
-// GHz.  The loop alone would leave the matrix pipes above 90 % busy; what takes the rest (a chunk's wait and barrier, the
-// output stage, 268 MB of results) has not been separated.  4096^3 w1a4 58.2 -> 45.2 us (48.0 with FP6 digits alone), over 8192 bits 81.6 (83 with the other order):
-// one round of tiles, whose 67 MB of results leave the chip after the last product.
+// 226 -> 220 us, 206 to 210 in graph replay (212 with LDS rows permuted for 32 banks).  Of its busy clocks there: matrix pipes 69 %,
+// vector pipes 68 %, waves waiting 13 % of their lifetime, 1.89 GHz.  Over 1024 to 16384 bits the time is a line of 22.1 us per
+// 1024 bits, 21.6 ns a matrix instruction and SIMD (17.8 in a loop of such instructions with six vector operations and nothing
+// else, 13.3 by the clock), and 37 us beside it, in which the 268 MB of results leave.  4096^3 w1a4 58.2 -> 45.2 us (48.0 with FP6
+// digits alone), over 8192 bits 81.6 (83 with the other order): 8.4 us per 1024 bits, 33 ns a matrix instruction, vector pipes
+// 57 % busy, and 15 us beside it for 67 MB of results.  What holds the loops up beyond the expansion is not known.
 // Convolution: a load's lane decodes the tap of its 16 bytes once per chunk; padding pixels are disabled loads, which
 // write zeros.  Two tiles of 128x256 per compute unit, three of 128x128.  3x3 convolutions at batch
 // 64: 56x56x256 76 -> 66 us, 28x28x512 78 -> 64, 14x14x512 28 -> 23 (bounded by vector work, 9.8 operations per matrix

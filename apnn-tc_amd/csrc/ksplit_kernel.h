@@ -19,8 +19,9 @@
 //
 // us in graph replay, the tiles these products took before first: w4a4 4096x333x4096 (64x64 tiles, 384 on 256 units) 25.5 ->
 // 13.6, over 8192 bits 43.9 -> 20.4; w2a2 1000x2016x2048 packed (128x64) 11.1 -> 8.3, over 8192 bits 27.5 -> 15.6; w1a4 and
-// w1a8 there 12.1 -> 8.3 and 18.6 -> 11.3.  Left: a chunk of 1024 bits takes 1.2 us (w2a2) where its vector and matrix work
-// is 0.65; about 6 us are spent outside the loop, the meeting of the partial tiles and the first fetch the most of it.  Words
+// w1a8 there 12.1 -> 8.3 and 18.6 -> 11.3.  Left (profiles/ksplit_wide_patch_counters.md): a chunk of 1024 bits takes 1.1
+// us (w2a2, the slope over 3072 to 8192 bits; w4a4 on 64x96 tiles 1.7), vector pipes a third and matrix pipes a tenth of the
+// launch busy, waves waiting half of their time; 5 to 7 us lie beside the loop, launch included, not taken apart further.  Words
 // of the next chunk held in a second register set gained 2 % and spilled with four activation planes: taken out.
 #pragma once
 #include "mfma_kernel.h"
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(64 * WA * KS, 1) void apnn_ksplit_kernel(const KPar
     }
   };
   // Units are permuted by the row; for eight waves, which read half units, the halves are too (by the whole index: by half of
-  // it 4096x333 over 4096 and 8192 bits took 15.1 and 22.6 us instead of 14.6 and 22.1).
+  // it 4096x333 over 4096 and 8192 bits took 2 to 3 % longer).
   const int wrow = wave * 8 + sr;
   const uint32_t swr = (uint32_t)(wrow * 32 + (KS == 8 ? (2 * su ^ (wrow & 15)) * 2 : (su ^ ((wrow >> 1) & 7)) * 4));
   auto stage = [&](uint32_t *buf) {

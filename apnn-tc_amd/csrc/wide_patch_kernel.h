@@ -17,7 +17,8 @@
 // 128x128 tiles only: of 128x256 tiles one or two fit a compute unit (the patch is the same, the weights twice as long), and
 // they were 4 to 20 % slower everywhere but near 784 tiles.  Graph replay at batch 64, implicit GEMM first: 14x14x512 to 512
 // w1a2 20.5 -> 18.9 us, w1a3 27.7 -> 23.3, w1a4 34.5 -> 26.8, w2a2 23.4 -> 21.7; 28x28x512 to 512 w1a2 57.3 -> 54.2, w1a3
-// 78.7 -> 72.4, w1a4 94.3 -> 84.5, w2a2 73.8 -> 62.4.
+// 78.7 -> 72.4, w1a4 94.3 -> 84.5, w2a2 73.8 -> 62.4.  Of the busy clocks of 28x28x512 w1a2: matrix pipes 51 %, vector pipes
+// 61 %, LDS 44 %, of which 45 % bank conflicts whose source is not known (profiles/ksplit_wide_patch_counters.md).
 #pragma once
 #include "async_kernel.h"
 #include "quotient.h"
