@@ -580,7 +580,7 @@ int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, i
   // the 32x64 split-K tile is the other one, up to half a tile per unit and a little beyond with tiles partly empty, w2a2 stays
   // there (408x2272, 144 tiles, 1.19), w4a4 up to 2400 bits (898x1044 over 1152 1.16, 782x1216 over 3072 0.92), and a chunk
   // that is begun costs w1a2 and w1a3 more than it gains (96 to 140 tiles: w1a2 1024 / 2048 / 4096 bits 0.97 / 0.96 / 0.91, all
-  // lengths between and up to 5248 1.02 to 1.14, w1a3 1.00 to 1.08 up to 1920 and 0.95 to 1.02 up to 3328, 0.93 to 0.98
+  // lengths between and up to 5248 1.02 to 1.14, w1a3 1.00 to 1.08 up to 2304, 0.92 to 1.03
   // beyond; w1a4 0.71 to 0.98).
   // w4a4 takes 64x96 tiles where they fill three quarters of a round (half from 4096 bits): 4096x333 over 4096 bits, 256
   // tiles, 25.5 on 64x64, 18.8 on 128x64, 13.6.
@@ -592,7 +592,7 @@ int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, i
     const bool few = ntiles(apnn::MT_32x64_K4) <= 2 * cus;  // that tile is the other one (below)
     // there: whole chunks of 32 words, or more words than a chunk's cost shows in
     const bool half = 2 * n10 > cus;
-    const bool length = planesW == 1 ? (KW & 31) == 0 || planes > 4 || (planes == 4 ? KW >= 108 : half && KW >= 92)
+    const bool length = planesW == 1 ? (KW & 31) == 0 || planes > 4 || (planes == 4 ? KW >= 76 : half && KW >= 92)
                                      : w4 && half && KW >= 76;
     if (16 * n10 >= (w1a8 ? 3 : 6) * cus && n10 <= (w1a8 ? 3 : 1) * cus && (planesW != 2 || KW > 32) &&
         (!few || length) && fill(apnn::MT_128x64_K4) >= 0.75)
@@ -625,15 +625,16 @@ int choose_mfma_tile(int rowsA, int rowsB, int KW, bool conv, int vw, bool i8, i
       return 8;
     // 32x32 blocks, one work-group each, while every compute unit gets at most one (256 blocks: 32x64 takes 1.04 to 1.18 of
     // it); beyond, the 32x64 tile, whose wave expands an activation block once for two channel blocks and loads it once.
-    // With four and five planes over more than 72 words: while that tile still gives no unit two, up to two 32x32 blocks a
-    // unit (1239 layers, all results: median w1a3 .89, w1a4 .88, w2a2 .95, five above 1.03; 13x13x384 to 256 at batch 8 6.9 -> 6.2,
-    // 8.0 -> 7.1, 6.5 -> 5.8 us), where it would 1.0 to 1.4 of 32x32; up to 2.5 while little of the last 64 channels is
-    // empty (293 layers with one weight plane .90 to .97, 1.00 at most; with one block of 32 channels 1.1 to 1.2), w2a2 none of
-    // it and up to 216 words (.99; 1.03 beyond, to 1.14).
-    // 72 words are level; wider precisions, shorter reductions and narrower loads keep 32x32 up to 2.5 per unit.
+    // With four and five planes: over more than 72 words while that tile still gives no unit two, up to two 32x32 blocks a
+    // unit (1252 layers, all results: median w1a3 .89, w1a4 .89, w2a2 .95, five above 1.03; 13x13x384 to 256 at batch 8 6.9 -> 6.2,
+    // 8.0 -> 7.1, 6.5 -> 5.8 us; over 72 words level), where it would 1.0 to 1.4 of 32x32; up to 2.5 from 72 words on with
+    // one weight plane unless its columns are half empty (.82 to 1.00; half empty 1.1 to 1.2), w2a2 where they are full and up
+    // to 216 words (.99; 1.03 beyond, to 1.14).  Wider precisions, shorter reductions and narrower loads keep 32x32 up to 2.5 per unit.
     const long long nb64 = ntiles(5);
-    const bool shared = planes <= 5 && vw == 4 && KW > 72 &&
-                        (nb32 <= 2 * cus ? nb64 <= cus : planesW == 1 ? 20 * nb64 < 13 * nb32 : KW <= 216 && 25 * nb64 < 13 * nb32);
+    const bool shared = planes <= 5 && vw == 4 &&
+                        (nb32 <= 2 * cus ? KW > 72 && nb64 <= cus
+                         : planesW == 1  ? KW >= 72 && 10 * nb64 < 7 * nb32
+                                         : KW > 72 && KW <= 216 && 25 * nb64 < 13 * nb32);
     if (KW >= 32 && nb32 <= (planes <= 3 ? 256 : 640) && !(planes > 3 && nb32 > 256 && shared)) return 4;
     if (KW >= 32 && nb32 <= 640) return 5;
     if (KW >= 64 && nb32 <= 14 * cus) return 5;  // up to 3584 blocks: 16x16 maps at batch 16, 896 channels
@@ -930,12 +931,14 @@ bool wide_patch_fits(const KParams &q, int R, int per_unit, int pixels = apnn::k
 // work-group or stage 304 pixels of 24 bytes for nine taps, w2a2 1.0, w1a3 1.03, w1a4 1.0.
 // Not for 1x1 filters (every pixel is read once: 1.03 to 1.33), nor where 128x256 tiles, two a unit, need one round and
 // these, three a unit, a second (784 and 980 tiles on 256 units: w1a2 1.09 to 1.12, w2a2 .98 to 1.02, w1a3 1.02 to 1.07, w1a4
-// .99; 1029 tiles .89, .78, .86, .84), nor, w1a2 and w1a3, where further rounds of filled 128x256 tiles leave less than half a
-// unit's tile idle (79 layers 1.02, to 1.11; of the other 1042 three beyond 1.03).  Instead of the tiles that split K beyond three of them to four units: 14x14x512 at
+// .99; 1029 tiles .89, .78, .86, .84), nor, w1a2 and w1a3, where the last of further rounds of filled 128x256 tiles, counted one a
+// unit, is more than half full (66 layers 1.03 in the median, to 1.11; w1a3's general results .90 to .98; of the other 1051 layers three beyond 1.03).  Instead of the tiles that split K beyond three of them to four units: 14x14x512 at
 // batch 32, 28x28x512 at batch 8 and 7x7 of 512 to 1024 at batch 64 (196 to 200 tiles) w1a2 .82 to .85, w1a3 .89 to .92, w1a4
 // .88 to .91, w2a2 .93 to .95; 192 tiles w1a2 .98, w1a3 1.02; 148 tiles 1.04 to 1.15, 100 tiles 1.2 to 1.4.  Of the 32x64 tile
-// its own blocks count, eight to a tile: from 6 a unit on 453 layers of all results w1a2 to 1.00, w1a4 1.02, w2a2 .96, where
-// the last column of 128 channels is mostly empty (32, 64, 160 channels) 1.1 to 1.6; w1a3's general results (the output
+// its own blocks count, eight to a full tile: where the last column of 128 channels is mostly empty (32, 64, 160 channels)
+// the wide tile takes 1.1 to 1.6.  From 4.5 a unit over multiples of 1024 channels, where the split tile's rows lie 4 KB apart (w1a2
+// .61 to .98, w1a3 .58 to .95, w1a4 .56 to .93, w2a2 .58 to .83), 5.25 over 400 words and more (.65 to 1.00), below that 5
+// with two weight planes (.7 to 1.05), 5.5 w1a2 (.76 to 1.05), 6 w1a3 and w1a4 (.75 to 1.02); w1a3's general results (the output
 // stage's path over LDS) 1.05 to 1.09 over 144 words, .95 to 1.05 over 216, .80 to .85 over 288.
 int prefer_wide_patch(const KParams &p, int R, int tile) {
   const bool split = tile == apnn::MT_32x64_K4 || tile == apnn::MT_32x128_K4 || tile == apnn::MT_128x128_G2;
@@ -944,15 +947,21 @@ int prefer_wide_patch(const KParams &p, int R, int tile) {
     return tile;
   const long long cus = device_cus() > 0 ? device_cus() : 256;
   const long long rows = (p.rowsA + 127) / 128, n = rows * ((p.rowsB + 127) / 128), n256 = rows * ((p.rowsB + 255) / 256);
+  const bool general = p.epi != APNN_EPI_INT32 && !apnn::conv_float_codes(p, p.planesA >= 3 ? 4 : 2);
   if (split) {
-    // counted in the blocks of the 32x64 tile: what is empty of the last column of 128 channels, that tile does not compute
-    const long long used = tile == apnn::MT_128x128_G2 ? 8 * n : (long long)((p.rowsA + 31) / 32) * ((p.rowsB + 63) / 64);
-    const bool general = p.epi != APNN_EPI_INT32 && !apnn::conv_float_codes(p, p.planesA >= 3 ? 4 : 2);
-    if (used <= 6 * cus || n >= cus || (p.planesA == 3 && general && p.KW <= 216 && tile != apnn::MT_128x128_G2)) return tile;
+    if (4 * n <= 3 * cus || n >= cus) return tile;
+    if (tile != apnn::MT_128x128_G2) {
+      // counted in the blocks of the 32x64 tile, which does not compute what is empty of the last column of 128 channels
+      const long long blocks = (long long)((p.rowsA + 31) / 32) * ((p.rowsB + 63) / 64);
+      const int least = p.C32 % 32 == 0 ? 18 : p.KW >= 400 ? 21 : p.planesB > 1 ? 20 : p.planesA == 2 ? 22 : 24;  // quarters of a unit
+      if (4 * blocks <= (long long)least * cus || (p.planesA == 3 && general && p.KW <= 216)) return tile;
+    }
   }
   if (tile == apnn::MT_128x256 && n > 3 * cus && n256 <= 2 * cus) return tile;
   const bool filled = 25 * (2 * n256 - n) <= n;  // columns of 256
-  if (tile == apnn::MT_128x256 && p.planesB == 1 && p.planesA <= 3 && n256 > 2 * cus && filled && n256 % cus >= cus / 2) return tile;
+  if (tile == apnn::MT_128x256 && p.planesB == 1 && p.planesA <= 3 && n256 > 2 * cus && filled &&
+      2 * (n256 % cus) > cus && !(p.planesA == 3 && general))
+    return tile;
   return apnn::MT_128x128_P;
 }
 

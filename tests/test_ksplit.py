@@ -106,7 +106,7 @@ def test_ksplit_packed(G, tile, wb, xb, bits, form):
     (8192, 16, 2048, 1, 2, None), (16, 8192, 2048, 1, 2, None),
     # up to half a tile per unit a begun chunk costs w1a2 and w1a3 more than it gains
     (1024, 768, 1024, 1, 2, K4), (1024, 768, 1152, 1, 2, None), (1000, 1000, 1920, 1, 2, None), (1000, 1000, 4224, 1, 2, None),
-    (1024, 768, 2048, 1, 3, K4), (1024, 768, 1152, 1, 3, None), (1000, 1000, 3328, 1, 3, None), (1000, 1000, 3456, 1, 3, K4),
+    (1024, 768, 2048, 1, 3, K4), (1024, 768, 1152, 1, 3, None), (1000, 1000, 2304, 1, 3, None), (1000, 1000, 2432, 1, 3, K4),
     (1000, 1000, 1152, 1, 4, K4), (768, 1536, 1152, 1, 2, K4), (768, 1536, 1152, 1, 3, K4),
     # a little more than half a tile per unit, partly empty: the 32x64 tile has 512 blocks at most
     (408, 2272, 2304, 2, 2, None), (898, 1044, 1152, 4, 4, None), (348, 2720, 1152, 1, 2, None), (348, 2720, 2048, 1, 2, K4),

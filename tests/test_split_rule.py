@@ -25,7 +25,8 @@ def test_split_tiles_beyond_one_block_a_unit(B, H, C, cout, blocks):
 @pytest.mark.parametrize("B,H,C,cout,wb,xb,cols", [
     (50, 14, 512, 32, 1, 4, 32), (22, 14, 512, 96, 1, 3, 32),                               # a second 32x64 tile for a unit
     (15, 14, 512, 96, 1, 3, 64), (15, 14, 512, 96, 2, 2, 64), (7, 14, 512, 224, 1, 4, 64),  # none, a quarter or an eighth empty
-    (7, 14, 512, 416, 1, 3, 64), (30, 14, 512, 96, 1, 4, 32),                               # up to 2.5 blocks: little empty, a third
+    (7, 14, 512, 416, 1, 3, 64), (30, 14, 512, 96, 1, 4, 64), (90, 14, 512, 32, 1, 4, 32),  # up to 2.5 blocks: little, a quarter, half empty
+    (12, 14, 256, 256, 1, 4, 64), (12, 14, 256, 256, 2, 2, 32),                             # 72 words there
     (29, 13, 768, 128, 2, 2, 64), (29, 13, 1024, 128, 2, 2, 32), (6, 14, 512, 544, 2, 2, 32),
     (8, 14, 256, 256, 1, 3, 32),                                                            # 72 words
 ])

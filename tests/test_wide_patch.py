@@ -159,6 +159,7 @@ def _plan(batch, H, W, C, cout, R, S, stride, pad, wb, xb, path=A.PATH_AUTO, poo
     (31, 14, 512, 512, 3, 1, []), (16, 16, 1024, 1024, 3, 1, []), (64, 7, 512, 512, 3, 1, []),    # the split tiles keep theirs
     (35, 28, 768, 32, 3, 1, []), (33, 28, 256, 64, 3, 1, []), (50, 16, 512, 160, 3, 1, []),       # columns mostly empty
     (31, 28, 512, 96, 3, 1, []), (40, 28, 512, 96, 3, 1, COMBOS),                                 # three quarters full, below and above
+    (18, 28, 1024, 160, 3, 1, COMBOS), (18, 28, 768, 160, 3, 1, [(2, 2)]), (12, 28, 768, 288, 5, 1, COMBOS[:3]),  # 1323 and 1470 blocks of 32x64: by the reduction
 ])
 def test_wide_patch_rule(B, H, C, cout, R, stride, combos):
     for wb, xb in COMBOS + [(1, 8), (2, 8), (1, 1), (4, 4)]:
