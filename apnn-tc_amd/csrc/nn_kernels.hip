@@ -1011,17 +1011,25 @@ hipError_t launch_conv_i8_bn(const int8_t *X, const int8_t *Wt, const int32_t *t
     Shape sh = best(2);
     const bool two = !wide_patch && patch_of(sh) <= 64 * (nks == 2 ? 4 : 6) && blocks_of(sh) >= 2 * cus;
     if (!two) sh = best(1);
-    // A patch beyond the slots of the form for the number of k-steps: strides beyond the filter put rows and pixels that no
-    // output reads between those of a block.  The shape that stages least, 32 pixels of a row among them, a wave's patch counting
-    // alone while the chip holds all blocks at once, and a form of 8 or 18 slots (7x7 stride 32 on one channel, 96x96 at
-    // batch 64: 54 us in blocks of 16x2 pixels, 12 in rows; 11x11 stride 24 fits the LDS only so).
+    // A patch beyond the slots of the form for the number of k-steps is staged in place, and strides beyond the filter put rows
+    // and pixels that no output reads between those of a block.  The shape that stages least, 32 pixels of a row among them, and a
+    // form of 8 or 18 slots, where that is less by more than the form for the number of k-steps saves (a wave's patch, times the
+    // rounds of sixteen waves a unit; 7x7 stride 32 on one channel, 96x96 at batch 64: 54 us in blocks of 16x2 pixels, 12 in
+    // rows; 4x4 stride 4 on four channels at batch 64, 516 dwords of 520: 15.3 so, 11.6 in place), or where only it fits the LDS.
     const int own_slots = 64 * (wide_patch ? 12 : nks == 7 || nks == 2 ? 6 : 8);
+    bool more = false;
     if (!two && patch_of(sh) > own_slots) {
       auto cost = [&](const Shape &c) { return std::max(blocks_of(c), 16LL * cus) * patch_of(c); };
+      auto staged = [&](const Shape &c) { return (blocks_of(c) + 16 * cus - 1) / (16 * cus) * patch_of(c); };
+      Shape least = sh;
       for (const Shape &c : {shape(1, 3), shape(1, 4), shape(1, 5)})
-        if (lds_of(c) <= lds_limit && (lds_of(sh) > lds_limit || cost(c) < cost(sh))) sh = c;
+        if (lds_of(c) <= lds_limit && (lds_of(least) > lds_limit || cost(c) < cost(least))) least = c;
+      const int percent = nks == 2 ? 70 : nks == 7 ? 90 : nks == 17 ? 85 : 95;
+      if (lds_of(sh) > lds_limit || 100 * staged(least) <= percent * staged(sh)) {
+        sh = least;
+        more = patch_of(sh) > own_slots;
+      }
     }
-    const bool more = !two && patch_of(sh) > own_slots;
     const long long blocks = blocks_of(sh);
     const size_t all = lds_of(sh);
     if (all <= lds_limit && blocks < 0x7fffffffLL) {

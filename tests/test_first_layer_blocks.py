@@ -23,6 +23,7 @@ def G():
     (3, 40, 44, 4, 64, 11, 2, 5), (1, 8, 8, 2, 32, 1, 1, 0),
     # strides beyond the filter: 32 pixels of a row, also where no other block fits the LDS
     (2, 64, 64, 1, 64, 16, 16, 0), (1, 96, 96, 1, 32, 11, 24, 5), (3, 100, 100, 3, 64, 4, 32, 2), (40, 69, 72, 3, 96, 5, 16, 2),
+    (2, 64, 64, 4, 64, 4, 4, 0), (1, 70, 72, 3, 32, 7, 7, 0), (40, 64, 64, 1, 32, 14, 7, 0), (3, 80, 84, 4, 64, 11, 5, 2),  # in place
     (1, 9, 1100, 1, 64, 7, 32, 3), (2, 40, 700, 4, 32, 2, 8, 1), (1, 16, 1056, 3, 64, 3, 16, 1),
 ])
 @pytest.mark.parametrize("bits,zero", [(2, 128), (1, 128), (2, 0)])
